@@ -217,70 +217,30 @@ DEVI void chunk_offsets(const u64 *m, const ChunkScan &c, Out out)
 
 // ---- numeric forms ---------------------------------------------------------------------
 //
-// A slot is 8 bytes in both forms, so the LDS layout and the bins are the same.
-// PrecF64 (plain): FP64 values, slot = one double, ds_add_f64 per product.
-// PrecF32C (compensated FP32): FP32 values; the product is split exactly into
-// p = fl(a*b) and e = fma(a, b, -p) (TwoProduct); the slot holds a float pair (s, c),
-// updated by one 64-bit compare-and-swap: s becomes the VALU's round-to-nearest-even
-// fl(s + p), and the exact rounding error of that addition (TwoSum, Knuth) plus e goes
-// into c.  The result is fl(s + c): c carries every rounding error of the products and
-// of the additions into s, so the sum is accurate to about one FP32 rounding of the
-// result plus O(n u^2) of sum |a*b| (u = 2^-24).  (Memory-side float atomic adds return
-// old values that are not a serial history of the stored sums when lanes collide, so
-// they cannot feed TwoSum.)
+// A slot is one double in both forms, so the LDS layout, the bins and the adds
+// (ds_add_f64) are the same.
+// PrecF64 (plain): FP64 values.
+// PrecF32C (compensated FP32): FP32 values.  The product of two FP32 values is exact in
+// FP64 (24 + 24 bits), so a double slot takes the place of a (sum, compensation) pair of
+// floats: it carries 53 bits where the pair carries 48, and one ds_add_f64 takes the place
+// of a read, TwoProduct, TwoSum and a 64-bit compare-and-swap loop.  The sum is rounded to
+// FP32 once, at the end.  One CU retires a wave's ds_add_f64 on random slots in 24 cycles;
+// the compare-and-swap form measured 1.9 times the numeric time of this one on a banded
+// matrix.
 struct PrecF64 {
     typedef double V;
-    typedef double T; // a product ready to be added
-    static DEVI T prep(double a, V b) { return a * b; }
-    static DEVI void put(double *vals, unsigned slot, T p) { atomicAdd(&vals[slot], p); }
+    static DEVI double prep(double a, V b) { return a * b; }
+    static DEVI void put(double *vals, unsigned slot, double p) { atomicAdd(&vals[slot], p); }
     static DEVI void add(double *vals, unsigned slot, double a, V b) { put(vals, slot, prep(a, b)); }
     static DEVI V result(const double *vals, unsigned slot) { return vals[slot]; }
 };
 
 struct PrecF32C {
     typedef float V;
-    // (s, c) += p with one 64-bit compare-and-swap on the pair: the VALU forms
-    // t = fl(s + p) (round to nearest even), recovers that addition's exact error
-    // (TwoSum, Knuth) and adds it and e into c; the swap succeeds only if no other lane
-    // changed the pair meanwhile, so the error always describes the addition stored.
-    // c's own rounding is second order (|c| ~ u |s|).
-    struct T { // the product split exactly: p + e = a * b
-        float p, e;
-    };
-    static DEVI T prep(double a, V b)
-    {
-        const float af = (float)a;
-        const float p = __fmul_rn(af, b);
-        return T{p, __builtin_fmaf(af, b, -p)};
-    }
+    static DEVI double prep(double a, V b) { return a * (double)b; }
+    static DEVI void put(double *vals, unsigned slot, double p) { atomicAdd(&vals[slot], p); }
     static DEVI void add(double *vals, unsigned slot, double a, V b) { put(vals, slot, prep(a, b)); }
-    static DEVI void put(double *vals, unsigned slot, T pe)
-    {
-        // no contraction: t must be fl(s + p), not fma(a, b, s), for the error to be exact
-#pragma clang fp contract(off)
-        const float p = pe.p, e = pe.e;
-        unsigned long long *w = (unsigned long long *)vals + slot;
-        unsigned long long old = *w;
-        while (true) {
-            const float sv = __uint_as_float((unsigned)old);
-            const float cv = __uint_as_float((unsigned)(old >> 32));
-            const float t = sv + p;
-            const float bb = t - sv;
-            const float err = (sv - (t - bb)) + (p - bb);
-            const float c2 = cv + (err + e);
-            const unsigned long long nw =
-                (unsigned long long)__float_as_uint(t) | ((unsigned long long)__float_as_uint(c2) << 32);
-            const unsigned long long prev = atomicCAS(w, old, nw);
-            if (prev == old)
-                break;
-            old = prev;
-        }
-    }
-    static DEVI V result(const double *vals, unsigned slot)
-    {
-        const float *f = (const float *)vals + 2 * slot;
-        return f[0] + f[1];
-    }
+    static DEVI V result(const double *vals, unsigned slot) { return (float)vals[slot]; }
 };
 
 // Slot of column c in the row's accumulator, by directory form.
@@ -320,34 +280,25 @@ DEVI void add_walk(const Operands &op, int kb, int ke, int gw, int gl, double a,
                 return foff[kk] + (unsigned)__popcll(fm[kk] & below(col & 63));
             }
         };
-        if constexpr (std::is_same<P, PrecF64>::value) {
-            // every slot and product of the step first, then the adds: a product computed
-            // between two adds reuses the registers the add before it still reads, so each
-            // add waited for the previous one to leave the LDS queue (measured on banded:
-            // 2.5% off the step, 3% off the dominant kernel)
-            unsigned slot[UNROLL];
-            double pv[UNROLL];
+        // every slot and product of the step first, then the adds: a product computed
+        // between two adds reuses the registers the add before it still reads, so each add
+        // waited for the previous one to leave the LDS queue (measured on banded: 2.5% off
+        // the step, 3% off the dominant kernel)
+        unsigned slot[UNROLL];
+        double pv[UNROLL];
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-                slot[u] = 0;
-                pv[u] = 0.0;
-                if (c[u] >= 0) {
-                    slot[u] = slot_of(c[u]);
-                    pv[u] = P::prep(a, v[u]);
-                }
+        for (int u = 0; u < UNROLL; ++u) {
+            slot[u] = 0;
+            pv[u] = 0.0;
+            if (c[u] >= 0) {
+                slot[u] = slot_of(c[u]);
+                pv[u] = P::prep(a, v[u]);
             }
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
-                if (c[u] >= 0)
-                    P::put(vals, slot[u], pv[u]);
-        } else {
-            // compensated FP32: each add is a compare-and-swap loop that waits for its own
-            // result anyway; separating the steps measured 1.5% slower
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
-                if (c[u] >= 0)
-                    P::add(vals, slot_of(c[u]), a, v[u]);
         }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+            if (c[u] >= 0)
+                P::put(vals, slot[u], pv[u]);
     }
 }
 
@@ -1443,7 +1394,6 @@ __global__ __launch_bounds__(WC_BS) void k_wide_cols(const int *__restrict__ row
 // sums into C (zeroed by k_wide_cols, which also writes every wide row's columns) with
 // atomics; the other rows store them.
 constexpr int WS_COARSE = 256;
-constexpr int WS_BS = 768;   // lanes of a workgroup (two fit a CU: 6 waves per SIMD)
 constexpr int WS_WIN = 256;  // window starts listed at a time
 constexpr int WS_LV = 8;     // directory entries per lane when listing window starts
 constexpr int WS_GL = 16;    // lanes of a chunk group
@@ -1464,21 +1414,15 @@ static_assert(ws_lds(WS_VALS_BIG) + 256 <= 160 * 1024, "one workgroup of the lar
 constexpr u64 WS_NOPOS = 0xffffffffull << 32; // (position, column) with no position
 static_assert(2 + 2 * WS_CLASSES <= WIDE_CTRS, "wide-row counters");
 
-// Lanes of a workgroup, by form, window and density.  The default window runs two
-// workgroups per CU, the large one a single workgroup.  A window's phases share one
-// barrier and one LDS whose atomics queue up, so fewer waves than the CU could hold are
-// faster, the more so the sparser the rows (R-MAT scale 20, wide-row bin, default window,
-// four chunk tasks in flight per group: FP64 192 / 256 / 320 lanes 258 / 246 / 340 ms,
-// compensated FP32 256 / 320 / 384 lanes 266 / 261 / 265 ms; one task at a time: FP64
-// 128 / 256 / 512 lanes 355 / 263 / 290 ms; large window, 512 lanes: 287 and 301 ms).
-// Dense rows want more lanes (a Zipf A·Aᵀ panel's wide rows, FP64 256 / 384 / 512 / 768
-// lanes 41.4 / 38.0 / 37.2 / 39.4 ms; compensated 384 / 512 / 768 lanes 38.2 / 35.0 /
-// 34.6 ms).
-template <typename P, int VW, bool SPARSE> constexpr int ws_bs()
-{
-    return VW == WS_VALS_BIG ? 512
-                             : (std::is_same<P, PrecF64>::value ? (SPARSE ? 256 : 512) : (SPARSE ? 320 : WS_BS));
-}
+// Lanes of a workgroup, by window and density (both value types accumulate in FP64).  The
+// default window runs two workgroups per CU, the large one a single workgroup.  A window's
+// phases share one barrier and one LDS whose atomics queue up, so fewer waves than the CU
+// could hold are faster, the more so the sparser the rows (R-MAT scale 20, wide-row bin,
+// default window, four chunk tasks in flight per group, FP64: 192 / 256 / 320 lanes 258 /
+// 246 / 340 ms; one task at a time: 128 / 256 / 512 lanes 355 / 263 / 290 ms; large
+// window, 512 lanes: 287 ms).  Dense rows want more lanes (a Zipf A·Aᵀ panel's wide rows,
+// FP64 256 / 384 / 512 / 768 lanes 41.4 / 38.0 / 37.2 / 39.4 ms).
+template <int VW, bool SPARSE> constexpr int ws_bs() { return VW == WS_VALS_BIG || !SPARSE ? 512 : 256; }
 // waves per SIMD the launch holds (its workgroups per CU x waves / 4 SIMDs), for the
 // compiler's register budget
 template <int VW, int BS> constexpr int ws_waves()
@@ -1497,9 +1441,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu((ws_waves<VW
     constexpr int WT = VW / 2; // directory entries of a window
     // chunk tasks a 16-lane group loads before it adds any: a narrow (sparse-row)
     // workgroup has few groups, each with many tasks per round, and the registers for
-    // four (R-MAT scale 20 wide-row bin 263 -> 244 ms FP64, 275 -> 265 ms compensated;
-    // eight: no better for FP64, 384 ms compensated; two for the dense FP64 launch: within
-    // 1% on a Zipf panel)
+    // four (R-MAT scale 20 wide-row bin 263 -> 244 ms; eight: no better; two for the dense
+    // launch: within 1% on a Zipf panel)
     constexpr int NTS = BS < 512 ? 4 : 1;
     constexpr int SPLIT = wide_split_max(VW); // entries of an item, at most
     constexpr int EPL = (SPLIT + BS - 1) / BS; // entries a lane posts and moves
@@ -1815,31 +1758,18 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu((ws_waves<VW
                 }
             }
             // Output: the window's values (its columns were written by k_wide_cols).  Split
-            // rows add theirs into C (FP64) or, compensated, s + c into the FP64 scratch.
-            if constexpr (F32C) {
-                const float *fv = (const float *)vals;
-                if (split) {
-                    // the item's compensated sums meet in FP64 (s + c is exact in a double),
-                    // one atomic add each, no retries; rounded to FP32 once, at the end
-                    double *sd = (double *)scratch + sbase + base;
-                    for (int q = l; q < cnt; q += BS) {
-                        const float sv = fv[2 * q], cv = fv[2 * q + 1];
-                        if (sv != 0.0f || cv != 0.0f)
-                            unsafeAtomicAdd(&sd[q], (double)sv + (double)cv);
-                    }
-                } else {
-                    for (int q = l; q < cnt; q += BS)
-                        Cval[cb + base + q] = fv[2 * q] + fv[2 * q + 1];
-                }
-            } else if (split) {
+            // rows add theirs into C (FP64) or, with FP32 values, into the FP64 scratch, which
+            // is rounded into C once at the end.
+            if (split) {
+                double *to = F32C ? (double *)scratch + sbase + base : (double *)Cval + cb + base;
                 for (int q = l; q < cnt; q += BS) {
                     const double v = vals[q];
                     if (v != 0.0)
-                        unsafeAtomicAdd(&Cval[cb + base + q], v);
+                        unsafeAtomicAdd(&to[q], v);
                 }
             } else {
                 for (int q = l; q < cnt; q += BS)
-                    Cval[cb + base + q] = vals[q];
+                    Cval[cb + base + q] = P::result(vals, (unsigned)q);
             }
             done += cnt;
             __syncthreads();
@@ -2010,8 +1940,8 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
                                count_dev, op, crp, Ccol, F32C ? nullptr : (double *)Cval, wide.sym_row_max,
                                wide.sym_all_global, wide.long_rows, vals);
 #define WSPLIT(VW, SPARSE)                                                                                           \
-    hipLaunchKernelGGL((k_numeric_wsplit<P, VW, ws_bs<P, VW, SPARSE>()>), dim3((unsigned)wide.blocks),                 \
-                       dim3(ws_bs<P, VW, SPARSE>()), ws_lds(VW), s, wide.items, wide.ctr, wide.ctr + 1, op, crp,        \
+    hipLaunchKernelGGL((k_numeric_wsplit<P, VW, ws_bs<VW, SPARSE>()>), dim3((unsigned)wide.blocks),                 \
+                       dim3(ws_bs<VW, SPARSE>()), ws_lds(VW), s, wide.items, wide.ctr, wide.ctr + 1, op, crp,        \
                        (typename P::V *)Cval, (u64 *)wide.scratch, wide.ws, wide.ft_stride, wide.sym_row_max,           \
                        wide.sym_all_global, wide.long_rows, err)
             if (vals == WS_VALS_BIG)
@@ -2093,9 +2023,9 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
     CFG(k_numeric_window<PrecF64>) CFG(k_numeric_window<PrecF32C>)
     CFG(k_numeric_wcompact<PrecF64>) CFG(k_numeric_wcompact<PrecF32C>) 
 #define CFGW(P)                                                                                                        \
-    CFG((k_numeric_wsplit<P, WS_VALS, ws_bs<P, WS_VALS, false>()>))                                                    \
-    CFG((k_numeric_wsplit<P, WS_VALS, ws_bs<P, WS_VALS, true>()>))                                                     \
-    CFG((k_numeric_wsplit<P, WS_VALS_BIG, ws_bs<P, WS_VALS_BIG, false>()>))
+    CFG((k_numeric_wsplit<P, WS_VALS, ws_bs<WS_VALS, false>()>))                                                    \
+    CFG((k_numeric_wsplit<P, WS_VALS, ws_bs<WS_VALS, true>()>))                                                     \
+    CFG((k_numeric_wsplit<P, WS_VALS_BIG, ws_bs<WS_VALS_BIG, false>()>))
     CFGW(PrecF64) CFGW(PrecF32C)
 #undef CFGW
 #undef CFG

@@ -56,7 +56,9 @@ enum hsmu_status {
 /* numeric form */
 enum hsmu_precision {
     HSMU_FP64 = 0,      /* plain: FP64 products, FP64 LDS accumulation (the reference's value_t) */
-    HSMU_FP32_COMP = 1  /* FP32 products, compensated (two-sum) FP32 accumulation, FP32 values */
+    HSMU_FP32_COMP = 1  /* compensated FP32: FP32 values; products exact and their sums carried with
+                           more bits than a compensated FP32 pair (accumulated in FP64), rounded to
+                           FP32 once: within one FP32 rounding of the exact sum */
 };
 
 /* ---- matrices ---------------------------------------------------------------- */
