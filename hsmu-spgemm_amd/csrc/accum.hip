@@ -16,11 +16,13 @@
 // (compressed_Ccol_symbolic.cuh:4-63); for the wide rows of the FP64 path a separate
 // streaming kernel (k_wide_cols) writes them from the kept directories.
 //
-// LDS row kernels stage the row's A entries (B row range, first tile, a_ij) in LDS once;
-// sub-groups of lanes then take one entry each and walk B_j, several elements per lane
-// with all loads issued first; rows of B longer than LONG_SEG (tiles: LONG_TILES) are
-// walked by whole waves.  Rows whose slice does not fit LDS (wide rows) use the windowed
-// kernels at the end of this file.
+// The kernels of rows that share a wave, and the symbolic ones, stage the row's A entries (B
+// row range, first tile, a_ij) in LDS once; sub-groups of lanes then take one entry each
+// and walk B_j, several elements per lane with all loads issued first; rows of B longer
+// than LONG_SEG (tiles: LONG_TILES) are walked by whole waves.  The numeric kernels of rows
+// with a workgroup to themselves walk all their B rows as one stream of element pairs.
+// Rows whose slice does not fit LDS (wide rows) use the windowed kernels at the end of this
+// file.
 
 #include <hip/hip_runtime.h>
 
@@ -325,6 +327,223 @@ DEVI void add_products(const Operands &op, const int *b0, const int *blen, const
     }
 }
 
+// ---- the element stream of a row ------------------------------------------------------------
+//
+// One workgroup of G lanes (64 or more) walks the B rows of its row's A entries as one
+// stream of slots (hsmu_internal.h).  stage() takes one entry per lane, mark() lays out the
+// bits of a window of slots, run() goes over all of a row's entries: entry(e) gives entry
+// e's first element, length and payload, body(st, w0) walks the window of slots from w0.
+struct Segment {
+    int start, len;
+    u64 payload;
+};
+
+template <int G> struct Stream {
+    static constexpr int NW = G / 64;
+    static constexpr int WINDOW = stream_window(G);
+    uint4 *rec;
+    u64 *bits, *red;
+    unsigned short *wb;
+    long long first, total; // this lane's first slot, slots in all
+    int cnt, nrec;          // this lane's slots, entries with slots
+    unsigned rank;
+
+    DEVI void stage(const Segment &g)
+    {
+        cnt = (int)(((unsigned)g.len + STREAM_V - 1) / STREAM_V);
+        u64 tot;
+        const u64 ex = group_excl_scan<G, u64>((u64)(unsigned)cnt | (cnt ? 1ull << 48 : 0ull), red, tot);
+        first = (long long)(ex & ((1ull << 48) - 1));
+        rank = (unsigned)(ex >> 48);
+        total = (long long)uniform64(tot & ((1ull << 48) - 1));
+        nrec = (int)uniform((unsigned)(tot >> 48));
+        if (cnt)
+            rec[rank] = make_uint4((unsigned)g.start - STREAM_V * (unsigned)first, (unsigned)(g.start + g.len),
+                                   (unsigned)g.payload, (unsigned)(g.payload >> 32));
+    }
+    DEVI void mark(long long w0)
+    {
+        if (!cnt)
+            return;
+        const long long f = first - w0, last = f + cnt - 1;
+        if (last >= 0 && last < WINDOW)
+            atomicOr(&bits[last >> 6], 1ull << (last & 63));
+        const int s0 = f > 0 ? (f < WINDOW ? (int)((f + 63) >> 6) : WINDOW / 64) : 0;
+        const int s1 = last < 0 ? -1 : (last < WINDOW ? (int)(last >> 6) : WINDOW / 64 - 1);
+        for (int s = s0; s <= s1; ++s)
+            wb[s] = (unsigned short)rank;
+    }
+    // steps of 64 slots in the window from w0
+    DEVI int steps(long long w0) const
+    {
+        const long long n = total - w0 < WINDOW ? total - w0 : WINDOW;
+        return (int)((n + 63) >> 6);
+    }
+    // the entry of this lane's slot in step s of the window (past the last slot: any)
+    DEVI uint4 entry(int s) const { return entry(wb[s], bits[s]); }
+    DEVI uint4 entry(int base, u64 word) const
+    {
+        int e = base + mbcnt(word);
+        e = e < nrec ? e : nrec - 1;
+        return rec[e];
+    }
+    // The bits must be zero, and a barrier passed since.
+    template <typename Entry, typename Body> DEVI void run(int nA, Entry entry_of, Body body)
+    {
+        const int l = threadIdx.x;
+        for (int c = 0; c < nA; c += G) {
+            stage(c + l < nA ? entry_of(c + l) : Segment{0, 0, 0});
+            for (long long w0 = 0; w0 < total; w0 += WINDOW) {
+                mark(w0);
+                __syncthreads();
+                body(*this, w0);
+                __syncthreads();
+                if (c + G < nA || w0 + WINDOW < total) {
+                    const int n = steps(w0);
+                    for (int q = l; q < n; q += G)
+                        bits[q] = 0;
+                    __syncthreads();
+                }
+            }
+        }
+    }
+};
+
+// STREAM_V consecutive elements in one load, at the alignment of a single element.
+template <typename T> struct Vec2 {
+    typedef T type __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+};
+template <typename T> DEVI typename Vec2<T>::type load2(const T *p) { return *(const typename Vec2<T>::type *)p; }
+
+// A lane's elements k, k + 1 of an array of n: loaded from k or, at the array's end, from
+// n - 2; in0 / in1: element 0 / 1 of the load belongs to [k, end).
+struct Pair {
+    unsigned at;
+    bool in0, in1;
+    DEVI Pair(unsigned k, unsigned end, unsigned n)
+    {
+        at = k < n - 2 ? k : n - 2;
+        in0 = at == k && k < end;
+        in1 = at + 1 >= k && at + 1 < end;
+    }
+};
+
+// Add the products of a window of the row's stream into their slots, STREAM_U steps of a
+// wave loaded while the STREAM_U before them are added (the loads are not predicated, so
+// that a wait for one set is not a wait for the other).
+constexpr int STREAM_U = 2;
+template <int G, int FORM, typename P>
+DEVI void stream_add(const Stream<G> &st, long long w0, const Operands &op, const u64 *cm, const unsigned *coff,
+                     const u64 *fm, const unsigned *foff, double *vals, int mn)
+{
+    typedef typename P::V V;
+    constexpr int NW = G / 64, U = STREAM_U;
+    const V *__restrict__ Bval = (const V *)op.Bval;
+    const unsigned nB = (unsigned)op.nnzB;
+    const int c0 = mn << 6;
+    const int lane = threadIdx.x & 63;
+    const int nst = st.steps(w0);
+    int s = NW > 1 ? uniform((int)(threadIdx.x >> 6)) : 0;
+    if (s >= nst)
+        return;
+    typename Vec2<int>::type c[2][U];
+    typename Vec2<V>::type v[2][U];
+    double a[2][U];
+    bool in0[2][U], in1[2][U];
+    // lane i holds the bits and the first entry of the wave's i-th next step
+    static_assert(Stream<G>::WINDOW / 64 <= 64 * NW, "a wave's steps fit its lanes");
+    u64 lw = 0;
+    int lb = 0;
+    if (s + lane * NW < nst) {
+        lw = st.bits[s + lane * NW];
+        lb = st.wb[s + lane * NW];
+    }
+    int i = 0; // the wave's next step
+    auto load = [&](int h) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // past the wave's last step: some entry, with nothing in it
+            const uint4 r = st.entry(__builtin_amdgcn_readlane(lb, (i + u) & 63), readlane_u64(lw, (i + u) & 63));
+            const int su = s + u * NW;
+            const unsigned k = r.x + STREAM_V * ((unsigned)w0 + 64 * su + lane);
+            const Pair q(k, su < nst ? r.y : 0u, nB);
+            c[h][u] = load2(op.Bcol + q.at);
+            v[h][u] = load2(Bval + q.at);
+            a[h][u] = __longlong_as_double((long long)(((u64)r.w << 32) | r.z));
+            in0[h][u] = q.in0;
+            in1[h][u] = q.in1;
+        }
+        i += U;
+        s += U * NW;
+    };
+    auto slot_of = [&](int col) -> unsigned {
+        const int q = col - c0;
+        if constexpr (FORM == SLOT_DENSE) {
+            return (unsigned)q;
+        } else {
+            const unsigned kk = FORM == SLOT_TWO_LEVEL ? fine_index(cm, coff, q >> 6) : (unsigned)(q >> 6);
+            return foff[kk] + (unsigned)__popcll(fm[kk] & below(q & 63));
+        }
+    };
+    auto add = [&](int h) {
+        unsigned s0[U], s1[U];
+        double p0[U], p1[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (FORM == SLOT_DENSE || in0[h][u])
+                s0[u] = slot_of(c[h][u].x);
+            if (FORM == SLOT_DENSE || in1[h][u])
+                s1[u] = slot_of(c[h][u].y);
+            p0[u] = P::prep(a[h][u], v[h][u].x);
+            p1[u] = P::prep(a[h][u], v[h][u].y);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (in0[h][u])
+                P::put(vals, s0[u], p0[u]);
+            if (in1[h][u])
+                P::put(vals, s1[u], p1[u]);
+        }
+    };
+    load(0);
+    while (true) {
+        const bool m1 = s < nst;
+        if (m1)
+            load(1);
+        add(0);
+        if (!m1)
+            break;
+        const bool m0 = s < nst;
+        if (m0)
+            load(0);
+        add(1);
+        if (!m0)
+            break;
+    }
+}
+
+// OR a window of the row's tile stream (entries are tile ranges) into its directory.
+template <int G, int MODE>
+DEVI void stream_or(const Stream<G> &st, long long w0, const Operands &op, u64 *dm, const unsigned *coff, u64 *fm, int mn)
+{
+    constexpr int NW = G / 64;
+    const unsigned nB = (unsigned)op.nnzB;
+    const int lane = threadIdx.x & 63;
+    const int nst = st.steps(w0);
+    for (int s = NW > 1 ? uniform((int)(threadIdx.x >> 6)) : 0; s < nst; s += NW) {
+        const uint4 r = st.entry(s);
+        const Pair q(r.x + STREAM_V * (unsigned)((unsigned)w0 + 64 * s + lane), r.y, nB);
+        const Vec2<int>::type c = load2(op.tcol + q.at);
+        Vec2<u64>::type m = {0, 0};
+        if constexpr (MODE != OR_COARSE)
+            m = load2(op.tmask + q.at);
+        if (q.in0)
+            or_put<MODE>(dm, coff, fm, c.x - mn, m.x);
+        if (q.in1)
+            or_put<MODE>(dm, coff, fm, c.y - mn, m.y);
+    }
+}
+
 // ---- symbolic ------------------------------------------------------------------------------
 
 // nnz(C_i) for rows kept in LDS: stage the row, OR the tile masks with ds_or_b64 into the
@@ -573,23 +792,23 @@ __global__ __launch_bounds__(1024) void k_symbolic_wide(const int *__restrict__ 
 
 // ---- numeric -------------------------------------------------------------------------------
 
-// The HSMU accumulator in LDS (slice layout: row_layout).  The row's tile directory is
-// loaded (kept by the symbolic phase) or rebuilt as there, every product is added with
-// ds_add_f64 into its slot, and the row of C is written in column order: for G >= 64 one
-// wave per tile, lane b writing column 64*(rmin+t)+b if present (coalesced); for G < 64
-// one lane per tile walking its set bits.  Directory forms: flat (slot from the tile's
-// entry), dense (one slot per column of the span) and two-level (the tile's entry found
-// through the coarse bitmap first); two_level = 0 when no row of the launch uses it.
+// The HSMU accumulator in LDS for rows that share a workgroup of one wave (G = 8, 16 or 32
+// lanes per row; slice layout: row_layout).  The row's tile directory is loaded (kept by
+// the symbolic phase) or rebuilt as there, every product is added with ds_add_f64 into its
+// slot, and the row of C is written in column order, a lane per tile walking its set bits.
+// Directory forms: flat (slot from the tile's entry), dense (one slot per column of the
+// span) and two-level (the tile's entry found through the coarse bitmap first); two_level =
+// 0 when no row of the launch uses it.
 template <int G, typename P, bool LONG>
-__global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_numeric_lds(const int *__restrict__ rows,
+__global__ __launch_bounds__(BLOCK) void k_numeric_lds(const int *__restrict__ rows,
                                                                       const int *__restrict__ count_p, int slice_bytes,
                                                                       Operands op, const long long *__restrict__ crp,
                                                                       int *__restrict__ Ccol, typename P::V *__restrict__ Cval,
                                                                       int bshift, int tshift, int two_level, int *err,
                                                                       unsigned *queue)
 {
-    constexpr int BS = G < BLOCK ? BLOCK : G;
-    constexpr int RPB = BS / G;
+    static_assert(G < BLOCK, "rows that share a workgroup");
+    constexpr int RPB = BLOCK / G;
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ unsigned redu[16];
     __shared__ int grp_s[2];
@@ -609,15 +828,6 @@ __global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_numeric_lds(const int
             a0 = op.Arp[row];
             nA = op.Arp[row + 1] - a0;
             tp = op.rtp[row];
-        }
-        if constexpr (G >= 64) { // one row per workgroup: its scalars in scalar registers
-            S = uniform(S);
-            mn = uniform(mn);
-            n = uniform(n);
-            a0 = uniform(a0);
-            nA = uniform(nA);
-            tp = uniform(tp);
-            cb = uniform64(cb);
         }
         const bool sparse = use_sparse(S, tp);
         const int W = sparse ? (S + 63) >> 6 : S; // entries of the first level
@@ -662,10 +872,6 @@ __global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_numeric_lds(const int
                 if (blen[k] >= LONG_SEG)
                     lidx[atomicAdd(lcnt, 1)] = k;
         }
-        // One row per workgroup with its directory kept (a uniform condition): the slot
-        // offsets and totals are loaded, so neither the tile OR with its barrier nor the
-        // popcount scans run.
-        const bool known = G >= 64 && rd >= 0;
         if (rd < 0) {
             if (sparse)
                 or_tiles<G, OR_COARSE>(op, t0, tlen, nA, nullptr, 0, dm, nullptr, nullptr, mn, tshift);
@@ -674,16 +880,11 @@ __global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_numeric_lds(const int
         }
         // first level: flat slot offsets (rebuilt) or coarse compact indices (rebuilt), and
         // the total (flat: nnz(C_i); two-level: non-empty tiles)
-        unsigned tot;
-        if (known) {
-            tot = sparse ? (W > 0 ? doff[W - 1] + (unsigned)__popcll(dm[W - 1]) : 0u) : (unsigned)n;
-        } else {
-            __syncthreads();
-            const ChunkScan cs = scan_popcounts<G>(dm, W, redu);
-            tot = cs.tot;
-            if (rd < 0)
-                chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64) { doff[t] = p; });
-        }
+        __syncthreads();
+        const ChunkScan cs = scan_popcounts<G>(dm, W, redu);
+        const unsigned tot = cs.tot;
+        if (rd < 0)
+            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64) { doff[t] = p; });
         unsigned nnz = tot;
         const int F = sparse ? (int)tot : S; // fine entries
         if (two_level) {
@@ -711,17 +912,12 @@ __global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_numeric_lds(const int
             __syncthreads();
             if (sparse && rd < 0)
                 or_tiles<G, OR_FINE>(op, t0, tlen, nA, nullptr, 0, dm, doff, fm, mn, tshift);
-            if (known) {
-                if (sparse)
-                    nnz = (unsigned)n;
-            } else {
-                __syncthreads();
-                const ChunkScan fs = scan_popcounts<G>(fm, sparse ? F : 0, redu);
-                if (sparse) {
-                    nnz = fs.tot;
-                    if (rd < 0)
-                        chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64) { foff[k] = p; });
-                }
+            __syncthreads();
+            const ChunkScan fs = scan_popcounts<G>(fm, sparse ? F : 0, redu);
+            if (sparse) {
+                nnz = fs.tot;
+                if (rd < 0)
+                    chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64) { foff[k] = p; });
             }
         }
         const bool ok = (int)nnz == n;
@@ -742,37 +938,238 @@ __global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_numeric_lds(const int
         }
         __syncthreads();
         if (row >= 0 && ok) {
-            if (G >= 64 && (dense || (unsigned)n >= 16u * (unsigned)F)) {
-                // tiles holding 16 columns or more on average: a wave per tile, a lane per column
-                constexpr int NW = G < 64 ? 1 : G / 64;
-                const int w = l >> 6, lane = l & 63;
-                for (int k = w; k < F; k += NW) {
-                    const u64 m = fm[k];
-                    if ((m >> lane) & 1ull) {
-                        const int t = sparse ? (int)ft[k] : k;
-                        const unsigned pos = foff[k] + (unsigned)__popcll(m & below(lane));
-                        Ccol[cb + pos] = ((mn + t) << 6) + lane;
-                        Cval[cb + pos] = P::result(vals, dense ? (t << 6) + lane : pos);
+            // a lane per tile, then the values in slot order
+            for (int t0 = l; t0 < F; t0 += G) {
+                u64 m = fm[t0];
+                unsigned pos = foff[t0];
+                const int t = sparse ? (int)ft[t0] : t0;
+                const int c0 = (mn + t) << 6;
+                while (m) {
+                    const int b = __ffsll((unsigned long long)m) - 1;
+                    Ccol[cb + pos] = c0 + b;
+                    if (dense)
+                        Cval[cb + pos] = P::result(vals, (t << 6) + b);
+                    ++pos;
+                    m &= m - 1;
+                }
+            }
+            if (!dense)
+                for (int q = l; q < n; q += G)
+                    Cval[cb + q] = P::result(vals, q);
+        }
+        __syncthreads();
+    }
+}
+
+// The same for a row with a workgroup to itself (G = 64 to 1024 lanes): its B rows are
+// walked as one element stream.  What bounds it: the L1's rate for loads (12 bytes per
+// product; see the stream's loads), the LDS's for ds_add_f64 (24 cycles per 64 products),
+// C's stores, and the chain of short phases of a row, which several workgroups per CU
+// overlap (ablation on banded: staging and zeroing 130 us, adds 250, output 200 of 560).
+// Against the walk it replaced (a sub-group of lanes per B row, 4- and 8-byte loads):
+// banded 62,451 rows 594 -> 512 us of numeric time; R-MAT scale 16, compensated FP32, rows
+// of 256 to 1024 lanes 1,950 -> 1,150 us; R-MAT scale 18, FP64, rows of 512 lanes 5.35 ->
+// 3.31 ms.
+// TL: some row of the launch has a two-level directory (the form costs registers, so
+// launches without one run a kernel without it).  At 5 waves per SIMD (96 registers) ten
+// banded rows of 128 lanes fit a CU as their LDS does.
+template <int G, typename P, bool TL>
+__global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5))) void k_numeric_row(
+    const int *__restrict__ rows, const int *__restrict__ count_p, Operands op, const long long *__restrict__ crp,
+    int *__restrict__ Ccol, typename P::V *__restrict__ Cval, int *err, unsigned *queue)
+{
+    typedef typename P::V V;
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ u64 red[16];
+    __shared__ int grp_s[2];
+    const int l = threadIdx.x;
+    const V *__restrict__ Aval = (const V *)op.Aval;
+    const int nrows = *count_p;
+    for (GroupWalk gw(queue, nrows, grp_s, c_nxcd); gw.more(); gw.next()) {
+        const int row = uniform(rows[gw.grp]);
+        const int mn = uniform(op.rmin[row]);
+        const int S = uniform(op.rmax[row]) - mn + 1;
+        const long long cb = uniform64(crp[row]);
+        const int n = (int)(uniform64(crp[row + 1]) - cb);
+        const int a0 = uniform(op.Arp[row]), nA = uniform(op.Arp[row + 1]) - a0;
+        const int tp = uniform(op.rtp[row]);
+        const bool sparse = TL && use_sparse(S, tp);
+        const int W = sparse ? (S + 63) >> 6 : S; // entries of the first level
+        const StreamLayout L = stream_layout(G, S, n, nA, tp, uniform64(op.rprod[row]));
+        double *vals = (double *)(lds + L.vals);
+        u64 *dm = (u64 *)(lds + L.dm);
+        unsigned *doff = (unsigned *)(lds + L.doff);
+        unsigned *ft = (unsigned *)(lds + L.ft);
+        Stream<G> st;
+        st.rec = (uint4 *)(lds + L.rec);
+        st.bits = (u64 *)(lds + L.bits);
+        st.wb = (unsigned short *)(lds + L.wb);
+        st.red = red;
+        // fine level: the flat directory itself, or the compact entries after the coarse words
+        u64 *fm = sparse ? dm + W : dm;
+        unsigned *foff = sparse ? doff + W : doff;
+        const bool dense = !sparse && use_dense(S, n);
+        const int nv = dense ? 64 * S : n;
+        const long long rd = op.dir_mask ? uniform64(op.rdir[row]) : -1;
+        const int words = (L.doff - L.bits) >> 3;
+        for (int q = 2 * l; q < nv; q += 2 * G) // (the array is padded to 16 bytes)
+            *(double2 *)(vals + q) = make_double2(0.0, 0.0);
+        for (int q = l; q < words; q += G)
+            st.bits[q] = 0;
+        if (rd >= 0) { // directory kept by the symbolic phase: its first level
+            for (int t = l; t < W; t += G) {
+                dm[t] = op.dir_mask[rd + t];
+                doff[t] = op.dir_off[rd + t];
+            }
+        } else {
+            for (int t = l; t < W; t += G)
+                dm[t] = 0;
+        }
+        __syncthreads();
+        auto tiles_of = [&](int e) {
+            const int j = op.Acol[a0 + e];
+            const int t0 = op.tptr[j];
+            return Segment{t0, op.tptr[j + 1] - t0, 0};
+        };
+        auto rezero = [&]() { // the stream's bits, for its next run
+            __syncthreads();
+            for (int q = l; q < words; q += G)
+                st.bits[q] = 0;
+        };
+        // the first level: flat slot offsets or coarse compact indices, and its total
+        unsigned tot = (unsigned)n;
+        if (rd < 0) {
+            if constexpr (TL) {
+                if (sparse)
+                    st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                        stream_or<G, OR_COARSE>(t, w0, op, dm, nullptr, nullptr, mn);
+                    });
+            }
+            if (!sparse)
+                st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                    stream_or<G, OR_FLAT>(t, w0, op, dm, nullptr, nullptr, mn);
+                });
+            rezero();
+            const ChunkScan cs = scan_popcounts<G>(dm, W, (unsigned *)red);
+            tot = cs.tot;
+            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64) { doff[t] = p; });
+        } else if (sparse) {
+            tot = W > 0 ? doff[W - 1] + (unsigned)__popcll(dm[W - 1]) : 0u;
+        }
+        unsigned nnz = tot;
+        const int F = sparse ? (int)tot : S; // fine entries
+        if (sparse) { // (uniform: one row per workgroup)
+            __syncthreads();
+            if (rd >= 0) {
+                for (int k = l; k < F; k += G) {
+                    fm[k] = op.dir_mask[rd + W + k];
+                    foff[k] = op.dir_off[rd + W + k];
+                }
+                nnz = (unsigned)n;
+            } else {
+                for (int k = l; k < F; k += G)
+                    fm[k] = 0;
+            }
+            // tile of every fine entry, from the coarse bitmap
+            for (int w = l; w < W; w += G) {
+                u64 m = dm[w];
+                unsigned k = doff[w];
+                while (m) {
+                    ft[k++] = (unsigned)((w << 6) + __ffsll((unsigned long long)m) - 1);
+                    m &= m - 1;
+                }
+            }
+            __syncthreads();
+            if (rd < 0) {
+                st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                    stream_or<G, OR_FINE>(t, w0, op, dm, doff, fm, mn);
+                });
+                rezero();
+                const ChunkScan fs = scan_popcounts<G>(fm, F, (unsigned *)red);
+                nnz = fs.tot;
+                chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64) { foff[k] = p; });
+            }
+        }
+        const bool ok = (int)nnz == n;
+        if (!ok && l == 0)
+            atomicOr(err, ERR_INTERNAL);
+        __syncthreads();
+        if (ok) { // uniform
+            auto rows_of = [&](int e) {
+                const int j = op.Acol[a0 + e];
+                const int b0 = op.Brp[j];
+                const double a = (double)Aval[a0 + e];
+                return Segment{b0, op.Brp[j + 1] - b0, (u64)__double_as_longlong(a)};
+            };
+            if (dense)
+                st.run(nA, rows_of, [&](const Stream<G> &t, long long w0) {
+                    stream_add<G, SLOT_DENSE, P>(t, w0, op, nullptr, nullptr, fm, foff, vals, mn);
+                });
+            else if (!sparse)
+                st.run(nA, rows_of, [&](const Stream<G> &t, long long w0) {
+                    stream_add<G, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, fm, foff, vals, mn);
+                });
+            if constexpr (TL) {
+                if (sparse)
+                    st.run(nA, rows_of, [&](const Stream<G> &t, long long w0) {
+                        stream_add<G, SLOT_TWO_LEVEL, P>(t, w0, op, dm, doff, fm, foff, vals, mn);
+                    });
+            }
+            if (dense || (unsigned)n >= 16u * (unsigned)F) {
+                // tiles holding 16 columns or more on average: a wave per tile, a lane per
+                // column; OUT_U tiles' values are read before any is stored
+                constexpr int NW = G / 64, OUT_U = 4;
+                const int w = uniform(l >> 6), lane = l & 63;
+                int *__restrict__ oc = Ccol + cb;
+                V *__restrict__ ov = Cval + cb;
+                for (int kb = w; kb < F; kb += 64 * NW) {
+                    // lane i holds tile kb + i * NW
+                    const int kt = kb + lane * NW;
+                    u64 lm = 0;
+                    unsigned lo = 0;
+                    int lt = 0;
+                    if (kt < F) {
+                        lm = fm[kt];
+                        lo = foff[kt];
+                        lt = sparse ? (int)ft[kt] : kt;
+                    }
+                    const int left = (F - kb + NW - 1) / NW, cnt = left < 64 ? left : 64;
+                    for (int i = 0; i < cnt; i += OUT_U) {
+                        unsigned pos[OUT_U];
+                        int col[OUT_U];
+                        V val[OUT_U];
+                        bool has[OUT_U];
+#pragma unroll
+                        for (int u = 0; u < OUT_U; ++u) {
+                            const u64 m = readlane_u64(lm, i + u); // (0 past the last tile)
+                            const int t = __builtin_amdgcn_readlane(lt, i + u);
+                            has[u] = __builtin_amdgcn_inverse_ballot_w64(m);
+                            pos[u] = (unsigned)__builtin_amdgcn_readlane((int)lo, i + u) + (unsigned)mbcnt(m);
+                            col[u] = ((mn + t) << 6) + lane;
+                            if (has[u])
+                                val[u] = P::result(vals, dense ? (unsigned)((t << 6) + lane) : pos[u]);
+                        }
+#pragma unroll
+                        for (int u = 0; u < OUT_U; ++u)
+                            if (has[u]) {
+                                oc[pos[u]] = col[u];
+                                ov[pos[u]] = val[u];
+                            }
                     }
                 }
             } else { // a lane per tile, then the values in slot order
                 for (int k = l; k < F; k += G) {
                     u64 m = fm[k];
                     unsigned pos = foff[k];
-                    const int t = sparse ? (int)ft[k] : k;
-                    const int c0 = (mn + t) << 6;
+                    const int c0 = (mn + (sparse ? (int)ft[k] : k)) << 6;
                     while (m) {
-                        const int b = __ffsll((unsigned long long)m) - 1;
-                        Ccol[cb + pos] = c0 + b;
-                        if (dense)
-                            Cval[cb + pos] = P::result(vals, (t << 6) + b);
+                        Ccol[cb + pos] = c0 + __ffsll((unsigned long long)m) - 1;
                         ++pos;
                         m &= m - 1;
                     }
                 }
-                if (!dense)
-                    for (int q = l; q < n; q += G)
-                        Cval[cb + q] = P::result(vals, q);
+                for (int q = l; q < n; q += G)
+                    Cval[cb + q] = P::result(vals, q);
             }
         }
         __syncthreads();
@@ -1906,7 +2303,35 @@ static void numeric_l(int bin, const int *rows, const int *count_dev, int count,
                               num_cus, queue, lds_bytes, s);                                                           \
         break;
     switch (bin) {
-        NUM(0, 8) NUM(1, 16) NUM(2, 32) NUM(3, 64) NUM(4, 128) NUM(5, 256) NUM(6, 512) NUM(7, 1024)
+        NUM(0, 8) NUM(1, 16) NUM(2, 32)
+    }
+#undef NUM
+}
+
+template <int G, typename P, bool TL>
+static void numeric_row(const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
+                        const long long *crp, int *Ccol, void *Cval, int *err, int num_cus, unsigned *queue,
+                        unsigned long long *lds_bytes, hipStream_t s)
+{
+    const size_t lds = (size_t)((max_need + 15) & ~15);
+    const int64_t blocks = row_grid(k_numeric_row<G, P, TL>, G, lds, count, num_cus, queue);
+    *lds_bytes += (unsigned long long)blocks * lds;
+    hipLaunchKernelGGL((k_numeric_row<G, P, TL>), dim3((unsigned)blocks), dim3(G), lds, s, rows, count_dev, op, crp,
+                       Ccol, (typename P::V *)Cval, err, queue);
+}
+
+template <typename P, bool TL>
+static void numeric_rows(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
+                         const long long *crp, int *Ccol, void *Cval, int *err, int num_cus, unsigned *queue,
+                         unsigned long long *lds_bytes, hipStream_t s)
+{
+#define NUM(B, G)                                                                                                      \
+    case B:                                                                                                            \
+        numeric_row<G, P, TL>(rows, count_dev, count, max_need, op, crp, Ccol, Cval, err, num_cus, queue, lds_bytes,   \
+                              s);                                                                                      \
+        break;
+    switch (bin) {
+        NUM(3, 64) NUM(4, 128) NUM(5, 256) NUM(6, 512) NUM(7, 1024)
     }
 #undef NUM
 }
@@ -1962,6 +2387,13 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
             hipLaunchKernelGGL(k_numeric_window<P>, dim3(blocks), dim3(1024), WIN_LDS, s, rows, count_dev, op, crp, Ccol,
                                (typename P::V *)Cval, bshift > 6 ? 6 : bshift, wide.ws, wide.cur_stride, wide.ft_stride,
                                err);
+    } else if (bin >= 3 && bin < NLDS) {
+        if (two_level)
+            numeric_rows<P, true>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, err, num_cus, queue,
+                                  lds_bytes, s);
+        else
+            numeric_rows<P, false>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, err, num_cus, queue,
+                                   lds_bytes, s);
     } else if (bin >= 0 && bin < NLDS) {
         if (long_rows)
             numeric_l<P, true>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, tshift, two_level,
@@ -2012,11 +2444,14 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
     CFG((k_symbolic_lds<64, L>)) CFG((k_symbolic_lds<128, L>)) CFG((k_symbolic_lds<256, L>))                          \
     CFG((k_symbolic_lds<512, L>)) CFG((k_symbolic_lds<1024, L>))
 #define CFGP(P, L)                                                                                                     \
-    CFG((k_numeric_lds<8, P, L>)) CFG((k_numeric_lds<16, P, L>)) CFG((k_numeric_lds<32, P, L>))                       \
-    CFG((k_numeric_lds<64, P, L>)) CFG((k_numeric_lds<128, P, L>)) CFG((k_numeric_lds<256, P, L>))                    \
-    CFG((k_numeric_lds<512, P, L>)) CFG((k_numeric_lds<1024, P, L>))
+    CFG((k_numeric_lds<8, P, L>)) CFG((k_numeric_lds<16, P, L>)) CFG((k_numeric_lds<32, P, L>))
+#define CFGR(P, TL)                                                                                                    \
+    CFG((k_numeric_row<64, P, TL>)) CFG((k_numeric_row<128, P, TL>)) CFG((k_numeric_row<256, P, TL>))                  \
+    CFG((k_numeric_row<512, P, TL>)) CFG((k_numeric_row<1024, P, TL>))
     CFGL(false) CFGL(true)
     CFGP(PrecF64, false) CFGP(PrecF64, true) CFGP(PrecF32C, false) CFGP(PrecF32C, true)
+    CFGR(PrecF64, false) CFGR(PrecF32C, false) CFGR(PrecF64, true) CFGR(PrecF32C, true)
+#undef CFGR
 #undef CFGP
 #undef CFGL
     CFG(k_symbolic_wide)

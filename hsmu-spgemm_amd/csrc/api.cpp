@@ -701,8 +701,9 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
 
     int *tcnt = (int *)ar.get<char>(btiles_ws_bytes(P.nnzB));
     int *tptr = ar.get<int>((size_t)K + 1);
-    int *tcol = ar.get<int>((size_t)P.nnzB);
-    unsigned long long *tmask = ar.get<unsigned long long>((size_t)P.nnzB);
+    const size_t ntcap = P.nnzB > STREAM_V ? (size_t)P.nnzB : STREAM_V; // loaded STREAM_V at a time
+    int *tcol = ar.get<int>(ntcap);
+    unsigned long long *tmask = ar.get<unsigned long long>(ntcap);
     int64_t nmax = M > K ? M : K;
     nmax = nmax > P.nnzB ? nmax : P.nnzB;
     void *scan_ws = ar.get<char>(scan_ws_bytes(nmax + 1));
@@ -773,6 +774,17 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     op.Brp = P.Brp;
     op.Bcol = P.Bcol;
     op.Bval = P.Bval;
+    op.nnzB = (int)P.nnzB;
+    if (P.nnzB < STREAM_V) { // the element stream loads STREAM_V at a time
+        int *pcol = ar.get<int>(STREAM_V);
+        void *pval = ar.raw(STREAM_V * (size_t)vsz);
+        if (!pcol || !pval)
+            return fail(HSMU_ERR_NOMEM, "workspace allocation");
+        HIP_TRY(launch_pad_b(P.Bcol, P.Bval, fp32 ? 1 : 0, (int)P.nnzB, pcol, pval, s));
+        op.Bcol = pcol;
+        op.Bval = pval;
+        op.nnzB = STREAM_V;
+    }
     op.val32 = fp32 ? 1 : 0;
     op.tptr = tptr;
     op.tcol = tcol;
@@ -780,6 +792,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     op.rmin = rmin;
     op.rmax = rmax;
     op.rtp = rtp;
+    op.rprod = rprod;
     // Row directories (tile masks + slot offsets) are kept from the symbolic to the
     // numeric phase (12 bytes per directory entry) when that is cheaper than rebuilding
     // them -- the directories hold at most half as many entries as the tile-products that

@@ -31,6 +31,14 @@ DEVI long long uniform64(long long v)
 }
 DEVI u64 uniform64(u64 v) { return (u64)uniform64((long long)v); }
 
+// Lane k's value (k uniform), in scalar registers.
+DEVI u64 readlane_u64(u64 v, int k)
+{
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, k);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), k);
+    return ((u64)hi << 32) | lo;
+}
+
 // Reductions and scans over the 64 lanes of a wave (every lane must take part).
 template <typename T> DEVI T wave_sum(T v)
 {

@@ -196,9 +196,73 @@ HSMU_HD inline long long sym_need(long long S, long long nA, long long tp, bool 
 {
     return row_layout(0, S, 0, nA, tp, with_long).bytes;
 }
-HSMU_HD inline long long num_need(long long S, long long n, long long nA, long long tp, bool with_long)
+
+// ---- one row per workgroup (64 lanes or more): the element stream ------------------------
+//
+// The B rows of a row's A entries are walked as one stream of slots of STREAM_V consecutive
+// elements: entry e owns ceil(nnz(B_j) / STREAM_V) slots, and step s of the stream gives
+// lane i of a wave slot 64 s + i, so every lane works whatever the lengths of the B rows,
+// and each lane's elements come in one load.  (A load instruction costs a CU's L1 8.7
+// cycles for 4 bytes per lane, 17.6 for 8 and 22 for 16, however few of its lanes are
+// active: 29 bytes per cycle for full narrow loads, 46 for 16-byte ones.)  Up to G entries
+// at a time are staged in LDS (start, end, a_ij: 16 bytes each), with a bit per slot that
+// ends an entry and, per 64 slots, the entry of the first: a lane's entry is that number
+// plus the bits below its slot.
+constexpr int STREAM_V = 2;
+// slots whose bits are in LDS at a time, for a row with G lanes
+HSMU_HD constexpr int stream_window(int G) { return G * 32 > 4096 ? G * 32 : 4096; }
+
+// LDS of one row (byte offsets), for a row of C over S tiles with n entries, nA entries in
+// A, tp tile-products and p products:
+//   vals f64[n]     accumulators (64*S of them in the dense form)
+//   dm   u64[E]     tile masks (flat), or coarse words then fine masks (two-level)
+//   rec  16[...]    staged entries: first element less STREAM_V times the first slot, end,
+//                   a_ij; min(nA, G) of them
+//   bits u64[...]   a bit per slot of the window: it ends an entry
+//   doff u32[E]     slot of each tile's first column, coarse offsets (two-level)
+//   ft   u32[R]     two-level: tile of each fine entry, relative to rmin
+//   wb   u16[...]   entry of the first slot of each 64
+struct StreamLayout {
+    int vals, dm, rec, bits, doff, ft, wb, bytes;
+};
+HSMU_HD inline StreamLayout stream_layout(int G, long long S, long long n, long long nA, long long tp, long long p)
 {
-    return row_layout(1, S, n, nA, tp, with_long).bytes;
+    StreamLayout L;
+    const bool sparse = use_sparse(S, tp);
+    const long long E = dir_entries(S, tp);
+    const long long slots = (p + nA * (STREAM_V - 1)) / STREAM_V;
+    const long long win = slots < stream_window(G) ? slots : stream_window(G);
+    const long long words = (win + 63) / 64;
+    const long long cap = 1LL << 30; // rows beyond LDS: any size past it will do
+    auto clip = [&](long long v) { return (int)(v < cap ? v : cap); };
+    long long o = 0;
+    L.vals = 0;
+    o += 8 * (!sparse && use_dense(S, n) ? 64 * S : n);
+    o = (o + 15) & ~15LL;
+    L.dm = clip(o);
+    o += 8 * E;
+    o = (o + 15) & ~15LL;
+    L.rec = clip(o);
+    o += 16 * (nA < G ? nA : G);
+    L.bits = clip(o);
+    o += 8 * words;
+    L.doff = clip(o);
+    o += 4 * E;
+    L.ft = clip(o);
+    if (sparse)
+        o += 4 * fine_cap(S, tp);
+    L.wb = clip(o);
+    o += 2 * words;
+    L.bytes = clip((o + 15) & ~15LL);
+    return L;
+}
+
+// LDS a row with p products needs in numeric bin `bin`
+HSMU_HD inline long long num_need(int bin, long long S, long long n, long long nA, long long tp, long long p,
+                                  bool with_long)
+{
+    return (8 << bin) >= BLOCK ? stream_layout(8 << bin, S, n, nA, tp, p).bytes
+                               : row_layout(1, S, n, nA, tp, with_long).bytes;
 }
 
 // LDS kept back from the dynamic allocation for the kernels' static __shared__ arrays
@@ -242,11 +306,13 @@ struct Operands {
     const void *Aval; // double, or float when val32
     const int *Brp, *Bcol;
     const void *Bval;
+    int nnzB;  // >= STREAM_V (the host pads a smaller B)
     int val32;
     const int *tptr, *tcol;
     const unsigned long long *tmask;
     const int *rmin, *rmax;
     const int *rtp; // tile-products per row (chooses the directory form)
+    const long long *rprod; // products per row
     // Row directories kept between the phases (nullptr when not kept): the symbolic LDS
     // kernel stores row i's directory (flat: tile masks and slot offsets; two-level: the
     // coarse words and compact indices, then the fine masks and slot offsets) at
@@ -347,6 +413,10 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
                           const WideRows &wide,
                           int *err, int num_cus, unsigned *queue, unsigned long long *lds_bytes,
                           hipStream_t s);
+
+// A B of fewer than STREAM_V entries (n of them, at least one), copied to arrays of
+// STREAM_V entries whose last one repeats: the element stream loads STREAM_V at a time.
+hipError_t launch_pad_b(const int *col, const void *val, int val32, int n, int *pcol, void *pval, hipStream_t s);
 
 hipError_t launch_rowptr_i64_to_i32(const long long *in, int64_t n, int *out, hipStream_t s);
 

@@ -540,11 +540,13 @@ hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, c
 
 // Bin of one row: lanes from work (per_lane items per lane, 8..1024 lanes), then fewer
 // rows per workgroup until the workgroup's LDS fits the budget; rows whose own need
-// exceeds lds_row_max go to the global-memory bin.  Reference ranges being replaced:
-// src/bining.cuh:12 (symbolic), :121 (tile OR), :228 (numeric).
-DEVI int choose_bin(long long work, long long need, const BinParams &bp)
+// exceeds lds_row_max go to the global-memory bin.  need(b): the row's LDS in bin b.
+// Reference ranges being replaced: src/bining.cuh:12 (symbolic), :121 (tile OR), :228
+// (numeric).
+template <typename Need>
+DEVI int choose_bin(long long work, Need need, const BinParams &bp)
 {
-    if (bp.force_global || need > bp.lds_row_max)
+    if (bp.force_global)
         return BIN_GLOBAL;
     const long long lanes = (work + bp.per_lane - 1) / bp.per_lane;
     int b = 0;
@@ -554,7 +556,7 @@ DEVI int choose_bin(long long work, long long need, const BinParams &bp)
     // the row's LDS whatever its width
     while (b < NLDS - 1) {
         const int G = 8 << b;
-        if (G >= BLOCK || need * (BLOCK / G) <= bp.lds_block_budget)
+        if (G >= BLOCK || (need(b) * (BLOCK / G) <= bp.lds_block_budget && need(b) <= bp.lds_row_max))
             break;
         ++b;
     }
@@ -562,11 +564,14 @@ DEVI int choose_bin(long long work, long long need, const BinParams &bp)
     // those workgroups hold min_waves waves, to hide the latency of the gathers from B
     while (b < NLDS - 1) {
         const int G = 8 << b;
-        if (G < BLOCK || need <= 0 || (long long)(G / 64) * (bp.lds_cu / need) >= bp.min_waves)
+        const long long nd = need(b);
+        if (G < BLOCK || nd <= 0 || (long long)(G / 64) * (bp.lds_cu / nd) >= bp.min_waves)
             break;
+        if (need(b + 1) > bp.lds_row_max)
+            break; // (the stream's tables grow a little with the width)
         ++b;
     }
-    return b;
+    return need(b) > bp.lds_row_max ? BIN_GLOBAL : b;
 }
 
 // One thread per row; appends are aggregated per workgroup in LDS, then one global
@@ -607,20 +612,23 @@ __global__ __launch_bounds__(BS) void k_bin(int numeric, int64_t M, const int *_
         S = rmax[i] - rmin[i] + 1;
         nA = Arp[i + 1] - Arp[i];
         const int tp = rtp[i];
+        const long long prod = rprod[i];
         if (numeric) {
             nc = rnnz[i];
-            need = num_need(S, nc, nA, tp, with_long);
-            work = rprod[i];
+            work = prod;
+            auto nd = [&](int bin) { return num_need(bin, S, nc, nA, tp, prod, with_long); };
+            b = choose_bin(work, nd, bp);
+            need = nd(b);
         } else {
             need = sym_need(S, nA, tp, with_long);
             work = tp;
+            b = choose_bin(work, [&](int) { return need; }, bp);
         }
-        b = choose_bin(work, need, bp);
         sp = use_sparse(S, tp) ? 1 : 0;
         if (!numeric) {
             // the numeric need with nnz(C_i) <= min(products, 64 * span)
-            const long long nub = rprod[i] < 64LL * S ? rprod[i] : 64LL * S;
-            wide = num_need(S, nub, nA, tp, with_long) > bp.lds_row_max;
+            const long long nub = prod < 64LL * S ? prod : 64LL * S;
+            wide = num_need(NLDS - 1, S, nub, nA, tp, prod, with_long) > bp.lds_row_max;
         }
         // directory entries kept for the numeric phase: the row's form in an LDS bin, the
         // flat span for rows the symbolic phase handles in global memory
@@ -744,6 +752,25 @@ hipError_t launch_rowptr_i64_to_i32(const long long *in, int64_t n, int *out, hi
     if (blocks < 1)
         blocks = 1;
     hipLaunchKernelGGL(k_i64_to_i32, dim3((unsigned)blocks), dim3(256), 0, s, in, n, out);
+    return hipGetLastError();
+}
+
+__global__ void k_pad_b(const int *col, const void *val, int val32, int n, int *pcol, void *pval)
+{
+    const int t = threadIdx.x;
+    if (t >= STREAM_V)
+        return;
+    const int q = t < n ? t : n - 1;
+    pcol[t] = col[q];
+    if (val32)
+        ((float *)pval)[t] = ((const float *)val)[q];
+    else
+        ((double *)pval)[t] = ((const double *)val)[q];
+}
+
+hipError_t launch_pad_b(const int *col, const void *val, int val32, int n, int *pcol, void *pval, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_pad_b, dim3(1), dim3(64), 0, s, col, val, val32, n, pcol, pval);
     return hipGetLastError();
 }
 

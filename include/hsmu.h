@@ -118,8 +118,9 @@ typedef struct hsmu_opts {
     int32_t timing;           /* hipEvents into hsmu_stats (each costs the device a few us):
                                  1 = per stage and per numeric bin (the default), 2 = per
                                  numeric bin only, 0 = none (stage and bin times read 0) */
-    int32_t b_lanes;          /* lanes that walk one row of B in the numeric phase (power of
-                                 two, 1..64); 0 = a quarter of the mean row length of B */
+    int32_t b_lanes;          /* lanes that walk one row of B in the numeric phase, for rows that
+                                 share a workgroup (power of two, 1..64); 0 = a quarter of the
+                                 mean row length of B */
     int32_t t_lanes;          /* lanes that walk one row of B's tiles in the tile OR (power
                                  of two, 1..64); 0 = from the mean tiles per row of B */
     int32_t rebuild_dirs;     /* 1: the numeric phase rebuilds each row's tile directory
