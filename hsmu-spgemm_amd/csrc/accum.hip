@@ -39,6 +39,9 @@ namespace hsmu {
 // it per device; each device holds its own copy).
 static __constant__ int c_nxcd = MAX_XCDS;
 
+// The one error these kernels raise; err may be host memory, hence a store.
+DEVI void raise_internal(int *err) { __hip_atomic_store(err, ERR_INTERNAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+
 // Stage the row's A entries a0 .. a0+nA-1 into LDS: first tile and tile count of B_j,
 // and (numeric) first element and length of B_j and a_ij.  One parallel step per row,
 // so the dependent loads Acol -> tptr/Brp are paid once per row rather than once per
@@ -922,7 +925,7 @@ __global__ __launch_bounds__(BLOCK) void k_numeric_lds(const int *__restrict__ r
         }
         const bool ok = (int)nnz == n;
         if (row >= 0 && !ok && l == 0)
-            atomicOr(err, ERR_INTERNAL);
+            raise_internal(err);
         __syncthreads();
         if (row >= 0 && ok) {
             const int nlong = LONG ? *lcnt : 0;
@@ -1092,7 +1095,7 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
         }
         const bool ok = (int)nnz == n;
         if (!ok && l == 0)
-            atomicOr(err, ERR_INTERNAL);
+            raise_internal(err);
         __syncthreads();
         if (ok) { // uniform
             auto rows_of = [&](int e) {
@@ -1370,7 +1373,7 @@ __global__ __launch_bounds__(1024) void k_numeric_window(const int *__restrict__
             __syncthreads();
         }
         if (l == 0 && written != n)
-            atomicOr(err, ERR_INTERNAL);
+            raise_internal(err);
         block_sync_global(); // workspace of the next row
     }
 }
@@ -1536,7 +1539,7 @@ __global__ __launch_bounds__(1024) void k_numeric_wcompact(const int *__restrict
             __syncthreads();
         }
         if (l == 0 && done != n)
-            atomicOr(err, ERR_INTERNAL);
+            raise_internal(err);
         block_sync_global(); // workspace of the next row
     }
 }
@@ -1629,7 +1632,7 @@ __global__ __launch_bounds__(256) void k_wide_fill(const int *__restrict__ rows,
         return;
     const unsigned base = lb[cls] + local;
     if ((long long)base + ns > cap) { // cannot happen: cap bounds count + nnz(A) / WS_MIN_SPLIT
-        atomicOr(err, ERR_INTERNAL);
+        raise_internal(err);
         return;
     }
     // a split row's range of the compensated scratch (sctr: nullptr for FP64)
@@ -1638,7 +1641,7 @@ __global__ __launch_bounds__(256) void k_wide_fill(const int *__restrict__ rows,
         const long long n = crp[row + 1] - crp[row];
         sbase = (long long)atomicAdd(sctr, (unsigned long long)n);
         if (sbase + n > scratch_n) { // cannot happen: scratch_n sums these rows' nnz
-            atomicOr(err, ERR_INTERNAL);
+            raise_internal(err);
             return;
         }
     }
@@ -2172,7 +2175,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu((ws_waves<VW
             __syncthreads();
         }
         if (l == 0 && done != n)
-            atomicOr(err, ERR_INTERNAL);
+            raise_internal(err);
         block_sync_global(); // ft and the LDS state of the next item
     }
 }

@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
@@ -170,11 +171,18 @@ int ilog2(int v)
 
 enum { EV_START, EV_CONV, EV_ANALYSIS, EV_SYMBOLIC, EV_ALLOC, EV_NUMERIC, EV_COUNT };
 
+// Pinned host memory the device writes: the counters of the last checkpoint, and the
+// numeric kernels' error word.
+struct HostBlock {
+    DevStats st;
+    int err;
+};
+
 struct hsmu_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     Pool pool;
-    DevStats *host_stats = nullptr; // pinned
+    HostBlock *host = nullptr; // pinned; the device writes its counters there
     hipEvent_t ev[EV_COUNT] = {};
     hipEvent_t evb[NBINS][2] = {};
     int num_cus = 0;
@@ -237,7 +245,7 @@ int hsmu_ctx_create(int device, hsmu_ctx **out)
     }
     // every failure from here on releases what was already created
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess &&
-              hipHostMalloc((void **)&c->host_stats, sizeof(DevStats), hipHostMallocDefault) == hipSuccess;
+              hipHostMalloc((void **)&c->host, sizeof(HostBlock), hipHostMallocDefault) == hipSuccess;
     for (int i = 0; ok && i < EV_COUNT; ++i)
         ok = hipEventCreate(&c->ev[i]) == hipSuccess;
     for (int b = 0; ok && b < NBINS; ++b)
@@ -289,8 +297,8 @@ void hsmu_ctx_destroy(hsmu_ctx *c)
         for (int k = 0; k < 2; ++k)
             if (c->evb[b][k])
                 (void)hipEventDestroy(c->evb[b][k]);
-    if (c->host_stats)
-        (void)hipHostFree(c->host_stats);
+    if (c->host)
+        (void)hipHostFree(c->host);
     if (c->stream)
         (void)hipStreamDestroy(c->stream);
     delete c;
@@ -382,6 +390,14 @@ int hsmu_copy_kernel(hsmu_ctx *c, void *dst, const void *src, size_t bytes, doub
 
 namespace {
 
+// Device memory of one call's zeroed counters, with the chained scans' words behind them.
+size_t dev_work_bytes(int64_t nnzB, int64_t M)
+{
+    return sizeof(DevWork) + (size_t)(btiles_blocks(nnzB) + rowptr_blocks(M)) * sizeof(unsigned long long);
+}
+unsigned long long *chain_words(DevWork *dw) { return (unsigned long long *)(dw + 1); }
+static_assert(sizeof(DevWork) % 8 == 0, "the scans' words follow the counters");
+
 int check_input(const hsmu_csr *X, const char *name, bool want_val32)
 {
     if (!X)
@@ -463,25 +479,24 @@ extern "C" int hsmu_btiles(hsmu_ctx *c, const hsmu_csr *B, hsmu_tiles *T)
     memset(T, 0, sizeof(*T));
     const int64_t K = B->M;
     Scratch ws(c->pool);
-    int *tcnt = (int *)ws.get<char>(btiles_ws_bytes(B->nnz));
-    void *scan_ws = ws.get<char>(scan_ws_bytes(B->nnz + 1));
-    DevStats *dst = ws.get<DevStats>(1);
+    const size_t work_bytes = dev_work_bytes(B->nnz, 0);
+    DevWork *dw = (DevWork *)ws.get<char>(work_bytes);
     int *tptr = (int *)c->pool.alloc(((size_t)K + 1) * sizeof(int));
     int *tcol = (int *)c->pool.alloc((size_t)(B->nnz > 0 ? B->nnz : 1) * sizeof(int));
     unsigned long long *tmask =
         (unsigned long long *)c->pool.alloc((size_t)(B->nnz > 0 ? B->nnz : 1) * sizeof(unsigned long long));
-    if (!tcnt || !scan_ws || !dst || !tptr || !tcol || !tmask) {
+    if (!dw || !tptr || !tcol || !tmask) {
         c->pool.release(tptr);
         c->pool.release(tcol);
         c->pool.release(tmask);
         return fail(HSMU_ERR_NOMEM, "hsmu_btiles: workspace");
     }
-    HIP_TRY(launch_fill_zero(dst, sizeof(DevStats), c->stream));
-    HIP_TRY(launch_btiles(K, B->N, B->nnz, (const int *)B->rowptr, B->col, tcnt, tptr, tcol, tmask, nullptr, scan_ws, dst,
-                          c->num_cus, c->stream));
-    HIP_TRY(hipMemcpyAsync(c->host_stats, dst, sizeof(DevStats), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(launch_fill_zero(dw, work_bytes, c->stream));
+    HIP_TRY(launch_btiles(K, B->N, B->nnz, (const int *)B->rowptr, B->col, tptr, tcol, tmask, nullptr, chain_words(dw),
+                          &dw->ticket[0], &dw->st, c->stream));
+    HIP_TRY(hipMemcpyAsync(&c->host->st, &dw->st, sizeof(DevStats), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    rc = device_error_status(c->host_stats->err);
+    rc = device_error_status(c->host->st.err);
     if (rc) {
         c->pool.release(tptr);
         c->pool.release(tcol);
@@ -489,7 +504,7 @@ extern "C" int hsmu_btiles(hsmu_ctx *c, const hsmu_csr *B, hsmu_tiles *T)
         return rc;
     }
     T->M = K;
-    T->ntiles = c->host_stats->ntiles_b;
+    T->ntiles = c->host->st.ntiles_b;
     T->tptr = tptr;
     T->tcol = tcol;
     T->tmask = (uint64_t *)tmask;
@@ -630,8 +645,9 @@ class Arena {
     int64_t want_nnz_ = 0;
 };
 
-// How a pipeline run meets its two checkpoints: eagerly (copy the device counters to
-// the host and synchronise; a plan's recording run keeps them), or, while a plan is
+// How a pipeline run meets its two checkpoints: eagerly (synchronise; the binning kernels
+// have written the device counters to pinned host memory; a plan's recording run keeps
+// them), or, while a plan is
 // being captured, with no synchronisation at all: the recorded counters stand in for the
 // device's, and a check kernel compares the two when the graph is replayed.
 struct RunMode {
@@ -647,9 +663,8 @@ int checkpoint(hsmu_ctx *c, const RunMode &m, DevStats *dst, int k, DevStats &ou
         out = m.plan->rec[k];
         return HSMU_OK;
     }
-    HIP_TRY(hipMemcpyAsync(c->host_stats, dst, sizeof(DevStats), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    out = *c->host_stats;
+    HIP_TRY(hipStreamSynchronize(s)); // the last kernel has written the counters to the host
+    out = c->host->st;
     if (m.plan)
         m.plan->rec[k] = out;
     return device_error_status(out.err);
@@ -680,9 +695,9 @@ struct Output {
     void *val = nullptr;
 };
 
-// B -> tiles, row analysis, symbolic, C allocation, numeric.  *dst must be zeroed on the
-// stream before the call (the batch stacking kernels report into it first).
-int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, const RunMode &mode, DevStats *dst,
+// B -> tiles, row analysis, symbolic, C allocation, numeric.  *dw (dev_work_bytes) must be
+// zeroed on the stream before the call (the batch stacking kernels report into it first).
+int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, const RunMode &mode, DevWork *dw,
              BatchSplit *batch, Output &res, hsmu_stats *stats)
 {
     const bool fp32 = opts.precision == HSMU_FP32_COMP;
@@ -698,15 +713,13 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     const bool stage_timing = opts.timing == 1 && !cap;
     auto mark = [&](hipEvent_t e) -> hipError_t { return stage_timing ? hipEventRecord(e, s) : hipSuccess; };
     int rc;
+    DevStats *dst = &dw->st;
+    DevStats *host = cap ? nullptr : &c->host->st;
 
-    int *tcnt = (int *)ar.get<char>(btiles_ws_bytes(P.nnzB));
     int *tptr = ar.get<int>((size_t)K + 1);
     const size_t ntcap = P.nnzB > STREAM_V ? (size_t)P.nnzB : STREAM_V; // loaded STREAM_V at a time
     int *tcol = ar.get<int>(ntcap);
     unsigned long long *tmask = ar.get<unsigned long long>(ntcap);
-    int64_t nmax = M > K ? M : K;
-    nmax = nmax > P.nnzB ? nmax : P.nnzB;
-    void *scan_ws = ar.get<char>(scan_ws_bytes(nmax + 1));
     long long *rprod = ar.get<long long>((size_t)M);
     int *rtp = ar.get<int>((size_t)M);
     int *rmin = ar.get<int>((size_t)M);
@@ -715,19 +728,18 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     int *binrows = ar.get<int>((size_t)NBINS * (size_t)M);
     long long *rdir = ar.get<long long>((size_t)M);
     BRow *brow = ar.get<BRow>((size_t)(K > 0 ? K : 1));
-    if (!tcnt || !tptr || !tcol || !tmask || !scan_ws || !rprod || !rtp || !rmin || !rmax || !rnnz || !binrows || !rdir ||
+    const int64_t nsums = std::max(row_info_blocks(M, P.nnzA, c->num_cus), rowptr_blocks(M));
+    BinSum *sums = ar.get<BinSum>((size_t)nsums * NBINS);
+    if (!sums || !tptr || !tcol || !tmask || !rprod || !rtp || !rmin || !rmax || !rnnz || !binrows || !rdir ||
         !brow)
         return fail(HSMU_ERR_NOMEM, "workspace allocation");
 
     // ---- 1. B -> tiles ----
-    HIP_TRY(launch_btiles(K, N, P.nnzB, P.Brp, P.Bcol, tcnt, tptr, tcol, tmask, brow, scan_ws, dst, c->num_cus, s));
+    unsigned long long *words = chain_words(dw);
+    HIP_TRY(launch_btiles(K, N, P.nnzB, P.Brp, P.Bcol, tptr, tcol, tmask, brow, words, &dw->ticket[0], dst, s));
     HIP_TRY(mark(c->ev[EV_CONV]));
 
     // ---- 2. row analysis + symbolic binning ----
-    const int avg_a = (int)(P.nnzA / (M > 0 ? M : 1));
-    // the spare bin region (bin 9) holds the list of long rows until binning runs
-    HIP_TRY(launch_row_info(M, K, P.nnzA, P.Arp, P.Acol, brow, rprod, rtp, rmin, rmax, rnnz,
-                            binrows + (size_t)(NBINS - 1) * M, dst, avg_a, c->num_cus, s));
     BinParams bp;
     const int lds_dyn = c->lds_max - LDS_STATIC_RESERVE;
     bp.lds_row_max = opts.lds_row_max > 0 ? opts.lds_row_max : lds_dyn;
@@ -744,7 +756,8 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     bp.force_global = opts.force_global;
     bp.lds_cu = lds_dyn;
     bp.min_waves = opts.min_waves > 0 ? opts.min_waves : 8;
-    HIP_TRY(launch_bin(0, M, P.Arp, rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, dst, c->num_cus, s));
+    HIP_TRY(launch_row_info(M, K, P.nnzA, P.Arp, P.Acol, brow, tptr, rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, dst,
+                            sums, &dw->done[0], host, c->num_cus, s));
     HIP_TRY(mark(c->ev[EV_ANALYSIS]));
     DevStats h1;
     rc = checkpoint(c, mode, dst, 0, h1);
@@ -876,9 +889,19 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     }
     if (!crp)
         return fail(HSMU_ERR_NOMEM, "C row pointers");
-    HIP_TRY(launch_scan_i32_i64(rnnz, M, crp, scan_ws, &dst->nnz_c, s));
+    // C's int32 row pointers, when they are the caller's (a batch splits them afterwards)
+    void *Crp = nullptr;
+    if (rp64 && !batch) {
+        Crp = crp;
+    } else if (!batch) {
+        Crp = ar.out(((size_t)M + 1) * sizeof(int), plain, OUT_ROWPTR);
+        if (!Crp)
+            return fail(HSMU_ERR_NOMEM, "C row pointers");
+        outs.p.push_back(Crp);
+    }
     bp.per_lane = opts.products_per_lane > 0 ? opts.products_per_lane : 32;
-    HIP_TRY(launch_bin(1, M, P.Arp, rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, dst, c->num_cus, s));
+    HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp, rp64 || batch ? nullptr : (int *)Crp, bp,
+                              binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, sums, &dw->done[1], host, s));
     HIP_TRY(mark(c->ev[EV_SYMBOLIC]));
     DevStats h2;
     rc = checkpoint(c, mode, dst, 1, h2);
@@ -894,18 +917,12 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     outs.p.push_back(Ccol);
     void *Cval = ar.out((size_t)nnzc * (size_t)vsz, plain, OUT_VAL);
     outs.p.push_back(Cval);
-    void *Crp;
     long long *bases = nullptr;
     if (batch) {
         Crp = ar.out((size_t)(M + batch->count) * (rp64 ? 8 : 4), plain, OUT_ROWPTR);
         outs.p.push_back(Crp);
         bases = ar.get<long long>((size_t)batch->count + 1);
         batch->bases_dev = bases;
-    } else if (rp64) {
-        Crp = crp;
-    } else {
-        Crp = ar.out(((size_t)M + 1) * sizeof(int), plain, OUT_ROWPTR);
-        outs.p.push_back(Crp);
     }
     if (!Ccol || !Cval || !Crp || (batch && !bases))
         return fail(HSMU_ERR_NOMEM, "allocating C (nnz %lld)", nnzc);
@@ -914,7 +931,9 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     HIP_TRY(mark(c->ev[EV_ALLOC]));
 
     // ---- 5. numeric ----
-    int *errp = &dst->err;
+    if (!cap)
+        c->host->err = 0;
+    int *errp = cap ? &dst->err : &c->host->err;
     unsigned long long lds_launched = 0;
     for (int b = 0; b < NBINS; ++b) {
         const int cnt = h2.num.count[b];
@@ -971,18 +990,15 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     }
     if (batch)
         HIP_TRY(launch_batch_split(batch->count, batch->off, crp, Crp, rp64 ? 1 : 0, bases, M + batch->count, s));
-    else if (!rp64)
-        HIP_TRY(launch_rowptr_i64_to_i32(crp, M + 1, (int *)Crp, s));
     HIP_TRY(mark(c->ev[EV_NUMERIC]));
     if (!cap) {
-        HIP_TRY(hipMemcpyAsync(&c->host_stats->err, errp, sizeof(int), hipMemcpyDeviceToHost, s));
         if (batch) {
             batch->bases->assign((size_t)batch->count + 1, 0);
             HIP_TRY(hipMemcpyAsync(batch->bases->data(), bases, ((size_t)batch->count + 1) * sizeof(long long),
                                    hipMemcpyDeviceToHost, s));
         }
         HIP_TRY(hipStreamSynchronize(s));
-        rc = device_error_status(c->host_stats->err);
+        rc = device_error_status(*(volatile int *)&c->host->err);
         if (rc)
             return rc;
     }
@@ -1284,11 +1300,12 @@ int run_batch(hsmu_ctx *c, int64_t count, const hsmu_csr *A, const hsmu_csr *B, 
         }
         return HSMU_OK;
     }
-    DevStats *dst = ar.get<DevStats>(1);
-    if (!dst)
+    const size_t work_bytes = dev_work_bytes(nnzB, M);
+    DevWork *dw = (DevWork *)ar.raw(work_bytes);
+    if (!dw)
         return fail(HSMU_ERR_NOMEM, "workspace allocation");
     if (mode.plan && !mode.capture) {
-        mode.plan->dst = dst;
+        mode.plan->dst = &dw->st;
         mode.plan->expect = ar.get<DevStats>(2);
         if (!mode.plan->expect)
             return fail(HSMU_ERR_NOMEM, "workspace allocation");
@@ -1297,10 +1314,10 @@ int run_batch(hsmu_ctx *c, int64_t count, const hsmu_csr *A, const hsmu_csr *B, 
     }
     if (!mode.capture && opts.timing == 1)
         HIP_TRY(hipEventRecord(c->ev[EV_START], s));
-    HIP_TRY(launch_fill_zero(dst, sizeof(DevStats), s));
+    HIP_TRY(launch_fill_zero(dw, work_bytes, s));
     Output r;
     if (count == 1) {
-        rc = pipeline(c, single_problem(A, B), opts, ar, mode, dst, nullptr, r, stats);
+        rc = pipeline(c, single_problem(A, B), opts, ar, mode, dw, nullptr, r, stats);
         if (rc)
             return rc;
         if (!mode.capture)
@@ -1312,10 +1329,10 @@ int run_batch(hsmu_ctx *c, int64_t count, const hsmu_csr *A, const hsmu_csr *B, 
     std::vector<long long> bases;
     split.count = count;
     split.bases = &bases;
-    rc = stack_inputs(c, bp, opts, ar, mode, dst, P, split.off);
+    rc = stack_inputs(c, bp, opts, ar, mode, &dw->st, P, split.off);
     if (rc)
         return rc;
-    rc = pipeline(c, P, opts, ar, mode, dst, &split, r, stats);
+    rc = pipeline(c, P, opts, ar, mode, dw, &split, r, stats);
     if (rc)
         return rc;
     if (mode.plan) {
@@ -1324,7 +1341,7 @@ int run_batch(hsmu_ctx *c, int64_t count, const hsmu_csr *A, const hsmu_csr *B, 
         if (!want)
             return fail(HSMU_ERR_NOMEM, "plan workspace");
         if (mode.capture) {
-            HIP_TRY(launch_plan_bases(split.bases_dev, want, count + 1, dst, s));
+            HIP_TRY(launch_plan_bases(split.bases_dev, want, count + 1, &dw->st, s));
         } else {
             HIP_TRY(hipMemcpyAsync(want, bases.data(), bases.size() * sizeof(long long), hipMemcpyHostToDevice, s));
             HIP_TRY(hipStreamSynchronize(s));
@@ -1623,9 +1640,9 @@ extern "C" int hsmu_plan_execute(hsmu_plan *p, hsmu_stats *stats)
     HIP_TRY(hipEventRecord(c->ev[EV_START], s));
     HIP_TRY(hipGraphLaunch(p->exec, s));
     HIP_TRY(hipEventRecord(c->ev[EV_NUMERIC], s));
-    HIP_TRY(hipMemcpyAsync(&c->host_stats->err, &p->dst->err, sizeof(int), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(&c->host->err, &p->dst->err, sizeof(int), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    const int err = c->host_stats->err;
+    const int err = c->host->err;
     if (err & ERR_PLAN)
         return fail(HSMU_ERR_PLAN, "the plan's inputs changed structure since it was made");
     int rc = device_error_status(err);

@@ -39,35 +39,62 @@ DEVI u64 readlane_u64(u64 v, int k)
     return ((u64)hi << 32) | lo;
 }
 
-// Reductions and scans over the 64 lanes of a wave (every lane must take part).
-template <typename T> DEVI T wave_sum(T v)
+// One step of a scan over the wave: the value of the lane the DPP control names, or `none`
+// where it names no lane (or the row mask leaves the row out).
+template <int CTRL, int ROWS> DEVI unsigned dpp_step(unsigned none, unsigned v)
+{
+    return (unsigned)__builtin_amdgcn_update_dpp((int)none, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS> DEVI int dpp_step(int none, int v)
+{
+    return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS> DEVI u64 dpp_step(u64 none, u64 v)
+{
+    const unsigned lo = dpp_step<CTRL, ROWS>((unsigned)none, (unsigned)v);
+    const unsigned hi = dpp_step<CTRL, ROWS>((unsigned)(none >> 32), (unsigned)(v >> 32));
+    return ((u64)hi << 32) | lo;
+}
+template <int CTRL, int ROWS> DEVI long long dpp_step(long long none, long long v)
+{
+    return (long long)dpp_step<CTRL, ROWS>((u64)none, (u64)v);
+}
+
+// Inclusive scan over the 64 lanes (every lane must take part) with DPP moves: within rows
+// of 16 lanes by 1, 2, 4, 8, then across rows.  No LDS round trip, unlike shuffles.
+template <typename T, typename Op> DEVI T wave_incl_scan(T v, T none, Op op)
+{
+    v = op(v, dpp_step<0x111, 0xf>(none, v)); // row_shr:1
+    v = op(v, dpp_step<0x112, 0xf>(none, v));
+    v = op(v, dpp_step<0x114, 0xf>(none, v));
+    v = op(v, dpp_step<0x118, 0xf>(none, v));
+    v = op(v, dpp_step<0x142, 0xa>(none, v)); // row_bcast:15
+    v = op(v, dpp_step<0x143, 0xc>(none, v)); // row_bcast:31
+    return v;
+}
+template <typename T> DEVI T wave_incl_scan(T v)
+{
+    return wave_incl_scan(v, (T)0, [](T a, T b) { return a + b; });
+}
+
+DEVI unsigned wave_last(unsigned v) { return (unsigned)__builtin_amdgcn_readlane((int)v, 63); }
+DEVI int wave_last(int v) { return __builtin_amdgcn_readlane(v, 63); }
+DEVI u64 wave_last(u64 v) { return readlane_u64(v, 63); }
+DEVI long long wave_last(long long v) { return (long long)readlane_u64((u64)v, 63); }
+
+// Reductions over the 64 lanes (every lane must take part), the same in every lane.
+template <typename T> DEVI T wave_sum(T v) { return wave_last(wave_incl_scan(v)); }
+DEVI double wave_sum(double v)
 {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1)
         v += __shfl_xor(v, o, 64);
     return v;
 }
-
-template <typename T> DEVI T wave_max(T v)
+// of values that are not negative
+DEVI int wave_max(int v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const T u = __shfl_xor(v, o, 64);
-        v = u > v ? u : v;
-    }
-    return v;
-}
-
-template <typename T> DEVI T wave_incl_scan(T v)
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const T u = __shfl_up(v, o, 64);
-        if (lane >= o)
-            v += u;
-    }
-    return v;
+    return wave_last(wave_incl_scan(v, 0, [](int a, int b) { return a > b ? a : b; }));
 }
 
 // Map the hardware block index so that each XCD (blocks are dealt round-robin over the
@@ -150,53 +177,37 @@ struct GroupWalk {
     }
 };
 
-// Sum over a group of G consecutive lanes.  G <= 64: shuffles; G > 64: through LDS
-// (every thread of the block must call it).
-template <int G, typename T> DEVI T group_sum(T v, T *red)
+// Reduction over a group of G <= 64 consecutive lanes, the same in every lane: with DPP
+// moves up to 16 lanes (quad permutes, then the mirrors of half a row and of a row), which
+// need no LDS; two shuffles at most beyond.
+template <int G, typename T, typename Op> DEVI T group_reduce(T v, Op op)
 {
-    if constexpr (G <= 64) {
-#pragma unroll
-        for (int o = G / 2; o > 0; o >>= 1)
-            v += __shfl_xor(v, o, G);
-        return v;
-    } else {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1)
-            v += __shfl_xor(v, o, 64);
-        const int w = threadIdx.x >> 6;
-        __syncthreads();
-        if ((threadIdx.x & 63) == 0)
-            red[w] = v;
-        __syncthreads();
-        const int w0 = (threadIdx.x / G) * (G / 64);
-        T s = 0;
-#pragma unroll
-        for (int k = 0; k < G / 64; ++k)
-            s += red[w0 + k];
-        return s;
-    }
+    static_assert(G <= 64 && sizeof(T) <= 8, "a wave operation");
+    if constexpr (G >= 2)
+        v = op(v, dpp_step<0xB1, 0xf>(v, v)); // quad_perm:[1,0,3,2]
+    if constexpr (G >= 4)
+        v = op(v, dpp_step<0x4E, 0xf>(v, v)); // quad_perm:[2,3,0,1]
+    if constexpr (G >= 8)
+        v = op(v, dpp_step<0x141, 0xf>(v, v)); // row_half_mirror
+    if constexpr (G >= 16)
+        v = op(v, dpp_step<0x140, 0xf>(v, v)); // row_mirror
+    if constexpr (G >= 32)
+        v = op(v, __shfl_xor(v, 16, 64));
+    if constexpr (G >= 64)
+        v = op(v, __shfl_xor(v, 32, 64));
+    return v;
 }
-
+template <int G, typename T> DEVI T group_sum(T v)
+{
+    return group_reduce<G>(v, [](T a, T b) { return a + b; });
+}
 template <int G, typename T> DEVI T group_min(T v)
 {
-    static_assert(G <= 64, "group_min is a wave operation");
-#pragma unroll
-    for (int o = G / 2; o > 0; o >>= 1) {
-        T y = __shfl_xor(v, o, G);
-        v = y < v ? y : v;
-    }
-    return v;
+    return group_reduce<G>(v, [](T a, T b) { return a < b ? a : b; });
 }
-
 template <int G, typename T> DEVI T group_max(T v)
 {
-    static_assert(G <= 64, "group_max is a wave operation");
-#pragma unroll
-    for (int o = G / 2; o > 0; o >>= 1) {
-        T y = __shfl_xor(v, o, G);
-        v = y > v ? y : v;
-    }
-    return v;
+    return group_reduce<G>(v, [](T a, T b) { return a > b ? a : b; });
 }
 
 // Exclusive scan over a group of G lanes; total = group sum.  G > 64 goes through LDS
@@ -206,14 +217,31 @@ template <int G, typename T> DEVI T group_excl_scan(T v, T *red, T &total)
     constexpr int W = G < 64 ? G : 64;
     const int l = threadIdx.x & (W - 1);
     T x = v;
-#pragma unroll
-    for (int o = 1; o < W; o <<= 1) {
-        T y = __shfl_up(x, o, W);
-        if (l >= o)
-            x += y;
+    if constexpr (G >= 64) {
+        x = wave_incl_scan(v);
+    } else { // (a shift within a row of 16 lanes also moves values between its groups)
+        T y = dpp_step<0x111, 0xf>((T)0, x);
+        x += l >= 1 ? y : (T)0;
+        if constexpr (G >= 4) {
+            y = dpp_step<0x112, 0xf>((T)0, x);
+            x += l >= 2 ? y : (T)0;
+        }
+        if constexpr (G >= 8) {
+            y = dpp_step<0x114, 0xf>((T)0, x);
+            x += l >= 4 ? y : (T)0;
+        }
+        if constexpr (G >= 16) {
+            y = dpp_step<0x118, 0xf>((T)0, x);
+            x += l >= 8 ? y : (T)0;
+        }
+        if constexpr (G >= 32)
+            x += dpp_step<0x142, 0xa>((T)0, x); // row_bcast:15
     }
-    if constexpr (G <= 64) {
-        total = __shfl(x, W - 1, W);
+    if constexpr (G == 64) {
+        total = wave_last(x);
+        return x - v;
+    } else if constexpr (G < 64) {
+        total = group_sum<G>(v);
         return x - v;
     } else {
         const int w = threadIdx.x >> 6;

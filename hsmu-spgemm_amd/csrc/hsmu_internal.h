@@ -32,10 +32,10 @@ constexpr int ERR_INTERNAL = 16;// symbolic and numeric counts disagree (a bug)
 constexpr int ERR_PLAN = 32;    // a replayed plan's inputs changed structure
 
 struct BinParams {
-    long long lds_block_budget; // LDS bytes per workgroup for bins with several rows per workgroup
-    long long lds_row_max;      // LDS bytes one row may use
-    long long per_lane;         // work items per lane
-    long long lds_cu;           // LDS bytes of a CU
+    int lds_block_budget; // LDS bytes per workgroup for bins with several rows per workgroup
+    int lds_row_max;      // LDS bytes one row may use
+    int per_lane;         // work items per lane
+    int lds_cu;           // LDS bytes of a CU
     int force_global;
     int min_waves;              // waves per CU a one-row workgroup's width should reach
 };
@@ -63,7 +63,7 @@ struct DevStats {
     long long nnz_c;
     int err;
     int ntiles_b;
-    int nlong; // rows of A set aside for the one-workgroup-per-row analysis
+    int pad;
     int max_brow; // longest row of B (counted from LONG_TILES on)
     unsigned long long num_wide_hint; // rows whose numeric need may exceed LDS (symbolic binning)
     unsigned long long wide_split_nnz; // nnz(C_i) summed over the wide rows split into several items
@@ -72,6 +72,21 @@ struct DevStats {
     BinStats num;
     // work-queue counters of the persistent LDS kernels: [phase][bin][XCD]
     unsigned queue[2][NBINS][MAX_XCDS];
+};
+
+// One block's part of a binning's sums and maxima, for one bin.
+struct BinSum {
+    unsigned long long work, nnz_c, nnz_a;
+    unsigned long long need_span; // max_need | max_span << 32
+    unsigned long long na_sparse; // max_na | nsparse << 32
+};
+
+// Everything on the device that a call needs zeroed: the counters, the blocks done and the
+// places taken of each binning or scan, and (behind it) the words of the two chained scans.
+struct DevWork {
+    DevStats st;
+    unsigned done[2], ticket[2];
+    // followed by btiles_blocks(nnz(B)) + rowptr_blocks(M) 64-bit words
 };
 
 // Batched form: instance i of a batch, as seen by the stacking kernels.  The stacked A
@@ -103,7 +118,7 @@ struct BatchOffsets {
 // one slot per column of the row's span, column c in slot c - 64*rmin, used when the
 // span is at least two-thirds full (then the dense array costs at most 1.5x the compact
 // one and saves the two directory reads per product) and at most 128 tiles wide.
-HSMU_HD inline bool use_dense(long long S, long long n) { return S <= 128 && 2 * 64 * S <= 3 * n; }
+HSMU_HD inline bool use_dense(int S, int n) { return S <= 128 && 2 * 64 * S <= 3 * n; }
 
 // Tile directory of a row of C over its span [rmin, rmax] of S tiles.
 // Flat: one entry (mask, first slot) per tile of the span, tile t at index t.
@@ -114,16 +129,16 @@ HSMU_HD inline bool use_dense(long long S, long long n) { return S <= 128 && 2 *
 // below(t&63)) -- the HSMU rank trick applied to tiles as well as to columns, so a slot
 // is still found in O(1).  At most R = min(S, tile-products) fine entries.  Chosen when
 // it at least halves the directory (never for spans of up to 64 tiles).
-HSMU_HD inline long long fine_cap(long long S, long long tp) { return tp < S ? tp : S; }
-HSMU_HD inline bool use_sparse(long long S, long long tp)
-{
-    return S > 64 && 2 * ((S + 63) / 64 + fine_cap(S, tp)) <= S;
-}
+// (S is at most 2^25, so 32 bits hold all of this.)
+HSMU_HD inline int fine_cap(int S, int tp) { return tp < S ? tp : S; }
+HSMU_HD inline bool use_sparse(int S, int tp) { return S > 64 && 2 * (((S + 63) >> 6) + fine_cap(S, tp)) <= S; }
 // directory entries of a row (12 bytes each when kept between the phases)
-HSMU_HD inline long long dir_entries(long long S, long long tp)
-{
-    return use_sparse(S, tp) ? (S + 63) / 64 + fine_cap(S, tp) : S;
-}
+HSMU_HD inline int dir_entries(int S, int tp) { return use_sparse(S, tp) ? ((S + 63) >> 6) + fine_cap(S, tp) : S; }
+
+// Sizes a row in LDS cannot have: layouts of larger rows are not worked out (32 bits) but
+// given this many bytes.
+constexpr int LAYOUT_CAP = 1 << 18;
+constexpr int LAYOUT_NONE = 1 << 30;
 
 // LDS slice of one row in the LDS kernels (byte offsets), for a row whose C row spans
 // S tiles, has n = nnz(C_i) entries, nA entries in A and tp tile-products; E =
@@ -142,7 +157,7 @@ HSMU_HD inline long long dir_entries(long long S, long long tp)
 //   lcnt i32        with_long: their number (16 bytes reserved)
 // The size is rounded up to 16 bytes so per-row slices of a workgroup stay aligned.
 struct RowLayout {
-    long long dm, doff, ft, vals, av, tlen, t0, blen, b0, lidx, lcnt, bytes;
+    int dm, doff, ft, vals, av, tlen, t0, blen, b0, lidx, lcnt, bytes;
 };
 
 // Rows of B at least this long (LONG_TILES for the tile OR) are walked by a whole wave:
@@ -150,12 +165,16 @@ struct RowLayout {
 constexpr int LONG_SEG = 256;
 constexpr int LONG_TILES = 128;
 
-HSMU_HD inline RowLayout row_layout(int numeric, long long S, long long n, long long nA, long long tp, bool with_long)
+HSMU_HD inline RowLayout row_layout(int numeric, int S, int n, int nA, int tp, bool with_long)
 {
-    RowLayout L;
+    RowLayout L = {};
     const bool sparse = use_sparse(S, tp);
-    const long long E = dir_entries(S, tp);
-    long long o = 0;
+    const int E = dir_entries(S, tp);
+    if (E > LAYOUT_CAP || n > LAYOUT_CAP || nA > LAYOUT_CAP) {
+        L.bytes = LAYOUT_NONE;
+        return L;
+    }
+    int o = 0;
     L.dm = o;
     o += 8 * E;
     L.doff = o;
@@ -164,7 +183,7 @@ HSMU_HD inline RowLayout row_layout(int numeric, long long S, long long n, long 
     L.ft = o;
     if (numeric && sparse)
         o += 4 * fine_cap(S, tp);
-    o = (o + 7) & ~7LL;
+    o = (o + 7) & ~7;
     L.vals = o;
     if (numeric)
         o += 8 * (!sparse && use_dense(S, n) ? 64 * S : n);
@@ -184,15 +203,15 @@ HSMU_HD inline RowLayout row_layout(int numeric, long long S, long long n, long 
     L.lidx = o;
     if (with_long)
         o += 4 * nA;
-    o = (o + 15) & ~15LL;
+    o = (o + 15) & ~15;
     L.lcnt = o;
     if (with_long)
         o += 16;
-    L.bytes = (o + 15) & ~15LL;
+    L.bytes = (o + 15) & ~15;
     return L;
 }
 
-HSMU_HD inline long long sym_need(long long S, long long nA, long long tp, bool with_long)
+HSMU_HD inline int sym_need(int S, int nA, int tp, bool with_long)
 {
     return row_layout(0, S, 0, nA, tp, with_long).bytes;
 }
@@ -225,41 +244,39 @@ HSMU_HD constexpr int stream_window(int G) { return G * 32 > 4096 ? G * 32 : 409
 struct StreamLayout {
     int vals, dm, rec, bits, doff, ft, wb, bytes;
 };
-HSMU_HD inline StreamLayout stream_layout(int G, long long S, long long n, long long nA, long long tp, long long p)
+HSMU_HD inline StreamLayout stream_layout(int G, int S, int n, int nA, int tp, long long p)
 {
-    StreamLayout L;
+    StreamLayout L = {};
     const bool sparse = use_sparse(S, tp);
-    const long long E = dir_entries(S, tp);
-    const long long slots = (p + nA * (STREAM_V - 1)) / STREAM_V;
-    const long long win = slots < stream_window(G) ? slots : stream_window(G);
-    const long long words = (win + 63) / 64;
-    const long long cap = 1LL << 30; // rows beyond LDS: any size past it will do
-    auto clip = [&](long long v) { return (int)(v < cap ? v : cap); };
-    long long o = 0;
-    L.vals = 0;
-    o += 8 * (!sparse && use_dense(S, n) ? 64 * S : n);
-    o = (o + 15) & ~15LL;
-    L.dm = clip(o);
+    const int E = dir_entries(S, tp);
+    if (E > LAYOUT_CAP || n > LAYOUT_CAP) {
+        L.bytes = LAYOUT_NONE;
+        return L;
+    }
+    const long long slots = (p + (long long)nA * (STREAM_V - 1)) / STREAM_V;
+    const int words = ((slots < stream_window(G) ? (int)slots : stream_window(G)) + 63) >> 6;
+    int o = 8 * (!sparse && use_dense(S, n) ? 64 * S : n);
+    o = (o + 15) & ~15;
+    L.dm = o;
     o += 8 * E;
-    o = (o + 15) & ~15LL;
-    L.rec = clip(o);
+    o = (o + 15) & ~15;
+    L.rec = o;
     o += 16 * (nA < G ? nA : G);
-    L.bits = clip(o);
+    L.bits = o;
     o += 8 * words;
-    L.doff = clip(o);
+    L.doff = o;
     o += 4 * E;
-    L.ft = clip(o);
+    L.ft = o;
     if (sparse)
         o += 4 * fine_cap(S, tp);
-    L.wb = clip(o);
+    L.wb = o;
     o += 2 * words;
-    L.bytes = clip((o + 15) & ~15LL);
+    L.bytes = (o + 15) & ~15;
     return L;
 }
 
 // LDS a row with p products needs in numeric bin `bin`
-HSMU_HD inline long long num_need(int bin, long long S, long long n, long long nA, long long tp, long long p,
-                                  bool with_long)
+HSMU_HD inline int num_need(int bin, int S, int n, int nA, int tp, long long p, bool with_long)
 {
     return (8 << bin) >= BLOCK ? stream_layout(8 << bin, S, n, nA, tp, p).bytes
                                : row_layout(1, S, n, nA, tp, with_long).bytes;
@@ -272,34 +289,37 @@ constexpr int LDS_STATIC_RESERVE = 256;
 
 hipError_t launch_fill_zero(void *p, size_t bytes, hipStream_t s);
 
-// B -> tiles: per-row tile counts, scan to tptr, fill tcol/tmask.
-// scan_ws must hold scan_ws_bytes(K) bytes.
-size_t scan_ws_bytes(int64_t n);
-// ws must hold btiles_ws_bytes(nnz) bytes, scan_ws scan_ws_bytes(nnz + 1).
-size_t btiles_ws_bytes(int64_t nnz);
-// One row of B as the row analysis needs it: entries, tiles, first and last tile column
-// (last = -1 for an empty row).
+// One row of B as the row analysis needs it: entries, tiles (-1: see the tile pointers), first
+// and last tile column (last = -1 for an empty row).
 struct alignas(16) BRow {
     int len, ntiles, first, last;
 };
-// brow (K entries, may be null): each row's BRow, written beside the tile row pointers.
-hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const int *col,
-                         int *ws, int *tptr, int *tcol, unsigned long long *tmask, BRow *brow,
-                         void *scan_ws, DevStats *st, int num_cus, hipStream_t s);
+// B -> tiles: tptr (K + 1), tcol and tmask (room for nnz), brow (K, may be null).  words:
+// btiles_blocks(nnz) zeroed words, *ticket = 0.
+int64_t btiles_blocks(int64_t nnz);
+hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const int *col, int *tptr,
+                         int *tcol, unsigned long long *tmask, BRow *brow, unsigned long long *words,
+                         unsigned *ticket, DevStats *st, hipStream_t s);
 
-// Per row of A: products, tile-products, tile span (from the BRow of each B_j it names).
-// longrows (M ints) is scratch for the list of long rows analysed one workgroup per row.
+// Per row of A: products, tile-products, tile span (from the BRow of each B_j it names), and
+// the rows' symbolic bins: binrows, and each LDS-bin row's directory range: rdir[i] = offset
+// (span entries), -1 for rows not in an LDS bin; st->dir_total = entries reserved.  host (may
+// be null): the counters are copied there at the end (device-accessible host memory).  sums:
+// NBINS per block (row_info_blocks).
 hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, const int *Acol,
-                           const BRow *brow, long long *rprod, int *rtp, int *rmin, int *rmax,
-                           int *rnnz, int *longrows, DevStats *st, int avg_a, int num_cus, hipStream_t s);
+                           const BRow *brow, const int *tptr, long long *rprod, int *rtp, int *rmin,
+                           int *rmax, int *rnnz, BinParams bp, int *binrows, long long *rdir, DevStats *st,
+                           BinSum *sums, unsigned *done, DevStats *host, int num_cus, hipStream_t s);
+int64_t row_info_blocks(int64_t M, int64_t nnzA, int num_cus);
 
-// Bin rows for the symbolic (numeric = 0) or numeric (numeric = 1) phase.  The symbolic
-// pass also reserves each LDS-bin row's directory range: rdir[i] = offset (span entries),
-// -1 for rows not in an LDS bin; st->dir_total = entries reserved.
-hipError_t launch_bin(int numeric, int64_t M, const int *Arp, const long long *rprod,
-                      const int *rtp, const int *rmin, const int *rmax, const int *rnnz,
-                      BinParams bp, int *binrows, long long *rdir, DevStats *st, int num_cus,
-                      hipStream_t s);
+// C's row pointers (crp, and out32 when given: M + 1 each) from rnnz, and the numeric bins.
+// words: rowptr_blocks(M) zeroed words, *ticket = 0.  sums, host as above (rowptr_blocks).
+int64_t rowptr_blocks(int64_t M);
+hipError_t launch_rowptr_bin(int64_t M, const int *Arp, const long long *rprod, const int *rtp,
+                             const int *rmin, const int *rmax, const int *rnnz, long long *crp,
+                             int *out32, BinParams bp, int *binrows, unsigned long long *words,
+                             unsigned *ticket, DevStats *st, BinSum *sums, unsigned *done,
+                             DevStats *host, hipStream_t s);
 
 struct Operands {
     const int *Arp, *Acol;
@@ -335,9 +355,6 @@ hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int c
                            int max_need, const Operands &op, int *rnnz, int tshift, int two_level, int long_rows,
                            unsigned long long *gws, long long gws_stride, int num_cus,
                            int gws_blocks, int lds_dyn, unsigned *queue, hipStream_t s);
-
-hipError_t launch_scan_i32_i64(const int *in, int64_t n, long long *out, void *scan_ws,
-                               long long *total_copy, hipStream_t s);
 
 // Wide rows (BIN_GLOBAL) in the numeric phase: blocks workgroups, each with a workspace of
 // 3 * cur_stride + ft_stride ints (cursors, ends and next columns of its row's A entries:
@@ -417,8 +434,6 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
 // A B of fewer than STREAM_V entries (n of them, at least one), copied to arrays of
 // STREAM_V entries whose last one repeats: the element stream loads STREAM_V at a time.
 hipError_t launch_pad_b(const int *col, const void *val, int val32, int n, int *pcol, void *pval, hipStream_t s);
-
-hipError_t launch_rowptr_i64_to_i32(const long long *in, int64_t n, int *out, hipStream_t s);
 
 // out[i] = in[i] - in[0] for i < n (row pointers of a row panel, rebased to 0)
 hipError_t launch_rowptr_rebase(const int *in, int64_t n, int *out, hipStream_t s);

@@ -2,18 +2,19 @@
 //
 // Pipeline for C = A * B (all on one stream; host synchronises twice, to validate the
 // input / size the symbolic launches and to size C):
-//   1. B -> 64-column tiles (k_btile_count, scan, k_btile_fill).
+//   1. B -> 64-column tiles (k_btiles: one pass, chained scan).
 //      Reference: src/compressed/compressed_mask64.cuh:61-424.  Tiles of a row come out
 //      sorted by tile column (the reference's order is whatever LDS atomics give).
 //   2. Row analysis of A (k_row_info): products, tile-products and the tile span
 //      [rmin, rmax] of each row of C.  Reference: k_compute_flop, src/small/mask.cuh:14-51.
-//   3. Binning (k_bin) by work and LDS need, wave/workgroup-aggregated appends.
-//      Reference: src/bining.cuh:1-395 (fixed ranges there; derived from LDS need here).
+//   3. Binning (in k_row_info, and in k_rowptr_bin for the numeric phase) by work and LDS
+//      need, wave/workgroup-aggregated appends.  Reference: src/bining.cuh:1-395 (fixed
+//      ranges there; derived from LDS need here).
 //   4. Symbolic (k_symbolic_lds / k_symbolic_global): OR of B's tile masks over the A row
 //      into a dense mask directory over the row's tile span, nnz(C_i) = sum popcount.
 //      Reference: compressed_tilePtr_symbolic.cuh + compressed_tileOR.cuh, which do the
 //      same in two hash passes; the dense directory needs one pass and no hashing.
-//   5. Scan of nnz(C_i) to int64 row pointers.
+//   5. Scan of nnz(C_i) to row pointers (k_rowptr_bin).
 //   6. Numeric (k_numeric_lds / k_numeric_window): the HSMU accumulator.  The row's
 //      value array is exactly nnz(C_i) long; the slot of column c is
 //        off[t] + popcount(mask[t] & ((1 << (c & 63)) - 1)),  t = (c >> 6) - rmin,
@@ -84,455 +85,287 @@ hipError_t launch_copy(const void *src, void *dst, size_t bytes, int num_cus, hi
     return hipGetLastError();
 }
 
-// ---- exclusive scan (three phases: block sums, scan of sums, apply) ---------------
-
-constexpr int SCAN_BS = 256;
-constexpr int SCAN_IPT = 16;
-constexpr int SCAN_TILE = SCAN_BS * SCAN_IPT;
-
-size_t scan_ws_bytes(int64_t n)
+// Loads and stores at the device's point of coherence, beside the atomics' updates.
+template <typename T> DEVI T device_load(const T *p)
 {
-    const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-    return (size_t)(nb + 2) * sizeof(long long);
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T> DEVI void device_store(T *p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename Tin>
-__global__ __launch_bounds__(SCAN_BS) void k_scan_reduce(const Tin *__restrict__ in, int64_t n, long long *__restrict__ bsum)
-{
-    __shared__ long long red[SCAN_BS / 64];
-    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE;
-    long long s = 0;
-    for (int i = threadIdx.x; i < SCAN_TILE; i += SCAN_BS) {
-        const int64_t k = base + i;
-        if (k < n)
-            s += (long long)in[k];
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0)
-        red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        long long t = 0;
-        for (int w = 0; w < SCAN_BS / 64; ++w)
-            t += red[w];
-        bsum[blockIdx.x] = t;
-    }
-}
+// ---- chained scan ---------------------------------------------------------------------
+//
+// Blocks take their place in a sequence from a counter (so that a block only ever waits for
+// blocks that are running), publish the sum of their part and then the prefix up to their
+// end, and read back over their predecessors' words until one holds a prefix.  A word holds
+// its state and its value together, so no other memory has to be ordered.
+constexpr u64 CHAIN_SUM = 1ull << 62, CHAIN_PREFIX = 2ull << 62, CHAIN_VALUE = CHAIN_SUM - 1;
 
-// One workgroup: exclusive scan of nb block sums in place; bsum[nb] = total.
-__global__ __launch_bounds__(1024) void k_scan_blocks(long long *bsum, int64_t nb)
+// The sum of the parts before place `b`; `part` is this block's.  Called by one whole wave.
+DEVI u64 chain_prefix(u64 *words, int b, u64 part)
 {
-    __shared__ long long red[16];
-    __shared__ long long carry_s;
-    if (threadIdx.x == 0)
-        carry_s = 0;
-    __syncthreads();
-    for (int64_t base = 0; base < nb; base += 1024) {
-        const int64_t k = base + threadIdx.x;
-        const long long v = k < nb ? bsum[k] : 0;
-        long long total;
-        const long long ex = group_excl_scan<1024>(v, red, total);
-        const long long carry = carry_s;
-        if (k < nb)
-            bsum[k] = carry + ex;
-        __syncthreads();
-        if (threadIdx.x == 0)
-            carry_s = carry + total;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        bsum[nb] = carry_s;
-}
-
-// Each thread scans SCAN_IPT consecutive elements; the block's tile passes through LDS
-// (padded by one element per SCAN_IPT, so a thread's run and a wave's coalesced row both
-// spread over the banks) so that global loads and stores stay coalesced.
-DEVI int scan_pad(int k) { return k + k / SCAN_IPT; }
-
-template <typename Tin, typename Tout>
-__global__ __launch_bounds__(SCAN_BS) void k_scan_apply(const Tin *__restrict__ in, int64_t n, const long long *__restrict__ bsum,
-                                                         int64_t nb, Tout *__restrict__ out, long long *total_copy)
-{
-    __shared__ long long red[SCAN_BS / 64];
-    __shared__ Tout tile[SCAN_TILE + SCAN_TILE / SCAN_IPT];
-    const int64_t b0 = (int64_t)blockIdx.x * SCAN_TILE;
-    const int t = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    if (lane == 0)
+        device_store(&words[b], (b ? CHAIN_SUM : CHAIN_PREFIX) | part);
+    // CHAIN_W words per lane at a time: blocks of one launch publish together, so most find
+    // sums only, all the way back, and every round costs a trip to memory
+    constexpr int CHAIN_W = 4;
+    u64 before = 0;
+    for (int e = b; e > 0;) { // words [e - 64 CHAIN_W, e), the nearest first
+        u64 w[CHAIN_W];
 #pragma unroll
-    for (int i = 0; i < SCAN_IPT; ++i) {
-        const int q = i * SCAN_BS + t;
-        tile[scan_pad(q)] = b0 + q < n ? (Tout)in[b0 + q] : (Tout)0;
-    }
-    __syncthreads();
-    long long v[SCAN_IPT];
-    long long loc = 0;
+        for (int i = 0; i < CHAIN_W; ++i) {
+            const int q = e - 1 - lane - 64 * i;
+            w[i] = q >= 0 ? device_load(&words[q]) : CHAIN_PREFIX; // before the first: a prefix of 0
+        }
+        bool wait = false, found = false;
+        u64 sum = 0;
+        int used = 0;
 #pragma unroll
-    for (int i = 0; i < SCAN_IPT; ++i) {
-        v[i] = (long long)tile[scan_pad(t * SCAN_IPT + i)];
-        loc += v[i];
+        for (int i = 0; i < CHAIN_W; ++i) {
+            if (wait || found)
+                continue;
+            if (__ballot(w[i] < CHAIN_SUM)) { // one is not published yet
+                wait = true;
+                continue;
+            }
+            const u64 pre = __ballot(w[i] >= CHAIN_PREFIX);
+            const int stop = pre ? (int)__builtin_ctzll(pre) : 63; // nearest prefix
+            sum += wave_sum(lane <= stop ? w[i] & CHAIN_VALUE : 0ull);
+            found = pre != 0;
+            used += 64;
+        }
+        before += sum;
+        if (found)
+            break;
+        e -= used;
+        if (wait && !used)
+            __builtin_amdgcn_s_sleep(1);
     }
-    long long total;
-    long long pre = group_excl_scan<SCAN_BS>(loc, red, total) + bsum[blockIdx.x];
-#pragma unroll
-    for (int i = 0; i < SCAN_IPT; ++i) {
-        tile[scan_pad(t * SCAN_IPT + i)] = (Tout)pre;
-        pre += v[i];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < SCAN_IPT; ++i) {
-        const int q = i * SCAN_BS + t;
-        if (b0 + q < n)
-            out[b0 + q] = tile[scan_pad(q)];
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        out[n] = (Tout)bsum[nb];
-        if (total_copy)
-            *total_copy = bsum[nb];
-    }
-}
-
-template <typename Tin, typename Tout>
-static hipError_t scan_excl(const Tin *in, int64_t n, Tout *out, void *ws, long long *total_copy, hipStream_t s)
-{
-    const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-    long long *bsum = (long long *)ws;
-    if (nb > 0)
-        hipLaunchKernelGGL((k_scan_reduce<Tin>), dim3((unsigned)nb), dim3(SCAN_BS), 0, s, in, n, bsum);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, s, bsum, nb);
-    hipLaunchKernelGGL((k_scan_apply<Tin, Tout>), dim3((unsigned)(nb > 0 ? nb : 1)), dim3(SCAN_BS), 0, s, in, n, bsum, nb,
-                       out, total_copy);
-    return hipGetLastError();
-}
-
-hipError_t launch_scan_i32_i64(const int *in, int64_t n, long long *out, void *scan_ws, long long *total_copy,
-                               hipStream_t s)
-{
-    return scan_excl<int, long long>(in, n, out, scan_ws, total_copy, s);
+    if (lane == 0 && b)
+        device_store(&words[b], CHAIN_PREFIX | (before + part));
+    return before;
 }
 
 // ---- B -> tiles ------------------------------------------------------------------------
 //
-// Element-parallel, so a row of any length costs the same per element (R-MAT's hub rows
-// made a row-per-group conversion wait on its longest row):
-//   1. k_bmark:  per row, validate the row pointers and mark the row's first element in a
-//                bitmap (only the bitmap is cleared beforehand, not the flags);
-//   2. k_bhead:  per element, validate the column and sortedness and flag tile heads
-//                (first element of a row, or tile column different from the left neighbour);
-//   3. exclusive scan of the flags: the tile index of every head;
-//   4. k_bfill:  per head, write its tile column and OR the bits of its run (k_bcarry
-//                adds the parts of runs that cross a wave);
-//      k_btptr:  per row, tptr[j] = tile index at the row's first element.
+// One pass over B's entries (a row of any length costs the same per entry: R-MAT's hub rows
+// made a row-per-group conversion wait on its longest row).  A block takes BT_N consecutive
+// entries; it finds the rows that start among them by searching the row pointers, marks
+// their first entries in LDS, flags tile heads (first entry of a row, or another tile than
+// the left neighbour's), counts them with ballots, learns the tiles before it from the
+// chained scan, and writes its tiles and its rows' tile pointers.  A tile's bits are OR-ed
+// in LDS by the block that holds its head, which reads on past its end for them.  Every
+// block also validates a share of the row pointers.
+// What bounds it: HBM (4 bytes read per entry, 12 written per tile) and, for small B, the
+// latency of the search and the chain.  It takes the place of nine kernels (row marks, head
+// flags, a three-kernel scan, fill, carry, tile pointers and a clear), which read the
+// entries and the flags several times over.
 // Reference: compute_tile64_nums / compute_tile64_col / compute_tile64_mask_num,
 // src/compressed/compressed_mask64.cuh:61-342.
+constexpr int BT_BS = 256;
+constexpr int BT_STEPS = 8;                      // entries per thread
+constexpr int BT_N = BT_BS * BT_STEPS;           // entries per block
+constexpr int BT_WAVE = BT_N / (BT_BS / 64);     // entries per wave, 64 per step
+static_assert(BT_WAVE == 64 * BT_STEPS, "a wave's entries are its steps");
 
-__global__ __launch_bounds__(256) void k_bmark(int64_t K, int64_t nnz, const int *__restrict__ rp,
-                                               unsigned *__restrict__ starts, DevStats *st)
+// The first r in [0, n) with rp[r] >= x (n if none), for nondecreasing rp, by one wave: each
+// round cuts the range to a 65th.  (Any rp: the result is some r in [0, n].)
+DEVI int first_row(const int *__restrict__ rp, long long n, long long x)
 {
-    const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    int len = 0;
-    if (j < K) {
-        const int s = rp[j], e = rp[j + 1];
-        if (s < 0 || e < s || (int64_t)e > nnz) {
-            atomicOr(&st->err, ERR_ROWPTR);
-        } else {
-            len = e - s;
-            if (e > s)
-                atomicOr(&starts[s >> 5], 1u << (s & 31));
-        }
-    }
-    // longest row, counted only from LONG_TILES on (all the kernels need to know): no
-    // atomic at all for inputs without long rows, one per wave that has one otherwise
-    if (len >= LONG_TILES) {
-        const int m = wave_max<int>(len);
-        if (len == m)
-            atomicMax(&st->max_brow, len);
-    }
-}
-
-__global__ __launch_bounds__(256) void k_bhead(int64_t nnz, int64_t N, const int *__restrict__ col,
-                                               const unsigned *__restrict__ starts, int *__restrict__ flag, DevStats *st)
-{
-    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    int bad = 0;
-    if (k < nnz) {
-        const int c = col[k];
-        if ((unsigned)c >= (unsigned long long)N)
-            bad |= ERR_BCOL;
-        const bool start = (starts[k >> 5] >> (k & 31)) & 1u;
-        int head = 1;
-        if (!start && k > 0) {
-            const int pc = col[k - 1];
-            if (pc > c)
-                bad |= ERR_UNSORTED;
-            head = (pc >> 6) != (c >> 6);
-        }
-        flag[k] = head;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        bad |= __shfl_xor(bad, o, 64);
-    if (bad && (threadIdx.x & 63) == 0)
-        atomicOr(&st->err, bad);
-}
-
-// The bits of a run are OR-ed across the wave with shuffles (a segmented suffix OR: lane
-// i gathers [i, end of its run within the wave) in six doubling steps).  A run that goes
-// on past the wave's last lane is finished by k_bcarry: every wave whose first element is
-// not a head leaves the OR of its lanes up to its first head in part[wave].
-__global__ __launch_bounds__(256) void k_bfill(int64_t nnz, const int *__restrict__ col, const int *__restrict__ flag,
-                                               const int *__restrict__ tix, int *__restrict__ tcol, u64 *__restrict__ tmask,
-                                               u64 *__restrict__ part)
-{
-    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    const bool valid = k < nnz;
-    const int c = valid ? col[k] : 0;
-    const bool head = !valid || flag[k] != 0; // past the end counts as a head: runs stop there
-    const u64 H = __ballot(head);
-    // first head after this lane within the wave (64: none)
-    const u64 after = lane < 63 ? (H >> (lane + 1)) : 0ull;
-    const int send = after ? lane + 1 + (int)__builtin_ctzll(after) : 64;
-    u64 acc = valid ? (1ull << (c & 63)) : 0ull;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const u64 other = __shfl_down(acc, o, 64);
-        if (lane + o < send)
-            acc |= other;
-    }
-    if (lane == 0 && !head)
-        part[k >> 6] = acc;
-    if (!valid || !head)
-        return;
-    const int t = tix[k];
-    tcol[t] = c >> 6;
-    tmask[t] = acc;
-}
-
-// Per wave of k_bfill whose first element continues a run: OR its part into that run's
-// tile (number tix - 1: the heads before it, less one).  Several waves may continue one
-// run (a tile with repeated columns), hence the atomic.
-__global__ __launch_bounds__(256) void k_bcarry(int64_t nnz, const int *__restrict__ flag, const int *__restrict__ tix,
-                                                const u64 *__restrict__ part, u64 *__restrict__ tmask)
-{
-    const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t k = w << 6;
-    if (k >= nnz || flag[k] != 0)
-        return;
-    atomicOr((unsigned long long *)&tmask[tix[k] - 1], (unsigned long long)part[w]);
-}
-
-__global__ __launch_bounds__(256) void k_btptr(int64_t K, int64_t nnz, const int *__restrict__ rp,
-                                               const int *__restrict__ col, const int *__restrict__ tix,
-                                               int *__restrict__ tptr, BRow *__restrict__ brow, DevStats *st)
-{
-    const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (j > K)
-        return;
-    // a row pointer outside [0, nnz] has already raised ERR_ROWPTR in k_bmark; keep
-    // the reads in bounds until the host sees the error
-    auto clamp = [&](int r) { return r < 0 ? 0 : (r > nnz ? (int)nnz : r); };
-    const int r = clamp(rp[j]);
-    tptr[j] = tix[r];
-    if (j == K) {
-        st->ntiles_b = tix[r];
-    } else if (brow) {
-        const int r1 = clamp(rp[j + 1]);
-        BRow q = {0, 0, 0, -1};
-        if (r1 > r) {
-            q.len = r1 - r;
-            q.ntiles = tix[r1] - tix[r];
-            q.first = col[r] >> 6; // rows are sorted: their first and last tiles
-            q.last = col[r1 - 1] >> 6;
+    long long lo = 0, hi = n; // the answer lies in [lo, hi]
+    while (hi > lo) {
+        const long long step = (hi - lo + 63) / 64;
+        const long long q = lo + lane * step;
+        const bool ge = q >= hi || (long long)rp[q] >= x;
+        const u64 m = __ballot(ge); // lanes from the first set one on (sorted rp)
+        const int f = m ? (int)__builtin_ctzll(m) : 64;
+        if (f == 0) {
+            hi = lo;
+        } else {
+            const long long l2 = lo + (f - 1) * step + 1, h2 = lo + f * step;
+            hi = h2 < hi ? h2 : hi;
+            lo = l2;
         }
-        brow[j] = q;
     }
+    return (int)uniform64(lo);
 }
 
-size_t btiles_ws_bytes(int64_t nnz)
+__global__ __launch_bounds__(BT_BS) void k_btiles(int64_t K, int64_t N, int64_t nnz, const int *__restrict__ rp,
+                                                  const int *__restrict__ col, int *__restrict__ tptr,
+                                                  int *__restrict__ tcol, u64 *__restrict__ tmask,
+                                                  BRow *__restrict__ brow, u64 *words, unsigned *ticket, DevStats *st)
 {
-    return (size_t)(2 * nnz + 2) * sizeof(int) + (size_t)(nnz / 64 + 1) * sizeof(u64) +
-           (size_t)(nnz / 32 + 1) * sizeof(unsigned);
-}
-
-hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const int *col, int *ws, int *tptr,
-                         int *tcol, u64 *tmask, BRow *brow, void *scan_ws, DevStats *st, int num_cus, hipStream_t s)
-{
-    (void)num_cus;
-    int *flag = ws;           // nnz + 1
-    int *tix = ws + nnz + 1;  // nnz + 1
-    u64 *part = (u64 *)(ws + 2 * nnz + 2); // nnz / 64 + 1 (8-byte aligned: 2 nnz + 2 ints before it)
-    unsigned *starts = (unsigned *)(part + nnz / 64 + 1); // nnz / 32 + 1 bits of row starts
-    const unsigned gk = (unsigned)((K + 256) / 256);
-    const unsigned ge = (unsigned)((nnz + 255) / 256 > 0 ? (nnz + 255) / 256 : 1);
-    hipError_t e = launch_fill_zero(starts, (size_t)(nnz / 32 + 1) * sizeof(unsigned), s);
-    if (e != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(k_bmark, dim3(gk), dim3(256), 0, s, K, nnz, rp, starts, st);
-    hipLaunchKernelGGL(k_bhead, dim3(ge), dim3(256), 0, s, nnz, N, col, starts, flag, st);
-    e = scan_excl<int, int>(flag, nnz, tix, scan_ws, nullptr, s);
-    if (e != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(k_bfill, dim3(ge), dim3(256), 0, s, nnz, col, flag, tix, tcol, tmask, part);
-    hipLaunchKernelGGL(k_bcarry, dim3((unsigned)((nnz / 64 + 256) / 256)), dim3(256), 0, s, nnz, flag, tix, part, tmask);
-    hipLaunchKernelGGL(k_btptr, dim3(gk), dim3(256), 0, s, K, nnz, rp, col, tix, tptr, brow, st);
-    return hipGetLastError();
-}
-
-// ---- row analysis of A ---------------------------------------------------------------
-
-// Per row i of A: products sum_j nnz(B_j), tile-products sum_j tiles(B_j), and the span
-// [rmin, rmax] of tile columns of row i of C (rows of B are sorted, so each B row's
-// first and last tile bound it).  Reference: k_compute_flop, src/small/mask.cuh:14-51.
-// One group of G lanes per row, one row per group (no grid-stride loop, so the latency
-// of the dependent loads Acol -> Brp/tptr -> tcol is paid once per row in parallel).
-// Totals are summed per bin by k_bin; only the rare error bits use a global atomic.
-constexpr int LONG_A = 2048; // rows of A longer than this are analysed by a whole workgroup
-
-template <int G>
-__global__ __launch_bounds__(256) void k_row_info(int64_t M, int64_t K, int64_t nnzA, const int *__restrict__ Arp,
-                                                  const int *__restrict__ Acol, const BRow *__restrict__ brow,
-                                                  long long *__restrict__ rprod, int *__restrict__ rtp,
-                                                  int *__restrict__ rmin, int *__restrict__ rmax, int *__restrict__ rnnz,
-                                                  int *__restrict__ longrows, DevStats *st)
-{
-    constexpr int RPB = 256 / G;
-    const int g = threadIdx.x / G, l = threadIdx.x & (G - 1);
-    const int64_t i = (int64_t)blockIdx.x * RPB + g;
-    if (i >= M)
-        return;
+    __shared__ u64 s_mask[BT_N]; // bits of the block's tiles
+    __shared__ u64 s_start[BT_N / 64];
+    __shared__ u64 s_head[BT_N / 64];
+    __shared__ int s_before[BT_N / 64]; // heads before each 64 entries, within the block
+    __shared__ int s_b, s_r0, s_r1, s_prefix, s_tiles;
+    const int t = threadIdx.x, lane = t & 63, w = uniform(t >> 6);
+    if (t == 0) // (a lone block has no place to take)
+        s_b = gridDim.x > 1 ? (int)atomicAdd(ticket, 1u) : 0;
+    for (int q = t; q < BT_N; q += BT_BS)
+        s_mask[q] = 0;
+    if (t < BT_N / 64)
+        s_start[t] = 0;
+    __syncthreads();
+    const int b = uniform(s_b);
+    const int nb = (int)gridDim.x;
+    const int64_t e0 = (int64_t)b * BT_N;
+    const int64_t e1 = e0 + BT_N < nnz ? e0 + BT_N : nnz;
     int bad = 0;
-    const int s = Arp[i], e = Arp[i + 1];
-    long long p = 0;
-    int tp = 0, mn = INT_MAX, mx = -1;
-    if (s < 0 || e < s || (int64_t)e > nnzA) {
-        bad |= ERR_ROWPTR;
-    } else if (e - s > LONG_A) {
-        if (l == 0)
-            longrows[atomicAdd(&st->nlong, 1)] = (int)i;
-        return;
-    } else {
-        for (int k = s + l; k < e; k += G) {
-            const int j = Acol[k];
-            if ((unsigned)j >= (unsigned long long)K) {
-                bad |= ERR_ACOL;
-                continue;
-            }
-            const BRow q = brow[j];
-            if (q.len > 0) {
-                p += q.len;
-                tp += q.ntiles;
-                mn = q.first < mn ? q.first : mn;
-                mx = q.last > mx ? q.last : mx;
-            }
+    // this block's share of the row pointers: in range and nondecreasing; the longest row,
+    // counted only from LONG_TILES on (all the kernels need to know)
+    {
+        const int64_t v0 = K * b / nb, v1 = K * (b + 1) / nb;
+        int longest = 0;
+        for (int64_t r = v0 + t; r < v1; r += BT_BS) {
+            const int s = rp[r], e = rp[r + 1];
+            if (s < 0 || e < s || (int64_t)e > nnz)
+                bad |= ERR_ROWPTR;
+            else if (e - s >= LONG_TILES)
+                longest = e - s > longest ? e - s : longest;
         }
+        longest = wave_max(longest);
+        if (lane == 0 && longest)
+            atomicMax(&st->max_brow, longest);
     }
-    p = group_sum<G>(p, (long long *)nullptr);
-    tp = group_sum<G>(tp, (int *)nullptr);
-    mn = group_min<G>(mn);
-    mx = group_max<G>(mx);
-    if (l == 0) {
-        rprod[i] = p;
-        rtp[i] = tp;
-        rmin[i] = mn;
-        rmax[i] = mx;
-        if (p == 0)
-            rnnz[i] = 0;
+    // rows whose first entry is in [e0, e1): [r0, r1); the last block takes the rest
+    if (w == 0) {
+        const int r = first_row(rp, K + 1, e0);
+        if (lane == 0)
+            s_r0 = b == 0 ? 0 : r;
+    } else if (w == 1) {
+        const int r = first_row(rp, K + 1, e1);
+        if (lane == 0)
+            s_r1 = b == nb - 1 ? (int)(K + 1) : r;
+    }
+    // the wave's columns, and each one's left neighbour through the lanes
+    int c[BT_STEPS], pc[BT_STEPS];
+    const int64_t k0 = e0 + (int64_t)w * BT_WAVE;
+#pragma unroll
+    for (int i = 0; i < BT_STEPS; ++i) {
+        const int64_t k = k0 + 64 * i + lane;
+        c[i] = k < e1 ? col[k] : 0;
+    }
+    int carry = k0 > 0 && k0 < e1 ? col[k0 - 1] : 0;
+#pragma unroll
+    for (int i = 0; i < BT_STEPS; ++i) {
+        pc[i] = __builtin_amdgcn_update_dpp(carry, c[i], 0x138, 0xf, 0xf, false); // wave_shr:1
+        carry = __builtin_amdgcn_readlane(c[i], 63);
+    }
+    __syncthreads();
+    const int r0 = uniform(s_r0), r1 = uniform(s_r1);
+    for (int64_t r = (int64_t)r0 + t; r < r1; r += BT_BS) {
+        const int64_t p = rp[r];
+        if (p >= e0 && p < e1)
+            atomicOr(&s_start[(p - e0) >> 6], 1ull << ((p - e0) & 63));
+    }
+    __syncthreads();
+    u64 H[BT_STEPS];
+#pragma unroll
+    for (int i = 0; i < BT_STEPS; ++i) {
+        const int64_t k = k0 + 64 * i + lane;
+        const bool in = k < e1;
+        const bool start = __builtin_amdgcn_inverse_ballot_w64(uniform64(s_start[w * BT_STEPS + i])) || k == 0;
+        if (in && (unsigned)c[i] >= (unsigned long long)N)
+            bad |= ERR_BCOL;
+        if (in && !start && pc[i] > c[i])
+            bad |= ERR_UNSORTED;
+        H[i] = __ballot(in && (start || (pc[i] >> 6) != (c[i] >> 6)));
+        if (lane == 0)
+            s_head[w * BT_STEPS + i] = H[i];
     }
     if (bad)
         atomicOr(&st->err, bad);
-}
-
-// The rows k_row_info set aside (more than LONG_A entries): one 1024-lane workgroup per
-// row, grid-stride over the device-side list.
-__global__ __launch_bounds__(1024) void k_row_info_long(int64_t K, const int *__restrict__ longrows,
-                                                        const int *__restrict__ Arp, const int *__restrict__ Acol,
-                                                        const BRow *__restrict__ brow, long long *__restrict__ rprod,
-                                                        int *__restrict__ rtp, int *__restrict__ rmin,
-                                                        int *__restrict__ rmax, int *__restrict__ rnnz, DevStats *st)
-{
-    __shared__ long long s_p[16];
-    __shared__ int s_tp[16], s_mn[16], s_mx[16], s_bad[16];
-    const int n = st->nlong;
-    const int w = threadIdx.x >> 6;
-    for (int idx = blockIdx.x; idx < n; idx += gridDim.x) {
-        const int i = longrows[idx];
-        const int s = Arp[i], e = Arp[i + 1];
-        long long p = 0;
-        int tp = 0, mn = INT_MAX, mx = -1, bad = 0;
-        for (int k = s + threadIdx.x; k < e; k += 1024) {
-            const int j = Acol[k];
-            if ((unsigned)j >= (unsigned long long)K) {
-                bad |= ERR_ACOL;
-                continue;
-            }
-            const BRow q = brow[j];
-            if (q.len > 0) {
-                p += q.len;
-                tp += q.ntiles;
-                mn = q.first < mn ? q.first : mn;
-                mx = q.last > mx ? q.last : mx;
-            }
+    __syncthreads();
+    // heads before each 64 entries, the block's tiles and the tiles before it
+    if (w == 0) {
+        static_assert(BT_N / 64 <= 64, "one wave scans the block's heads");
+        const int n = lane < BT_N / 64 ? __popcll(s_head[lane]) : 0;
+        const int incl = wave_incl_scan(n);
+        if (lane < BT_N / 64)
+            s_before[lane] = incl - n;
+        const int tiles = wave_last(incl);
+        const u64 pre = chain_prefix(words, b, (u64)tiles);
+        if (lane == 0) {
+            s_tiles = tiles;
+            s_prefix = (int)pre;
         }
-        p = group_sum<64>(p, (long long *)nullptr);
-        tp = group_sum<64>(tp, (int *)nullptr);
-        mn = group_min<64>(mn);
-        mx = group_max<64>(mx);
+    }
+    __syncthreads();
+    const int prefix = uniform(s_prefix), tiles = uniform(s_tiles);
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1)
-            bad |= __shfl_xor(bad, o, 64);
-        if ((threadIdx.x & 63) == 0) {
-            s_p[w] = p;
-            s_tp[w] = tp;
-            s_mn[w] = mn;
-            s_mx[w] = mx;
-            s_bad[w] = bad;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int k = 1; k < 16; ++k) {
-                p += s_p[k];
-                tp += s_tp[k];
-                mn = s_mn[k] < mn ? s_mn[k] : mn;
-                mx = s_mx[k] > mx ? s_mx[k] : mx;
-                bad |= s_bad[k];
-            }
-            rprod[i] = p;
-            rtp[i] = tp;
-            rmin[i] = mn;
-            rmax[i] = mx;
-            if (p == 0)
-                rnnz[i] = 0;
-            if (bad)
-                atomicOr(&st->err, bad);
-        }
-        __syncthreads();
+    for (int i = 0; i < BT_STEPS; ++i) {
+        const int64_t k = k0 + 64 * i + lane;
+        const bool head = __builtin_amdgcn_inverse_ballot_w64(H[i]);
+        const int at = s_before[w * BT_STEPS + i] + mbcnt(H[i]) + (head ? 1 : 0) - 1; // this entry's tile
+        if (k < e1 && at >= 0) // (before the first head: another block's tile)
+            atomicOr(&s_mask[at], 1ull << (c[i] & 63));
+        if (head)
+            tcol[prefix + at] = c[i] >> 6;
     }
+    // entries past the block that belong to its last tile: the same row and tile
+    if (w == 0 && tiles > 0 && e1 < nnz) {
+        const int64_t row_end = r1 <= K ? (int64_t)rp[r1] : nnz; // of the row of entry e1 - 1
+        const int64_t end = row_end < nnz ? row_end : nnz;
+        const int last = col[e1 - 1] >> 6;
+        for (int64_t k = e1 + lane;; k += 64) {
+            const int cc = k < end ? col[k] : 0;
+            const bool mine = k < end && (cc >> 6) == last;
+            if (mine)
+                atomicOr(&s_mask[tiles - 1], 1ull << (cc & 63));
+            if (__ballot(mine) != ~0ull)
+                break;
+        }
+    }
+    // the block's rows: tiles before entry p of this block
+    for (int64_t r = (int64_t)r0 + t; r < r1; r += BT_BS) {
+        const int64_t p = rp[r];
+        if (p < e0 || p > e1 || (p == e1 && e1 < nnz))
+            continue; // (row pointers out of order: reported)
+        int tp = tiles;
+        if (p < e1) {
+            const int q = (int)(p - e0);
+            tp = s_before[q >> 6] + __popcll(s_head[q >> 6] & below(q & 63));
+        }
+        tp += prefix;
+        tptr[r] = tp;
+        if (r == K) {
+            st->ntiles_b = tp;
+        } else if (brow) {
+            const int64_t e = rp[r + 1];
+            BRow q = {0, 0, INT_MAX, -1};
+            if (e > p && e <= nnz) { // rows are sorted: their first and last tiles
+                q.len = (int)(e - p);
+                q.ntiles = -1; // known if the row ends in this block
+                if (e < e1) {
+                    const int f = (int)(e - e0);
+                    q.ntiles = prefix + s_before[f >> 6] + __popcll(s_head[f >> 6] & below(f & 63)) - tp;
+                } else if (e == e1) {
+                    q.ntiles = prefix + tiles - tp;
+                }
+                q.first = col[p] >> 6;
+                q.last = col[e - 1] >> 6;
+            }
+            brow[r] = q;
+        }
+    }
+    __syncthreads();
+    for (int q = t; q < tiles; q += BT_BS)
+        tmask[prefix + q] = s_mask[q];
 }
 
-hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, const int *Acol, const BRow *brow,
-                           long long *rprod, int *rtp, int *rmin, int *rmax, int *rnnz, int *longrows, DevStats *st,
-                           int avg_a, int num_cus, hipStream_t s)
+int64_t btiles_blocks(int64_t nnz) { return nnz > 0 ? (nnz + BT_N - 1) / BT_N : 1; }
+
+hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const int *col, int *tptr, int *tcol,
+                         u64 *tmask, BRow *brow, u64 *words, unsigned *ticket, DevStats *st, hipStream_t s)
 {
-#define ROW_INFO(G)                                                                                                    \
-    {                                                                                                                  \
-        constexpr int RPB = 256 / G;                                                                                   \
-        const int64_t blocks = (M + RPB - 1) / RPB;                                                                    \
-        hipLaunchKernelGGL((k_row_info<G>), dim3((unsigned)(blocks > 0 ? blocks : 1)), dim3(256), 0, s, M, K, nnzA,    \
-                           Arp, Acol, brow, rprod, rtp, rmin, rmax, rnnz, longrows, st);                               \
-    }
-    if (avg_a <= 12)
-        ROW_INFO(8)
-    else if (avg_a <= 24)
-        ROW_INFO(16)
-    else if (avg_a <= 48)
-        ROW_INFO(32)
-    else
-        ROW_INFO(64)
-#undef ROW_INFO
-    hipLaunchKernelGGL(k_row_info_long, dim3((unsigned)num_cus), dim3(1024), 0, s, K, longrows, Arp, Acol, brow, rprod,
-                       rtp, rmin, rmax, rnnz, st);
+    hipLaunchKernelGGL(k_btiles, dim3((unsigned)btiles_blocks(nnz)), dim3(BT_BS), 0, s, K, N, nnz, rp, col, tptr, tcol,
+                       tmask, brow, words, ticket, st);
     return hipGetLastError();
 }
 
@@ -548,212 +381,558 @@ DEVI int choose_bin(long long work, Need need, const BinParams &bp)
 {
     if (bp.force_global)
         return BIN_GLOBAL;
-    const long long lanes = (work + bp.per_lane - 1) / bp.per_lane;
     int b = 0;
-    while (b < NLDS - 1 && (8LL << b) < lanes)
+    while (b < NLDS - 1 && (8LL << b) * bp.per_lane < work)
         ++b;
     // the budget limits only workgroups that pack several rows: a one-row workgroup needs
     // the row's LDS whatever its width
-    while (b < NLDS - 1) {
-        const int G = 8 << b;
-        if (G >= BLOCK || (need(b) * (BLOCK / G) <= bp.lds_block_budget && need(b) <= bp.lds_row_max))
+    while ((8 << b) < BLOCK) {
+        const int nd = need(b);
+        if (nd <= bp.lds_row_max && nd * (BLOCK >> (b + 3)) <= bp.lds_block_budget)
             break;
         ++b;
     }
     // a one-row workgroup's LDS decides how many fit a CU: widen the row's group until
     // those workgroups hold min_waves waves, to hide the latency of the gathers from B
-    while (b < NLDS - 1) {
-        const int G = 8 << b;
-        const long long nd = need(b);
-        if (G < BLOCK || nd <= 0 || (long long)(G / 64) * (bp.lds_cu / nd) >= bp.min_waves)
+    int nd = need(b);
+    while (b < NLDS - 1 && (8 << b) >= BLOCK) {
+        const int waves = (8 << b) / 64, wgs = (bp.min_waves + waves - 1) / waves;
+        if ((long long)nd * wgs <= bp.lds_cu)
             break;
-        if (need(b + 1) > bp.lds_row_max)
+        const int wider = need(b + 1);
+        if (wider > bp.lds_row_max)
             break; // (the stream's tables grow a little with the width)
+        nd = wider;
         ++b;
     }
-    return need(b) > bp.lds_row_max ? BIN_GLOBAL : b;
+    return nd > bp.lds_row_max ? BIN_GLOBAL : b;
 }
 
-// One thread per row; appends are aggregated per workgroup in LDS, then one global
-// atomic per bin per workgroup reserves the range.  Also sums each bin's work, nnz(A)
-// and (numeric) nnz(C) for the per-kernel algorithmic byte counts.  Workgroups of BS
-// lanes: 256 while that makes at most four per CU (62K rows then occupy every CU, where
-// 1024-lane ones left three quarters idle), 1024 beyond (millions of rows would otherwise
-// queue four times as many atomics on the same bin counters).
-template <int BS>
-__global__ __launch_bounds__(BS) void k_bin(int numeric, int64_t M, const int *__restrict__ Arp,
-                                              const long long *__restrict__ rprod, const int *__restrict__ rtp,
-                                              const int *__restrict__ rmin, const int *__restrict__ rmax,
-                                              const int *__restrict__ rnnz, BinParams bp, int *__restrict__ binrows,
-                                              long long *__restrict__ rdir, DevStats *st)
+// One row as the binning sees it.
+struct BinRow {
+    long long prod;
+    int S, nA, tp, nc; // tiles spanned, entries of A, tile-products, entries of C
+};
+
+// The blocks of one binning: their counts in LDS, then one global atomic per bin and block
+// for the rows' places (atomics on one address retire one every few nanoseconds
+// device-wide: with one more for each sum and maximum they were the binning's whole time).
+// The sums and maxima go to the block's own BinSum, and the last block to finish adds those
+// up and, given `host`, writes the totals there.
+struct BinBlock {
+    int cnt[NBINS], need[NBINS], span[NBINS], base[NBINS], sparse[NBINS], na_max[NBINS];
+    u64 work[NBINS], nc[NBINS], na[NBINS];
+    u64 dir, dir_base;
+    int last;
+};
+
+DEVI void bin_clear(BinBlock &B)
 {
-    __shared__ int s_cnt[NBINS], s_need[NBINS], s_span[NBINS], s_base[NBINS], s_sparse[NBINS], s_na_max[NBINS];
-    __shared__ unsigned long long s_work[NBINS], s_nc[NBINS], s_na[NBINS];
-    __shared__ unsigned long long s_dir, s_dir_base;
-    if (threadIdx.x < NBINS) {
-        s_cnt[threadIdx.x] = 0;
-        s_need[threadIdx.x] = 0;
-        s_span[threadIdx.x] = 0;
-        s_work[threadIdx.x] = 0;
-        s_nc[threadIdx.x] = 0;
-        s_na[threadIdx.x] = 0;
-        s_sparse[threadIdx.x] = 0;
-        s_na_max[threadIdx.x] = 0;
+    const int t = threadIdx.x;
+    if (t < NBINS) {
+        B.cnt[t] = B.need[t] = B.span[t] = B.sparse[t] = B.na_max[t] = 0;
+        B.work[t] = B.nc[t] = B.na[t] = 0;
     }
-    if (threadIdx.x == 0)
-        s_dir = 0;
-    __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * BS + threadIdx.x;
-    const bool with_long = st->max_brow >= LONG_TILES;
-    int b = -1, S = 0, nA = 0, nc = 0, sp = 0;
+    if (t == 0)
+        B.dir = 0;
+}
+
+// Where one of the block's rows goes.
+struct BinPlace {
+    int b = -1, pos = 0;
+    long long dloc = -1;
+};
+
+// One row per lane of a wave (every lane of the wave calls it; r.prod == 0: no row).
+DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, bool with_long, const BinParams &bp, DevStats *st)
+{
+    BinPlace at;
+    int sp = 0;
     bool wide = false;
-    long long work = 0, need = 0, E = 0;
-    if (i < M && rprod[i] > 0) {
-        S = rmax[i] - rmin[i] + 1;
-        nA = Arp[i + 1] - Arp[i];
-        const int tp = rtp[i];
-        const long long prod = rprod[i];
+    long long work = 0;
+    int need = 0, E = 0;
+    if (r.prod > 0) {
         if (numeric) {
-            nc = rnnz[i];
-            work = prod;
-            auto nd = [&](int bin) { return num_need(bin, S, nc, nA, tp, prod, with_long); };
-            b = choose_bin(work, nd, bp);
-            need = nd(b);
+            work = r.prod;
+            auto nd = [&](int bin) { return num_need(bin, r.S, r.nc, r.nA, r.tp, r.prod, with_long); };
+            at.b = choose_bin(work, nd, bp);
+            need = nd(at.b);
         } else {
-            need = sym_need(S, nA, tp, with_long);
-            work = tp;
-            b = choose_bin(work, [&](int) { return need; }, bp);
-        }
-        sp = use_sparse(S, tp) ? 1 : 0;
-        if (!numeric) {
+            work = r.tp;
+            need = sym_need(r.S, r.nA, r.tp, with_long);
+            at.b = choose_bin(work, [&](int) { return need; }, bp);
             // the numeric need with nnz(C_i) <= min(products, 64 * span)
-            const long long nub = prod < 64LL * S ? prod : 64LL * S;
-            wide = num_need(NLDS - 1, S, nub, nA, tp, prod, with_long) > bp.lds_row_max;
+            const long long nub = r.prod < 64LL * r.S ? r.prod : 64LL * r.S;
+            wide = num_need(NLDS - 1, r.S, (int)(nub < INT_MAX ? nub : INT_MAX), r.nA, r.tp, r.prod, with_long) > bp.lds_row_max;
+            // directory entries kept for the numeric phase: the row's form in an LDS bin, the
+            // flat span for rows the symbolic phase handles in global memory
+            E = at.b < BIN_GLOBAL ? dir_entries(r.S, r.tp) : r.S;
         }
-        // directory entries kept for the numeric phase: the row's form in an LDS bin, the
-        // flat span for rows the symbolic phase handles in global memory
-        if (!numeric)
-            E = b < BIN_GLOBAL ? dir_entries(S, tp) : S;
+        sp = use_sparse(r.S, r.tp) ? 1 : 0;
     }
-    // Aggregate per wave first: the lanes that chose one bin (neighbouring rows usually
-    // share it) add their counts and sums with one LDS atomic per bin per wave, instead
-    // of one per lane on the same LDS word.
     const int lane = threadIdx.x & 63;
     const u64 wides = __ballot(wide);
     if (lane == 0 && wides)
-        atomicAdd(&st->num_wide_hint, (unsigned long long)__popcll(wides));
-    // nonzeros of the wide rows whose work is split into several items (their compensated
-    // FP32 partial sums meet in a scratch buffer of this size)
-    if (numeric) {
-        const unsigned long long sn =
-            wave_sum<unsigned long long>(b == BIN_GLOBAL && nA > wide_split(nc) ? (unsigned long long)nc : 0ull);
+        atomicAdd(&st->num_wide_hint, (u64)__popcll(wides));
+    // nonzeros of the wide rows whose work is split into several items (their partial sums
+    // meet in a scratch buffer of this size when C holds FP32), and the tiles they span
+    if (numeric && __ballot(at.b == BIN_GLOBAL)) {
+        const u64 sn = wave_sum(at.b == BIN_GLOBAL && r.nA > wide_split(r.nc) ? (u64)r.nc : 0ull);
+        const u64 ss = wave_sum(at.b == BIN_GLOBAL ? (u64)r.S : 0ull);
         if (lane == 0 && sn)
             atomicAdd(&st->wide_split_nnz, sn);
-        const unsigned long long ss = wave_sum<unsigned long long>(b == BIN_GLOBAL ? (unsigned long long)S : 0ull);
         if (lane == 0 && ss)
             atomicAdd(&st->wide_span, ss);
     }
-    int pos = 0;
-    long long dloc = -1;
-    u64 pending = __ballot(b >= 0);
+    // the lanes that chose one bin (neighbouring rows usually share it) add up first
+    u64 pending = __ballot(at.b >= 0);
     while (pending) {
-        const int leader = __ffsll((unsigned long long)pending) - 1;
-        const int bb = __shfl(b, leader, 64);
-        const u64 same = __ballot(b == bb);
+        const int leader = (int)__builtin_ctzll(pending);
+        const int bb = __builtin_amdgcn_readlane(at.b, leader);
+        const bool mine = at.b == bb;
+        const u64 same = __ballot(mine);
         pending &= ~same;
-        const bool mine = b == bb;
-        const unsigned long long wsum = wave_sum<unsigned long long>(mine ? (unsigned long long)work : 0ull);
-        const unsigned long long ncs = wave_sum<unsigned long long>(mine ? (unsigned long long)nc : 0ull);
-        const unsigned long long nas = wave_sum<unsigned long long>(mine ? (unsigned long long)nA : 0ull);
-        const int needm = wave_max<int>(mine ? (int)(need < INT_MAX ? need : INT_MAX) : 0);
-        const int spanm = wave_max<int>(mine ? S : 0);
-        const int nam = wave_max<int>(mine ? nA : 0);
-        const int sps = wave_sum<int>(mine ? sp : 0);
-        const unsigned long long dincl = wave_incl_scan<unsigned long long>(mine ? (unsigned long long)E : 0ull);
-        const unsigned long long dtot = __shfl(dincl, 63, 64);
+        const u64 wsum = wave_sum(mine ? (u64)work : 0ull);
+        const u64 nas = wave_sum(mine ? (u64)r.nA : 0ull);
+        const u64 ncs = numeric ? wave_sum(mine ? (u64)r.nc : 0ull) : 0ull;
+        const int needm = wave_max(mine ? need : 0);
+        const int spanm = wave_max(mine ? r.S : 0);
+        const int nam = wave_max(mine ? r.nA : 0);
+        const int sps = (int)__popcll(__ballot(mine && sp));
+        const u64 dincl = numeric ? 0ull : wave_incl_scan(mine ? (u64)E : 0ull);
+        const u64 dtot = numeric ? 0ull : wave_last(dincl);
         int base = 0;
-        unsigned long long dbase = 0;
+        u64 dbase = 0;
         if (lane == leader) {
-            base = atomicAdd(&s_cnt[bb], __popcll(same));
-            atomicMax(&s_need[bb], needm);
-            atomicMax(&s_span[bb], spanm);
-            atomicMax(&s_na_max[bb], nam);
-            atomicAdd(&s_work[bb], wsum);
-            atomicAdd(&s_nc[bb], ncs);
-            atomicAdd(&s_na[bb], nas);
+            base = atomicAdd(&B.cnt[bb], (int)__popcll(same));
+            atomicMax(&B.need[bb], needm);
+            atomicMax(&B.span[bb], spanm);
+            atomicMax(&B.na_max[bb], nam);
+            atomicAdd(&B.work[bb], wsum);
+            atomicAdd(&B.na[bb], nas);
+            if (ncs)
+                atomicAdd(&B.nc[bb], ncs);
             if (sps)
-                atomicAdd(&s_sparse[bb], sps);
+                atomicAdd(&B.sparse[bb], sps);
             if (dtot)
-                dbase = atomicAdd(&s_dir, dtot);
+                dbase = atomicAdd(&B.dir, dtot);
         }
-        base = __shfl(base, leader, 64);
-        dbase = __shfl(dbase, leader, 64);
+        base = __builtin_amdgcn_readlane(base, leader);
+        dbase = readlane_u64(dbase, leader);
         if (mine) {
-            pos = base + mbcnt(same);
+            at.pos = base + mbcnt(same);
             if (E > 0)
-                dloc = (long long)(dbase + dincl) - E;
+                at.dloc = (long long)(dbase + dincl) - E;
         }
     }
-    __syncthreads();
-    BinStats *bs = numeric ? &st->num : &st->sym;
-    if (threadIdx.x < NBINS) {
-        const int c = s_cnt[threadIdx.x];
-        s_base[threadIdx.x] = c ? atomicAdd(&bs->count[threadIdx.x], c) : 0;
-        if (c) {
-            atomicMax(&bs->max_need[threadIdx.x], s_need[threadIdx.x]);
-            atomicMax(&bs->max_span[threadIdx.x], s_span[threadIdx.x]);
-            atomicMax(&bs->max_na[threadIdx.x], s_na_max[threadIdx.x]);
-            atomicAdd(&bs->work[threadIdx.x], s_work[threadIdx.x]);
-            atomicAdd(&bs->nnz_c[threadIdx.x], s_nc[threadIdx.x]);
-            atomicAdd(&bs->nnz_a[threadIdx.x], s_na[threadIdx.x]);
-            if (s_sparse[threadIdx.x])
-                atomicAdd(&bs->nsparse[threadIdx.x], s_sparse[threadIdx.x]);
-        }
-    }
-    if (!numeric && threadIdx.x == NBINS)
-        s_dir_base = s_dir ? atomicAdd(&st->dir_total, s_dir) : 0;
-    __syncthreads();
-    if (b >= 0)
-        binrows[(int64_t)b * M + s_base[b] + pos] = (int)i;
-    if (!numeric && i < M)
-        rdir[i] = dloc >= 0 ? (long long)s_dir_base + dloc : -1;
+    return at;
 }
 
-hipError_t launch_bin(int numeric, int64_t M, const int *Arp, const long long *rprod, const int *rtp, const int *rmin,
-                      const int *rmax, const int *rnnz, BinParams bp, int *binrows, long long *rdir, DevStats *st,
-                      int num_cus, hipStream_t s)
+// Reserve the places of the block's rows (every thread of the block; after a barrier).
+DEVI void bin_reserve(BinBlock &B, int numeric, DevStats *st, BinSum *sums)
+{
+    const int t = threadIdx.x;
+    BinStats *bs = numeric ? &st->num : &st->sym;
+    if (t < NBINS) {
+        const int c = B.cnt[t];
+        B.base[t] = c ? atomicAdd(&bs->count[t], c) : 0;
+        BinSum *s = sums + (size_t)blockIdx.x * NBINS + t;
+        device_store(&s->work, B.work[t]);
+        device_store(&s->nnz_c, B.nc[t]);
+        device_store(&s->nnz_a, B.na[t]);
+        device_store(&s->need_span, (u64)(unsigned)B.need[t] | ((u64)(unsigned)B.span[t] << 32));
+        device_store(&s->na_sparse, (u64)(unsigned)B.na_max[t] | ((u64)(unsigned)B.sparse[t] << 32));
+    }
+    if (!numeric && t == NBINS)
+        B.dir_base = B.dir ? atomicAdd(&st->dir_total, B.dir) : 0;
+    __syncthreads();
+}
+
+// The end of a binning: the last block adds the blocks' sums up and hands the counters to
+// the host.  Every thread of the block (of blockDim.x >= NBINS).
+DEVI void bin_finish(BinBlock &B, int numeric, DevStats *st, const BinSum *sums, unsigned *done, DevStats *host)
+{
+    const int t = threadIdx.x;
+    const int nblk = (int)gridDim.x;
+    if (nblk > 1) {
+        // each thread's own updates are done (at the device's point of coherence: no cache
+        // has to be written back)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (t == 0)
+            B.last = atomicAdd(done, 1u) == (unsigned)nblk - 1;
+        __syncthreads();
+        if (!B.last)
+            return;
+        bin_clear(B);
+        __syncthreads();
+        const int parts = (int)blockDim.x / NBINS, bin = t % NBINS;
+        if (t / NBINS < parts) {
+            u64 w = 0, nc = 0, na = 0;
+            unsigned need = 0, span = 0, nam = 0, sp = 0;
+#pragma unroll 4
+            for (int q = t / NBINS; q < nblk; q += parts) {
+                const BinSum *s = sums + (size_t)q * NBINS + bin;
+                w += device_load(&s->work);
+                nc += device_load(&s->nnz_c);
+                na += device_load(&s->nnz_a);
+                const u64 x = device_load(&s->need_span), y = device_load(&s->na_sparse);
+                need = (unsigned)x > need ? (unsigned)x : need;
+                span = (unsigned)(x >> 32) > span ? (unsigned)(x >> 32) : span;
+                nam = (unsigned)y > nam ? (unsigned)y : nam;
+                sp += (unsigned)(y >> 32);
+            }
+            atomicAdd(&B.work[bin], w);
+            atomicAdd(&B.nc[bin], nc);
+            atomicAdd(&B.na[bin], na);
+            atomicMax(&B.need[bin], (int)need);
+            atomicMax(&B.span[bin], (int)span);
+            atomicMax(&B.na_max[bin], (int)nam);
+            atomicAdd(&B.sparse[bin], (int)sp);
+        }
+        __syncthreads();
+    }
+    BinStats *bs = numeric ? &st->num : &st->sym;
+    if (t < NBINS) {
+        device_store(&bs->work[t], B.work[t]);
+        device_store(&bs->nnz_c[t], B.nc[t]);
+        device_store(&bs->nnz_a[t], B.na[t]);
+        device_store(&bs->max_need[t], B.need[t]);
+        device_store(&bs->max_span[t], B.span[t]);
+        device_store(&bs->max_na[t], B.na_max[t]);
+        device_store(&bs->nsparse[t], B.sparse[t]);
+    }
+    if (!host)
+        return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const unsigned *from = (const unsigned *)st;
+    unsigned *to = (unsigned *)host;
+    for (unsigned q = t; q < sizeof(DevStats) / sizeof(unsigned); q += blockDim.x)
+        to[q] = device_load(&from[q]);
+}
+
+// ---- row analysis of A ---------------------------------------------------------------
+
+// Per row i of A: products sum_j nnz(B_j), tile-products sum_j tiles(B_j), and the span
+// [rmin, rmax] of tile columns of row i of C (rows of B are sorted, so each B row's first
+// and last tile bound it); then the symbolic binning of the block's rows.  Reference:
+// k_compute_flop, src/small/mask.cuh:14-51.
+// A group of G lanes per row; a block takes `rows` rows, 256 / G at a time, and bins them
+// together, so that the binning's atomics are few and hide behind other blocks' gathers.
+// Rows of more than LONG_A entries per lane are listed and left to whole waves, those of
+// more than LONG_WAVE entries to the whole block (at 2,048 entries for every group width,
+// a hub row's 16 lanes kept an R-MAT graph's analysis waiting).
+constexpr int LONG_A = 16;
+constexpr int LONG_WAVE = 4096;
+constexpr int RI_BS = 1024;
+constexpr int ROWS_MAX = 2048; // rows of a block
+
+template <int G>
+__global__ __launch_bounds__(RI_BS) void k_row_info(int64_t M, int64_t K, int64_t nnzA, int rows,
+                                                  const int *__restrict__ Arp, const int *__restrict__ Acol,
+                                                  const BRow *__restrict__ brow, const int *__restrict__ tptr,
+                                                  long long *__restrict__ rprod, int *__restrict__ rtp, int *__restrict__ rmin,
+                                                  int *__restrict__ rmax, int *__restrict__ rnnz, BinParams bp,
+                                                  int *__restrict__ binrows, long long *__restrict__ rdir,
+                                                  DevStats *st, BinSum *sums, unsigned *done, DevStats *host)
+{
+    constexpr int RPB = RI_BS / G, NW = RI_BS / 64;
+    __shared__ long long s_prod[ROWS_MAX];
+    __shared__ int s_tp[ROWS_MAX], s_mn[ROWS_MAX], s_mx[ROWS_MAX];
+    __shared__ BinBlock B;
+    __shared__ long long s_p[NW];
+    __shared__ int s_t[NW], s_n[NW], s_x[NW];
+    __shared__ int s_long;
+    __shared__ unsigned short s_list[ROWS_MAX];
+    const int t = threadIdx.x, g = t / G, l = t & (G - 1);
+    const int64_t i0 = (int64_t)blockIdx.x * rows;
+    const int n = (int)(M - i0 < rows ? M - i0 : rows);
+    int bad = 0;
+    bin_clear(B);
+    if (t == 0)
+        s_long = 0;
+    __syncthreads();
+    auto entry = [&](int j, long long &p, int &tp, int &mn, int &mx) {
+        if ((unsigned)j >= (unsigned long long)K) {
+            bad |= ERR_ACOL;
+            return;
+        }
+        const BRow q = brow[j];
+        p += q.len;
+        tp += q.ntiles >= 0 ? q.ntiles : tptr[j + 1] - tptr[j];
+        mn = q.first < mn ? q.first : mn;
+        mx = q.last > mx ? q.last : mx;
+    };
+    // RU rows per group at a time: their dependent loads (row extent, column, record of B's
+    // row) are issued together
+    constexpr int RU = 4;
+    for (int q0 = g; q0 < n; q0 += RU * RPB) {
+        int s[RU], e[RU], tp[RU], mn[RU], mx[RU];
+        long long p[RU];
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            const int q = q0 + u * RPB;
+            s[u] = e[u] = 0;
+            if (q < n) {
+                s[u] = Arp[i0 + q];
+                e[u] = Arp[i0 + q + 1];
+            }
+        }
+        int j[RU];
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            p[u] = 0;
+            tp[u] = 0;
+            mn[u] = INT_MAX;
+            mx[u] = -1;
+            if (s[u] < 0 || e[u] < s[u] || (int64_t)e[u] > nnzA) {
+                bad |= ERR_ROWPTR;
+                e[u] = s[u] = 0;
+            } else if (e[u] - s[u] > LONG_A * G) {
+                if (l == 0)
+                    s_list[atomicAdd(&s_long, 1)] = (unsigned short)(q0 + u * RPB);
+                e[u] = s[u];
+            }
+            j[u] = s[u] + l < e[u] ? Acol[s[u] + l] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+            if (s[u] + l < e[u])
+                entry(j[u], p[u], tp[u], mn[u], mx[u]);
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+            for (int k = s[u] + l + G; k < e[u]; k += G)
+                entry(Acol[k], p[u], tp[u], mn[u], mx[u]);
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            const int q = q0 + u * RPB;
+            const long long ps = group_sum<G>(p[u]);
+            const int ts = group_sum<G>(tp[u]), ms = group_min<G>(mn[u]), xs = group_max<G>(mx[u]);
+            if (q < n && l == 0) {
+                s_prod[q] = ps;
+                s_tp[q] = ts;
+                s_mn[q] = ms;
+                s_mx[q] = xs;
+            }
+        }
+    }
+    __syncthreads();
+    const int nlong = s_long;
+    for (int i = t >> 6; i < nlong; i += NW) { // listed rows: a wave each
+        const int q = s_list[i], lane = t & 63;
+        const int s = Arp[i0 + q], e = Arp[i0 + q + 1];
+        if (e - s > LONG_WAVE)
+            continue;
+        long long p = 0;
+        int tp = 0, mn = INT_MAX, mx = -1;
+#pragma unroll 4
+        for (int k = s + lane; k < e; k += 64)
+            entry(Acol[k], p, tp, mn, mx);
+        p = wave_sum(p);
+        tp = wave_sum(tp);
+        mn = group_min<64>(mn);
+        mx = group_max<64>(mx);
+        if (lane == 0) {
+            s_prod[q] = p;
+            s_tp[q] = tp;
+            s_mn[q] = mn;
+            s_mx[q] = mx;
+        }
+    }
+    for (int i = 0; i < nlong; ++i) { // the longest: the block each
+        const int q = s_list[i];
+        const int s = Arp[i0 + q], e = Arp[i0 + q + 1];
+        if (e - s <= LONG_WAVE)
+            continue;
+        long long p = 0;
+        int tp = 0, mn = INT_MAX, mx = -1;
+#pragma unroll 4
+        for (int k = s + t; k < e; k += RI_BS)
+            entry(Acol[k], p, tp, mn, mx);
+        p = wave_sum(p);
+        tp = wave_sum(tp);
+        mn = group_min<64>(mn);
+        mx = group_max<64>(mx);
+        if ((t & 63) == 0) {
+            s_p[t >> 6] = p;
+            s_t[t >> 6] = tp;
+            s_n[t >> 6] = mn;
+            s_x[t >> 6] = mx;
+        }
+        __syncthreads();
+        if (t == 0) {
+            for (int w = 1; w < NW; ++w) {
+                p += s_p[w];
+                tp += s_t[w];
+                mn = s_n[w] < mn ? s_n[w] : mn;
+                mx = s_x[w] > mx ? s_x[w] : mx;
+            }
+            s_prod[q] = p;
+            s_tp[q] = tp;
+            s_mn[q] = mn;
+            s_mx[q] = mx;
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    if (bad)
+        atomicOr(&st->err, bad);
+    // the rows' values, and their bins
+    const bool with_long = st->max_brow >= LONG_TILES;
+    BinPlace at[ROWS_MAX / RI_BS];
+#pragma unroll
+    for (int u = 0; u < ROWS_MAX / RI_BS; ++u) {
+        if (u * RI_BS >= n) // uniform
+            break;
+        const int q = u * RI_BS + t;
+        BinRow r = {0, 0, 0, 0, 0};
+        if (q < n) {
+            const int64_t i = i0 + q;
+            const int mn = s_mn[q], mx = s_mx[q];
+            r.prod = s_prod[q];
+            r.S = mx - mn + 1;
+            r.tp = s_tp[q];
+            r.nA = Arp[i + 1] - Arp[i];
+            rprod[i] = r.prod;
+            rtp[i] = r.tp;
+            rmin[i] = mn;
+            rmax[i] = mx;
+            if (r.prod == 0)
+                rnnz[i] = 0;
+        }
+        at[u] = bin_row(B, 0, r, with_long, bp, st);
+    }
+    __syncthreads();
+    bin_reserve(B, 0, st, sums);
+#pragma unroll
+    for (int u = 0; u < ROWS_MAX / RI_BS; ++u) {
+        const int q = u * RI_BS + t;
+        if (q >= n)
+            break;
+        if (at[u].b >= 0)
+            binrows[(int64_t)at[u].b * M + B.base[at[u].b] + at[u].pos] = (int)(i0 + q);
+        rdir[i0 + q] = at[u].dloc >= 0 ? (long long)B.dir_base + at[u].dloc : -1;
+    }
+    bin_finish(B, 0, st, sums, done, host);
+}
+
+static int row_info_lanes(int64_t M, int64_t nnzA)
+{
+    const int64_t avg = nnzA / (M > 0 ? M : 1);
+    return avg <= 12 ? 8 : (avg <= 24 ? 16 : (avg <= 48 ? 32 : 64));
+}
+
+// Rows per block: two blocks per CU hold all its waves; beyond that, as many rows as the
+// block's LDS holds, for fewer atomics per row.
+static int row_info_rows(int64_t M, int64_t nnzA, int num_cus)
+{
+    const int rpb = RI_BS / row_info_lanes(M, nnzA);
+    const int64_t full = (int64_t)rpb * 2 * num_cus;
+    int64_t passes = (M + full - 1) / full;
+    passes = passes < 1 ? 1 : (passes > ROWS_MAX / rpb ? ROWS_MAX / rpb : passes);
+    return (int)passes * rpb;
+}
+
+int64_t row_info_blocks(int64_t M, int64_t nnzA, int num_cus)
+{
+    const int rows = row_info_rows(M, nnzA, num_cus);
+    return (M + rows - 1) / rows;
+}
+
+hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, const int *Acol, const BRow *brow,
+                           const int *tptr, long long *rprod, int *rtp, int *rmin, int *rmax, int *rnnz, BinParams bp,
+                           int *binrows, long long *rdir, DevStats *st, BinSum *sums, unsigned *done, DevStats *host,
+                           int num_cus, hipStream_t s)
+{
+    const int rows = row_info_rows(M, nnzA, num_cus);
+    const unsigned blocks = (unsigned)row_info_blocks(M, nnzA, num_cus);
+#define ROW_INFO(G)                                                                                                    \
+    case G:                                                                                                            \
+        hipLaunchKernelGGL((k_row_info<G>), dim3(blocks), dim3(RI_BS), 0, s, M, K, nnzA, rows, Arp, Acol, brow, tptr,  \
+                           rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, st, sums, done, host);                     \
+        break;
+    switch (row_info_lanes(M, nnzA)) {
+        ROW_INFO(8) ROW_INFO(16) ROW_INFO(32) ROW_INFO(64)
+    }
+#undef ROW_INFO
+    return hipGetLastError();
+}
+
+// C's row pointers from nnz(C_i) (chained scan) and the numeric binning, a lane per row.  out32 (may be null): the row pointers as int32 too, for the caller.
+constexpr int RP_BS = 1024;
+
+__global__ __launch_bounds__(RP_BS) void k_rowptr_bin(int64_t M, const int *__restrict__ Arp,
+                                                    const long long *__restrict__ rprod, const int *__restrict__ rtp,
+                                                    const int *__restrict__ rmin, const int *__restrict__ rmax,
+                                                    const int *__restrict__ rnnz, long long *__restrict__ crp,
+                                                    int *__restrict__ out32, BinParams bp, int *__restrict__ binrows,
+                                                    u64 *words, unsigned *ticket, DevStats *st, BinSum *sums,
+                                                    unsigned *done, DevStats *host)
+{
+    __shared__ BinBlock B;
+    __shared__ u64 red[RP_BS / 64];
+    __shared__ u64 s_pre;
+    __shared__ int s_b;
+    const int t = threadIdx.x;
+    bin_clear(B);
+    if (t == 0)
+        s_b = gridDim.x > 1 ? (int)atomicAdd(ticket, 1u) : 0;
+    __syncthreads();
+    const int b = uniform(s_b);
+    const int64_t i = (int64_t)b * RP_BS + t;
+    const int nc = i < M ? rnnz[i] : 0;
+    u64 total;
+    const u64 pre = group_excl_scan<RP_BS, u64>((u64)(unsigned)nc, red, total);
+    if (t < 64) {
+        const u64 before = chain_prefix(words, b, total);
+        if (t == 0)
+            s_pre = before;
+    }
+    const bool with_long = st->max_brow >= LONG_TILES;
+    BinRow r = {0, 0, 0, 0, 0};
+    if (i < M) {
+        r.prod = rprod[i];
+        r.nc = nc;
+        r.S = rmax[i] - rmin[i] + 1;
+        r.nA = Arp[i + 1] - Arp[i];
+        r.tp = rtp[i];
+    }
+    const BinPlace at = bin_row(B, 1, r, with_long, bp, st);
+    __syncthreads();
+    if (i < M) {
+        const u64 at0 = s_pre + pre, end = at0 + (u64)(unsigned)nc;
+        crp[i] = (long long)at0;
+        if (out32)
+            out32[i] = (int)at0;
+        if (i == M - 1) {
+            crp[M] = (long long)end;
+            if (out32)
+                out32[M] = (int)end;
+            device_store(&st->nnz_c, (long long)end);
+        }
+    }
+    bin_reserve(B, 1, st, sums);
+    if (at.b >= 0)
+        binrows[(int64_t)at.b * M + B.base[at.b] + at.pos] = (int)i;
+    bin_finish(B, 1, st, sums, done, host);
+}
+
+int64_t rowptr_blocks(int64_t M) { return (M + RP_BS - 1) / RP_BS; }
+
+hipError_t launch_rowptr_bin(int64_t M, const int *Arp, const long long *rprod, const int *rtp, const int *rmin,
+                             const int *rmax, const int *rnnz, long long *crp, int *out32, BinParams bp, int *binrows,
+                             u64 *words, unsigned *ticket, DevStats *st, BinSum *sums, unsigned *done, DevStats *host,
+                             hipStream_t s)
 {
     if (M <= 0)
         return hipSuccess;
-    const int64_t small = (M + 255) / 256;
-    if (small <= 4LL * num_cus)
-        hipLaunchKernelGGL(k_bin<256>, dim3((unsigned)small), dim3(256), 0, s, numeric, M, Arp, rprod, rtp, rmin, rmax,
-                           rnnz, bp, binrows, rdir, st);
-    else
-        hipLaunchKernelGGL(k_bin<1024>, dim3((unsigned)((M + 1023) / 1024)), dim3(1024), 0, s, numeric, M, Arp, rprod,
-                           rtp, rmin, rmax, rnnz, bp, binrows, rdir, st);
+    hipLaunchKernelGGL(k_rowptr_bin, dim3((unsigned)rowptr_blocks(M)), dim3(RP_BS), 0, s, M, Arp, rprod, rtp, rmin, rmax,
+                       rnnz, crp, out32, bp, binrows, words, ticket, st, sums, done, host);
     return hipGetLastError();
 }
 
 // ---- misc ------------------------------------------------------------------------------------
-
-__global__ __launch_bounds__(256) void k_i64_to_i32(const long long *__restrict__ in, int64_t n, int *__restrict__ out)
-{
-    const int64_t stride = (int64_t)gridDim.x * 256;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride)
-        out[i] = (int)in[i];
-}
-
-hipError_t launch_rowptr_i64_to_i32(const long long *in, int64_t n, int *out, hipStream_t s)
-{
-    int64_t blocks = (n + 255) / 256;
-    if (blocks > 8192)
-        blocks = 8192;
-    if (blocks < 1)
-        blocks = 1;
-    hipLaunchKernelGGL(k_i64_to_i32, dim3((unsigned)blocks), dim3(256), 0, s, in, n, out);
-    return hipGetLastError();
-}
 
 __global__ void k_pad_b(const int *col, const void *val, int val32, int n, int *pcol, void *pval)
 {
@@ -806,8 +985,8 @@ __global__ __launch_bounds__(256) void k_row_sums(int64_t M, const RP *__restric
             s += v;
             a += v < 0 ? -v : v;
         }
-        s = wave_sum<double>(s);
-        a = wave_sum<double>(a);
+        s = wave_sum(s);
+        a = wave_sum(a);
         if (lane == 0) {
             sum[i] = s;
             asum[i] = a;
