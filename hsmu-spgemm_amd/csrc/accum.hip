@@ -13,8 +13,8 @@
 // column list, src/compressed/compressed_Cval.cuh:5-69 and src/small/numeric.cuh:233-253);
 // a dense form (one slot per column of a short, full span) skips the directory.  The
 // numeric kernels also write C's sorted columns, replacing the reference's rank-sort pass
-// (compressed_Ccol_symbolic.cuh:4-63); for the wide rows of the FP64 path a separate
-// streaming kernel (k_wide_cols) writes them from the kept directories.
+// (compressed_Ccol_symbolic.cuh:4-63); for the wide rows a separate streaming kernel
+// (k_wide_cols) writes them from the kept directories.
 //
 // The kernels of rows that share a wave, and the symbolic ones, stage the row's A entries (B
 // row range, first tile, a_ij) in LDS once; sub-groups of lanes then take one entry each
@@ -435,9 +435,9 @@ struct Pair {
 // wave loaded while the STREAM_U before them are added (the loads are not predicated, so
 // that a wait for one set is not a wait for the other).
 constexpr int STREAM_U = 2;
-template <int G, int FORM, typename P>
+template <int G, int FORM, typename P, typename Off>
 DEVI void stream_add(const Stream<G> &st, long long w0, const Operands &op, const u64 *cm, const unsigned *coff,
-                     const u64 *fm, const unsigned *foff, double *vals, int mn)
+                     const u64 *fm, const Off *foff, double *vals, int mn)
 {
     typedef typename P::V V;
     constexpr int NW = G / 64, U = STREAM_U;
@@ -1544,122 +1544,180 @@ __global__ __launch_bounds__(1024) void k_numeric_wcompact(const int *__restrict
     }
 }
 
-// Work items of the split wide-row kernel: each row's entries in runs of
-// wide_split(nnz(C_i)), listed largest rows first (classes of half an octave of nnz(C_i),
-// by a counting sort): the big rows start early (their items bound the tail), and the
-// workgroups that run together work on rows of similar size, which move through their
-// columns, and so through the shared rows of B, at similar paces.
-// ctr: [0] items listed, [1] items taken, [2, 2 + WS_CLASSES) items per class,
-// [2 + WS_CLASSES, 2 + 2 WS_CLASSES) first item of each class.
-constexpr int WS_CLASSES = 32;
-DEVI int wide_class(long long n)
-{
-    const int lg2 = n > 1 ? 2 * (63 - __builtin_clzll((unsigned long long)n)) +
-                                (((unsigned long long)n >> (62 - __builtin_clzll((unsigned long long)n))) & 1)
-                          : 0; // 2 log2(n), rounded down to half octaves
-    const int c = lg2 - 20; // below 2^10: class 0
-    return c < 0 ? 0 : (c >= WS_CLASSES ? WS_CLASSES - 1 : c);
-}
+// ---- wide rows as windows -----------------------------------------------------------------
 
-DEVI void wide_row_items(const int *rows, int idx, const int *Arp, const long long *crp, int vals, int &row, int &nA,
-                         int &sz, int &ns, int &cls)
+// The first element of every B row at each unit's start (and the row's end): index[j * (U + 1)
+// + u] = first element of row j with a column of unit u or later.  A lane per (row, unit),
+// binary search in the row (neighbouring lanes search one row).
+__global__ __launch_bounds__(256) void k_wide_index(long long K, long long U, const int *__restrict__ rp,
+                                                    const int *__restrict__ col, int *__restrict__ index)
 {
-    row = rows[idx];
-    nA = Arp[row + 1] - Arp[row];
-    const long long n = crp[row + 1] - crp[row];
-    sz = wide_split(n, vals);
-    ns = nA > 0 ? (nA + sz - 1) / sz : 1;
-    cls = wide_class(n);
-}
-
-// pass 1: items per class (per-workgroup counts in LDS, one global atomic per class)
-__global__ __launch_bounds__(256) void k_wide_count(const int *__restrict__ rows, const int *__restrict__ count_p,
-                                                    const int *__restrict__ Arp, const long long *__restrict__ crp,
-                                                    int vals, unsigned *ctr)
-{
-    __shared__ unsigned lc[WS_CLASSES];
-    if (threadIdx.x < WS_CLASSES)
-        lc[threadIdx.x] = 0;
-    __syncthreads();
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (idx < *count_p) {
-        int row, nA, sz, ns, cls;
-        wide_row_items(rows, idx, Arp, crp, vals, row, nA, sz, ns, cls);
-        atomicAdd(&lc[cls], (unsigned)ns);
+    const long long n = K * (U + 1), stride = (long long)gridDim.x * 256;
+    for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < n; q += stride) {
+        const long long j = q / (U + 1), u = q - j * (U + 1);
+        int lo = rp[j], hi = rp[j + 1];
+        if (u == 0)
+            hi = lo;
+        else if (u == U)
+            lo = hi;
+        const int c = (int)(u * WIDE_UNIT < INT_MAX ? u * WIDE_UNIT : INT_MAX);
+        while (lo < hi) {
+            const int mid = lo + ((hi - lo) >> 1);
+            if (col[mid] < c)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        index[q] = lo;
     }
-    __syncthreads();
-    if (threadIdx.x < WS_CLASSES && lc[threadIdx.x])
-        atomicAdd(&ctr[2 + threadIdx.x], lc[threadIdx.x]);
 }
 
-// pass 2 (one thread): first item of each class, largest class first; the total
+// A wide row's directory in global memory, flat or two-level.
+struct WideDir {
+    const u64 *cm, *fm;
+    const unsigned *co, *fo;
+    int mn, S, F; // first tile, tiles spanned, fine entries
+    unsigned n;   // entries of C_i
+    bool two;
+
+    DEVI WideDir(const Operands &op, const long long *crp, int row, long long sym_row_max, int sym_all_global,
+                 int long_rows)
+    {
+        const int nA = uniform(op.Arp[row + 1]) - uniform(op.Arp[row]);
+        const long long cb = uniform64(crp[row]);
+        n = (unsigned)(uniform64(crp[row + 1]) - cb);
+        mn = uniform(op.rmin[row]);
+        S = uniform(op.rmax[row]) - mn + 1;
+        two = wide_two_level(S, nA, uniform(op.rtp[row]), sym_row_max, sym_all_global, long_rows);
+        const int W = two ? (S + 63) >> 6 : 0;
+        const long long rd = uniform64(op.rdir[row]);
+        cm = op.dir_mask + rd;
+        co = op.dir_off + rd;
+        fm = cm + W;
+        fo = co + W;
+        F = two ? (int)(uniform(co[W - 1]) + (unsigned)__popcll(uniform64(cm[W - 1]))) : S;
+    }
+    // entries of C_i before tile t (relative to mn, any integer)
+    DEVI unsigned before(int t) const
+    {
+        if (t <= 0)
+            return 0;
+        if (t >= S)
+            return n;
+        int k = t;
+        if (two) {
+            k = (int)(co[t >> 6] + (unsigned)__popcll(cm[t >> 6] & below(t & 63)));
+            if (k >= F)
+                return n;
+        }
+        return fo[k];
+    }
+    // tile t's mask (0 outside the row's span) and the entries before it
+    DEVI u64 tile(int t, unsigned &off) const
+    {
+        off = 0;
+        if (t < 0 || t >= S)
+            return 0;
+        int k = t;
+        if (two) {
+            const u64 w = cm[t >> 6];
+            if (!((w >> (t & 63)) & 1ull))
+                return 0;
+            k = (int)(co[t >> 6] + (unsigned)__popcll(w & below(t & 63)));
+        }
+        off = fo[k];
+        return fm[k];
+    }
+};
+
+// The windows of the wide rows, a wave per row: greedy runs of units.  FILL = false counts
+// them per bucket (a bucket is a range of first units), FILL = true writes them, so that the
+// list goes through C's columns in order and the workgroups that run together read the same
+// part of B, which then stays in the L2s (R-MAT scale 18: 1/32 of B is 1.5 MB).
+template <bool FILL>
+__global__ __launch_bounds__(256) void k_wide_items(const int *__restrict__ rows, const int *__restrict__ count_p,
+                                                    Operands op, const long long *__restrict__ crp, long long U,
+                                                    long long sym_row_max, int sym_all_global, int long_rows,
+                                                    WideItem *__restrict__ items, long long cap, unsigned *ctr, int *err)
+{
+    __shared__ unsigned cnt[WIDE_BUCKETS], base[WIDE_BUCKETS];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int nrows = *count_p;
+    unsigned *total = ctr + 2, *next = ctr + 2 + WIDE_BUCKETS;
+    // each workgroup takes a contiguous run of rows, twice over: count, then (FILL) write
+    const int per = (nrows + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int i0 = (int)blockIdx.x * per, i1 = i0 + per < nrows ? i0 + per : nrows;
+    for (int pass = 0; pass < (FILL ? 2 : 1); ++pass) {
+        if (threadIdx.x < WIDE_BUCKETS) {
+            if (pass == 1)
+                base[threadIdx.x] = cnt[threadIdx.x] ? atomicAdd(&next[threadIdx.x], cnt[threadIdx.x]) : 0u;
+            cnt[threadIdx.x] = 0;
+        }
+        __syncthreads();
+        for (int i = i0 + w; i < i1; i += 4) {
+            const int row = uniform(rows[i]);
+            const WideDir d(op, crp, row, sym_row_max, sym_all_global, long_rows);
+            const int U0 = d.mn / WIDE_TILES, U1 = (d.mn + d.S - 1) / WIDE_TILES + 1; // units of the row
+            int u = U0;                   // first unit of the open window
+            unsigned at = 0;              // entries before it
+            auto close = [&](int v, unsigned end) { // window [u, v)
+                if (end > at) {
+                    const int b = (int)((long long)u * WIDE_BUCKETS / U);
+                    if (lane == 0) {
+                        const unsigned p = atomicAdd(&cnt[b], 1u);
+                        if (pass == 1) {
+                            const unsigned q = base[b] + p;
+                            if (q < cap)
+                                items[q] = WideItem{row, (unsigned)u | ((unsigned)(v - u) << 24), at, end - at};
+                            else // cannot happen: wide_row_items bounds them
+                                raise_internal(err);
+                        }
+                    }
+                }
+                u = v;
+                at = end;
+            };
+            // lane q holds the entries before unit vb + q
+            for (int vb = U0 + 1; vb <= U1; vb += 64) {
+                const int v = vb + lane;
+                const unsigned off = v < U1 ? d.before(v * WIDE_TILES - d.mn) : d.n;
+                unsigned prev = at; // entries before unit vb + q - 1
+                if (vb > U0 + 1)
+                    prev = d.before((vb - 1) * WIDE_TILES - d.mn);
+                for (int q = 0; q < 64 && vb + q <= U1; ++q) {
+                    const unsigned o = (unsigned)__builtin_amdgcn_readlane((int)off, q);
+                    const int x = vb + q; // unit x - 1 is the one to take in
+                    if (o - at > WIDE_UNIT || x - u > WIDE_UMAX)
+                        close(x - 1, prev);
+                    prev = o;
+                }
+            }
+            close(U1, d.n);
+        }
+        __syncthreads();
+    }
+    if (!FILL && threadIdx.x < WIDE_BUCKETS && cnt[threadIdx.x])
+        atomicAdd(&total[threadIdx.x], cnt[threadIdx.x]);
+}
+
+// one wave: the first window of each bucket; the total
 __global__ void k_wide_order(unsigned *ctr)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0)
-        return;
-    unsigned o = 0;
-    for (int c = WS_CLASSES - 1; c >= 0; --c) {
-        ctr[2 + WS_CLASSES + c] = o;
-        o += ctr[2 + c];
-    }
-    ctr[0] = o;
-}
-
-// pass 3: the items, at per-workgroup ranges of their class
-__global__ __launch_bounds__(256) void k_wide_fill(const int *__restrict__ rows, const int *__restrict__ count_p,
-                                                   const int *__restrict__ Arp, const long long *__restrict__ crp,
-                                                   int vals, WideItem *__restrict__ items, long long cap,
-                                                   unsigned *ctr, unsigned long long *sctr, long long scratch_n,
-                                                   int *err)
-{
-    __shared__ unsigned lc[WS_CLASSES], lb[WS_CLASSES];
-    if (threadIdx.x < WS_CLASSES)
-        lc[threadIdx.x] = 0;
-    __syncthreads();
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    const bool have = idx < *count_p;
-    int row = 0, nA = 0, sz = 1, ns = 0, cls = 0;
-    unsigned local = 0;
-    if (have) {
-        wide_row_items(rows, idx, Arp, crp, vals, row, nA, sz, ns, cls);
-        local = atomicAdd(&lc[cls], (unsigned)ns);
-    }
-    __syncthreads();
-    if (threadIdx.x < WS_CLASSES && lc[threadIdx.x])
-        lb[threadIdx.x] = atomicAdd(&ctr[2 + WS_CLASSES + threadIdx.x], lc[threadIdx.x]);
-    __syncthreads();
-    if (!have)
-        return;
-    const unsigned base = lb[cls] + local;
-    if ((long long)base + ns > cap) { // cannot happen: cap bounds count + nnz(A) / WS_MIN_SPLIT
-        raise_internal(err);
-        return;
-    }
-    // a split row's range of the compensated scratch (sctr: nullptr for FP64)
-    long long sbase = 0;
-    if (sctr && ns > 1) {
-        const long long n = crp[row + 1] - crp[row];
-        sbase = (long long)atomicAdd(sctr, (unsigned long long)n);
-        if (sbase + n > scratch_n) { // cannot happen: scratch_n sums these rows' nnz
-            raise_internal(err);
-            return;
-        }
-    }
-    for (int q = 0; q < ns; ++q) {
-        const int e0 = q * sz;
-        const int e1 = e0 + sz < nA ? e0 + sz : nA;
-        items[base + q] = WideItem{row, e0, e1, ns, sbase};
-    }
+    const int l = threadIdx.x;
+    const unsigned n = l < WIDE_BUCKETS ? ctr[2 + l] : 0u;
+    const unsigned incl = wave_incl_scan(n);
+    if (l < WIDE_BUCKETS)
+        ctr[2 + WIDE_BUCKETS + l] = incl - n;
+    if (l == 63)
+        ctr[0] = incl;
 }
 
 constexpr int WC_BS = 256;     // lanes of a k_wide_cols workgroup
 constexpr int WC_DENSE = 1024; // dense tiles listed per pass (more are written by their lane)
 constexpr int WC_STAGE = 4096; // columns of a flat chunk staged in LDS for coalesced stores
 
-// Columns of the wide rows, from their kept directories, before k_numeric_wsplit adds the
-// values; and, for FP64 (Cval given), zeroed values for the rows split into several items
-// (their items add into C; the compensated form's meet in a zeroed scratch instead).  One
-// workgroup per row.  Flat directory: WC_BS consecutive tiles' columns are one contiguous
+// Columns of the wide rows, from their kept directories (k_numeric_windows writes the
+// values).  One workgroup per row.  Flat directory: WC_BS consecutive tiles' columns are one contiguous
 // range of C, so a scan of the tiles' popcounts places each lane's columns in an LDS stage
 // that the workgroup then stores coalesced.  Chunks of more than WC_STAGE columns, and
 // two-level rows, take the direct path: a lane per tile (flat) or per coarse word,
@@ -1667,9 +1725,8 @@ constexpr int WC_STAGE = 4096; // columns of a flat chunk staged in LDS for coal
 // denser tiles are listed in LDS and written by a wave each, one lane per column.
 __global__ __launch_bounds__(WC_BS) void k_wide_cols(const int *__restrict__ rows, const int *__restrict__ count_p,
                                                      Operands op, const long long *__restrict__ crp,
-                                                     int *__restrict__ Ccol, double *__restrict__ Cval,
-                                                     long long sym_row_max, int sym_all_global, int long_rows,
-                                                     int vals)
+                                                     int *__restrict__ Ccol, long long sym_row_max,
+                                                     int sym_all_global, int long_rows)
 {
     // one buffer, used by one path per chunk: the staged chunk's columns, or the list of
     // its dense tiles (mask, first slot, absolute tile), so that the waves writing them
@@ -1691,9 +1748,6 @@ __global__ __launch_bounds__(WC_BS) void k_wide_cols(const int *__restrict__ row
         const long long n = uniform64(crp[row + 1]) - cb;
         if (n <= 0)
             continue;
-        if (Cval && nA > wide_split(n, vals)) // a split row: its items add into C
-            for (long long q = l; q < n; q += WC_BS)
-                Cval[cb + q] = 0.0;
         const int mn = uniform(op.rmin[row]);
         const int S = uniform(op.rmax[row]) - mn + 1;
         const bool two = wide_two_level(S, nA, uniform(op.rtp[row]), sym_row_max, sym_all_global, long_rows);
@@ -1777,428 +1831,89 @@ __global__ __launch_bounds__(WC_BS) void k_wide_cols(const int *__restrict__ row
     }
 }
 
-// Wide rows (FP64, directory kept): the compact windowed accumulator of k_numeric_wcompact,
-// on work items pulled from a queue.  An item holds at most SPLIT entries of one row, so
-// their cursors into the B rows live in LDS.  Windows are runs of directory entries that
-// share both k / (VW / 2) and (slot of k) / (VW - 64), so a window holds at most VW / 2
-// entries and VW slots (VW: WS_VALS, or WS_VALS_BIG for sparse rows); their starts are listed in parallel (WS_LV entries
-// per lane, a workgroup scan), WS_WIN at a time.  In a window, the elements of the active
-// B rows are spread over the whole workgroup: each active entry gets chunks of WS_CH
-// elements from its cursor, as many as its density (elements left / columns left to its
-// last column) predicts for the window, and every group of WS_GL lanes takes chunks from
-// that list.  B rows are sorted, so a chunk's in-window elements are a prefix of it; the
-// smallest (position, column) after a prefix, kept by a 64-bit LDS atomicMin, is the
-// entry's new cursor and the column there.  An entry whose chunks were all inside the
-// window gets twice as many chunks in another round.  A two-level row's coarse words are staged
-// in LDS when there are at most WS_COARSE of them.  Items of a split row add their window
-// sums into C (zeroed by k_wide_cols, which also writes every wide row's columns) with
-// atomics; the other rows store them.
-constexpr int WS_COARSE = 256;
-constexpr int WS_WIN = 256;  // window starts listed at a time
-constexpr int WS_LV = 8;     // directory entries per lane when listing window starts
-constexpr int WS_GL = 16;    // lanes of a chunk group
-constexpr int WS_CH = 4 * WS_GL; // elements of a chunk (WS_GL lanes x 4)
-constexpr int WS_TCAP = 1024; // chunks listed per round
-// dynamic LDS of a workgroup with windows of vw slots (vw / 2 directory entries) and items
-// of up to wide_split_max(vw) entries
-constexpr int ws_lds(int vw)
+// Wide rows as windows: the compact accumulator over one window's entries of C_i, its part
+// of the row's directory (expanded to one mask and slot per tile of the window) and its
+// elements of the B rows as one stream, their ranges read from the index.  Workgroups take
+// windows from the list until it is used up.  Neither a search nor atomics in C nor a
+// second round: every window's elements are known when it starts, and a window belongs to
+// one workgroup.
+// What bounds it: the chain of a window's phases (item, row, directory; A's entries, index;
+// stream; output), three workgroups per CU.  Against items of up to 512 A entries that kept
+// cursors into the B rows and posted chunks of them window by window (in rounds, with split
+// rows meeting by atomics): R-MAT scale 18 wide rows 22.4 -> 8.9 ms (this kernel 20.5 ->
+// 6.5), a 2,000-row Zipf panel 7.6 -> 4.6 ms.  256 lanes: Zipf 128 / 256 / 512 / 1,024
+// lanes 5.7 / 4.6 / 5.0 / 7.3 ms, R-MAT scale 18 11.2 / 8.9 / 9.0 / 11.9 ms.
+constexpr int WW_TILES = WIDE_TILES * WIDE_UMAX;
+constexpr int WW_BS = 256; // lanes of a workgroup
+template <int BS> constexpr int ww_lds()
 {
-    const int sp = wide_split_max(vw);
-    return (vw * 8 + (vw / 2) * 8 + sp * 8 /* av */ + sp * 8 /* pos:col */ + WS_COARSE * 8 +
-            sp * 4 * 5 /* cur kend last, two act lists */ + WS_COARSE * 4 + (WS_WIN + 1) * 4 + WS_TCAP * 4 +
-            (vw / 2) * 2 + sp * 2 + 15) & ~15;
-}
-// (the kernel's static LDS is under 256 bytes)
-static_assert(2 * (ws_lds(WS_VALS) + 256) <= 160 * 1024, "two workgroups of the default window per CU");
-static_assert(ws_lds(WS_VALS_BIG) + 256 <= 160 * 1024, "one workgroup of the large window per CU");
-constexpr u64 WS_NOPOS = 0xffffffffull << 32; // (position, column) with no position
-static_assert(2 + 2 * WS_CLASSES <= WIDE_CTRS, "wide-row counters");
-
-// Lanes of a workgroup, by window and density (both value types accumulate in FP64).  The
-// default window runs two workgroups per CU, the large one a single workgroup.  A window's
-// phases share one barrier and one LDS whose atomics queue up, so fewer waves than the CU
-// could hold are faster, the more so the sparser the rows (R-MAT scale 20, wide-row bin,
-// default window, four chunk tasks in flight per group, FP64: 192 / 256 / 320 lanes 258 /
-// 246 / 340 ms; one task at a time: 128 / 256 / 512 lanes 355 / 263 / 290 ms; large
-// window, 512 lanes: 287 ms).  Dense rows want more lanes (a Zipf A·Aᵀ panel's wide rows,
-// FP64 256 / 384 / 512 / 768 lanes 41.4 / 38.0 / 37.2 / 39.4 ms).
-template <int VW, bool SPARSE> constexpr int ws_bs() { return VW == WS_VALS_BIG || !SPARSE ? 512 : 256; }
-// waves per SIMD the launch holds (its workgroups per CU x waves / 4 SIMDs), for the
-// compiler's register budget
-template <int VW, int BS> constexpr int ws_waves()
-{
-    return (BS / 64) * (VW == WS_VALS_BIG ? 1 : 2) / 4 > 0 ? (BS / 64) * (VW == WS_VALS_BIG ? 1 : 2) / 4 : 1;
+    constexpr int words = stream_window(BS) / 64;
+    return WIDE_UNIT * 8 + WW_TILES * 8 + BS * 16 + words * 8 + WW_TILES * 2 + words * 2;
 }
 
-template <typename P, int VW, int BS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu((ws_waves<VW, BS>())))) void k_numeric_wsplit(
-    const WideItem *__restrict__ items, const unsigned *__restrict__ ctr_listed, unsigned *ctr_taken, Operands op,
-    const long long *__restrict__ crp, typename P::V *__restrict__ Cval, u64 *__restrict__ scratch, int *ws,
-    long long ft_stride, long long sym_row_max, int sym_all_global, int long_rows, int *err)
+template <typename P, int BS>
+__global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restrict__ items,
+                                                        const unsigned *__restrict__ ctr_listed, unsigned *ctr_taken,
+                                                        Operands op, const int *__restrict__ index, long long U,
+                                                        const long long *__restrict__ crp,
+                                                        typename P::V *__restrict__ Cval, long long sym_row_max,
+                                                        int sym_all_global, int long_rows)
 {
     typedef typename P::V V;
-    constexpr bool F32C = std::is_same<P, PrecF32C>::value;
-    constexpr int WT = VW / 2; // directory entries of a window
-    // chunk tasks a 16-lane group loads before it adds any: a narrow (sparse-row)
-    // workgroup has few groups, each with many tasks per round, and the registers for
-    // four (R-MAT scale 20 wide-row bin 263 -> 244 ms; eight: no better; two for the dense
-    // launch: within 1% on a Zipf panel)
-    constexpr int NTS = BS < 512 ? 4 : 1;
-    constexpr int SPLIT = wide_split_max(VW); // entries of an item, at most
-    constexpr int EPL = (SPLIT + BS - 1) / BS; // entries a lane posts and moves
-    static_assert(SPLIT <= 1024 && WS_TCAP <= 1024, "task: entry in bits 0-9, chunk in 10-19");
-    const V *__restrict__ Aval = (const V *)op.Aval;
-    const V *__restrict__ Bval = (const V *)op.Bval;
     extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ u64 red[16];
+    __shared__ unsigned next_s;
+    constexpr int words = stream_window(BS) / 64;
     double *vals = (double *)lds;
-    u64 *wm = (u64 *)(vals + VW);
-    double *av = (double *)(wm + WT);
-    u64 *pc = (u64 *)(av + SPLIT); // (position of the next element << 32) | its column
-    u64 *cm = pc + SPLIT;
-    int *cur = (int *)(cm + WS_COARSE);
-    int *kend = cur + SPLIT;
-    int *last = kend + SPLIT; // last column of B_j
-    int *act = last + SPLIT; // two lists (rounds alternate)
-    unsigned *co = (unsigned *)(act + 2 * SPLIT);
-    unsigned *wst = co + WS_COARSE;
-    unsigned *task = wst + WS_WIN + 1;
-    unsigned short *wo = (unsigned short *)(task + WS_TCAP);
-    unsigned short *nch = wo + WT; // chunks listed for an entry in this round
-    __shared__ int item_s, nact_s[2], ntask_s[2];
-    __shared__ unsigned red[16];
-    const int l = threadIdx.x, lane = l & 63;
-    const int ll = l & (WS_GL - 1), lg0 = lane & ~(WS_GL - 1);
-    int *ft = ws + (size_t)blockIdx.x * ft_stride; // tile of every fine entry of a two-level row
+    u64 *wm = (u64 *)(vals + WIDE_UNIT);
+    Stream<BS> st;
+    st.rec = (uint4 *)(wm + WW_TILES);
+    st.bits = (u64 *)(st.rec + BS);
+    unsigned short *wo = (unsigned short *)(st.bits + words);
+    st.wb = wo + WW_TILES;
+    st.red = red;
+    const int l = threadIdx.x;
+    const V *__restrict__ Aval = (const V *)op.Aval;
     const unsigned nitems = *ctr_listed;
-    while (true) {
-        if (l == 0)
-            item_s = (int)atomicAdd(ctr_taken, 1u);
-        __syncthreads();
-        // item and row scalars are uniform: keep them in scalar registers
-        const unsigned it = (unsigned)uniform(item_s);
-        if (it >= nitems)
-            break;
-        const int row = uniform(items[it].row), ie0 = uniform(items[it].e0);
-        const int ne = uniform(items[it].e1) - ie0, nsplit = uniform(items[it].nsplit);
-        const long long sbase = uniform64(items[it].sbase);
+    if (l == 0)
+        next_s = atomicAdd(ctr_taken, 1u);
+    __syncthreads();
+    unsigned it = uniform(next_s);
+    while (it < nitems) {
+        const int row = uniform(items[it].row);
+        const unsigned units = uniform(items[it].units);
+        const unsigned base = uniform(items[it].base);
+        const int cnt = (int)uniform(items[it].cnt);
+        const int u0 = (int)(units & 0xffffffu), u1 = u0 + (int)(units >> 24);
         const int a0 = uniform(op.Arp[row]), nA = uniform(op.Arp[row + 1]) - a0;
-        const long long cb = uniform64(crp[row]);
-        const long long n = uniform64(crp[row + 1]) - cb;
-        const int mn = uniform(op.rmin[row]);
-        const int S = uniform(op.rmax[row]) - mn + 1;
-        const int tp = uniform(op.rtp[row]);
-        const long long rd = uniform64(op.rdir[row]);
-        const bool two = wide_two_level(S, nA, tp, sym_row_max, sym_all_global, long_rows);
-        const int W = two ? (S + 63) >> 6 : 0;
-        const u64 *cmg = op.dir_mask + rd;
-        const unsigned *cog = op.dir_off + rd;
-        const u64 *fm = op.dir_mask + rd + W;
-        const unsigned *foff = op.dir_off + rd + W;
-        const bool clds = W <= WS_COARSE;
-        for (int q = l; q < W && clds; q += BS) {
-            cm[q] = cmg[q];
-            co[q] = cog[q];
+        const WideDir d(op, crp, row, sym_row_max, sym_all_global, long_rows);
+        const long long cb = uniform64(crp[row]) + base;
+        const int T0 = u0 * WIDE_TILES, nt = (u1 - u0) * WIDE_TILES;
+        for (int t = l; t < nt; t += BS) {
+            unsigned off;
+            wm[t] = d.tile(T0 + t - d.mn, off);
+            wo[t] = (unsigned short)(off - base);
         }
-        const int F = two ? (int)(uniform(cog[W - 1]) + (unsigned)__popcll(uniform64(cmg[W - 1]))) : S;
-        const unsigned off0 = F > 0 ? uniform(foff[0]) : 0u;
-        if (two) {
-            for (int q = l; q < W; q += BS) {
-                u64 m = cmg[q];
-                unsigned k = cog[q];
-                while (m) {
-                    ft[k++] = (q << 6) + __ffsll((unsigned long long)m) - 1;
-                    m &= m - 1;
-                }
-            }
-        }
-        for (int e = l; e < ne; e += BS) {
-            const int j = op.Acol[a0 + ie0 + e];
-            const int k0 = op.Brp[j], k1 = op.Brp[j + 1];
-            cur[e] = k0;
-            kend[e] = k1;
-            const int c0 = k0 < k1 ? op.Bcol[k0] : INT_MAX;
-            last[e] = k0 < k1 ? op.Bcol[k1 - 1] : 0;
-            pc[e] = WS_NOPOS | (unsigned)c0;
-            av[e] = Aval[a0 + ie0 + e];
-        }
-        block_sync_global();
-        const bool split = nsplit > 1;
-        long long done = 0;
-        int kb = 0;         // first entry whose window start is not listed yet
-        int nw = 0, wi = 0; // windows listed, current window
-        while (true) {
-            if (wi == nw) { // list the next window starts (WS_WIN at a time, in order)
-                if (kb >= F)
-                    break;
-                int cnt_st = 0; // starts listed so far
-                // WS_LV consecutive entries per lane, their offsets loaded together: one
-                // round trip covers BS * WS_LV entries
-                for (int kk = kb; kk < F && cnt_st <= WS_WIN; kk += BS * WS_LV) {
-                    const int kl = kk + l * WS_LV;
-                    unsigned f[WS_LV + 1]; // foff[kl - 1 + i]
-#pragma unroll
-                    for (int i = 0; i <= WS_LV; ++i) {
-                        const int k = kl - 1 + i;
-                        f[i] = k >= kb && k < F ? foff[k] : 0u;
-                    }
-                    unsigned bits = 0;
-#pragma unroll
-                    for (int i = 0; i < WS_LV; ++i) {
-                        const int k = kl + i;
-                        bool st = false;
-                        if (k < F) {
-                            if (k == kb || (k % WT) == 0)
-                                st = true;
-                            else
-                                st = (f[i + 1] - off0) / (unsigned)(VW - 64) != (f[i] - off0) / (unsigned)(VW - 64);
-                        }
-                        bits |= (st ? 1u : 0u) << i;
-                    }
-                    unsigned tot;
-                    unsigned pos = group_excl_scan<BS>((unsigned)__popc(bits), red, tot);
-                    while (bits) { // this lane's starts, in order
-                        if (cnt_st + (int)pos <= WS_WIN)
-                            wst[cnt_st + pos] = (unsigned)(kl + __ffs(bits) - 1);
-                        ++pos;
-                        bits &= bits - 1;
-                    }
-                    cnt_st += (int)uniform(tot);
-                    __syncthreads(); // red is reused by the next scan
-                }
-                // windows: starts 0..m-1 complete; the last listed start (or F) ends them
-                int m;
-                if (cnt_st > WS_WIN) {
-                    m = WS_WIN;
-                    kb = (int)uniform(wst[WS_WIN]);
-                } else {
-                    m = cnt_st;
-                    if (l == 0)
-                        wst[m] = (unsigned)F;
-                    kb = F;
-                }
-                nw = m;
-                wi = 0;
-                __syncthreads();
-                if (nw == 0)
-                    break;
-            }
-            const int k0 = (int)uniform(wst[wi]), k1 = (int)uniform(wst[wi + 1]);
-            ++wi;
-            const int nk = k1 - k0;
-            const unsigned base = uniform(foff[k0]);
-            const int cnt = (int)((k1 == F ? n : (long long)uniform(foff[k1])) - base);
-            if (l == 0) {
-                nact_s[0] = 0;
-                ntask_s[0] = 0;
-            }
-            for (int q = l; q < nk; q += BS) {
-                wm[q] = fm[k0 + q];
-                wo[q] = (unsigned short)(foff[k0 + q] - base);
-            }
-            for (int q = l; q < cnt; q += BS)
-                vals[q] = 0.0;
-            const int lastt = two ? uniform(ft[k1 - 1]) : k1 - 1;
-            const int chi = (mn + lastt + 1) << 6; // end of the window's last tile
-            __syncthreads();
-            // Chunks of entry e (has) for round r into the lists of buffer r & 1: as many as
-            // its density predicts for the window, doubled in every further round (the
-            // density was too low for this window).  Every lane of every wave calls it: the
-            // chunk counts are laid out with one wave scan and one LDS atomic per wave.
-            auto post = [&](bool has, int e, int r) {
-                const int buf = r & 1;
-                int want = 0;
-                if (has) {
-                    const int c0 = (int)(unsigned)pc[e];
-                    const long long rem = kend[e] - cur[e];
-                    long long est = rem;
-                    if (last[e] >= chi) { // the row goes past the window: scale by its columns
-                        const long long span = (long long)last[e] - c0 + 1;
-                        est = rem * (long long)(chi - c0) / span;
-                        est = ((est + est / 4 + 8) << (r < 8 ? r : 8));
-                        est = est < rem ? est : rem;
-                    }
-                    want = (int)((est + WS_CH - 1) / WS_CH);
-                    want = want < 1 ? 1 : want;
-                }
-                const int incl = wave_incl_scan(want);
-                const int wtot = __shfl(incl, 63, 64);
-                const u64 mh = __ballot(has);
-                int tb = 0, ab = 0;
-                if (lane == 0) {
-                    if (wtot)
-                        tb = atomicAdd(&ntask_s[buf], wtot);
-                    if (mh)
-                        ab = atomicAdd(&nact_s[buf], __popcll(mh));
-                }
-                tb = __shfl(tb, 0, 64);
-                ab = __shfl(ab, 0, 64);
-                if (has) {
-                    const int off = tb + incl - want;
-                    const int got = off >= WS_TCAP ? 0 : (off + want > WS_TCAP ? WS_TCAP - off : want);
-                    nch[e] = (unsigned short)got;
-                    for (int c = 0; c < got; ++c)
-                        task[off + c] = (unsigned)e | ((unsigned)c << 10);
-                    act[buf * SPLIT + ab + mbcnt(mh)] = e;
-                }
-            };
-            auto add_c = [&](int c, V v, double a) {
-                const int tt = (c >> 6) - mn;
-                int r = tt - k0;
-                if (two) {
-                    const int q = tt >> 6;
-                    const u64 m = clds ? cm[q] : cmg[q];
-                    const unsigned o = clds ? co[q] : cog[q];
-                    r = (int)(o + (unsigned)__popcll(m & below(tt & 63))) - k0;
-                }
-                P::add(vals, (unsigned)wo[r] + (unsigned)__popcll(wm[r] & below(c & 63)), a, v);
-            };
-            // round 0: the entries with elements in this window; then those that go again
-            // (EPL entries per lane)
-            bool has[EPL];
-            int e[EPL];
-#pragma unroll
-            for (int q = 0; q < EPL; ++q) {
-                e[q] = l + q * BS;
-                has[q] = e[q] < ne && (int)(unsigned)pc[e[q]] < chi;
-            }
-            for (int round = 0;; ++round) {
-#pragma unroll
-                for (int q = 0; q < EPL; ++q)
-                    post(has[q], e[q], round);
-                __syncthreads();
-                const int buf = round & 1;
-                const int nact = uniform(nact_s[buf]);
-                if (nact == 0)
-                    break;
-                const int nt = uniform(ntask_s[buf]);
-                const int ntask = nt < WS_TCAP ? nt : WS_TCAP;
-                if (l == 0) { // the other buffer's counters, for the next round
-                    nact_s[buf ^ 1] = 0;
-                    ntask_s[buf ^ 1] = 0;
-                }
-                // a group loads the chunks of NTS tasks before it adds any of them
-                constexpr int NG = BS / WS_GL;
-                for (int t = l / WS_GL; t < ntask; t += NTS * NG) {
-                    int te[NTS], k[NTS], ke[NTS];
-                    double a[NTS];
-                    int c[NTS][4];
-                    V v[NTS][4];
-#pragma unroll
-                    for (int h = 0; h < NTS; ++h) {
-                        const int th = t + h * NG;
-                        te[h] = 0;
-                        k[h] = 0;
-                        ke[h] = 0; // no task: no element loaded
-                        a[h] = 0.0;
-                        if (th < ntask) {
-                            const unsigned tk = task[th];
-                            te[h] = (int)(tk & 1023u);
-                            k[h] = cur[te[h]] + (int)(tk >> 10) * WS_CH;
-                            ke[h] = kend[te[h]];
-                            a[h] = av[te[h]];
-                        }
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            const int p = k[h] + ll + WS_GL * u;
-                            c[h][u] = INT_MAX;
-                            v[h][u] = 0;
-                            if (p < ke[h]) {
-                                c[h][u] = op.Bcol[p];
-                                v[h][u] = Bval[p];
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int h = 0; h < NTS; ++h) {
-                        if (t + h * NG >= ntask) // uniform in the group (t is)
-                            break;
-                        int took = 0;
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            const bool in = c[h][u] < chi;
-                            if (in)
-                                add_c(c[h][u], v[h][u], a[h]);
-                            took += __popcll((__ballot(in) >> lg0) & ((1ull << WS_GL) - 1ull));
-                        }
-                        if (took < WS_CH) { // the prefix ends here: offer (position, column) after it
-#pragma unroll
-                            for (int u = 0; u < 4; ++u)
-                                if (ll + WS_GL * u == took)
-                                    atomicMin((unsigned long long *)&pc[te[h]],
-                                              ((u64)(unsigned)(k[h] + took) << 32) | (unsigned)c[h][u]);
-                        }
-                    }
-                }
-                __syncthreads();
-                // move the cursors; entries whose chunks were all inside the window go again
-#pragma unroll
-                for (int q = 0; q < EPL; ++q) {
-                    const int idx = l + q * BS;
-                    bool again = false;
-                    int ee = -1;
-                    if (idx < nact) {
-                        ee = act[buf * SPLIT + idx];
-                        const u64 r = pc[ee];
-                        if ((r >> 32) != 0xffffffffull) {
-                            cur[ee] = (int)(r >> 32);
-                            pc[ee] = WS_NOPOS | (r & 0xffffffffull);
-                        } else {
-                            const int kn = cur[ee] + (int)nch[ee] * WS_CH;
-                            if (kn >= kend[ee]) {
-                                cur[ee] = kend[ee];
-                                pc[ee] = WS_NOPOS | (unsigned)INT_MAX;
-                            } else {
-                                cur[ee] = kn;
-                                again = true;
-                            }
-                        }
-                    }
-                    has[q] = again;
-                    e[q] = ee;
-                }
-            }
-            // Output: the window's values (its columns were written by k_wide_cols).  Split
-            // rows add theirs into C (FP64) or, with FP32 values, into the FP64 scratch, which
-            // is rounded into C once at the end.
-            if (split) {
-                double *to = F32C ? (double *)scratch + sbase + base : (double *)Cval + cb + base;
-                for (int q = l; q < cnt; q += BS) {
-                    const double v = vals[q];
-                    if (v != 0.0)
-                        unsafeAtomicAdd(&to[q], v);
-                }
-            } else {
-                for (int q = l; q < cnt; q += BS)
-                    Cval[cb + base + q] = P::result(vals, (unsigned)q);
-            }
-            done += cnt;
-            __syncthreads();
-        }
-        if (l == 0 && done != n)
-            raise_internal(err);
-        block_sync_global(); // ft and the LDS state of the next item
-    }
-}
-
-// Compensated FP32, rows split into several items: C's values, rounded once from the
-// FP64 sums the items added into the scratch.  A workgroup per row; the row's first item
-// names it and its scratch range.
-__global__ __launch_bounds__(256) void k_wide_final(const WideItem *__restrict__ items,
-                                                    const unsigned *__restrict__ ctr_listed,
-                                                    const long long *__restrict__ crp, float *__restrict__ Cval,
-                                                    const u64 *__restrict__ scratch)
-{
-    const unsigned nitems = *ctr_listed;
-    for (unsigned idx = blockIdx.x; idx < nitems; idx += gridDim.x) {
-        const int e0 = uniform(items[idx].e0), ns = uniform(items[idx].nsplit);
-        if (e0 != 0 || ns <= 1)
-            continue;
-        const int row = uniform(items[idx].row);
-        const long long sb = uniform64(items[idx].sbase);
-        const long long cb = uniform64(crp[row]), n = uniform64(crp[row + 1]) - cb;
-        const double *sd = (const double *)scratch + sb;
-        for (long long q = threadIdx.x; q < n; q += 256)
-            Cval[cb + q] = (float)sd[q];
+        for (int q = 2 * l; q < cnt; q += 2 * BS) // (WIDE_UNIT is even)
+            *(double2 *)(vals + q) = make_double2(0.0, 0.0);
+        for (int q = l; q < words; q += BS)
+            st.bits[q] = 0;
+        if (l == 0)
+            next_s = atomicAdd(ctr_taken, 1u);
+        __syncthreads();
+        auto rows_of = [&](int e) {
+            const int j = op.Acol[a0 + e];
+            const int *ix = index + (long long)j * (U + 1);
+            const int s0 = ix[u0];
+            return Segment{s0, ix[u1] - s0, (u64)__double_as_longlong((double)Aval[a0 + e])};
+        };
+        st.run(nA, rows_of, [&](const Stream<BS> &t, long long w0) {
+            stream_add<BS, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, wm, wo, vals, T0);
+        });
+        for (int q = l; q < cnt; q += BS)
+            Cval[cb + q] = P::result(vals, (unsigned)q);
+        it = uniform(next_s);
+        __syncthreads();
     }
 }
 
@@ -2347,41 +2062,27 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
 {
     if (bin == BIN_GLOBAL) {
         const int blocks = count < wide.blocks ? count : wide.blocks;
-        if (op.dir_mask && wide.items) { // split work items (FP64, or compensated with its scratch)
-            constexpr bool F32C = std::is_same<P, PrecF32C>::value;
+        if (op.dir_mask && wide.items) { // windows
             hipError_t e = launch_fill_zero(wide.ctr, WIDE_CTRS * sizeof(unsigned), s);
-            if (e == hipSuccess && F32C)
-                e = launch_fill_zero(wide.sctr, sizeof(unsigned long long), s);
-            if (e == hipSuccess && F32C && wide.scratch_n > 0)
-                e = launch_fill_zero(wide.scratch, (size_t)wide.scratch_n * sizeof(u64), s);
             if (e != hipSuccess)
                 return e;
-            const unsigned gr = (unsigned)((count + 255) / 256);
-            // (the compensated scratch is sized by wide_split at WS_VALS in the binning; the
-            // large window splits a subset of those rows, in fewer items)
-            const int vals = wide.vals == WS_VALS_BIG ? WS_VALS_BIG : WS_VALS;
-            hipLaunchKernelGGL(k_wide_count, dim3(gr), dim3(256), 0, s, rows, count_dev, op.Arp, crp, vals, wide.ctr);
+            const long long nix = wide.K * (wide.nunits + 1);
+            const long long gx = (nix + 255) / 256;
+            hipLaunchKernelGGL(k_wide_index, dim3((unsigned)(gx < 65536 ? gx : 65536)), dim3(256), 0, s, wide.K,
+                               wide.nunits, op.Brp, op.Bcol, wide.index);
+            const unsigned gi = (unsigned)(count < 4 * num_cus ? (count + 3) / 4 : num_cus);
+            hipLaunchKernelGGL(k_wide_items<false>, dim3(gi), dim3(256), 0, s, rows, count_dev, op, crp, wide.nunits,
+                               wide.sym_row_max, wide.sym_all_global, wide.long_rows, wide.items, wide.items_cap,
+                               wide.ctr, err);
             hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(64), 0, s, wide.ctr);
-            hipLaunchKernelGGL(k_wide_fill, dim3(gr), dim3(256), 0, s, rows, count_dev, op.Arp, crp, vals, wide.items,
-                               wide.items_cap, wide.ctr, F32C ? wide.sctr : nullptr, wide.scratch_n, err);
+            hipLaunchKernelGGL(k_wide_items<true>, dim3(gi), dim3(256), 0, s, rows, count_dev, op, crp, wide.nunits,
+                               wide.sym_row_max, wide.sym_all_global, wide.long_rows, wide.items, wide.items_cap,
+                               wide.ctr, err);
             hipLaunchKernelGGL(k_wide_cols, dim3((unsigned)(count < 8192 ? count : 8192)), dim3(WC_BS), 0, s, rows,
-                               count_dev, op, crp, Ccol, F32C ? nullptr : (double *)Cval, wide.sym_row_max,
-                               wide.sym_all_global, wide.long_rows, vals);
-#define WSPLIT(VW, SPARSE)                                                                                           \
-    hipLaunchKernelGGL((k_numeric_wsplit<P, VW, ws_bs<VW, SPARSE>()>), dim3((unsigned)wide.blocks),                 \
-                       dim3(ws_bs<VW, SPARSE>()), ws_lds(VW), s, wide.items, wide.ctr, wide.ctr + 1, op, crp,        \
-                       (typename P::V *)Cval, (u64 *)wide.scratch, wide.ws, wide.ft_stride, wide.sym_row_max,           \
-                       wide.sym_all_global, wide.long_rows, err)
-            if (vals == WS_VALS_BIG)
-                WSPLIT(WS_VALS_BIG, false);
-            else if (wide.sparse)
-                WSPLIT(WS_VALS, true);
-            else
-                WSPLIT(WS_VALS, false);
-#undef WSPLIT
-            if (F32C)
-                hipLaunchKernelGGL(k_wide_final, dim3(2048), dim3(256), 0, s, wide.items, wide.ctr, crp, (float *)Cval,
-                                   (const u64 *)wide.scratch);
+                               count_dev, op, crp, Ccol, wide.sym_row_max, wide.sym_all_global, wide.long_rows);
+            hipLaunchKernelGGL((k_numeric_windows<P, WW_BS>), dim3((unsigned)wide.blocks), dim3(WW_BS),
+                               ww_lds<WW_BS>(), s, wide.items, wide.ctr, wide.ctr + 1, op, wide.index, wide.nunits, crp,
+                               (typename P::V *)Cval, wide.sym_row_max, wide.sym_all_global, wide.long_rows);
         } else if (op.dir_mask)
             hipLaunchKernelGGL(k_numeric_wcompact<P>, dim3(blocks), dim3(1024), CW_LDS, s, rows, count_dev, op, crp,
                                Ccol, (typename P::V *)Cval, bshift > 6 ? 6 : bshift, wide.ws, wide.cur_stride,
@@ -2427,6 +2128,11 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
                               long_rows, wide, err, num_cus, queue, lds_bytes, s);
 }
 
+int wide_window_blocks(int num_cus)
+{
+    return num_cus * (160 * 1024 / (ww_lds<WW_BS>() + LDS_STATIC_RESERVE));
+}
+
 size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks)
 {
     return (size_t)blocks * (size_t)(3 * cur_stride + ft_stride);
@@ -2460,10 +2166,7 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
     CFG(k_symbolic_wide)
     CFG(k_numeric_window<PrecF64>) CFG(k_numeric_window<PrecF32C>)
     CFG(k_numeric_wcompact<PrecF64>) CFG(k_numeric_wcompact<PrecF32C>) 
-#define CFGW(P)                                                                                                        \
-    CFG((k_numeric_wsplit<P, WS_VALS, ws_bs<WS_VALS, false>()>))                                                    \
-    CFG((k_numeric_wsplit<P, WS_VALS, ws_bs<WS_VALS, true>()>))                                                     \
-    CFG((k_numeric_wsplit<P, WS_VALS_BIG, ws_bs<WS_VALS_BIG, false>()>))
+#define CFGW(P) CFG((k_numeric_windows<P, WW_BS>))
     CFGW(PrecF64) CFGW(PrecF32C)
 #undef CFGW
 #undef CFG

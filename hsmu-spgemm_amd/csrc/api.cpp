@@ -939,44 +939,36 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         const int cnt = h2.num.count[b];
         if (cnt <= 0)
             continue;
-        // wide rows: a workspace per window workgroup (two 1024-lane workgroups fit a CU's
-        // LDS) for the tiles of a two-level directory and, without split items, the cursors
-        // of its row's A entries.  Rows with kept directories (FP64, and the compensated form
-        // when its scratch fits) run as split work items (at most count + nnz(A) /
-        // WS_MIN_SPLIT of them) on a full persistent grid.
+        // wide rows: with kept directories and room for the index of B, windows of their
+        // columns on a persistent grid; else a workgroup per row, with a workspace for the
+        // tiles of a two-level directory and the cursors of its row's A entries
         WideRows wide = {};
         if (b == BIN_GLOBAL) {
-            // the compensated form's split rows need an FP64 sum per nonzero of theirs
-            const unsigned long long scratch_bytes = h2.wide_split_nnz * sizeof(unsigned long long);
-            unsigned long long scratch_max =
+            const long long units = wide_units(N);
+            const long long index_n = K * (units + 1);
+            unsigned long long index_max =
                 opts.wide_scratch_mb > 0 ? (unsigned long long)opts.wide_scratch_mb << 20 : c->total_mem / 4;
-            if (scratch_max > ar.remaining() / 2) // allocation-free: what the workspace has left
-                scratch_max = ar.remaining() / 2;
-            const bool split_items = keep_dirs && (!fp32 || scratch_bytes <= scratch_max);
-            // split items: the window size asked for (the default one otherwise), and
-            // narrow workgroups for sparse rows (few columns per tile spanned)
-            wide.vals = split_items && opts.wide_window ? opts.wide_window : WS_VALS;
-            wide.sparse =
-                (unsigned long long)h2.num.nnz_c[b] < (unsigned long long)WS_SPARSE_DENSITY * h2.wide_span ? 1 : 0;
-            const int per_cu = wide.vals == WS_VALS ? 2 : 1; // workgroups of the window kernel a CU holds
-            wide.blocks = split_items ? per_cu * c->num_cus : (cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt);
-            wide.cur_stride = split_items ? 0 : ((long long)h2.num.max_na[b] + 63) & ~63LL;
-            wide.ft_stride = keep_dirs ? (((long long)h2.num.max_span[b] + 63) & ~63LL) : 0;
+            if (index_max > ar.remaining() / 2) // allocation-free: what the workspace has left
+                index_max = ar.remaining() / 2;
+            const bool windows = keep_dirs && (unsigned long long)index_n * sizeof(int) <= index_max &&
+                                 units < (1 << 24) && h2.wide_items < (1ull << 31);
+            wide.blocks = windows ? wide_window_blocks(c->num_cus) : (cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt);
             wide.sym_row_max = bp_sym_row_max;
             wide.sym_all_global = opts.force_global ? 1 : 0;
             wide.long_rows = long_rows;
-            wide.ws = ar.get<int>(wide_ws_ints(wide.cur_stride, wide.ft_stride, wide.blocks) + 1);
-            if (split_items) {
-                wide.items_cap = (long long)cnt + P.nnzA / WS_MIN_SPLIT + 1;
+            if (windows) {
+                wide.nunits = units;
+                wide.K = K;
+                wide.index = ar.get<int>((size_t)index_n);
+                wide.items_cap = (long long)h2.wide_items;
                 wide.items = ar.get<WideItem>((size_t)wide.items_cap);
                 wide.ctr = ar.get<unsigned>(WIDE_CTRS);
-                if (fp32) {
-                    wide.scratch_n = (long long)h2.wide_split_nnz;
-                    wide.scratch = ar.get<unsigned long long>((size_t)(wide.scratch_n > 0 ? wide.scratch_n : 1));
-                    wide.sctr = ar.get<unsigned long long>(1);
-                }
+            } else {
+                wide.cur_stride = ((long long)h2.num.max_na[b] + 63) & ~63LL;
+                wide.ft_stride = keep_dirs ? (((long long)h2.num.max_span[b] + 63) & ~63LL) : 0;
+                wide.ws = ar.get<int>(wide_ws_ints(wide.cur_stride, wide.ft_stride, wide.blocks) + 1);
             }
-            if (!wide.ws || (split_items && (!wide.items || !wide.ctr || (fp32 && (!wide.scratch || !wide.sctr)))))
+            if (windows ? (!wide.index || !wide.items || !wide.ctr) : !wide.ws)
                 return fail(HSMU_ERR_NOMEM, "wide-row workspace");
         }
         if (timing)
@@ -1081,8 +1073,8 @@ int check_opts(const hsmu_opts &o)
 {
     if (o.precision != HSMU_FP64 && o.precision != HSMU_FP32_COMP)
         return fail(HSMU_ERR_INVALID, "unknown precision %d", o.precision);
-    if (o.wide_window != 0 && o.wide_window != WS_VALS && o.wide_window != WS_VALS_BIG)
-        return fail(HSMU_ERR_INVALID, "wide_window %d: 0, %d or %d", o.wide_window, WS_VALS, WS_VALS_BIG);
+    if (o.wide_window != 0 && o.wide_window != 4096 && o.wide_window != 8192)
+        return fail(HSMU_ERR_INVALID, "wide_window %d: 0, 4096 or 8192", o.wide_window);
     return HSMU_OK;
 }
 

@@ -66,8 +66,7 @@ struct DevStats {
     int pad;
     int max_brow; // longest row of B (counted from LONG_TILES on)
     unsigned long long num_wide_hint; // rows whose numeric need may exceed LDS (symbolic binning)
-    unsigned long long wide_split_nnz; // nnz(C_i) summed over the wide rows split into several items
-    unsigned long long wide_span; // tiles spanned, summed over the wide rows (numeric binning)
+    unsigned long long wide_items; // windows the wide rows may need, at most (numeric binning)
     BinStats sym;
     BinStats num;
     // work-queue counters of the persistent LDS kernels: [phase][bin][XCD]
@@ -356,46 +355,34 @@ hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int c
                            unsigned long long *gws, long long gws_stride, int num_cus,
                            int gws_blocks, int lds_dyn, unsigned *queue, hipStream_t s);
 
-// Wide rows (BIN_GLOBAL) in the numeric phase: blocks workgroups, each with a workspace of
-// 3 * cur_stride + ft_stride ints (cursors, ends and next columns of its row's A entries:
-// cur_stride >= the longest row of A in the bin; tiles of the fine directory entries of
-// a two-level row: ft_stride >= the widest span in the bin).  With kept directories the
-// compact windowed kernel runs, and needs to know which rows the symbolic phase held in
-// global memory (their directories are flat): sym_row_max (LDS bytes a row may use) and
-// sym_all_global (every row was global: force_global).
-// Wide rows with kept directories (FP64) are processed as work items: entries [e0, e1) of
-// A row `row`.  A row whose entries x windows exceed WS_VISITS is split into several items
-// (nsplit > 1); their partial sums meet in C's values by atomic adds (C zeroed first).
+// Wide rows (BIN_GLOBAL) in the numeric phase.  With kept directories and room for the index
+// (below) they are processed as windows: a window is a run of units of WIDE_UNIT columns
+// (aligned, so that all rows' windows share their boundaries) that holds at most WIDE_UNIT
+// entries of C_i and spans at most WIDE_UMAX units, one workgroup each.  The index gives
+// every B row's first element at each unit's start, so a window's elements are known without
+// a search.  (Which rows' directories are flat depends on what the symbolic phase held in
+// global memory: sym_row_max, sym_all_global, long_rows.)
+constexpr int WIDE_UNIT = 4096;
+constexpr int WIDE_UMAX = 16;
+constexpr int WIDE_TILES = WIDE_UNIT / 64;     // tiles of a unit
+constexpr int WIDE_BUCKETS = 32;               // windows are listed by their place in C's columns
 struct WideItem {
-    int row, e0, e1, nsplit;
-    long long sbase; // compensated FP32, split rows: the row's first sum in the scratch
+    int row;
+    unsigned units;     // first unit | number of units << 24
+    unsigned base, cnt; // the row's entries before the window, and in it
 };
-constexpr int WIDE_CTRS = 66;
-// A window holds at most `vals` value slots and vals / 2 directory entries: WS_VALS (two
-// workgroups per CU, the default), or WS_VALS_BIG (one per CU, on request).  Launches
-// whose wide rows hold fewer than WS_SPARSE_DENSITY columns of C per tile they span take
-// narrower workgroups (the sparse lane counts of k_numeric_wsplit).
-constexpr int WS_VALS = 4096;
-constexpr int WS_VALS_BIG = 8192;
-constexpr int WS_SPARSE_DENSITY = 16;
-// A entries of one item, at most: WS_SPLIT with the default window, twice as many with
-// the large one (its workgroup has the CU's LDS to itself), so that the fixed cost of a
-// window (its directory, its output) is shared by more entries
-constexpr int WS_SPLIT = 512;
-constexpr int WS_SPLIT_BIG = 1024;
-constexpr int WS_MIN_SPLIT = 64;     // A entries of one item, at least (unless the row has fewer)
-constexpr long long WS_VISITS = 65536; // target of entries x windows per item (per WS_SPLIT)
-HSMU_HD constexpr int wide_split_max(int vals) { return vals == WS_VALS_BIG ? WS_SPLIT_BIG : WS_SPLIT; }
-// A entries per item for a row with nA entries and n = nnz(C_i), windows of `vals` slots
-HSMU_HD inline int wide_split(long long n, int vals = WS_VALS)
+HSMU_HD inline long long wide_units(long long N) { return (N + WIDE_UNIT - 1) / WIDE_UNIT; }
+// windows of a row of n entries over S tiles, at most: two neighbouring ones hold more than
+// WIDE_UNIT entries or span more than WIDE_UMAX units
+HSMU_HD inline long long wide_row_items(int n, int S)
 {
-    const long long win = n / (vals - 64) + 1; // windows, about
-    const long long mx = wide_split_max(vals);
-    long long sz = WS_VISITS * (mx / WS_SPLIT) / win;
-    sz = sz < WS_MIN_SPLIT ? WS_MIN_SPLIT : (sz > mx ? mx : sz);
-    return (int)(sz & ~63LL);
+    return 2LL * (n / WIDE_UNIT) + 2LL * (S / (WIDE_TILES * WIDE_UMAX)) + 4;
 }
 
+// Otherwise one workgroup per row (blocks workgroups), each with a workspace of 3 *
+// cur_stride + ft_stride ints (cursors, ends and next columns of its row's A entries:
+// cur_stride >= the longest row of A in the bin; tiles of the fine directory entries of a
+// two-level row: ft_stride >= the widest span in the bin).
 struct WideRows {
     int *ws;
     long long cur_stride, ft_stride;
@@ -403,21 +390,19 @@ struct WideRows {
     long long sym_row_max;
     int sym_all_global;
     int long_rows; // the with_long the symbolic binning used
-    int vals;      // split work items: value slots of a window (WS_VALS or WS_VALS_BIG)
-    int sparse;    // split work items: the wide rows hold few columns per tile (narrow workgroups)
-    // split work items (FP64 with kept directories): capacity, list, WIDE_CTRS counters
-    // (ctr[0] = items listed, ctr[1] = items taken, then per size class)
+    // windows: their capacity and list, and counters: windows listed, taken, then per bucket
+    // the windows and the place of the next one (null items: one workgroup per row)
     long long items_cap;
     WideItem *items;
     unsigned *ctr;
-    // compensated FP32 split rows: one FP64 sum per nonzero of those rows (zeroed before
-    // the items add their windows into it), and the counter that hands out each row's
-    // range
-    unsigned long long *scratch;
-    long long scratch_n;
-    unsigned long long *sctr;
+    int *index; // K rows of nunits + 1
+    long long nunits;
+    long long K;
 };
+constexpr int WIDE_CTRS = 2 + 2 * WIDE_BUCKETS;
 size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks);
+// workgroups of the windows' kernel that the device holds
+int wide_window_blocks(int num_cus);
 
 // Numeric phase of one bin.  fp32c = 0: FP64 values (Cval double); fp32c = 1: compensated
 // FP32 (Cval float).  lds_bytes (may be null): += the dynamic LDS of an LDS-bin launch,

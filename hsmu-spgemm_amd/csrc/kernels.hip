@@ -474,15 +474,10 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, bool with_long,
     const u64 wides = __ballot(wide);
     if (lane == 0 && wides)
         atomicAdd(&st->num_wide_hint, (u64)__popcll(wides));
-    // nonzeros of the wide rows whose work is split into several items (their partial sums
-    // meet in a scratch buffer of this size when C holds FP32), and the tiles they span
-    if (numeric && __ballot(at.b == BIN_GLOBAL)) {
-        const u64 sn = wave_sum(at.b == BIN_GLOBAL && r.nA > wide_split(r.nc) ? (u64)r.nc : 0ull);
-        const u64 ss = wave_sum(at.b == BIN_GLOBAL ? (u64)r.S : 0ull);
-        if (lane == 0 && sn)
-            atomicAdd(&st->wide_split_nnz, sn);
-        if (lane == 0 && ss)
-            atomicAdd(&st->wide_span, ss);
+    if (numeric && __ballot(at.b == BIN_GLOBAL)) { // room for the wide rows' windows
+        const u64 items = wave_sum(at.b == BIN_GLOBAL ? (u64)wide_row_items(r.nc, r.S) : 0ull);
+        if (lane == 0)
+            atomicAdd(&st->wide_items, items);
     }
     // the lanes that chose one bin (neighbouring rows usually share it) add up first
     u64 pending = __ballot(at.b >= 0);
@@ -1173,7 +1168,7 @@ __global__ void k_plan_check(DevStats *st, const DevStats *expect, int stage)
         same = same && st->dir_total == expect->dir_total && st->ntiles_b == expect->ntiles_b &&
                st->max_brow == expect->max_brow;
     else
-        same = same && st->nnz_c == expect->nnz_c && st->wide_split_nnz == expect->wide_split_nnz;
+        same = same && st->nnz_c == expect->nnz_c && st->wide_items == expect->wide_items;
     if (!same)
         st->err |= ERR_PLAN;
     if (st->err) {

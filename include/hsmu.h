@@ -131,14 +131,12 @@ typedef struct hsmu_opts {
     int32_t min_waves;        /* a row that has a workgroup to itself gets enough lanes for
                                  this many waves per CU at the occupancy its LDS allows (at
                                  most 1024 lanes); 0 = 8 */
-    int32_t wide_scratch_mb;  /* compensated FP32: MiB the FP64 scratch of wide rows split
-                                 into several work items may take; 0 = a quarter of device
-                                 memory.  Beyond it those rows take one workgroup each */
-    int32_t wide_window;      /* rows wider than LDS, split into work items: value slots of
-                                 one window of the windowed accumulator, 4096 (two
-                                 workgroups per CU) or 8192 (one); 0 = 4096.  Workgroups
-                                 are narrower when those rows hold fewer than 16 columns of
-                                 C per 64-column tile they span */
+    int32_t wide_scratch_mb;  /* rows wider than LDS: MiB the column index of B may take that cuts
+                                 them into windows (4 bytes per row of B and 4,096 columns);
+                                 0 = a quarter of device memory.  Beyond it those rows take one
+                                 workgroup each, which is slower */
+    int32_t wide_window;      /* accepted, without effect: 0, 4096 or 8192 (windows of rows wider
+                                 than LDS hold 4,096 entries of C) */
 } hsmu_opts;
 
 #define HSMU_NBINS 10 /* 8 LDS bins (8..1024 lanes per row), global fallback, wide rows */
