@@ -127,30 +127,15 @@ DEVI void or_walk(const Operands &op, int tb, int te, int gw, int gl, u64 *dm, c
     }
 }
 
-template <int G, int MODE, bool LIST = false>
-DEVI void or_tiles(const Operands &op, const int *t0, const int *tlen, int nA, const int *lidx, int nlong, u64 *dm,
-                   const unsigned *coff, u64 *fm, int mn, int tshift)
+template <int G, int MODE>
+DEVI void or_tiles(const Operands &op, const int *t0, const int *tlen, int nA, u64 *dm, const unsigned *coff, u64 *fm,
+                   int mn, int tshift)
 {
     const int l = threadIdx.x & (G - 1);
-    // LIST: entries with many tiles (listed in lidx), one wave each (the whole group if
-    // smaller); the sub-group walks below skip them
-    // 1024-lane groups hold a row per CU (LDS bounds their occupancy), so each lane keeps
-    // twice as many tile loads in flight
-    constexpr int U = G >= 1024 ? 2 * UNROLL : UNROLL;
-    if constexpr (LIST) {
-        constexpr int LW = G < 64 ? G : 64;
-        for (int i = l / LW; i < nlong; i += G / LW) {
-            const int e = lidx[i];
-            or_walk<MODE, U>(op, t0[e], t0[e] + tlen[e], LW, l & (LW - 1), dm, coff, fm, mn);
-        }
-    }
     // sub-groups of 2^tshift lanes take one entry each
     const int SG = 1 << tshift, sl = l & (SG - 1), NSG = G >> tshift;
-    for (int e = l >> tshift; e < nA; e += NSG) {
-        if (LIST && tlen[e] >= LONG_TILES)
-            continue;
-        or_walk<MODE, U>(op, t0[e], t0[e] + tlen[e], SG, sl, dm, coff, fm, mn);
-    }
+    for (int e = l >> tshift; e < nA; e += NSG)
+        or_walk<MODE>(op, t0[e], t0[e] + tlen[e], SG, sl, dm, coff, fm, mn);
 }
 
 // Each lane scans a contiguous chunk [ta, tb) of the n directory entries; groups of 256
@@ -218,6 +203,14 @@ DEVI void chunk_offsets(const u64 *m, const ChunkScan &c, Out out)
             p += (unsigned)__popcll(w);
         }
     }
+}
+
+// Where row's kept directory lies, -1 if it has none in the form the row takes here (a row
+// the symbolic phase held in global memory keeps a flat one).
+DEVI long long kept_dir(const Operands &op, int row, bool two)
+{
+    const long long rd = op.rdir[row];
+    return rd >= 0 && ((rd & RDIR_TWO) != 0) == two ? rd & ~RDIR_TWO : -1;
 }
 
 // ---- numeric forms ---------------------------------------------------------------------
@@ -525,7 +518,9 @@ DEVI void stream_add(const Stream<G> &st, long long w0, const Operands &op, cons
     }
 }
 
-// OR a window of the row's tile stream (entries are tile ranges) into its directory.
+// OR a window of the row's tile stream (entries are tile ranges) into its directory, OR_U
+// steps of a wave loaded together.
+constexpr int OR_U = 4;
 template <int G, int MODE>
 DEVI void stream_or(const Stream<G> &st, long long w0, const Operands &op, u64 *dm, const unsigned *coff, u64 *fm, int mn)
 {
@@ -533,17 +528,37 @@ DEVI void stream_or(const Stream<G> &st, long long w0, const Operands &op, u64 *
     const unsigned nB = (unsigned)op.nnzB;
     const int lane = threadIdx.x & 63;
     const int nst = st.steps(w0);
-    for (int s = NW > 1 ? uniform((int)(threadIdx.x >> 6)) : 0; s < nst; s += NW) {
-        const uint4 r = st.entry(s);
-        const Pair q(r.x + STREAM_V * (unsigned)((unsigned)w0 + 64 * s + lane), r.y, nB);
-        const Vec2<int>::type c = load2(op.tcol + q.at);
-        Vec2<u64>::type m = {0, 0};
-        if constexpr (MODE != OR_COARSE)
-            m = load2(op.tmask + q.at);
-        if (q.in0)
-            or_put<MODE>(dm, coff, fm, c.x - mn, m.x);
-        if (q.in1)
-            or_put<MODE>(dm, coff, fm, c.y - mn, m.y);
+    const int s0 = NW > 1 ? uniform((int)(threadIdx.x >> 6)) : 0;
+    u64 lw = 0; // lane i holds the wave's i-th step
+    int lb = 0;
+    if (s0 + lane * NW < nst) {
+        lw = st.bits[s0 + lane * NW];
+        lb = st.wb[s0 + lane * NW];
+    }
+    for (int i = 0, s = s0; s < nst; i += OR_U, s += OR_U * NW) {
+        Vec2<int>::type c[OR_U];
+        Vec2<u64>::type m[OR_U];
+        bool in0[OR_U], in1[OR_U];
+#pragma unroll
+        for (int u = 0; u < OR_U; ++u) {
+            const uint4 r = st.entry(__builtin_amdgcn_readlane(lb, (i + u) & 63), readlane_u64(lw, (i + u) & 63));
+            const int su = s + u * NW;
+            const Pair q(r.x + STREAM_V * ((unsigned)w0 + 64 * su + lane), su < nst ? r.y : 0u, nB);
+            c[u] = load2(op.tcol + q.at);
+            if constexpr (MODE != OR_COARSE)
+                m[u] = load2(op.tmask + q.at);
+            else
+                m[u] = Vec2<u64>::type{0, 0};
+            in0[u] = q.in0;
+            in1[u] = q.in1;
+        }
+#pragma unroll
+        for (int u = 0; u < OR_U; ++u) {
+            if (in0[u])
+                or_put<MODE>(dm, coff, fm, c[u].x - mn, m[u].x);
+            if (in1[u])
+                or_put<MODE>(dm, coff, fm, c[u].y - mn, m[u].y);
+        }
     }
 }
 
@@ -557,13 +572,13 @@ DEVI void stream_or(const Stream<G> &st, long long w0, const Operands &op, u64 *
 // When the directory is kept, it goes out with each entry's exclusive prefix (coarse:
 // first compact index; fine or flat: first slot) for the numeric phase.
 template <int G, bool LONG>
-__global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_symbolic_lds(const int *__restrict__ rows,
+__global__ __launch_bounds__(BLOCK) void k_symbolic_lds(const int *__restrict__ rows,
                                                                        const int *__restrict__ count_p, int slice_bytes,
                                                                        Operands op, int *__restrict__ rnnz, int tshift,
                                                                        int two_level, unsigned *queue)
 {
-    constexpr int BS = G < BLOCK ? BLOCK : G;
-    constexpr int RPB = BS / G;
+    static_assert(G < BLOCK, "rows that share a workgroup");
+    constexpr int RPB = BLOCK / G;
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ unsigned redu[16];
     __shared__ int grp_s[2];
@@ -581,13 +596,6 @@ __global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_symbolic_lds(const in
             nA = op.Arp[row + 1] - a0;
             tp = op.rtp[row];
         }
-        if constexpr (G >= 64) { // one row per workgroup: its scalars in scalar registers
-            S = uniform(S);
-            mn = uniform(mn);
-            a0 = uniform(a0);
-            nA = uniform(nA);
-            tp = uniform(tp);
-        }
         const bool sparse = use_sparse(S, tp);
         const int W = sparse ? (S + 63) >> 6 : S; // entries of the first level
         const RowLayout L = row_layout(0, S, 0, nA, tp, LONG);
@@ -595,78 +603,32 @@ __global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_symbolic_lds(const in
         unsigned *doff = (unsigned *)(slice + L.doff);
         int *tlen = (int *)(slice + L.tlen);
         int *t0 = (int *)(slice + L.t0);
-        int *lidx = (int *)(slice + L.lidx);
-        int *lcnt = (int *)(slice + L.lcnt);
         for (int t = l; t < W; t += G)
             dm[t] = 0;
-        if (LONG && G >= 128 && l == 0)
-            *lcnt = 0;
         stage_row<G, false>(op, a0, nA, t0, tlen, nullptr, nullptr, nullptr);
         __syncthreads();
-        // rows of the wide bins: entries with many tiles, one wave each
-        int nlong = 0;
-        if constexpr (LONG && G >= 128) {
-            for (int k = l; k < nA; k += G)
-                if (tlen[k] >= LONG_TILES)
-                    lidx[atomicAdd(lcnt, 1)] = k;
-            __syncthreads();
-            nlong = *lcnt;
-        }
-        // the list, when there is one, takes the long entries out of the sub-group walks
-        constexpr bool LIST = LONG && G >= 128;
         if (sparse)
-            or_tiles<G, OR_COARSE, LIST>(op, t0, tlen, nA, lidx, nlong, dm, nullptr, nullptr, mn, tshift);
+            or_tiles<G, OR_COARSE>(op, t0, tlen, nA, dm, nullptr, nullptr, mn, tshift);
         else
-            or_tiles<G, OR_FLAT, LIST>(op, t0, tlen, nA, lidx, nlong, dm, nullptr, nullptr, mn, tshift);
+            or_tiles<G, OR_FLAT>(op, t0, tlen, nA, dm, nullptr, nullptr, mn, tshift);
         __syncthreads();
         const ChunkScan cs = scan_popcounts<G>(dm, W, redu);
         const unsigned tot = cs.tot;
-        const long long rd = (row >= 0 && op.dir_mask) ? op.rdir[row] : -1;
-        // Kept directories of groups of 256 lanes or more (chunks of many entries) go out
-        // coalesced: the masks first, then each entry's slot offset (flat rows: written
-        // over its mask in LDS; coarse level: into doff, which the fine pass reads) after a
-        // barrier.  keep is uniform over the launch, so every thread takes the barriers.
-        // Smaller groups store each entry from the chunk walk.
-        constexpr bool COAL = G >= 256;
-        const bool keep = COAL && op.dir_mask != nullptr;
+        const long long rd = (row >= 0 && op.dir_mask) ? op.rdir[row] & ~RDIR_TWO : -1;
         unsigned nnz = tot;
-        if (COAL && !sparse && rd >= 0)
-            for (int t = l; t < W; t += G)
-                op.dir_mask[rd + t] = dm[t];
-        if (keep)
-            __syncthreads();
-        if (!COAL) {
-            if (sparse)
-                chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64 w) {
-                    doff[t] = p;
-                    if (rd >= 0) {
-                        op.dir_mask[rd + t] = w;
-                        op.dir_off[rd + t] = p;
-                    }
-                });
-            else if (rd >= 0)
-                chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64 w) {
+        if (sparse)
+            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64 w) {
+                doff[t] = p;
+                if (rd >= 0) {
                     op.dir_mask[rd + t] = w;
                     op.dir_off[rd + t] = p;
-                });
-        } else if (sparse) {
-            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64) { doff[t] = p; });
-        } else if (rd >= 0) {
-            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64) { dm[t] = p; });
-        }
-        if (keep)
-            __syncthreads();
-        if (COAL && rd >= 0) {
-            if (sparse) {
-                for (int t = l; t < W; t += G) {
-                    op.dir_mask[rd + t] = dm[t];
-                    op.dir_off[rd + t] = doff[t];
                 }
-            } else {
-                for (int t = l; t < W; t += G)
-                    op.dir_off[rd + t] = (unsigned)dm[t];
-            }
-        }
+            });
+        else if (rd >= 0)
+            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64 w) {
+                op.dir_mask[rd + t] = w;
+                op.dir_off[rd + t] = p;
+            });
         if (two_level) {
             // two-level rows: tot = non-empty tiles; build and count the fine level
             u64 *fm = dm + W;
@@ -676,34 +638,119 @@ __global__ __launch_bounds__(G < BLOCK ? BLOCK : G) void k_symbolic_lds(const in
                     fm[k] = 0;
             __syncthreads();
             if (sparse)
-                or_tiles<G, OR_FINE, LIST>(op, t0, tlen, nA, lidx, nlong, dm, doff, fm, mn, tshift);
+                or_tiles<G, OR_FINE>(op, t0, tlen, nA, dm, doff, fm, mn, tshift);
             __syncthreads();
             const int F = sparse ? (int)tot : 0;
             const ChunkScan fs = scan_popcounts<G>(fm, F, redu);
             if (sparse)
                 nnz = fs.tot;
-            // the fine level goes out as the flat directory does
-            if (COAL && rd >= 0)
-                for (int k = l; k < F; k += G)
-                    op.dir_mask[rd + W + k] = fm[k];
-            if (keep)
-                __syncthreads();
-            if (rd >= 0) {
-                if (COAL)
-                    chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64) { fm[k] = p; });
-                else
-                    chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64 w) {
-                        op.dir_mask[rd + W + k] = w;
-                        op.dir_off[rd + W + k] = p;
-                    });
-            }
-            if (keep)
-                __syncthreads();
-            if (COAL && rd >= 0)
-                for (int k = l; k < F; k += G)
-                    op.dir_off[rd + W + k] = (unsigned)fm[k];
+            if (rd >= 0)
+                chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64 w) {
+                    op.dir_mask[rd + W + k] = w;
+                    op.dir_off[rd + W + k] = p;
+                });
         }
         if (row >= 0 && l == 0)
+            rnnz[row] = (int)nnz;
+        __syncthreads();
+    }
+}
+
+// The same for a row with a workgroup to itself: the tiles of its B rows are walked as one
+// stream of pairs.  Bound by the loads of column and mask per tile (a load instruction costs
+// the same for any number of active lanes: B rows of a few tiles left most of a sub-group
+// idle, and staging entries in LDS doubled a row's need) and then by the LDS ORs.  Symbolic
+// stage of R-MAT squares, before and after: scale 16 938 and 434 us, scale 18 8.5 and
+// 3.5 ms; banded rows of 100 tiles 147 and 131 us.  TL: some row of the launch has a two-level directory.  A kept directory
+// goes out coalesced: the masks first, then each entry's slot offset, written over its mask
+// in LDS (coarse level: into doff, which the fine pass reads).
+template <int G, bool TL>
+__global__ __launch_bounds__(G) void k_symbolic_row(const int *__restrict__ rows, const int *__restrict__ count_p,
+                                                    Operands op, int *__restrict__ rnnz, unsigned *queue)
+{
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ u64 red[16];
+    __shared__ int grp_s[2];
+    const int l = threadIdx.x;
+    const int nrows = *count_p;
+    for (GroupWalk gw(queue, nrows, grp_s, c_nxcd); gw.more(); gw.next()) {
+        const int row = uniform(rows[gw.grp]);
+        const int mn = uniform(op.rmin[row]);
+        const int S = uniform(op.rmax[row]) - mn + 1;
+        const int a0 = uniform(op.Arp[row]), nA = uniform(op.Arp[row + 1]) - a0;
+        const int tp = uniform(op.rtp[row]);
+        const bool sparse = TL && use_sparse(S, tp);
+        const int W = sparse ? (S + 63) >> 6 : S; // entries of the first level
+        const StreamLayout L = sym_stream_layout(G, S, nA, tp);
+        u64 *dm = (u64 *)lds;
+        unsigned *doff = (unsigned *)(lds + L.doff);
+        Stream<G> st;
+        st.rec = (uint4 *)(lds + L.rec);
+        st.bits = (u64 *)(lds + L.bits);
+        st.wb = (unsigned short *)(lds + L.wb);
+        st.red = red;
+        const int words = (L.doff - L.bits) >> 3;
+        const long long rd = op.dir_mask ? uniform64(op.rdir[row]) & ~RDIR_TWO : -1;
+        for (int t = l; t < W; t += G)
+            dm[t] = 0;
+        for (int q = l; q < words; q += G)
+            st.bits[q] = 0;
+        __syncthreads();
+        auto tiles_of = [&](int e) {
+            const int j = op.Acol[a0 + e];
+            const typename Vec2<int>::type t = load2(op.tptr + j);
+            return Segment{t.x, t.y - t.x, 0};
+        };
+        if (!sparse)
+            st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                stream_or<G, OR_FLAT>(t, w0, op, dm, nullptr, nullptr, mn);
+            });
+        if constexpr (TL) {
+            if (sparse)
+                st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                    stream_or<G, OR_COARSE>(t, w0, op, dm, nullptr, nullptr, mn);
+                });
+        }
+        const ChunkScan cs = scan_popcounts<G>(dm, W, (unsigned *)red);
+        unsigned nnz = cs.tot;
+        if (rd >= 0)
+            for (int t = l; t < W; t += G)
+                op.dir_mask[rd + t] = dm[t];
+        __syncthreads();
+        if (sparse)
+            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64) { doff[t] = p; });
+        else if (rd >= 0)
+            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64) { dm[t] = p; });
+        __syncthreads();
+        if (rd >= 0)
+            for (int t = l; t < W; t += G)
+                op.dir_off[rd + t] = sparse ? doff[t] : (unsigned)dm[t];
+        if constexpr (TL) {
+            if (sparse) { // (uniform) the non-empty tiles' masks
+                const int F = (int)cs.tot;
+                u64 *fm = dm + W;
+                for (int k = l; k < F; k += G)
+                    fm[k] = 0;
+                for (int q = l; q < words; q += G)
+                    st.bits[q] = 0;
+                __syncthreads();
+                st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                    stream_or<G, OR_FINE>(t, w0, op, dm, doff, fm, mn);
+                });
+                const ChunkScan fs = scan_popcounts<G>(fm, F, (unsigned *)red);
+                nnz = fs.tot;
+                if (rd >= 0) {
+                    for (int k = l; k < F; k += G)
+                        op.dir_mask[rd + W + k] = fm[k];
+                    __syncthreads();
+                    chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64) { fm[k] = p; });
+                    __syncthreads();
+                    for (int k = l; k < F; k += G)
+                        op.dir_off[rd + W + k] = (unsigned)fm[k];
+                }
+            }
+        }
+        if (l == 0)
             rnnz[row] = (int)nnz;
         __syncthreads();
     }
@@ -726,7 +773,7 @@ __global__ __launch_bounds__(1024) void k_symbolic_global(const int *__restrict_
         const int row = rows[idx];
         const int mn = op.rmin[row];
         const int S = op.rmax[row] - mn + 1;
-        const long long rd = op.dir_mask ? op.rdir[row] : -1;
+        const long long rd = op.dir_mask ? op.rdir[row] & ~RDIR_TWO : -1;
         u64 *dm = rd >= 0 ? op.dir_mask + rd : gws + (size_t)blockIdx.x * gws_stride;
         for (int t = l; t < S; t += 1024)
             dm[t] = 0;
@@ -766,7 +813,7 @@ __global__ __launch_bounds__(1024) void k_symbolic_wide(const int *__restrict__ 
         const int row = uniform(rows[idx]);
         const int mn = uniform(op.rmin[row]);
         const int S = uniform(op.rmax[row]) - mn + 1;
-        const long long rd = op.dir_mask ? uniform64(op.rdir[row]) : -1;
+        const long long rd = op.dir_mask ? uniform64(op.rdir[row]) & ~RDIR_TWO : -1;
         for (int t = l; t < S; t += 1024)
             dm[t] = 0;
         __syncthreads();
@@ -851,7 +898,7 @@ __global__ __launch_bounds__(BLOCK) void k_numeric_lds(const int *__restrict__ r
         unsigned *foff = sparse ? doff + W : doff;
         const bool dense = !sparse && use_dense(S, n);
         const int nv = dense ? 64 * S : n;
-        const long long rd = (row >= 0 && op.dir_mask) ? op.rdir[row] : -1;
+        const long long rd = (row >= 0 && op.dir_mask) ? kept_dir(op, row, sparse) : -1;
         for (int q = l; q < nv; q += G)
             vals[q] = 0.0;
         if (LONG && l == 0)
@@ -877,9 +924,9 @@ __global__ __launch_bounds__(BLOCK) void k_numeric_lds(const int *__restrict__ r
         }
         if (rd < 0) {
             if (sparse)
-                or_tiles<G, OR_COARSE>(op, t0, tlen, nA, nullptr, 0, dm, nullptr, nullptr, mn, tshift);
+                or_tiles<G, OR_COARSE>(op, t0, tlen, nA, dm, nullptr, nullptr, mn, tshift);
             else
-                or_tiles<G, OR_FLAT>(op, t0, tlen, nA, nullptr, 0, dm, nullptr, nullptr, mn, tshift);
+                or_tiles<G, OR_FLAT>(op, t0, tlen, nA, dm, nullptr, nullptr, mn, tshift);
         }
         // first level: flat slot offsets (rebuilt) or coarse compact indices (rebuilt), and
         // the total (flat: nnz(C_i); two-level: non-empty tiles)
@@ -914,7 +961,7 @@ __global__ __launch_bounds__(BLOCK) void k_numeric_lds(const int *__restrict__ r
             }
             __syncthreads();
             if (sparse && rd < 0)
-                or_tiles<G, OR_FINE>(op, t0, tlen, nA, nullptr, 0, dm, doff, fm, mn, tshift);
+                or_tiles<G, OR_FINE>(op, t0, tlen, nA, dm, doff, fm, mn, tshift);
             __syncthreads();
             const ChunkScan fs = scan_popcounts<G>(fm, sparse ? F : 0, redu);
             if (sparse) {
@@ -1013,7 +1060,7 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
         unsigned *foff = sparse ? doff + W : doff;
         const bool dense = !sparse && use_dense(S, n);
         const int nv = dense ? 64 * S : n;
-        const long long rd = op.dir_mask ? uniform64(op.rdir[row]) : -1;
+        const long long rd = op.dir_mask ? uniform64(kept_dir(op, row, sparse)) : -1;
         const int words = (L.doff - L.bits) >> 3;
         for (int q = 2 * l; q < nv; q += 2 * G) // (the array is padded to 16 bytes)
             *(double2 *)(vals + q) = make_double2(0.0, 0.0);
@@ -1031,8 +1078,8 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
         __syncthreads();
         auto tiles_of = [&](int e) {
             const int j = op.Acol[a0 + e];
-            const int t0 = op.tptr[j];
-            return Segment{t0, op.tptr[j + 1] - t0, 0};
+            const typename Vec2<int>::type t = load2(op.tptr + j);
+            return Segment{t.x, t.y - t.x, 0};
         };
         auto rezero = [&]() { // the stream's bits, for its next run
             __syncthreads();
@@ -1100,9 +1147,9 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
         if (ok) { // uniform
             auto rows_of = [&](int e) {
                 const int j = op.Acol[a0 + e];
-                const int b0 = op.Brp[j];
+                const typename Vec2<int>::type b = load2(op.Brp + j);
                 const double a = (double)Aval[a0 + e];
-                return Segment{b0, op.Brp[j + 1] - b0, (u64)__double_as_longlong(a)};
+                return Segment{b.x, b.y - b.x, (u64)__double_as_longlong(a)};
             };
             if (dense)
                 st.run(nA, rows_of, [&](const Stream<G> &t, long long w0) {
@@ -1262,13 +1309,6 @@ DEVI void collect_active(const int *nxt, const int *cur, const int *kend, int b0
     }
 }
 
-// The directory form the symbolic kernels stored for a row of the wide bin: two-level
-// (coarse words, then compact fine entries) or flat (one entry per tile of the span).
-DEVI bool wide_two_level(int S, int nA, int tp, long long sym_row_max, int sym_all_global, int long_rows)
-{
-    return use_sparse(S, tp) && !sym_all_global && sym_need(S, nA, tp, long_rows) <= sym_row_max;
-}
-
 template <typename P>
 __global__ __launch_bounds__(1024) void k_numeric_window(const int *__restrict__ rows, const int *__restrict__ count_p,
                                                          Operands op, const long long *__restrict__ crp,
@@ -1398,7 +1438,6 @@ __global__ __launch_bounds__(1024) void k_numeric_wcompact(const int *__restrict
                                                            Operands op, const long long *__restrict__ crp,
                                                            int *__restrict__ Ccol, typename P::V *__restrict__ Cval,
                                                            int bshift, int *ws, long long cur_stride, long long ft_stride,
-                                                           long long sym_row_max, int sym_all_global, int long_rows,
                                                            int *err)
 {
     typedef typename P::V V;
@@ -1427,10 +1466,9 @@ __global__ __launch_bounds__(1024) void k_numeric_wcompact(const int *__restrict
         const long long n = crp[row + 1] - cb;
         const int mn = op.rmin[row];
         const int S = op.rmax[row] - mn + 1;
-        const int tp = op.rtp[row];
-        const long long rd = op.rdir[row];
         // the form the symbolic phase kept: two-level only if the row was in an LDS bin there
-        const bool two = wide_two_level(S, nA, tp, sym_row_max, sym_all_global, long_rows);
+        const bool two = (op.rdir[row] & RDIR_TWO) != 0;
+        const long long rd = op.rdir[row] & ~RDIR_TWO;
         const int W = two ? (S + 63) >> 6 : 0;
         const u64 *cmask = op.dir_mask + rd;      // coarse words (two-level)
         const unsigned *coff = op.dir_off + rd;
@@ -1580,17 +1618,16 @@ struct WideDir {
     unsigned n;   // entries of C_i
     bool two;
 
-    DEVI WideDir(const Operands &op, const long long *crp, int row, long long sym_row_max, int sym_all_global,
-                 int long_rows)
+    DEVI WideDir(const Operands &op, const long long *crp, int row)
     {
-        const int nA = uniform(op.Arp[row + 1]) - uniform(op.Arp[row]);
         const long long cb = uniform64(crp[row]);
         n = (unsigned)(uniform64(crp[row + 1]) - cb);
         mn = uniform(op.rmin[row]);
         S = uniform(op.rmax[row]) - mn + 1;
-        two = wide_two_level(S, nA, uniform(op.rtp[row]), sym_row_max, sym_all_global, long_rows);
+        const long long r = uniform64(op.rdir[row]);
+        two = (r & RDIR_TWO) != 0;
         const int W = two ? (S + 63) >> 6 : 0;
-        const long long rd = uniform64(op.rdir[row]);
+        const long long rd = r & ~RDIR_TWO;
         cm = op.dir_mask + rd;
         co = op.dir_off + rd;
         fm = cm + W;
@@ -1637,7 +1674,6 @@ struct WideDir {
 template <bool FILL>
 __global__ __launch_bounds__(256) void k_wide_items(const int *__restrict__ rows, const int *__restrict__ count_p,
                                                     Operands op, const long long *__restrict__ crp, long long U,
-                                                    long long sym_row_max, int sym_all_global, int long_rows,
                                                     WideItem *__restrict__ items, long long cap, unsigned *ctr, int *err)
 {
     __shared__ unsigned cnt[WIDE_BUCKETS], base[WIDE_BUCKETS];
@@ -1656,7 +1692,7 @@ __global__ __launch_bounds__(256) void k_wide_items(const int *__restrict__ rows
         __syncthreads();
         for (int i = i0 + w; i < i1; i += 4) {
             const int row = uniform(rows[i]);
-            const WideDir d(op, crp, row, sym_row_max, sym_all_global, long_rows);
+            const WideDir d(op, crp, row);
             const int U0 = d.mn / WIDE_TILES, U1 = (d.mn + d.S - 1) / WIDE_TILES + 1; // units of the row
             int u = U0;                   // first unit of the open window
             unsigned at = 0;              // entries before it
@@ -1725,8 +1761,7 @@ constexpr int WC_STAGE = 4096; // columns of a flat chunk staged in LDS for coal
 // denser tiles are listed in LDS and written by a wave each, one lane per column.
 __global__ __launch_bounds__(WC_BS) void k_wide_cols(const int *__restrict__ rows, const int *__restrict__ count_p,
                                                      Operands op, const long long *__restrict__ crp,
-                                                     int *__restrict__ Ccol, long long sym_row_max,
-                                                     int sym_all_global, int long_rows)
+                                                     int *__restrict__ Ccol)
 {
     // one buffer, used by one path per chunk: the staged chunk's columns, or the list of
     // its dense tiles (mask, first slot, absolute tile), so that the waves writing them
@@ -1743,16 +1778,16 @@ __global__ __launch_bounds__(WC_BS) void k_wide_cols(const int *__restrict__ row
     const int nrows = *count_p;
     for (int idx = blockIdx.x; idx < nrows; idx += gridDim.x) {
         const int row = uniform(rows[idx]);
-        const int nA = uniform(op.Arp[row + 1]) - uniform(op.Arp[row]);
         const long long cb = uniform64(crp[row]);
         const long long n = uniform64(crp[row + 1]) - cb;
         if (n <= 0)
             continue;
         const int mn = uniform(op.rmin[row]);
         const int S = uniform(op.rmax[row]) - mn + 1;
-        const bool two = wide_two_level(S, nA, uniform(op.rtp[row]), sym_row_max, sym_all_global, long_rows);
+        const long long r = uniform64(op.rdir[row]);
+        const bool two = (r & RDIR_TWO) != 0;
         const int W = two ? (S + 63) >> 6 : 0;
-        const long long rd = uniform64(op.rdir[row]);
+        const long long rd = r & ~RDIR_TWO;
         const u64 *cmg = op.dir_mask + rd;
         const unsigned *cog = op.dir_off + rd;
         const u64 *fm = op.dir_mask + rd + W;
@@ -1856,8 +1891,7 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
                                                         const unsigned *__restrict__ ctr_listed, unsigned *ctr_taken,
                                                         Operands op, const int *__restrict__ index, long long U,
                                                         const long long *__restrict__ crp,
-                                                        typename P::V *__restrict__ Cval, long long sym_row_max,
-                                                        int sym_all_global, int long_rows)
+                                                        typename P::V *__restrict__ Cval)
 {
     typedef typename P::V V;
     extern __shared__ __align__(16) unsigned char lds[];
@@ -1886,7 +1920,7 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
         const int cnt = (int)uniform(items[it].cnt);
         const int u0 = (int)(units & 0xffffffu), u1 = u0 + (int)(units >> 24);
         const int a0 = uniform(op.Arp[row]), nA = uniform(op.Arp[row + 1]) - a0;
-        const WideDir d(op, crp, row, sym_row_max, sym_all_global, long_rows);
+        const WideDir d(op, crp, row);
         const long long cb = uniform64(crp[row]) + base;
         const int T0 = u0 * WIDE_TILES, nt = (u1 - u0) * WIDE_TILES;
         for (int t = l; t < nt; t += BS) {
@@ -1943,25 +1977,34 @@ template <int G, bool LONG>
 static void symbolic_g(const int *rows, const int *count_dev, int count, int max_need, const Operands &op, int *rnnz,
                        int tshift, int two_level, int num_cus, unsigned *queue, hipStream_t s)
 {
-    constexpr int BS = G < BLOCK ? BLOCK : G;
-    constexpr int RPB = BS / G;
+    constexpr int RPB = BLOCK / G;
     const int slice = (max_need + 15) & ~15;
     const size_t lds = (size_t)slice * RPB;
     const int64_t blocks =
-        row_grid(k_symbolic_lds<G, LONG>, BS, lds, ((int64_t)count + RPB - 1) / RPB, num_cus, queue);
+        row_grid(k_symbolic_lds<G, LONG>, BLOCK, lds, ((int64_t)count + RPB - 1) / RPB, num_cus, queue);
     const int lg = __builtin_ctz(G);
-    hipLaunchKernelGGL((k_symbolic_lds<G, LONG>), dim3((unsigned)blocks), dim3(BS), lds, s, rows, count_dev, slice, op,
-                       rnnz, tshift > lg ? lg : tshift, two_level, queue);
+    hipLaunchKernelGGL((k_symbolic_lds<G, LONG>), dim3((unsigned)blocks), dim3(BLOCK), lds, s, rows, count_dev, slice,
+                       op, rnnz, tshift > lg ? lg : tshift, two_level, queue);
 }
 
-template <bool LONG>
-static void symbolic_l(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
-                       int *rnnz, int tshift, int two_level, int num_cus, unsigned *queue, hipStream_t s)
+template <int G, bool TL>
+static void symbolic_row(const int *rows, const int *count_dev, int count, int max_need, const Operands &op, int *rnnz,
+                         int num_cus, unsigned *queue, hipStream_t s)
+{
+    const size_t lds = (size_t)((max_need + 15) & ~15);
+    const int64_t blocks = row_grid(k_symbolic_row<G, TL>, G, lds, count, num_cus, queue);
+    hipLaunchKernelGGL((k_symbolic_row<G, TL>), dim3((unsigned)blocks), dim3(G), lds, s, rows, count_dev, op, rnnz,
+                       queue);
+}
+
+template <bool TL>
+static void symbolic_rows(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
+                          int *rnnz, int num_cus, unsigned *queue, hipStream_t s)
 {
 #define SYM(B, G)                                                                                                      \
-    case B: symbolic_g<G, LONG>(rows, count_dev, count, max_need, op, rnnz, tshift, two_level, num_cus, queue, s); break;
+    case B: symbolic_row<G, TL>(rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s); break;
     switch (bin) {
-        SYM(0, 8) SYM(1, 16) SYM(2, 32) SYM(3, 64) SYM(4, 128) SYM(5, 256) SYM(6, 512) SYM(7, 1024)
+        SYM(3, 64) SYM(4, 128) SYM(5, 256) SYM(6, 512) SYM(7, 1024)
     }
 #undef SYM
 }
@@ -1982,10 +2025,17 @@ hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int c
             hipLaunchKernelGGL(k_symbolic_global, dim3(blocks), dim3(1024), 0, s, rows, count_dev, op, rnnz,
                                tshift > 10 ? 10 : tshift, gws, gws_stride);
     } else if (bin >= 0 && bin < NLDS) {
-        if (long_rows)
-            symbolic_l<true>(bin, rows, count_dev, count, max_need, op, rnnz, tshift, two_level, num_cus, queue, s);
+#define SYM(B, G, LONG)                                                                                                \
+    case B: symbolic_g<G, LONG>(rows, count_dev, count, max_need, op, rnnz, tshift, two_level, num_cus, queue, s); break;
+        if (bin >= 3 && two_level)
+            symbolic_rows<true>(bin, rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s);
+        else if (bin >= 3)
+            symbolic_rows<false>(bin, rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s);
+        else if (long_rows)
+            switch (bin) { SYM(0, 8, true) SYM(1, 16, true) SYM(2, 32, true) }
         else
-            symbolic_l<false>(bin, rows, count_dev, count, max_need, op, rnnz, tshift, two_level, num_cus, queue, s);
+            switch (bin) { SYM(0, 8, false) SYM(1, 16, false) SYM(2, 32, false) }
+#undef SYM
     } else {
         return hipErrorInvalidValue;
     }
@@ -2072,21 +2122,19 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
                                wide.nunits, op.Brp, op.Bcol, wide.index);
             const unsigned gi = (unsigned)(count < 4 * num_cus ? (count + 3) / 4 : num_cus);
             hipLaunchKernelGGL(k_wide_items<false>, dim3(gi), dim3(256), 0, s, rows, count_dev, op, crp, wide.nunits,
-                               wide.sym_row_max, wide.sym_all_global, wide.long_rows, wide.items, wide.items_cap,
-                               wide.ctr, err);
+                               wide.items, wide.items_cap, wide.ctr, err);
             hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(64), 0, s, wide.ctr);
             hipLaunchKernelGGL(k_wide_items<true>, dim3(gi), dim3(256), 0, s, rows, count_dev, op, crp, wide.nunits,
-                               wide.sym_row_max, wide.sym_all_global, wide.long_rows, wide.items, wide.items_cap,
-                               wide.ctr, err);
+                               wide.items, wide.items_cap, wide.ctr, err);
             hipLaunchKernelGGL(k_wide_cols, dim3((unsigned)(count < 8192 ? count : 8192)), dim3(WC_BS), 0, s, rows,
-                               count_dev, op, crp, Ccol, wide.sym_row_max, wide.sym_all_global, wide.long_rows);
+                               count_dev, op, crp, Ccol);
             hipLaunchKernelGGL((k_numeric_windows<P, WW_BS>), dim3((unsigned)wide.blocks), dim3(WW_BS),
                                ww_lds<WW_BS>(), s, wide.items, wide.ctr, wide.ctr + 1, op, wide.index, wide.nunits, crp,
-                               (typename P::V *)Cval, wide.sym_row_max, wide.sym_all_global, wide.long_rows);
+                               (typename P::V *)Cval);
         } else if (op.dir_mask)
             hipLaunchKernelGGL(k_numeric_wcompact<P>, dim3(blocks), dim3(1024), CW_LDS, s, rows, count_dev, op, crp,
                                Ccol, (typename P::V *)Cval, bshift > 6 ? 6 : bshift, wide.ws, wide.cur_stride,
-                               wide.ft_stride, wide.sym_row_max, wide.sym_all_global, wide.long_rows, err);
+                               wide.ft_stride, err);
         else
             hipLaunchKernelGGL(k_numeric_window<P>, dim3(blocks), dim3(1024), WIN_LDS, s, rows, count_dev, op, crp, Ccol,
                                (typename P::V *)Cval, bshift > 6 ? 6 : bshift, wide.ws, wide.cur_stride, wide.ft_stride,
@@ -2149,20 +2197,22 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
             e = r;                                                                                                     \
     }
 #define CFGL(L)                                                                                                        \
-    CFG((k_symbolic_lds<8, L>)) CFG((k_symbolic_lds<16, L>)) CFG((k_symbolic_lds<32, L>))                             \
-    CFG((k_symbolic_lds<64, L>)) CFG((k_symbolic_lds<128, L>)) CFG((k_symbolic_lds<256, L>))                          \
-    CFG((k_symbolic_lds<512, L>)) CFG((k_symbolic_lds<1024, L>))
+    CFG((k_symbolic_lds<8, L>)) CFG((k_symbolic_lds<16, L>)) CFG((k_symbolic_lds<32, L>))
+#define CFGS(TL)                                                                                                       \
+    CFG((k_symbolic_row<64, TL>)) CFG((k_symbolic_row<128, TL>)) CFG((k_symbolic_row<256, TL>))                        \
+    CFG((k_symbolic_row<512, TL>)) CFG((k_symbolic_row<1024, TL>))
 #define CFGP(P, L)                                                                                                     \
     CFG((k_numeric_lds<8, P, L>)) CFG((k_numeric_lds<16, P, L>)) CFG((k_numeric_lds<32, P, L>))
 #define CFGR(P, TL)                                                                                                    \
     CFG((k_numeric_row<64, P, TL>)) CFG((k_numeric_row<128, P, TL>)) CFG((k_numeric_row<256, P, TL>))                  \
     CFG((k_numeric_row<512, P, TL>)) CFG((k_numeric_row<1024, P, TL>))
-    CFGL(false) CFGL(true)
+    CFGL(false) CFGL(true) CFGS(false) CFGS(true)
     CFGP(PrecF64, false) CFGP(PrecF64, true) CFGP(PrecF32C, false) CFGP(PrecF32C, true)
     CFGR(PrecF64, false) CFGR(PrecF32C, false) CFGR(PrecF64, true) CFGR(PrecF32C, true)
 #undef CFGR
 #undef CFGP
 #undef CFGL
+#undef CFGS
     CFG(k_symbolic_wide)
     CFG(k_numeric_window<PrecF64>) CFG(k_numeric_window<PrecF32C>)
     CFG(k_numeric_wcompact<PrecF64>) CFG(k_numeric_wcompact<PrecF32C>) 

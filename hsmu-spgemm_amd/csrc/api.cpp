@@ -751,11 +751,10 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     bp.lds_block_budget = opts.lds_block_budget > 0 ? opts.lds_block_budget : 8 * 1024;
     if (bp.lds_block_budget > lds_dyn)
         bp.lds_block_budget = lds_dyn;
-    bp.per_lane = opts.tiles_per_lane > 0 ? opts.tiles_per_lane : 4;
-    const long long bp_sym_row_max = bp.lds_row_max;
+    bp.per_lane = opts.tiles_per_lane > 0 ? opts.tiles_per_lane : 32;
     bp.force_global = opts.force_global;
     bp.lds_cu = lds_dyn;
-    bp.min_waves = opts.min_waves > 0 ? opts.min_waves : 8;
+    bp.min_waves = opts.min_waves > 0 ? opts.min_waves : 16;
     HIP_TRY(launch_row_info(M, K, P.nnzA, P.Arp, P.Acol, brow, tptr, rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, dst,
                             sums, &dw->done[0], host, c->num_cus, s));
     HIP_TRY(mark(c->ev[EV_ANALYSIS]));
@@ -953,9 +952,6 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
             const bool windows = keep_dirs && (unsigned long long)index_n * sizeof(int) <= index_max &&
                                  units < (1 << 24) && h2.wide_items < (1ull << 31);
             wide.blocks = windows ? wide_window_blocks(c->num_cus) : (cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt);
-            wide.sym_row_max = bp_sym_row_max;
-            wide.sym_all_global = opts.force_global ? 1 : 0;
-            wide.long_rows = long_rows;
             if (windows) {
                 wide.nunits = units;
                 wide.K = K;

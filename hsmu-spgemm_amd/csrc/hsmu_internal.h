@@ -210,11 +210,6 @@ HSMU_HD inline RowLayout row_layout(int numeric, int S, int n, int nA, int tp, b
     return L;
 }
 
-HSMU_HD inline int sym_need(int S, int nA, int tp, bool with_long)
-{
-    return row_layout(0, S, 0, nA, tp, with_long).bytes;
-}
-
 // ---- one row per workgroup (64 lanes or more): the element stream ------------------------
 //
 // The B rows of a row's A entries are walked as one stream of slots of STREAM_V consecutive
@@ -274,6 +269,42 @@ HSMU_HD inline StreamLayout stream_layout(int G, int S, int n, int nA, int tp, l
     return L;
 }
 
+// The symbolic counterpart: the stream is of tile pairs.
+//   dm   u64[E]     tile masks (flat), or coarse words then fine masks (two-level)
+//   rec, bits       as above
+//   doff u32[E]     two-level: coarse offsets
+//   wb   u16[...]   as above
+HSMU_HD inline StreamLayout sym_stream_layout(int G, int S, int nA, int tp)
+{
+    StreamLayout L = {};
+    const int E = dir_entries(S, tp);
+    if (E > LAYOUT_CAP) {
+        L.bytes = LAYOUT_NONE;
+        return L;
+    }
+    const long long slots = ((long long)tp + (long long)nA * (STREAM_V - 1)) / STREAM_V;
+    const int words = ((slots < stream_window(G) ? (int)slots : stream_window(G)) + 63) >> 6;
+    int o = (8 * E + 15) & ~15;
+    L.rec = o;
+    o += 16 * (nA < G ? nA : G);
+    L.bits = o;
+    o += 8 * words;
+    L.doff = o;
+    if (use_sparse(S, tp))
+        o += 4 * E;
+    L.wb = o;
+    o += 2 * words;
+    L.bytes = (o + 15) & ~15;
+    return L;
+}
+
+// LDS a row needs in symbolic bin `bin`
+HSMU_HD inline int sym_need(int bin, int S, int nA, int tp, bool with_long)
+{
+    return (8 << bin) >= BLOCK ? sym_stream_layout(8 << bin, S, nA, tp).bytes
+                               : row_layout(0, S, 0, nA, tp, with_long).bytes;
+}
+
 // LDS a row with p products needs in numeric bin `bin`
 HSMU_HD inline int num_need(int bin, int S, int n, int nA, int tp, long long p, bool with_long)
 {
@@ -320,6 +351,10 @@ hipError_t launch_rowptr_bin(int64_t M, const int *Arp, const long long *rprod, 
                              unsigned *ticket, DevStats *st, BinSum *sums, unsigned *done,
                              DevStats *host, hipStream_t s);
 
+// A kept directory that is two-level has this bit in rdir (the form follows from use_sparse
+// for rows the symbolic phase held in LDS; it keeps flat ones for the others).
+constexpr long long RDIR_TWO = 1LL << 62;
+
 struct Operands {
     const int *Arp, *Acol;
     const void *Aval; // double, or float when val32
@@ -360,8 +395,7 @@ hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int c
 // (aligned, so that all rows' windows share their boundaries) that holds at most WIDE_UNIT
 // entries of C_i and spans at most WIDE_UMAX units, one workgroup each.  The index gives
 // every B row's first element at each unit's start, so a window's elements are known without
-// a search.  (Which rows' directories are flat depends on what the symbolic phase held in
-// global memory: sym_row_max, sym_all_global, long_rows.)
+// a search.
 constexpr int WIDE_UNIT = 4096;
 constexpr int WIDE_UMAX = 16;
 constexpr int WIDE_TILES = WIDE_UNIT / 64;     // tiles of a unit
@@ -387,9 +421,6 @@ struct WideRows {
     int *ws;
     long long cur_stride, ft_stride;
     int blocks;
-    long long sym_row_max;
-    int sym_all_global;
-    int long_rows; // the with_long the symbolic binning used
     // windows: their capacity and list, and counters: windows listed, taken, then per bucket
     // the windows and the place of the next one (null items: one workgroup per row)
     long long items_cap;

@@ -376,13 +376,23 @@ hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const
 // exceeds lds_row_max go to the global-memory bin.  need(b): the row's LDS in bin b.
 // Reference ranges being replaced: src/bining.cuh:12 (symbolic), :121 (tile OR), :228
 // (numeric).
+// Lanes per row: the stream that rows with a workgroup of their own walk costs about the
+// same per item at every width from 64 lanes, and a start and an end per row that narrow
+// groups spread over more rows, so both phases give a lane 32 items by default (symbolic
+// stage at 4 / 16 / 32 tiles per lane: R-MAT squares of scale 16 746 / 476 / 439 us and of
+// scale 18 6.67 / 4.28 / 3.52 ms, banded rows of 100 tiles 116 / 72 / 66 us).  Symbolic rows that share a wave walk their entries one after the other, in step
+// with the longest of them: beyond 16 tiles per lane their own wave is faster.  16 waves
+// per CU, where LDS limits the workgroups, take 17.8 ms on the square of scale 18 against
+// 19.2 ms with 8; 24 slow a banded square by 4%.
+constexpr int SHARED_PER_LANE = 16;
 template <typename Need>
-DEVI int choose_bin(long long work, Need need, const BinParams &bp)
+DEVI int choose_bin(int numeric, long long work, Need need, const BinParams &bp)
 {
     if (bp.force_global)
         return BIN_GLOBAL;
+    const int shared = !numeric && bp.per_lane > SHARED_PER_LANE ? SHARED_PER_LANE : bp.per_lane;
     int b = 0;
-    while (b < NLDS - 1 && (8LL << b) * bp.per_lane < work)
+    while (b < NLDS - 1 && (8LL << b) * ((8 << b) < BLOCK ? shared : bp.per_lane) < work)
         ++b;
     // the budget limits only workgroups that pack several rows: a one-row workgroup needs
     // the row's LDS whatever its width
@@ -455,12 +465,13 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, bool with_long,
         if (numeric) {
             work = r.prod;
             auto nd = [&](int bin) { return num_need(bin, r.S, r.nc, r.nA, r.tp, r.prod, with_long); };
-            at.b = choose_bin(work, nd, bp);
+            at.b = choose_bin(numeric, work, nd, bp);
             need = nd(at.b);
         } else {
             work = r.tp;
-            need = sym_need(r.S, r.nA, r.tp, with_long);
-            at.b = choose_bin(work, [&](int) { return need; }, bp);
+            auto nd = [&](int bin) { return sym_need(bin, r.S, r.nA, r.tp, with_long); };
+            at.b = choose_bin(numeric, work, nd, bp);
+            need = nd(at.b);
             // the numeric need with nnz(C_i) <= min(products, 64 * span)
             const long long nub = r.prod < 64LL * r.S ? r.prod : 64LL * r.S;
             wide = num_need(NLDS - 1, r.S, (int)(nub < INT_MAX ? nub : INT_MAX), r.nA, r.tp, r.prod, with_long) > bp.lds_row_max;
@@ -517,7 +528,7 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, bool with_long,
         if (mine) {
             at.pos = base + mbcnt(same);
             if (E > 0)
-                at.dloc = (long long)(dbase + dincl) - E;
+                at.dloc = ((long long)(dbase + dincl) - E) | (sp && bb < BIN_GLOBAL ? RDIR_TWO : 0);
         }
     }
     return at;

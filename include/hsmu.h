@@ -114,7 +114,8 @@ typedef struct hsmu_opts {
     int32_t lds_block_budget; /* LDS bytes per workgroup for bins that pack several rows
                                  into one workgroup (one wave); 0 = default (8 KiB) */
     int32_t products_per_lane;/* numeric work per lane that sets a row's lane count; 0 = 32 */
-    int32_t tiles_per_lane;   /* symbolic work per lane that sets a row's lane count; 0 = 4 */
+    int32_t tiles_per_lane;   /* symbolic work per lane that sets a row's lane count (rows that
+                                 share a wave: at most 16); 0 = 32 */
     int32_t timing;           /* hipEvents into hsmu_stats (each costs the device a few us):
                                  1 = per stage and per numeric bin (the default), 2 = per
                                  numeric bin only, 0 = none (stage and bin times read 0) */
@@ -130,7 +131,7 @@ typedef struct hsmu_opts {
                                  device work queues; 0: one workgroup per row group */
     int32_t min_waves;        /* a row that has a workgroup to itself gets enough lanes for
                                  this many waves per CU at the occupancy its LDS allows (at
-                                 most 1024 lanes); 0 = 8 */
+                                 most 1024 lanes); 0 = 16 */
     int32_t wide_scratch_mb;  /* rows wider than LDS: MiB the column index of B may take that cuts
                                  them into windows (4 bytes per row of B and 4,096 columns);
                                  0 = a quarter of device memory.  Beyond it those rows take one
