@@ -253,7 +253,7 @@ def bench_rmat(hsmu, ctx, steps, table):
              "frac_end_to_end": round(st["alg_bytes"] / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
              "frac_compulsory": round(st["compulsory_bytes"] / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
              "products": st["products"], "nnz_c": st["nnz_c"],
-             "wide_bin": {"kernels": "k_wide_index, k_wide_items, k_wide_order, k_wide_cols, k_numeric_windows",
+             "wide_bin": {"kernels": "k_wide_index, k_wide_items, k_wide_order, k_numeric_windows",
                           "rows": st["num_bin_rows"][wide], "ms": round(st["ms_numeric_bin"][wide], 2),
                           "alg_bytes": st["num_bin_bytes"][wide],
                           "alg_GBps": round(st["num_bin_bytes"][wide] / (st["ms_numeric_bin"][wide] * 1e-3) / 1e9, 1)

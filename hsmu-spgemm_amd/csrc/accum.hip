@@ -13,8 +13,7 @@
 // column list, src/compressed/compressed_Cval.cuh:5-69 and src/small/numeric.cuh:233-253);
 // a dense form (one slot per column of a short, full span) skips the directory.  The
 // numeric kernels also write C's sorted columns, replacing the reference's rank-sort pass
-// (compressed_Ccol_symbolic.cuh:4-63); for the wide rows a separate streaming kernel
-// (k_wide_cols) writes them from the kept directories.
+// (compressed_Ccol_symbolic.cuh:4-63).
 //
 // The kernels of rows that share a wave, and the symbolic ones, stage the row's A entries (B
 // row range, first tile, a_ij) in LDS once; sub-groups of lanes then take one entry each
@@ -383,7 +382,37 @@ template <int G> struct Stream {
         e = e < nrec ? e : nrec - 1;
         return rec[e];
     }
-    // The bits must be zero, and a barrier passed since.
+    // The bits must be zero, and a barrier passed since.  col_of(e) loads entry e's column
+    // and entry_of(e, col) the rest; past the row's end they give an empty entry.  Those of
+    // the next G entries, and the columns of the G after them, are loaded while the body
+    // walks these.
+    template <typename Col, typename Entry, typename Body>
+    DEVI void run(int nA, const Segment &s0, Col col_of, Entry entry_of, Body body)
+    {
+        const int l = threadIdx.x;
+        Segment g = s0;
+        int j = G < nA ? col_of(G + l) : 0;
+        for (int c = 0; c < nA; c += G) {
+            stage(g);
+            if (c + G < nA) {
+                g = entry_of(c + G + l, j);
+                if (c + 2 * G < nA)
+                    j = col_of(c + 2 * G + l);
+            }
+            for (long long w0 = 0; w0 < total; w0 += WINDOW) {
+                mark(w0);
+                __syncthreads();
+                body(*this, w0);
+                __syncthreads();
+                if (c + G < nA || w0 + WINDOW < total) {
+                    const int n = steps(w0);
+                    for (int q = l; q < n; q += G)
+                        bits[q] = 0;
+                    __syncthreads();
+                }
+            }
+        }
+    }
     template <typename Entry, typename Body> DEVI void run(int nA, Entry entry_of, Body body)
     {
         const int l = threadIdx.x;
@@ -1610,21 +1639,19 @@ __global__ __launch_bounds__(256) void k_wide_index(long long K, long long U, co
     }
 }
 
+constexpr int WI_BS = 256; // lanes of a k_wide_items workgroup
+
 // A wide row's directory in global memory, flat or two-level.
 struct WideDir {
     const u64 *cm, *fm;
     const unsigned *co, *fo;
-    int mn, S, F; // first tile, tiles spanned, fine entries
-    unsigned n;   // entries of C_i
+    int mn, S; // first tile, tiles spanned
     bool two;
 
-    DEVI WideDir(const Operands &op, const long long *crp, int row)
+    DEVI WideDir(const Operands &op, int first, int last, long long r)
     {
-        const long long cb = uniform64(crp[row]);
-        n = (unsigned)(uniform64(crp[row + 1]) - cb);
-        mn = uniform(op.rmin[row]);
-        S = uniform(op.rmax[row]) - mn + 1;
-        const long long r = uniform64(op.rdir[row]);
+        mn = first;
+        S = last - first + 1;
         two = (r & RDIR_TWO) != 0;
         const int W = two ? (S + 63) >> 6 : 0;
         const long long rd = r & ~RDIR_TWO;
@@ -1632,10 +1659,16 @@ struct WideDir {
         co = op.dir_off + rd;
         fm = cm + W;
         fo = co + W;
-        F = two ? (int)(uniform(co[W - 1]) + (unsigned)__popcll(uniform64(cm[W - 1]))) : S;
     }
-    // entries of C_i before tile t (relative to mn, any integer)
-    DEVI unsigned before(int t) const
+    // entries of the (fine) level
+    DEVI int entries() const
+    {
+        const int W = (S + 63) >> 6;
+        return two ? (int)(uniform(co[W - 1]) + (unsigned)__popcll(uniform64(cm[W - 1]))) : S;
+    }
+    // entries of C_i, n of them in F = entries() tiles, before tile t (relative to mn, any
+    // integer)
+    DEVI unsigned before(int t, int F, unsigned n) const
     {
         if (t <= 0)
             return 0;
@@ -1668,201 +1701,83 @@ struct WideDir {
 };
 
 // The windows of the wide rows, a wave per row: greedy runs of units.  FILL = false counts
-// them per bucket (a bucket is a range of first units), FILL = true writes them, so that the
-// list goes through C's columns in order and the workgroups that run together read the same
-// part of B, which then stays in the L2s (R-MAT scale 18: 1/32 of B is 1.5 MB).
+// them per bucket (a bucket is a range of first units) and workgroup, FILL = true writes
+// them, so that the list goes through C's columns in order and the workgroups that run
+// together read the same part of B, which then stays in the L2s (R-MAT scale 18: 1/32 of B
+// is 1.5 MB).  Bound by the chain of loads per row, so the grid fills the device.
 template <bool FILL>
-__global__ __launch_bounds__(256) void k_wide_items(const int *__restrict__ rows, const int *__restrict__ count_p,
-                                                    Operands op, const long long *__restrict__ crp, long long U,
-                                                    WideItem *__restrict__ items, long long cap, unsigned *ctr, int *err)
+__global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ rows, const int *__restrict__ count_p,
+                                                      Operands op, const long long *__restrict__ crp, long long U,
+                                                      WideItem *__restrict__ items, long long cap,
+                                                      unsigned *__restrict__ places, int *err)
 {
-    __shared__ unsigned cnt[WIDE_BUCKETS], base[WIDE_BUCKETS];
+    __shared__ unsigned cnt[WIDE_BUCKETS];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int nrows = *count_p;
-    unsigned *total = ctr + 2, *next = ctr + 2 + WIDE_BUCKETS;
-    // each workgroup takes a contiguous run of rows, twice over: count, then (FILL) write
-    const int per = (nrows + (int)gridDim.x - 1) / (int)gridDim.x;
-    const int i0 = (int)blockIdx.x * per, i1 = i0 + per < nrows ? i0 + per : nrows;
-    for (int pass = 0; pass < (FILL ? 2 : 1); ++pass) {
-        if (threadIdx.x < WIDE_BUCKETS) {
-            if (pass == 1)
-                base[threadIdx.x] = cnt[threadIdx.x] ? atomicAdd(&next[threadIdx.x], cnt[threadIdx.x]) : 0u;
-            cnt[threadIdx.x] = 0;
-        }
-        __syncthreads();
-        for (int i = i0 + w; i < i1; i += 4) {
-            const int row = uniform(rows[i]);
-            const WideDir d(op, crp, row);
-            const int U0 = d.mn / WIDE_TILES, U1 = (d.mn + d.S - 1) / WIDE_TILES + 1; // units of the row
-            int u = U0;                   // first unit of the open window
-            unsigned at = 0;              // entries before it
-            auto close = [&](int v, unsigned end) { // window [u, v)
-                if (end > at) {
-                    const int b = (int)((long long)u * WIDE_BUCKETS / U);
-                    if (lane == 0) {
-                        const unsigned p = atomicAdd(&cnt[b], 1u);
-                        if (pass == 1) {
-                            const unsigned q = base[b] + p;
-                            if (q < cap)
-                                items[q] = WideItem{row, (unsigned)u | ((unsigned)(v - u) << 24), at, end - at};
-                            else // cannot happen: wide_row_items bounds them
-                                raise_internal(err);
-                        }
-                    }
-                }
-                u = v;
-                at = end;
-            };
-            // lane q holds the entries before unit vb + q
-            for (int vb = U0 + 1; vb <= U1; vb += 64) {
-                const int v = vb + lane;
-                const unsigned off = v < U1 ? d.before(v * WIDE_TILES - d.mn) : d.n;
-                unsigned prev = at; // entries before unit vb + q - 1
-                if (vb > U0 + 1)
-                    prev = d.before((vb - 1) * WIDE_TILES - d.mn);
-                for (int q = 0; q < 64 && vb + q <= U1; ++q) {
-                    const unsigned o = (unsigned)__builtin_amdgcn_readlane((int)off, q);
-                    const int x = vb + q; // unit x - 1 is the one to take in
-                    if (o - at > WIDE_UNIT || x - u > WIDE_UMAX)
-                        close(x - 1, prev);
-                    prev = o;
+    unsigned *place = places + (size_t)threadIdx.x * gridDim.x + blockIdx.x; // bucket threadIdx.x's
+    if (threadIdx.x < WIDE_BUCKETS)
+        cnt[threadIdx.x] = FILL ? *place : 0u;
+    __syncthreads();
+    for (int i = blockIdx.x * (WI_BS / 64) + w; i < nrows; i += gridDim.x * (WI_BS / 64)) {
+        const int row = uniform(rows[i]);
+        const unsigned n = (unsigned)(uniform64(crp[row + 1]) - uniform64(crp[row]));
+        const WideDir d(op, uniform(op.rmin[row]), uniform(op.rmax[row]), uniform64(op.rdir[row]));
+        const int F = d.entries();
+        const int U0 = d.mn / WIDE_TILES, U1 = (d.mn + d.S - 1) / WIDE_TILES + 1; // units of the row
+        int u = U0;      // first unit of the open window
+        unsigned at = 0; // entries before it
+        auto close = [&](int v, unsigned end) { // window [u, v)
+            if (end > at && lane == 0) {
+                const unsigned q = atomicAdd(&cnt[(int)((long long)u * WIDE_BUCKETS / U)], 1u);
+                if (FILL) {
+                    if (q < cap)
+                        items[q] = WideItem{row, (unsigned)u | ((unsigned)(v - u) << 24), at, end - at};
+                    else // cannot happen: wide_row_items bounds them
+                        raise_internal(err);
                 }
             }
-            close(U1, d.n);
-        }
-        __syncthreads();
-    }
-    if (!FILL && threadIdx.x < WIDE_BUCKETS && cnt[threadIdx.x])
-        atomicAdd(&total[threadIdx.x], cnt[threadIdx.x]);
-}
-
-// one wave: the first window of each bucket; the total
-__global__ void k_wide_order(unsigned *ctr)
-{
-    const int l = threadIdx.x;
-    const unsigned n = l < WIDE_BUCKETS ? ctr[2 + l] : 0u;
-    const unsigned incl = wave_incl_scan(n);
-    if (l < WIDE_BUCKETS)
-        ctr[2 + WIDE_BUCKETS + l] = incl - n;
-    if (l == 63)
-        ctr[0] = incl;
-}
-
-constexpr int WC_BS = 256;     // lanes of a k_wide_cols workgroup
-constexpr int WC_DENSE = 1024; // dense tiles listed per pass (more are written by their lane)
-constexpr int WC_STAGE = 4096; // columns of a flat chunk staged in LDS for coalesced stores
-
-// Columns of the wide rows, from their kept directories (k_numeric_windows writes the
-// values).  One workgroup per row.  Flat directory: WC_BS consecutive tiles' columns are one contiguous
-// range of C, so a scan of the tiles' popcounts places each lane's columns in an LDS stage
-// that the workgroup then stores coalesced.  Chunks of more than WC_STAGE columns, and
-// two-level rows, take the direct path: a lane per tile (flat) or per coarse word,
-// walking its tiles (two-level); a tile with at most 4 columns is written by its lane,
-// denser tiles are listed in LDS and written by a wave each, one lane per column.
-__global__ __launch_bounds__(WC_BS) void k_wide_cols(const int *__restrict__ rows, const int *__restrict__ count_p,
-                                                     Operands op, const long long *__restrict__ crp,
-                                                     int *__restrict__ Ccol)
-{
-    // one buffer, used by one path per chunk: the staged chunk's columns, or the list of
-    // its dense tiles (mask, first slot, absolute tile), so that the waves writing them
-    // read LDS instead of going back to the directory in global memory
-    static_assert(WC_DENSE * (8 + 4 + 4) <= WC_STAGE * 4, "dense-tile list fits the stage");
-    __shared__ __align__(16) unsigned char buf[WC_STAGE * 4];
-    int *stage = (int *)buf;
-    u64 *dmask = (u64 *)buf;
-    unsigned *doff = (unsigned *)(buf + 8 * WC_DENSE);
-    int *dtile = (int *)(buf + 12 * WC_DENSE);
-    __shared__ unsigned red[WC_BS / 64];
-    __shared__ int nd_s;
-    const int l = threadIdx.x, lane = l & 63, w = l >> 6;
-    const int nrows = *count_p;
-    for (int idx = blockIdx.x; idx < nrows; idx += gridDim.x) {
-        const int row = uniform(rows[idx]);
-        const long long cb = uniform64(crp[row]);
-        const long long n = uniform64(crp[row + 1]) - cb;
-        if (n <= 0)
-            continue;
-        const int mn = uniform(op.rmin[row]);
-        const int S = uniform(op.rmax[row]) - mn + 1;
-        const long long r = uniform64(op.rdir[row]);
-        const bool two = (r & RDIR_TWO) != 0;
-        const int W = two ? (S + 63) >> 6 : 0;
-        const long long rd = r & ~RDIR_TWO;
-        const u64 *cmg = op.dir_mask + rd;
-        const unsigned *cog = op.dir_off + rd;
-        const u64 *fm = op.dir_mask + rd + W;
-        const unsigned *foff = op.dir_off + rd + W;
-        auto emit = [&](int k, int tile) {
-            u64 m = fm[k];
-            const unsigned o = foff[k];
-            if (__popcll(m) > 4) {
-                const int p = atomicAdd(&nd_s, 1);
-                if (p < WC_DENSE) {
-                    dmask[p] = m;
-                    doff[p] = o;
-                    dtile[p] = tile;
-                    return;
-                }
-            }
-            long long at = cb + o;
-            while (m) {
-                Ccol[at++] = (tile << 6) + __ffsll((unsigned long long)m) - 1;
-                m &= m - 1;
-            }
+            u = v;
+            at = end;
         };
-        const int U = two ? W : S; // units: coarse words, or tiles
-        // flat rows: each chunk's tile masks and first slot are loaded one chunk ahead, so
-        // the load overlaps the previous chunk's scan and stores
-        u64 m_next = !two && l < S ? fm[l] : 0ull;
-        unsigned base_next = !two && S > 0 ? uniform(foff[0]) : 0u;
-        for (int u0 = 0; u0 < U; u0 += WC_BS) {
-            const int u = u0 + l;
-            if (!two) { // staged: [foff[u0], foff[u0] + tot) holds this chunk's columns
-                const u64 m = m_next;
-                const unsigned base = base_next;
-                m_next = u + WC_BS < S ? fm[u + WC_BS] : 0ull;
-                base_next = u0 + WC_BS < S ? uniform(foff[u0 + WC_BS]) : 0u;
-                unsigned tot;
-                const unsigned pos = group_excl_scan<WC_BS>((unsigned)__popcll(m), red, tot);
-                if (uniform(tot) <= (unsigned)WC_STAGE) {
-                    const int c0 = (mn + u) << 6;
-                    u64 mm = m;
-                    unsigned q = pos;
-                    while (mm) {
-                        stage[q++] = c0 + __ffsll((unsigned long long)mm) - 1;
-                        mm &= mm - 1;
-                    }
-                    __syncthreads();
-                    for (unsigned i = l; i < tot; i += WC_BS)
-                        Ccol[cb + base + i] = stage[i];
-                    __syncthreads(); // the stage of the next chunk
-                    continue;
-                }
+        // lane q holds the entries before unit vb + q
+        unsigned prev = 0; // entries before the unit to take in
+        for (int vb = U0 + 1; vb <= U1; vb += 64) {
+            const int v = vb + lane;
+            const unsigned off = v < U1 ? d.before(v * WIDE_TILES - d.mn, F, n) : n;
+            for (int q = 0; q < 64 && vb + q <= U1; ++q) {
+                const unsigned o = (unsigned)__builtin_amdgcn_readlane((int)off, q);
+                const int x = vb + q; // unit x - 1 is the one to take in
+                if (o - at > WIDE_UNIT || x - u > WIDE_UMAX)
+                    close(x - 1, prev);
+                prev = o;
             }
-            if (l == 0)
-                nd_s = 0;
-            __syncthreads();
-            if (u < U) {
-                if (two) {
-                    u64 cw = cmg[u];
-                    int k = (int)cog[u];
-                    while (cw) {
-                        emit(k++, mn + (u << 6) + __ffsll((unsigned long long)cw) - 1);
-                        cw &= cw - 1;
-                    }
-                } else {
-                    emit(u, mn + u);
-                }
-            }
-            __syncthreads();
-            const int nd = min(uniform(nd_s), WC_DENSE);
-            for (int t = w; t < nd; t += WC_BS / 64) {
-                const u64 m = dmask[t];
-                if ((m >> lane) & 1ull)
-                    Ccol[cb + doff[t] + __popcll(m & below(lane))] = (dtile[t] << 6) + lane;
-            }
-            __syncthreads(); // the list and nd_s of the next pass
         }
+        close(U1, n);
+    }
+    __syncthreads();
+    if (!FILL && threadIdx.x < WIDE_BUCKETS)
+        *place = cnt[threadIdx.x];
+}
+
+// The place of each workgroup's first window in each bucket, from their numbers; the total.
+__global__ __launch_bounds__(1024) void k_wide_order(unsigned *__restrict__ places, int n, unsigned *ctr)
+{
+    __shared__ unsigned red[16];
+    const int per = (n + 1023) / 1024;
+    const int q0 = threadIdx.x * per, q1 = q0 + per < n ? q0 + per : n;
+    unsigned sum = 0;
+    for (int q = q0; q < q1; ++q)
+        sum += places[q];
+    unsigned tot;
+    unsigned at = group_excl_scan<1024>(sum, red, tot);
+    for (int q = q0; q < q1; ++q) {
+        const unsigned k = places[q];
+        places[q] = at;
+        at += k;
+    }
+    if (threadIdx.x == 0) {
+        ctr[0] = tot; // listed
+        ctr[1] = 0;   // taken
     }
 }
 
@@ -1872,14 +1787,20 @@ __global__ __launch_bounds__(WC_BS) void k_wide_cols(const int *__restrict__ row
 // windows from the list until it is used up.  Neither a search nor atomics in C nor a
 // second round: every window's elements are known when it starts, and a window belongs to
 // one workgroup.
-// What bounds it: the chain of a window's phases (item, row, directory; A's entries, index;
-// stream; output), three workgroups per CU.  Against items of up to 512 A entries that kept
-// cursors into the B rows and posted chunks of them window by window (in rounds, with split
-// rows meeting by atomics): R-MAT scale 18 wide rows 22.4 -> 8.9 ms (this kernel 20.5 ->
-// 6.5), a 2,000-row Zipf panel 7.6 -> 4.6 ms.  256 lanes: Zipf 128 / 256 / 512 / 1,024
-// lanes 5.7 / 4.6 / 5.0 / 7.3 ms, R-MAT scale 18 11.2 / 8.9 / 9.0 / 11.9 ms.
+// No single unit bounds it (Zipf panel: vector ALU 41%, LDS 32%, L1 47% of the time): a
+// window's phases follow one another and 48 KB of LDS leave three workgroups per CU, so the
+// next window's item, row and columns of A, and the next 256 entries' ranges, are loaded
+// during the stream.  The columns come from the window's masks, which are in LDS: read from
+// the directories in global memory by a kernel of its own they took 1.55 ms on the R-MAT
+// square of scale 18 and 0.95 ms on
+// the 2,000-row Zipf panel (4.94 -> 4.81 ms for the call).  Against items of up to 512 A
+// entries that kept cursors into the B rows and posted chunks of them window by window (in
+// rounds, with split rows meeting by atomics): scale 18 22.4 -> 8.6 ms, the Zipf panel
+// 7.6 -> 4.5 ms.  Zipf panel with 128 / 256 / 512 lanes 6.3 / 4.8 / 5.0 ms, scale 18
+// 20.8 / 17.4 / 17.5 ms; windows of 2,048 entries and twice the workgroups 6.1 and 18.4 ms.
 constexpr int WW_TILES = WIDE_TILES * WIDE_UMAX;
 constexpr int WW_BS = 256; // lanes of a workgroup
+constexpr int WW_DENSE = 16; // entries per tile from which a wave writes a tile's columns
 template <int BS> constexpr int ww_lds()
 {
     constexpr int words = stream_window(BS) / 64;
@@ -1890,7 +1811,7 @@ template <typename P, int BS>
 __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restrict__ items,
                                                         const unsigned *__restrict__ ctr_listed, unsigned *ctr_taken,
                                                         Operands op, const int *__restrict__ index, long long U,
-                                                        const long long *__restrict__ crp,
+                                                        const long long *__restrict__ crp, int *__restrict__ Ccol,
                                                         typename P::V *__restrict__ Cval)
 {
     typedef typename P::V V;
@@ -1906,23 +1827,36 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
     unsigned short *wo = (unsigned short *)(st.bits + words);
     st.wb = wo + WW_TILES;
     st.red = red;
-    const int l = threadIdx.x;
+    int *stage = (int *)vals; // columns, once the values are out
+    const int l = threadIdx.x, lane = l & 63, w = uniform((int)(threadIdx.x >> 6));
     const V *__restrict__ Aval = (const V *)op.Aval;
     const unsigned nitems = *ctr_listed;
-    if (l == 0)
-        next_s = atomicAdd(ctr_taken, 1u);
-    __syncthreads();
-    unsigned it = uniform(next_s);
+    if (blockIdx.x >= nitems)
+        return;
+    // a window's item, then its row's places, are loaded while the window before it is
+    // worked on: raw loads here, made scalars (which waits for them) where they are used
+    uint4 item = ((const uint4 *)items)[blockIdx.x];
+    int row = uniform((int)item.x);
+    int ra = op.Arp[row], rb = op.Arp[row + 1], rmn = op.rmin[row], rmx = op.rmax[row];
+    long long rcb = crp[row], rrd = op.rdir[row];
+    unsigned it = blockIdx.x;
+    int j = l < rb - ra ? op.Acol[ra + l] : 0; // column of the lane's entry of A
     while (it < nitems) {
-        const int row = uniform(items[it].row);
-        const unsigned units = uniform(items[it].units);
-        const unsigned base = uniform(items[it].base);
-        const int cnt = (int)uniform(items[it].cnt);
+        const unsigned units = uniform(item.y), base = uniform(item.z);
+        const int cnt = (int)uniform(item.w);
         const int u0 = (int)(units & 0xffffffu), u1 = u0 + (int)(units >> 24);
-        const int a0 = uniform(op.Arp[row]), nA = uniform(op.Arp[row + 1]) - a0;
-        const WideDir d(op, crp, row);
-        const long long cb = uniform64(crp[row]) + base;
+        const int a0 = uniform(ra), nA = uniform(rb) - a0;
+        const WideDir d(op, uniform(rmn), uniform(rmx), uniform64(rrd));
+        const long long cb = uniform64(rcb) + base;
         const int T0 = u0 * WIDE_TILES, nt = (u1 - u0) * WIDE_TILES;
+        auto segment = [&](int e, int col) {
+            if (e >= nA)
+                return Segment{0, 0, 0};
+            const int *ix = index + (long long)col * (U + 1);
+            const int s0 = ix[u0];
+            return Segment{s0, ix[u1] - s0, (u64)__double_as_longlong((double)Aval[a0 + e])};
+        };
+        const Segment first = segment(l, j);
         for (int t = l; t < nt; t += BS) {
             unsigned off;
             wm[t] = d.tile(T0 + t - d.mn, off);
@@ -1933,20 +1867,48 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
         for (int q = l; q < words; q += BS)
             st.bits[q] = 0;
         if (l == 0)
-            next_s = atomicAdd(ctr_taken, 1u);
+            next_s = atomicAdd(ctr_taken, 1u) + gridDim.x;
         __syncthreads();
-        auto rows_of = [&](int e) {
-            const int j = op.Acol[a0 + e];
-            const int *ix = index + (long long)j * (U + 1);
-            const int s0 = ix[u0];
-            return Segment{s0, ix[u1] - s0, (u64)__double_as_longlong((double)Aval[a0 + e])};
-        };
-        st.run(nA, rows_of, [&](const Stream<BS> &t, long long w0) {
-            stream_add<BS, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, wm, wo, vals, T0);
-        });
+        it = uniform(next_s);
+        item = ((const uint4 *)items)[it < nitems ? it : nitems - 1];
+        st.run(
+            nA, first, [&](int e) { return e < nA ? op.Acol[a0 + e] : 0; }, segment,
+            [&](const Stream<BS> &t, long long w0) {
+                stream_add<BS, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, wm, wo, vals, T0);
+            });
+        row = uniform((int)item.x);
+        ra = op.Arp[row];
+        rb = op.Arp[row + 1];
+        rmn = op.rmin[row];
+        rmx = op.rmax[row];
+        rcb = crp[row];
+        rrd = op.rdir[row];
         for (int q = l; q < cnt; q += BS)
             Cval[cb + q] = P::result(vals, (unsigned)q);
-        it = uniform(next_s);
+        j = l < rb - ra ? op.Acol[ra + l] : 0;
+        // dense tiles: a wave each, a lane per column; else a lane per tile and LDS, for
+        // stores in order
+        if (cnt >= WW_DENSE * nt) {
+            for (int t = w; t < nt; t += BS / 64) {
+                const u64 m = uniform64(wm[t]);
+                if ((m >> lane) & 1ull)
+                    Ccol[cb + wo[t] + __popcll(m & below(lane))] = ((T0 + t) << 6) + lane;
+            }
+        } else {
+            __syncthreads();
+            for (int t = l; t < nt; t += BS) {
+                u64 m = wm[t];
+                unsigned q = wo[t];
+                const int c = (T0 + t) << 6;
+                while (m) {
+                    stage[q++] = c + __ffsll((unsigned long long)m) - 1;
+                    m &= m - 1;
+                }
+            }
+            __syncthreads();
+            for (int q = l; q < cnt; q += BS)
+                Ccol[cb + q] = stage[q];
+        }
         __syncthreads();
     }
 }
@@ -2113,24 +2075,19 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
     if (bin == BIN_GLOBAL) {
         const int blocks = count < wide.blocks ? count : wide.blocks;
         if (op.dir_mask && wide.items) { // windows
-            hipError_t e = launch_fill_zero(wide.ctr, WIDE_CTRS * sizeof(unsigned), s);
-            if (e != hipSuccess)
-                return e;
             const long long nix = wide.K * (wide.nunits + 1);
             const long long gx = (nix + 255) / 256;
             hipLaunchKernelGGL(k_wide_index, dim3((unsigned)(gx < 65536 ? gx : 65536)), dim3(256), 0, s, wide.K,
                                wide.nunits, op.Brp, op.Bcol, wide.index);
-            const unsigned gi = (unsigned)(count < 4 * num_cus ? (count + 3) / 4 : num_cus);
-            hipLaunchKernelGGL(k_wide_items<false>, dim3(gi), dim3(256), 0, s, rows, count_dev, op, crp, wide.nunits,
-                               wide.items, wide.items_cap, wide.ctr, err);
-            hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(64), 0, s, wide.ctr);
-            hipLaunchKernelGGL(k_wide_items<true>, dim3(gi), dim3(256), 0, s, rows, count_dev, op, crp, wide.nunits,
-                               wide.items, wide.items_cap, wide.ctr, err);
-            hipLaunchKernelGGL(k_wide_cols, dim3((unsigned)(count < 8192 ? count : 8192)), dim3(WC_BS), 0, s, rows,
-                               count_dev, op, crp, Ccol);
+            const unsigned gi = (unsigned)wide_item_blocks(count, num_cus);
+            hipLaunchKernelGGL(k_wide_items<false>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
+                               wide.items, wide.items_cap, wide.places, err);
+            hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(1024), 0, s, wide.places, (int)gi * WIDE_BUCKETS, wide.ctr);
+            hipLaunchKernelGGL(k_wide_items<true>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
+                               wide.items, wide.items_cap, wide.places, err);
             hipLaunchKernelGGL((k_numeric_windows<P, WW_BS>), dim3((unsigned)wide.blocks), dim3(WW_BS),
                                ww_lds<WW_BS>(), s, wide.items, wide.ctr, wide.ctr + 1, op, wide.index, wide.nunits, crp,
-                               (typename P::V *)Cval);
+                               Ccol, (typename P::V *)Cval);
         } else if (op.dir_mask)
             hipLaunchKernelGGL(k_numeric_wcompact<P>, dim3(blocks), dim3(1024), CW_LDS, s, rows, count_dev, op, crp,
                                Ccol, (typename P::V *)Cval, bshift > 6 ? 6 : bshift, wide.ws, wide.cur_stride,
@@ -2174,6 +2131,12 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
                                    long_rows, wide, err, num_cus, queue, lds_bytes, s);
     return numeric_p<PrecF64>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, tshift, two_level,
                               long_rows, wide, err, num_cus, queue, lds_bytes, s);
+}
+
+int wide_item_blocks(int count, int num_cus)
+{
+    const int per = WI_BS / 64, most = 8 * num_cus; // 32 waves per CU
+    return (count + per - 1) / per < most ? (count + per - 1) / per : most;
 }
 
 int wide_window_blocks(int num_cus)

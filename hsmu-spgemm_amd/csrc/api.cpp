@@ -958,13 +958,14 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
                 wide.index = ar.get<int>((size_t)index_n);
                 wide.items_cap = (long long)h2.wide_items;
                 wide.items = ar.get<WideItem>((size_t)wide.items_cap);
-                wide.ctr = ar.get<unsigned>(WIDE_CTRS);
+                wide.places = ar.get<unsigned>((size_t)wide_item_blocks(cnt, c->num_cus) * WIDE_BUCKETS);
+                wide.ctr = ar.get<unsigned>(2);
             } else {
                 wide.cur_stride = ((long long)h2.num.max_na[b] + 63) & ~63LL;
                 wide.ft_stride = keep_dirs ? (((long long)h2.num.max_span[b] + 63) & ~63LL) : 0;
                 wide.ws = ar.get<int>(wide_ws_ints(wide.cur_stride, wide.ft_stride, wide.blocks) + 1);
             }
-            if (windows ? (!wide.index || !wide.items || !wide.ctr) : !wide.ws)
+            if (windows ? (!wide.index || !wide.items || !wide.places || !wide.ctr) : !wide.ws)
                 return fail(HSMU_ERR_NOMEM, "wide-row workspace");
         }
         if (timing)

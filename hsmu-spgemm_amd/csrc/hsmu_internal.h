@@ -400,7 +400,7 @@ constexpr int WIDE_UNIT = 4096;
 constexpr int WIDE_UMAX = 16;
 constexpr int WIDE_TILES = WIDE_UNIT / 64;     // tiles of a unit
 constexpr int WIDE_BUCKETS = 32;               // windows are listed by their place in C's columns
-struct WideItem {
+struct __attribute__((aligned(16))) WideItem {
     int row;
     unsigned units;     // first unit | number of units << 24
     unsigned base, cnt; // the row's entries before the window, and in it
@@ -421,16 +421,18 @@ struct WideRows {
     int *ws;
     long long cur_stride, ft_stride;
     int blocks;
-    // windows: their capacity and list, and counters: windows listed, taken, then per bucket
-    // the windows and the place of the next one (null items: one workgroup per row)
+    // windows: their capacity and list, the place of each listing workgroup's windows per
+    // bucket, and how many are listed and taken (null items: one workgroup per row)
     long long items_cap;
     WideItem *items;
+    unsigned *places;
     unsigned *ctr;
     int *index; // K rows of nunits + 1
     long long nunits;
     long long K;
 };
-constexpr int WIDE_CTRS = 2 + 2 * WIDE_BUCKETS;
+// workgroups that list the windows of count rows
+int wide_item_blocks(int count, int num_cus);
 size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks);
 // workgroups of the windows' kernel that the device holds
 int wide_window_blocks(int num_cus);
