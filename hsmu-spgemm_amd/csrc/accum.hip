@@ -1701,21 +1701,21 @@ struct WideDir {
 };
 
 // The windows of the wide rows, a wave per row: greedy runs of units.  FILL = false counts
-// them per bucket (a bucket is a range of first units) and workgroup, FILL = true writes
-// them, so that the list goes through C's columns in order and the workgroups that run
-// together read the same part of B, which then stays in the L2s (R-MAT scale 18: 1/32 of B
-// is 1.5 MB).  Bound by the chain of loads per row, so the grid fills the device.
+// them per bucket (the heavy ones, then the compact and the dense form's by ranges of first
+// units) and workgroup, FILL = true writes them, so that the list goes through C's columns
+// in order and the workgroups that run together read the same part of B, which then stays in
+// the L2s (R-MAT scale 18: 1/32 of B is 1.5 MB).  Bound by the chain of loads per row, so the grid fills the device.
 template <bool FILL>
 __global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ rows, const int *__restrict__ count_p,
                                                       Operands op, const long long *__restrict__ crp, long long U,
                                                       WideItem *__restrict__ items, long long cap,
                                                       unsigned *__restrict__ places, int *err)
 {
-    __shared__ unsigned cnt[WIDE_BUCKETS];
+    __shared__ unsigned cnt[WIDE_LISTS]; // heavy windows, others, dense ones
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int nrows = *count_p;
     unsigned *place = places + (size_t)threadIdx.x * gridDim.x + blockIdx.x; // bucket threadIdx.x's
-    if (threadIdx.x < WIDE_BUCKETS)
+    if (threadIdx.x < WIDE_LISTS)
         cnt[threadIdx.x] = FILL ? *place : 0u;
     __syncthreads();
     for (int i = blockIdx.x * (WI_BS / 64) + w; i < nrows; i += gridDim.x * (WI_BS / 64)) {
@@ -1723,12 +1723,17 @@ __global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ ro
         const unsigned n = (unsigned)(uniform64(crp[row + 1]) - uniform64(crp[row]));
         const WideDir d(op, uniform(op.rmin[row]), uniform(op.rmax[row]), uniform64(op.rdir[row]));
         const int F = d.entries();
+        const float work = (float)uniform64(op.rprod[row]) / (float)n; // products per entry of C_i
         const int U0 = d.mn / WIDE_TILES, U1 = (d.mn + d.S - 1) / WIDE_TILES + 1; // units of the row
         int u = U0;      // first unit of the open window
         unsigned at = 0; // entries before it
         auto close = [&](int v, unsigned end) { // window [u, v)
             if (end > at && lane == 0) {
-                const unsigned q = atomicAdd(&cnt[(int)((long long)u * WIDE_BUCKETS / U)], 1u);
+                const float p = work * (float)(end - at);
+                const bool dense = v - u == 1 && end - at >= WIDE_DENSE && p < (float)WIDE_DENSE_WORK;
+                const int b = (int)((long long)u * WIDE_BUCKETS / U);
+                const unsigned q =
+                    atomicAdd(&cnt[p > (float)WIDE_HEAVY ? 0 : dense ? WIDE_LISTS - WIDE_BUCKETS + b : 1 + b], 1u);
                 if (FILL) {
                     if (q < cap)
                         items[q] = WideItem{row, (unsigned)u | ((unsigned)(v - u) << 24), at, end - at};
@@ -1755,14 +1760,15 @@ __global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ ro
         close(U1, n);
     }
     __syncthreads();
-    if (!FILL && threadIdx.x < WIDE_BUCKETS)
+    if (!FILL && threadIdx.x < WIDE_LISTS)
         *place = cnt[threadIdx.x];
 }
 
-// The place of each workgroup's first window in each bucket, from their numbers; the total.
-__global__ __launch_bounds__(1024) void k_wide_order(unsigned *__restrict__ places, int n, unsigned *ctr)
+// The place of each workgroup's first window in each bucket, from their numbers; the totals.
+__global__ __launch_bounds__(1024) void k_wide_order(unsigned *__restrict__ places, int groups, WideCount *ctr)
 {
     __shared__ unsigned red[16];
+    const int n = WIDE_LISTS * groups;
     const int per = (n + 1023) / 1024;
     const int q0 = threadIdx.x * per, q1 = q0 + per < n ? q0 + per : n;
     unsigned sum = 0;
@@ -1773,11 +1779,13 @@ __global__ __launch_bounds__(1024) void k_wide_order(unsigned *__restrict__ plac
     for (int q = q0; q < q1; ++q) {
         const unsigned k = places[q];
         places[q] = at;
+        if (q == (WIDE_LISTS - WIDE_BUCKETS) * groups)
+            ctr->dense = tot - at >= WIDE_DENSE_MIN ? at : tot;
         at += k;
     }
     if (threadIdx.x == 0) {
-        ctr[0] = tot; // listed
-        ctr[1] = 0;   // taken
+        ctr->listed = tot;
+        ctr->taken[0] = ctr->taken[1] = 0;
     }
 }
 
@@ -1787,29 +1795,33 @@ __global__ __launch_bounds__(1024) void k_wide_order(unsigned *__restrict__ plac
 // windows from the list until it is used up.  Neither a search nor atomics in C nor a
 // second round: every window's elements are known when it starts, and a window belongs to
 // one workgroup.
-// No single unit bounds it (Zipf panel: vector ALU 41%, LDS 32%, L1 47% of the time): a
-// window's phases follow one another and 48 KB of LDS leave three workgroups per CU, so the
-// next window's item, row and columns of A, and the next 256 entries' ranges, are loaded
-// during the stream.  The columns come from the window's masks, which are in LDS: read from
-// the directories in global memory by a kernel of its own they took 1.55 ms on the R-MAT
-// square of scale 18 and 0.95 ms on
-// the 2,000-row Zipf panel (4.94 -> 4.81 ms for the call).  Against items of up to 512 A
-// entries that kept cursors into the B rows and posted chunks of them window by window (in
-// rounds, with split rows meeting by atomics): scale 18 22.4 -> 8.6 ms, the Zipf panel
-// 7.6 -> 4.5 ms.  Zipf panel with 128 / 256 / 512 lanes 6.3 / 4.8 / 5.0 ms, scale 18
-// 20.8 / 17.4 / 17.5 ms; windows of 2,048 entries and twice the workgroups 6.1 and 18.4 ms.
+// DENSE: a slot per column of the unit, with no masks in LDS: the element's column is its
+// slot, and a tile goes out as one store of columns and one of values by a wave.
+// No single unit bounds the compact form (Zipf panel: vector ALU 41%, LDS 32%, L1 47% of the
+// time): a window's phases follow one another and 48 KB of LDS leave three workgroups per
+// CU, so the next window's item, row and columns of A, and the next 256 entries' ranges, are
+// loaded during the stream.  The dense form takes about a third fewer instructions and leaves
+// room for four: Zipf panels of 2,000 rows 4.80 -> 4.25 ms, of 777 rows FP32 1.85 -> 1.55 ms
+// (the calls; about 2.9 TB/s of C).
+// The columns come from the window's masks: read from the directories in global memory by
+// a kernel of its own they took 1.55 ms on the R-MAT square of scale 18.  Against items of up
+// to 512 A entries that kept cursors into the B rows and posted chunks of them window by
+// window (in rounds, with split rows meeting by atomics): scale 18 22.4 -> 8.6 ms, the Zipf
+// panel 7.6 -> 3.9 ms.  Compact form with 128 / 256 / 512 lanes: Zipf 6.3 / 4.8 / 5.0 ms,
+// scale 18 20.8 / 17.4 / 17.5 ms; windows of 2,048 entries and twice the workgroups 6.1 and
+// 18.4 ms.  Dense form with 512 lanes: Zipf 4.6 ms.
 constexpr int WW_TILES = WIDE_TILES * WIDE_UMAX;
 constexpr int WW_BS = 256; // lanes of a workgroup
-constexpr int WW_DENSE = 16; // entries per tile from which a wave writes a tile's columns
-template <int BS> constexpr int ww_lds()
+constexpr int WW_PER_TILE = 16; // entries per tile from which a wave writes a tile's columns
+template <int BS, bool DENSE> constexpr int ww_lds()
 {
     constexpr int words = stream_window(BS) / 64;
-    return WIDE_UNIT * 8 + WW_TILES * 8 + BS * 16 + words * 8 + WW_TILES * 2 + words * 2;
+    return WIDE_UNIT * 8 + BS * 16 + words * 10 + (DENSE ? 0 : WW_TILES * 10);
 }
 
-template <typename P, int BS>
+template <typename P, int BS, bool DENSE>
 __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restrict__ items,
-                                                        const unsigned *__restrict__ ctr_listed, unsigned *ctr_taken,
+                                                        const WideCount *__restrict__ listed, unsigned *taken,
                                                         Operands op, const int *__restrict__ index, long long U,
                                                         const long long *__restrict__ crp, int *__restrict__ Ccol,
                                                         typename P::V *__restrict__ Cval)
@@ -1818,33 +1830,33 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ u64 red[16];
     __shared__ unsigned next_s;
-    constexpr int words = stream_window(BS) / 64;
+    constexpr int NW = BS / 64, words = stream_window(BS) / 64;
     double *vals = (double *)lds;
-    u64 *wm = (u64 *)(vals + WIDE_UNIT);
     Stream<BS> st;
-    st.rec = (uint4 *)(wm + WW_TILES);
+    st.rec = (uint4 *)(vals + WIDE_UNIT);
     st.bits = (u64 *)(st.rec + BS);
-    unsigned short *wo = (unsigned short *)(st.bits + words);
-    st.wb = wo + WW_TILES;
+    u64 *wm = st.bits + words;
+    unsigned short *wo = (unsigned short *)(wm + (DENSE ? 0 : WW_TILES));
+    st.wb = wo + (DENSE ? 0 : WW_TILES);
     st.red = red;
     int *stage = (int *)vals; // columns, once the values are out
     const int l = threadIdx.x, lane = l & 63, w = uniform((int)(threadIdx.x >> 6));
     const V *__restrict__ Aval = (const V *)op.Aval;
-    const unsigned nitems = *ctr_listed;
-    if (blockIdx.x >= nitems)
+    const unsigned i0 = DENSE ? listed->dense : 0u, i1 = DENSE ? listed->listed : listed->dense;
+    unsigned it = i0 + blockIdx.x;
+    if (it >= i1)
         return;
     // a window's item, then its row's places, are loaded while the window before it is
     // worked on: raw loads here, made scalars (which waits for them) where they are used
-    uint4 item = ((const uint4 *)items)[blockIdx.x];
+    uint4 item = ((const uint4 *)items)[it];
     int row = uniform((int)item.x);
     int ra = op.Arp[row], rb = op.Arp[row + 1], rmn = op.rmin[row], rmx = op.rmax[row];
     long long rcb = crp[row], rrd = op.rdir[row];
-    unsigned it = blockIdx.x;
     int j = l < rb - ra ? op.Acol[ra + l] : 0; // column of the lane's entry of A
-    while (it < nitems) {
+    while (it < i1) {
         const unsigned units = uniform(item.y), base = uniform(item.z);
         const int cnt = (int)uniform(item.w);
-        const int u0 = (int)(units & 0xffffffu), u1 = u0 + (int)(units >> 24);
+        const int u0 = (int)(units & 0xffffffu), u1 = DENSE ? u0 + 1 : u0 + (int)(units >> 24);
         const int a0 = uniform(ra), nA = uniform(rb) - a0;
         const WideDir d(op, uniform(rmn), uniform(rmx), uniform64(rrd));
         const long long cb = uniform64(rcb) + base;
@@ -1857,24 +1869,33 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
             return Segment{s0, ix[u1] - s0, (u64)__double_as_longlong((double)Aval[a0 + e])};
         };
         const Segment first = segment(l, j);
-        for (int t = l; t < nt; t += BS) {
-            unsigned off;
-            wm[t] = d.tile(T0 + t - d.mn, off);
-            wo[t] = (unsigned short)(off - base);
+        // dense: lane i of wave w holds tile w * TW + i
+        constexpr int TW = WIDE_TILES / NW;
+        u64 tm = 0;
+        unsigned to = 0;
+        if constexpr (DENSE) {
+            tm = d.tile(T0 + w * TW + (lane < TW ? lane : TW - 1) - d.mn, to);
+        } else {
+            for (int t = l; t < nt; t += BS) {
+                unsigned off;
+                wm[t] = d.tile(T0 + t - d.mn, off);
+                wo[t] = (unsigned short)(off - base);
+            }
         }
-        for (int q = 2 * l; q < cnt; q += 2 * BS) // (WIDE_UNIT is even)
+        const int nv = DENSE ? WIDE_UNIT : cnt;
+        for (int q = 2 * l; q < nv; q += 2 * BS) // (WIDE_UNIT is even)
             *(double2 *)(vals + q) = make_double2(0.0, 0.0);
         for (int q = l; q < words; q += BS)
             st.bits[q] = 0;
         if (l == 0)
-            next_s = atomicAdd(ctr_taken, 1u) + gridDim.x;
+            next_s = i0 + gridDim.x + atomicAdd(taken, 1u);
         __syncthreads();
         it = uniform(next_s);
-        item = ((const uint4 *)items)[it < nitems ? it : nitems - 1];
+        item = ((const uint4 *)items)[it < i1 ? it : i1 - 1];
         st.run(
             nA, first, [&](int e) { return e < nA ? op.Acol[a0 + e] : 0; }, segment,
             [&](const Stream<BS> &t, long long w0) {
-                stream_add<BS, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, wm, wo, vals, T0);
+                stream_add<BS, DENSE ? SLOT_DENSE : SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, wm, wo, vals, T0);
             });
         row = uniform((int)item.x);
         ra = op.Arp[row];
@@ -1883,35 +1904,55 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
         rmx = op.rmax[row];
         rcb = crp[row];
         rrd = op.rdir[row];
-        for (int q = l; q < cnt; q += BS)
-            Cval[cb + q] = P::result(vals, (unsigned)q);
-        j = l < rb - ra ? op.Acol[ra + l] : 0;
-        // dense tiles: a wave each, a lane per column; else a lane per tile and LDS, for
-        // stores in order
-        if (cnt >= WW_DENSE * nt) {
-            for (int t = w; t < nt; t += BS / 64) {
-                const u64 m = uniform64(wm[t]);
-                if ((m >> lane) & 1ull)
-                    Ccol[cb + wo[t] + __popcll(m & below(lane))] = ((T0 + t) << 6) + lane;
-            }
-        } else {
-            __syncthreads();
-            for (int t = l; t < nt; t += BS) {
-                u64 m = wm[t];
-                unsigned q = wo[t];
-                const int c = (T0 + t) << 6;
-                while (m) {
-                    stage[q++] = c + __ffsll((unsigned long long)m) - 1;
-                    m &= m - 1;
+        int *cc = Ccol + cb;
+        V *cv = Cval + cb;
+        if constexpr (DENSE) { // a tile per step of a wave, a lane per column
+#pragma unroll 4
+            for (int i = 0; i < TW; ++i) {
+                const u64 m = readlane_u64(tm, i);
+                const unsigned q = (unsigned)__builtin_amdgcn_readlane((int)to, i) - base + (unsigned)mbcnt(m);
+                const unsigned c = (unsigned)(w * TW + i) * 64 + lane;
+                const V v = P::result(vals, c);
+                if ((m >> lane) & 1ull) {
+                    cc[q] = (T0 << 6) + (int)c;
+                    cv[q] = v;
                 }
             }
-            __syncthreads();
+            j = l < rb - ra ? op.Acol[ra + l] : 0;
+        } else {
             for (int q = l; q < cnt; q += BS)
-                Ccol[cb + q] = stage[q];
+                cv[q] = P::result(vals, (unsigned)q);
+            j = l < rb - ra ? op.Acol[ra + l] : 0;
+            // many entries per tile: a wave each, a lane per column; else a lane per tile and
+            // LDS, for stores in order
+            if (cnt >= WW_PER_TILE * nt) {
+                for (int t = w; t < nt; t += NW) {
+                    const u64 m = uniform64(wm[t]);
+                    if ((m >> lane) & 1ull)
+                        cc[wo[t] + (unsigned)mbcnt(m)] = ((T0 + t) << 6) + lane;
+                }
+            } else {
+                __syncthreads();
+                for (int t = l; t < nt; t += BS) {
+                    u64 m = wm[t];
+                    unsigned q = wo[t];
+                    const int c = (T0 + t) << 6;
+                    while (m) {
+                        stage[q++] = c + __ffsll((unsigned long long)m) - 1;
+                        m &= m - 1;
+                    }
+                }
+                __syncthreads();
+                for (int q = l; q < cnt; q += BS)
+                    cc[q] = stage[q];
+            }
         }
         __syncthreads();
     }
 }
+
+// workgroups of a windows' kernel that a CU holds
+static int ww_per_cu(int lds) { return 160 * 1024 / (lds + LDS_STATIC_RESERVE); }
 
 // ---- launchers -------------------------------------------------------------------------------
 
@@ -2082,12 +2123,17 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
             const unsigned gi = (unsigned)wide_item_blocks(count, num_cus);
             hipLaunchKernelGGL(k_wide_items<false>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
                                wide.items, wide.items_cap, wide.places, err);
-            hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(1024), 0, s, wide.places, (int)gi * WIDE_BUCKETS, wide.ctr);
+            hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(1024), 0, s, wide.places, (int)gi, wide.ctr);
             hipLaunchKernelGGL(k_wide_items<true>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
                                wide.items, wide.items_cap, wide.places, err);
-            hipLaunchKernelGGL((k_numeric_windows<P, WW_BS>), dim3((unsigned)wide.blocks), dim3(WW_BS),
-                               ww_lds<WW_BS>(), s, wide.items, wide.ctr, wide.ctr + 1, op, wide.index, wide.nunits, crp,
-                               Ccol, (typename P::V *)Cval);
+            hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, true>),
+                               dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, true>()))), dim3(WW_BS),
+                               (ww_lds<WW_BS, true>()), s, wide.items, wide.ctr, wide.ctr->taken, op, wide.index,
+                               wide.nunits, crp, Ccol, (typename P::V *)Cval);
+            hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, false>),
+                               dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, false>()))), dim3(WW_BS),
+                               (ww_lds<WW_BS, false>()), s, wide.items, wide.ctr, wide.ctr->taken + 1, op, wide.index,
+                               wide.nunits, crp, Ccol, (typename P::V *)Cval);
         } else if (op.dir_mask)
             hipLaunchKernelGGL(k_numeric_wcompact<P>, dim3(blocks), dim3(1024), CW_LDS, s, rows, count_dev, op, crp,
                                Ccol, (typename P::V *)Cval, bshift > 6 ? 6 : bshift, wide.ws, wide.cur_stride,
@@ -2139,11 +2185,6 @@ int wide_item_blocks(int count, int num_cus)
     return (count + per - 1) / per < most ? (count + per - 1) / per : most;
 }
 
-int wide_window_blocks(int num_cus)
-{
-    return num_cus * (160 * 1024 / (ww_lds<WW_BS>() + LDS_STATIC_RESERVE));
-}
-
 size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks)
 {
     return (size_t)blocks * (size_t)(3 * cur_stride + ft_stride);
@@ -2179,7 +2220,9 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
     CFG(k_symbolic_wide)
     CFG(k_numeric_window<PrecF64>) CFG(k_numeric_window<PrecF32C>)
     CFG(k_numeric_wcompact<PrecF64>) CFG(k_numeric_wcompact<PrecF32C>) 
-#define CFGW(P) CFG((k_numeric_windows<P, WW_BS>))
+#define CFGW(P)                                                                                                        \
+    CFG((k_numeric_windows<P, WW_BS, false>))                                                                          \
+    CFG((k_numeric_windows<P, WW_BS, true>))
     CFGW(PrecF64) CFGW(PrecF32C)
 #undef CFGW
 #undef CFG

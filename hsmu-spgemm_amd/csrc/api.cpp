@@ -951,15 +951,15 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
                 index_max = ar.remaining() / 2;
             const bool windows = keep_dirs && (unsigned long long)index_n * sizeof(int) <= index_max &&
                                  units < (1 << 24) && h2.wide_items < (1ull << 31);
-            wide.blocks = windows ? wide_window_blocks(c->num_cus) : (cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt);
+            wide.blocks = cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt;
             if (windows) {
                 wide.nunits = units;
                 wide.K = K;
                 wide.index = ar.get<int>((size_t)index_n);
                 wide.items_cap = (long long)h2.wide_items;
                 wide.items = ar.get<WideItem>((size_t)wide.items_cap);
-                wide.places = ar.get<unsigned>((size_t)wide_item_blocks(cnt, c->num_cus) * WIDE_BUCKETS);
-                wide.ctr = ar.get<unsigned>(2);
+                wide.places = ar.get<unsigned>((size_t)wide_item_blocks(cnt, c->num_cus) * WIDE_LISTS);
+                wide.ctr = ar.get<WideCount>(1);
             } else {
                 wide.cur_stride = ((long long)h2.num.max_na[b] + 63) & ~63LL;
                 wide.ft_stride = keep_dirs ? (((long long)h2.num.max_span[b] + 63) & ~63LL) : 0;

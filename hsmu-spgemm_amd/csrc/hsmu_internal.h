@@ -400,10 +400,29 @@ constexpr int WIDE_UNIT = 4096;
 constexpr int WIDE_UMAX = 16;
 constexpr int WIDE_TILES = WIDE_UNIT / 64;     // tiles of a unit
 constexpr int WIDE_BUCKETS = 32;               // windows are listed by their place in C's columns
+constexpr int WIDE_LISTS = 1 + 2 * WIDE_BUCKETS;
+// Windows with a slot per column: of one unit, with at least WIDE_DENSE entries and fewer than
+// WIDE_DENSE_WORK products (by the mean of their row), if there are WIDE_DENSE_MIN of them (a
+// kernel of a few windows per workgroup is mostly its start and end).  They need neither
+// masks nor slots per tile: a Zipf panel, whose windows hold 1.1 products per entry, takes
+// 4.25 ms against 4.80.  Windows with more products are the hot columns of skewed graphs,
+// where a slot per column puts more adds on one LDS bank: R-MAT squares of scale 16 and 18
+// take 2.62 and 17.7 ms with them against 2.53 and 17.45.
+// Windows of more than WIDE_HEAVY products are listed first, so that none of them is the last
+// one running.
+constexpr int WIDE_DENSE = WIDE_UNIT / 4;
+constexpr int WIDE_DENSE_WORK = 3 * WIDE_UNIT;
+constexpr unsigned WIDE_DENSE_MIN = 8192;
+constexpr int WIDE_HEAVY = 16 * WIDE_UNIT;
 struct __attribute__((aligned(16))) WideItem {
     int row;
     unsigned units;     // first unit | number of units << 24
     unsigned base, cnt; // the row's entries before the window, and in it
+};
+// The list: windows with compact slots, from `dense` on those with a slot per column, its
+// end; how many of each form are taken.
+struct WideCount {
+    unsigned dense, listed, taken[2];
 };
 HSMU_HD inline long long wide_units(long long N) { return (N + WIDE_UNIT - 1) / WIDE_UNIT; }
 // windows of a row of n entries over S tiles, at most: two neighbouring ones hold more than
@@ -426,7 +445,7 @@ struct WideRows {
     long long items_cap;
     WideItem *items;
     unsigned *places;
-    unsigned *ctr;
+    WideCount *ctr;
     int *index; // K rows of nunits + 1
     long long nunits;
     long long K;
@@ -434,8 +453,6 @@ struct WideRows {
 // workgroups that list the windows of count rows
 int wide_item_blocks(int count, int num_cus);
 size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks);
-// workgroups of the windows' kernel that the device holds
-int wide_window_blocks(int num_cus);
 
 // Numeric phase of one bin.  fp32c = 0: FP64 values (Cval double); fp32c = 1: compensated
 // FP32 (Cval float).  lds_bytes (may be null): += the dynamic LDS of an LDS-bin launch,

@@ -50,3 +50,22 @@ def test_windows(ctx, case, opts, fp32):
     assert np.all(np.abs(C.val.astype(np.float64) - ref.val) <= bound)
     if "force_global" in opts:
         assert st["num_bin_rows"][8] == st["rows_nonempty"]
+
+
+@pytest.mark.parametrize("N", [4093, 2 * 4096])  # a unit that ends within a tile; two per row
+@pytest.mark.parametrize("fp32", [False, True])
+def test_dense_windows(ctx, N, fp32):
+    """Enough one-unit windows of at least 1,024 entries for the form with a slot per column,
+    with some of fewer entries and of many products among them."""
+    rng = np.random.default_rng(5)
+    print(f"[gpu-case] dense windows N {N} fp32 {fp32}", flush=True)
+    part = 1100 if N < 4096 else 5000
+    B = csr([rng.choice(N, part, replace=False) for _ in range(20)] + [np.arange(N), [0], [N - 1], [], np.arange(0, N, 5)],
+            N, rng)
+    light = [[i % 20, 21 + i % 3] for i in range(8500)]
+    A = csr(light + [[20], [24], [21, 22], [20] * 300, list(range(25)) * 30] + light[:300], 25, rng)
+    C, _ = ctx.spgemm(A, B, force_global=1, precision=hsmu.HSMU_FP32_COMP if fp32 else hsmu.HSMU_FP64)
+    ref = oracle.spgemm(A, B)
+    assert np.array_equal(np.asarray(C.rowptr, np.int64), ref.rowptr) and np.array_equal(C.col, ref.col)
+    bound = 2.0 ** -23 * np.abs(ref.val) + 1e-10 * ref.absval if fp32 else 1e-12 * ref.absval
+    assert np.all(np.abs(C.val.astype(np.float64) - ref.val) <= bound)
