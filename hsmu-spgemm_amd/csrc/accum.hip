@@ -1639,7 +1639,7 @@ __global__ __launch_bounds__(256) void k_wide_index(long long K, long long U, co
     }
 }
 
-constexpr int WI_BS = 256; // lanes of a k_wide_items workgroup
+constexpr int WI_BS = 1024; // lanes of a k_wide_items workgroup
 
 // A wide row's directory in global memory, flat or two-level.
 struct WideDir {
@@ -1725,39 +1725,56 @@ __global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ ro
         const int F = d.entries();
         const float work = (float)uniform64(op.rprod[row]) / (float)n; // products per entry of C_i
         const int U0 = d.mn / WIDE_TILES, U1 = (d.mn + d.S - 1) / WIDE_TILES + 1; // units of the row
-        int u = U0;      // first unit of the open window
-        unsigned at = 0; // entries before it
-        auto close = [&](int v, unsigned end) { // window [u, v)
-            if (end > at && lane == 0) {
-                const float p = work * (float)(end - at);
-                const bool dense = v - u == 1 && end - at >= WIDE_DENSE && p < (float)WIDE_DENSE_WORK;
-                const int b = (int)((long long)u * WIDE_BUCKETS / U);
+        int wu = 0, wv = 0; // lane i holds the i-th window found: its units [wu, wv) and
+        unsigned wa = 0, we = 0; // the entries before its start and end
+        int nw = 0;
+        auto list = [&]() { // those found, a lane each
+            if (lane < nw && we > wa) {
+                const float p = work * (float)(we - wa);
+                const bool dense = wv - wu == 1 && we - wa >= WIDE_DENSE && p < (float)WIDE_DENSE_WORK;
+                const int b = (int)((long long)wu * WIDE_BUCKETS / U);
                 const unsigned q =
                     atomicAdd(&cnt[p > (float)WIDE_HEAVY ? 0 : dense ? WIDE_LISTS - WIDE_BUCKETS + b : 1 + b], 1u);
                 if (FILL) {
                     if (q < cap)
-                        items[q] = WideItem{row, (unsigned)u | ((unsigned)(v - u) << 24), at, end - at};
+                        items[q] = WideItem{row, (unsigned)wu | ((unsigned)(wv - wu) << 24), wa, we - wa};
                     else // cannot happen: wide_row_items bounds them
                         raise_internal(err);
                 }
             }
+            nw = 0;
+        };
+        int u = U0;      // first unit of the open window
+        unsigned at = 0; // entries before it
+        auto close = [&](int v, unsigned end) { // window [u, v)
+            if (lane == nw) {
+                wu = u;
+                wv = v;
+                wa = at;
+                we = end;
+            }
             u = v;
             at = end;
+            if (++nw == 64)
+                list();
         };
-        // lane q holds the entries before unit vb + q
-        unsigned prev = 0; // entries before the unit to take in
+        unsigned prev = 0; // entries before unit vb - 1
         for (int vb = U0 + 1; vb <= U1; vb += 64) {
-            const int v = vb + lane;
+            const int v = vb + lane; // this lane's unit, and the entries before it
             const unsigned off = v < U1 ? d.before(v * WIDE_TILES - d.mn, F, n) : n;
-            for (int q = 0; q < 64 && vb + q <= U1; ++q) {
-                const unsigned o = (unsigned)__builtin_amdgcn_readlane((int)off, q);
-                const int x = vb + q; // unit x - 1 is the one to take in
-                if (o - at > WIDE_UNIT || x - u > WIDE_UMAX)
-                    close(x - 1, prev);
-                prev = o;
+            // the first unit that the open window cannot reach; a window has a unit at least
+            // (which holds at most WIDE_UNIT entries), so u grows each time
+            while (true) {
+                const u64 m = __ballot(v > u + 1 && v <= U1 && (off - at > WIDE_UNIT || v - u > WIDE_UMAX));
+                if (!m)
+                    break;
+                const int q = __ffsll((unsigned long long)m) - 1;
+                close(vb + q - 1, q > 0 ? (unsigned)__builtin_amdgcn_readlane((int)off, q - 1) : prev);
             }
+            prev = (unsigned)__builtin_amdgcn_readlane((int)off, 63);
         }
         close(U1, n);
+        list();
     }
     __syncthreads();
     if (!FILL && threadIdx.x < WIDE_LISTS)
@@ -1765,26 +1782,34 @@ __global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ ro
 }
 
 // The place of each workgroup's first window in each bucket, from their numbers; the totals.
+// One workgroup, in passes of 4,096 numbers.
 __global__ __launch_bounds__(1024) void k_wide_order(unsigned *__restrict__ places, int groups, WideCount *ctr)
 {
-    __shared__ unsigned red[16];
-    const int n = WIDE_LISTS * groups;
-    const int per = (n + 1023) / 1024;
-    const int q0 = threadIdx.x * per, q1 = q0 + per < n ? q0 + per : n;
-    unsigned sum = 0;
-    for (int q = q0; q < q1; ++q)
-        sum += places[q];
-    unsigned tot;
-    unsigned at = group_excl_scan<1024>(sum, red, tot);
-    for (int q = q0; q < q1; ++q) {
-        const unsigned k = places[q];
-        places[q] = at;
-        if (q == (WIDE_LISTS - WIDE_BUCKETS) * groups)
-            ctr->dense = tot - at >= WIDE_DENSE_MIN ? at : tot;
-        at += k;
+    __shared__ unsigned red[16], dense_s;
+    const int n = WIDE_LISTS * groups, dense = (WIDE_LISTS - WIDE_BUCKETS) * groups;
+    unsigned done = 0;
+    for (int q0 = 0; q0 < n; q0 += 4096) {
+        const int q = q0 + 4 * (int)threadIdx.x;
+        unsigned k[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            k[i] = q + i < n ? places[q + i] : 0u;
+        unsigned tot;
+        unsigned at = done + group_excl_scan<1024>(k[0] + k[1] + k[2] + k[3], red, tot);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (q + i < n)
+                places[q + i] = at;
+            if (q + i == dense)
+                dense_s = at;
+            at += k[i];
+        }
+        done += tot;
+        __syncthreads();
     }
     if (threadIdx.x == 0) {
-        ctr->listed = tot;
+        ctr->dense = done - dense_s >= WIDE_DENSE_MIN ? dense_s : done;
+        ctr->listed = done;
         ctr->taken[0] = ctr->taken[1] = 0;
     }
 }
@@ -2181,8 +2206,8 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
 
 int wide_item_blocks(int count, int num_cus)
 {
-    const int per = WI_BS / 64, most = 8 * num_cus; // 32 waves per CU
-    return (count + per - 1) / per < most ? (count + per - 1) / per : most;
+    const int per = WI_BS / 64, most = 2 * num_cus; // 32 waves per CU
+    return (count - 1) / per + 1 < most ? (count - 1) / per + 1 : most;
 }
 
 size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks)

@@ -899,6 +899,25 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         outs.p.push_back(Crp);
     }
     bp.per_lane = opts.products_per_lane > 0 ? opts.products_per_lane : 32;
+    // The column index of B that cuts wide rows into windows, and whether it and `list` bytes
+    // of the windows' lists can be had.
+    const long long units = wide_units(N);
+    const unsigned long long index_bytes = (unsigned long long)K * (units + 1) * sizeof(int);
+    auto windows_fit = [&](unsigned long long list) {
+        const unsigned long long left = ar.remaining(); // allocation-free: of the workspace
+        unsigned long long most =
+            opts.wide_scratch_mb > 0 ? (unsigned long long)opts.wide_scratch_mb << 20 : c->total_mem / 4;
+        if (most > left / 2)
+            most = left / 2;
+        return keep_dirs && index_bytes <= most && list <= left - index_bytes && units < (1 << 24);
+    };
+    // rows of more than WINDOW_ROW_MIN are wide where windows are certain: with room for the
+    // lists of M full rows
+    const int n_most = (int)(N < INT_MAX ? N : INT_MAX);
+    if (bp.lds_row_max > WINDOW_ROW_MIN &&
+        windows_fit((unsigned long long)M * wide_row_items(n_most, n_most / 64 + 1) * sizeof(WideItem) +
+                    wide_list_bytes(c->num_cus)))
+        bp.lds_row_max = WINDOW_ROW_MIN;
     HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp, rp64 || batch ? nullptr : (int *)Crp, bp,
                               binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, sums, &dw->done[1], host, s));
     HIP_TRY(mark(c->ev[EV_SYMBOLIC]));
@@ -943,19 +962,13 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         // tiles of a two-level directory and the cursors of its row's A entries
         WideRows wide = {};
         if (b == BIN_GLOBAL) {
-            const long long units = wide_units(N);
-            const long long index_n = K * (units + 1);
-            unsigned long long index_max =
-                opts.wide_scratch_mb > 0 ? (unsigned long long)opts.wide_scratch_mb << 20 : c->total_mem / 4;
-            if (index_max > ar.remaining() / 2) // allocation-free: what the workspace has left
-                index_max = ar.remaining() / 2;
-            const bool windows = keep_dirs && (unsigned long long)index_n * sizeof(int) <= index_max &&
-                                 units < (1 << 24) && h2.wide_items < (1ull << 31);
+            const bool windows = h2.wide_items < (1ull << 31) &&
+                                 windows_fit(h2.wide_items * sizeof(WideItem) + wide_list_bytes(c->num_cus));
             wide.blocks = cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt;
             if (windows) {
                 wide.nunits = units;
                 wide.K = K;
-                wide.index = ar.get<int>((size_t)index_n);
+                wide.index = (int *)ar.raw((size_t)index_bytes);
                 wide.items_cap = (long long)h2.wide_items;
                 wide.items = ar.get<WideItem>((size_t)wide.items_cap);
                 wide.places = ar.get<unsigned>((size_t)wide_item_blocks(cnt, c->num_cus) * WIDE_LISTS);

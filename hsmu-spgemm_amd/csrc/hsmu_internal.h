@@ -397,6 +397,10 @@ hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int c
 // every B row's first element at each unit's start, so a window's elements are known without
 // a search.
 constexpr int WIDE_UNIT = 4096;
+// Rows of more LDS than this are wide where windows can be had: with one or two workgroups
+// per CU they are slower in one piece.  R-MAT squares of scale 16 (FP32) / 18 with rows of up
+// to 160 KB in LDS 2.35 / 17.1 ms, 80 KB 2.34 / 16.9, 64 KB 2.11 / 16.5, 48 KB 2.11 / 16.7.
+constexpr int WINDOW_ROW_MIN = 64 * 1024;
 constexpr int WIDE_UMAX = 16;
 constexpr int WIDE_TILES = WIDE_UNIT / 64;     // tiles of a unit
 constexpr int WIDE_BUCKETS = 32;               // windows are listed by their place in C's columns
@@ -452,6 +456,11 @@ struct WideRows {
 };
 // workgroups that list the windows of count rows
 int wide_item_blocks(int count, int num_cus);
+// bytes of the lists besides the windows, at most (with what alignment adds)
+inline unsigned long long wide_list_bytes(int num_cus)
+{
+    return 4ull * WIDE_LISTS * wide_item_blocks(INT_MAX, num_cus) + 2048;
+}
 size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks);
 
 // Numeric phase of one bin.  fp32c = 0: FP64 values (Cval double); fp32c = 1: compensated

@@ -110,7 +110,8 @@ typedef struct hsmu_opts {
     int32_t force_global;     /* 1: every nonempty row takes the global-memory accumulator
                                  (exercises the fallback on small inputs) */
     int32_t lds_row_max;      /* bytes of LDS one row may use before it falls back to the
-                                 global-memory path; 0 = device maximum */
+                                 global-memory path; 0 = device maximum (in the numeric phase
+                                 64 KiB where wide rows can be cut into windows) */
     int32_t lds_block_budget; /* LDS bytes per workgroup for bins that pack several rows
                                  into one workgroup (one wave); 0 = default (8 KiB) */
     int32_t products_per_lane;/* numeric work per lane that sets a row's lane count; 0 = 32 */

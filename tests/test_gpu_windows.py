@@ -69,3 +69,19 @@ def test_dense_windows(ctx, N, fp32):
     assert np.array_equal(np.asarray(C.rowptr, np.int64), ref.rowptr) and np.array_equal(C.col, ref.col)
     bound = 2.0 ** -23 * np.abs(ref.val) + 1e-10 * ref.absval if fp32 else 1e-12 * ref.absval
     assert np.all(np.abs(C.val.astype(np.float64) - ref.val) <= bound)
+
+
+@pytest.mark.parametrize("opts", [dict(), dict(rebuild_dirs=1), dict(wide_scratch_mb=1)])
+def test_rows_of_64_kib(ctx, opts):
+    """Rows around the LDS need from which they are cut into windows, with windows, without
+    kept directories, and without room for the index (200 rows of B of 1,500 units)."""
+    rng = np.random.default_rng(9)
+    N = 4096 * 1500 if "wide_scratch_mb" in opts else 40000
+    print(f"[gpu-case] rows of 64 KiB {opts}", flush=True)
+    B = csr([rng.choice(40000, 100, replace=False) for _ in range(200)], N, rng)
+    A = csr([rng.choice(200, n, replace=False) for n in (70, 78, 80, 82, 84, 90, 100, 150, 200)], 200, rng)
+    C, st = ctx.spgemm(A, B, **opts)
+    ref = oracle.spgemm(A, B)
+    assert np.array_equal(np.asarray(C.rowptr, np.int64), ref.rowptr) and np.array_equal(C.col, ref.col)
+    assert np.all(np.abs(C.val - ref.val) <= 1e-12 * ref.absval)
+    assert (st["num_bin_rows"][8] > 0) == (not opts)
