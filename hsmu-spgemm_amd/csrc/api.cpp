@@ -1219,10 +1219,11 @@ int stack_inputs(hsmu_ctx *c, const BatchPrep &bp, const hsmu_opts &opts, Arena 
     off.eb = offs + 3 * n1;
     const int v32 = fp32 ? 1 : 0;
     HIP_TRY(launch_batch_rowptr(1, bp.count, inst, off, bp.K, bp.nnzB, Brp, dst, s));
-    HIP_TRY(launch_batch_entries(1, bp.count, inst, off, bp.nnzB, v32, Bcol, Bval, dst, s));
-    if (!bp.self)
+    HIP_TRY(launch_batch_entries(1, bp.count, inst, off, bp.nnzB, v32, bp.self ? Acol : nullptr, Bcol, Bval, dst, s));
+    if (!bp.self) {
         HIP_TRY(launch_batch_rowptr(0, bp.count, inst, off, bp.M, bp.nnzA, Arp, dst, s));
-    HIP_TRY(launch_batch_entries(0, bp.count, inst, off, bp.nnzA, v32, Acol, bp.self ? nullptr : Aval, dst, s));
+        HIP_TRY(launch_batch_entries(0, bp.count, inst, off, bp.nnzA, v32, Acol, nullptr, Aval, dst, s));
+    }
     P.M = bp.M;
     P.K = bp.K;
     P.N = bp.N;

@@ -491,10 +491,11 @@ hipError_t launch_row_sums(int64_t M, const void *rp, int rp64, const void *val,
 // ERR_ROWPTR when an instance's rp[0] != 0 or rp[rows] != its nnz.
 hipError_t launch_batch_rowptr(int which, int64_t count, const BatchInst *inst, BatchOffsets off,
                                int64_t nrows, int64_t nnz, int *out, DevStats *st, hipStream_t s);
-// Stacked columns (A: + ko_i; B: unchanged) and values (val may be nullptr: not copied).
-// Raises ERR_ACOL / ERR_BCOL for a column outside instance i's range (and writes 0).
+// Stacked columns and values of B (which = 1) or A (0): Acol + ko_i, Bcol unchanged; either
+// array may be nullptr (a batch of A_i * A_i takes both from one pass).  Raises ERR_ACOL /
+// ERR_BCOL for a column outside instance i's range (and writes 0).
 hipError_t launch_batch_entries(int which, int64_t count, const BatchInst *inst, BatchOffsets off,
-                                int64_t nnz, int val32, int *col, void *val, DevStats *st,
+                                int64_t nnz, int val32, int *Acol, int *Bcol, void *val, DevStats *st,
                                 hipStream_t s);
 // Row pointers of every C_i from the stacked C's (crp, int64): instance i's M_i + 1 entries
 // at out + mo_i + i, rebased to start at 0; out is int64 (rp64) or int32.  Also
