@@ -15,11 +15,9 @@
 // numeric kernels also write C's sorted columns, replacing the reference's rank-sort pass
 // (compressed_Ccol_symbolic.cuh:4-63).
 //
-// The kernels of rows that share a wave, and the symbolic ones, stage the row's A entries (B
-// row range, first tile, a_ij) in LDS once; sub-groups of lanes then take one entry each
-// and walk B_j, several elements per lane with all loads issued first; rows of B longer
-// than LONG_SEG (tiles: LONG_TILES) are walked by whole waves.  The numeric kernels of rows
-// with a workgroup to themselves walk all their B rows as one stream of element pairs.
+// Rows of few products share a wave and keep their elements in registers; rows with a
+// workgroup to themselves walk all their B rows as one stream of pairs of elements
+// (symbolic: of tiles).
 // Rows whose slice does not fit LDS (wide rows) use the windowed kernels at the end of this
 // file.
 
@@ -41,37 +39,7 @@ static __constant__ int c_nxcd = MAX_XCDS;
 // The one error these kernels raise; err may be host memory, hence a store.
 DEVI void raise_internal(int *err) { __hip_atomic_store(err, ERR_INTERNAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 
-// Stage the row's A entries a0 .. a0+nA-1 into LDS: first tile and tile count of B_j,
-// and (numeric) first element and length of B_j and a_ij.  One parallel step per row,
-// so the dependent loads Acol -> tptr/Brp are paid once per row rather than once per
-// entry inside the accumulation loops.
-template <int G, bool NUMERIC>
-DEVI void stage_row(const Operands &op, int a0, int nA, int *t0, int *tlen, int *b0, int *blen, double *av)
-{
-    const int l = threadIdx.x & (G - 1);
-    for (int k = l; k < nA; k += G) {
-        const int j = op.Acol[a0 + k];
-        if (t0) {
-            const int tt = op.tptr[j];
-            t0[k] = tt;
-            tlen[k] = op.tptr[j + 1] - tt;
-        }
-        if constexpr (NUMERIC) {
-            const int bb = op.Brp[j];
-            b0[k] = bb;
-            blen[k] = op.Brp[j + 1] - bb;
-            av[k] = op.val32 ? (double)((const float *)op.Aval)[a0 + k] : ((const double *)op.Aval)[a0 + k];
-        }
-    }
-}
-
 constexpr int UNROLL = 4;
-
-// A B row with at least LONG_SEG elements (left; LONG_TILES tiles in the tile OR) is
-// walked by a whole wave, shorter ones by sub-groups: R-MAT's hub rows of B hold tens of
-// thousands of entries and would otherwise leave one sub-group walking while the rest of
-// the workgroup waits.  The LDS kernels list such entries only in their LONG variants,
-// launched when B has a row that long.
 
 // Compact index of tile t (relative to rmin) in a two-level directory: the rank of t
 // among the row's non-empty tiles.
@@ -87,8 +55,6 @@ DEVI unsigned fine_index(const u64 *cm, const unsigned *coff, int t)
 //   OR_FINE    fm[fine_index(t)] |= mask      two-level, pass 2
 enum { OR_FLAT, OR_COARSE, OR_FINE };
 
-// Sub-groups of 2^tshift lanes take one entry j each and walk the tiles of B_j, UNROLL
-// tiles per lane per iteration with all loads issued before the ds_or_b64s.
 template <int MODE>
 DEVI void or_put(u64 *dm, const unsigned *coff, u64 *fm, int tt, u64 m)
 {
@@ -124,17 +90,6 @@ DEVI void or_walk(const Operands &op, int tb, int te, int gw, int gl, u64 *dm, c
             if (c[u] >= 0)
                 or_put<MODE>(dm, coff, fm, c[u] - mn, m[u]);
     }
-}
-
-template <int G, int MODE>
-DEVI void or_tiles(const Operands &op, const int *t0, const int *tlen, int nA, u64 *dm, const unsigned *coff, u64 *fm,
-                   int mn, int tshift)
-{
-    const int l = threadIdx.x & (G - 1);
-    // sub-groups of 2^tshift lanes take one entry each
-    const int SG = 1 << tshift, sl = l & (SG - 1), NSG = G >> tshift;
-    for (int e = l >> tshift; e < nA; e += NSG)
-        or_walk<MODE>(op, t0[e], t0[e] + tlen[e], SG, sl, dm, coff, fm, mn);
 }
 
 // Each lane scans a contiguous chunk [ta, tb) of the n directory entries; groups of 256
@@ -242,85 +197,6 @@ struct PrecF32C {
 
 // Slot of column c in the row's accumulator, by directory form.
 enum { SLOT_FLAT, SLOT_DENSE, SLOT_TWO_LEVEL };
-
-// Add every product a_ij * b_jc of the row into its slot: sub-groups of 2^bshift lanes
-// take one entry each and walk B_j, UNROLL elements per lane per iteration with all
-// loads issued before the ds_add_f64s.  fm/foff: the (fine) tile masks and first slots;
-// cm/coff: the coarse level of a two-level directory.
-// B_j's elements [kb, ke) by a group of gw lanes (this lane the gl-th), each product added
-// into its slot.
-template <int FORM, typename P>
-DEVI void add_walk(const Operands &op, int kb, int ke, int gw, int gl, double a, const u64 *cm, const unsigned *coff,
-                   const u64 *fm, const unsigned *foff, double *vals, int mn)
-{
-    typedef typename P::V V;
-    const V *__restrict__ Bval = (const V *)op.Bval;
-    for (int k = kb + gl; k < ke; k += UNROLL * gw) {
-        int c[UNROLL];
-        V v[UNROLL];
-#pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
-            const int ku = k + u * gw;
-            c[u] = -1;
-            v[u] = 0;
-            if (ku < ke) {
-                c[u] = op.Bcol[ku];
-                v[u] = Bval[ku];
-            }
-        }
-        auto slot_of = [&](int col) -> unsigned {
-            if constexpr (FORM == SLOT_DENSE) {
-                return (unsigned)(col - (mn << 6));
-            } else {
-                const int t = (col >> 6) - mn;
-                const unsigned kk = FORM == SLOT_TWO_LEVEL ? fine_index(cm, coff, t) : (unsigned)t;
-                return foff[kk] + (unsigned)__popcll(fm[kk] & below(col & 63));
-            }
-        };
-        // every slot and product of the step first, then the adds: a product computed
-        // between two adds reuses the registers the add before it still reads, so each add
-        // waited for the previous one to leave the LDS queue (measured on banded: 2.5% off
-        // the step, 3% off the dominant kernel)
-        unsigned slot[UNROLL];
-        double pv[UNROLL];
-#pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
-            slot[u] = 0;
-            pv[u] = 0.0;
-            if (c[u] >= 0) {
-                slot[u] = slot_of(c[u]);
-                pv[u] = P::prep(a, v[u]);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < UNROLL; ++u)
-            if (c[u] >= 0)
-                P::put(vals, slot[u], pv[u]);
-    }
-}
-
-template <int G, int FORM, typename P, bool LIST>
-DEVI void add_products(const Operands &op, const int *b0, const int *blen, const double *av, int nA, const int *lidx,
-                       int nlong, const u64 *cm, const unsigned *coff, const u64 *fm, const unsigned *foff, double *vals,
-                       int mn, int bshift)
-{
-    const int l = threadIdx.x & (G - 1);
-    // LIST: long B rows (listed in lidx), one wave each (the whole group if smaller)
-    if constexpr (LIST) {
-        constexpr int LW = G < 64 ? G : 64;
-        for (int i = l / LW; i < nlong; i += G / LW) {
-            const int e = lidx[i];
-            add_walk<FORM, P>(op, b0[e], b0[e] + blen[e], LW, l & (LW - 1), av[e], cm, coff, fm, foff, vals, mn);
-        }
-    }
-    // sub-groups of SG lanes take one entry each
-    const int SG = 1 << bshift, sl = l & (SG - 1), NSG = G >> bshift;
-    for (int e = l >> bshift; e < nA; e += NSG) {
-        if (LIST && blen[e] >= LONG_SEG)
-            continue;
-        add_walk<FORM, P>(op, b0[e], b0[e] + blen[e], SG, sl, av[e], cm, coff, fm, foff, vals, mn);
-    }
-}
 
 // ---- the element stream of a row ------------------------------------------------------------
 //
@@ -593,100 +469,219 @@ DEVI void stream_or(const Stream<G> &st, long long w0, const Operands &op, u64 *
 
 // ---- symbolic ------------------------------------------------------------------------------
 
-// nnz(C_i) for rows kept in LDS: stage the row, OR the tile masks with ds_or_b64 into the
-// row's tile directory, popcount.  Flat rows: one pass into a directory over the whole
-// span.  Two-level rows: pass 1 marks the non-empty tiles in the coarse bitmap, a scan
-// gives their compact indices, pass 2 ORs the masks into the compact fine level.
-// two_level = 0 when no row of the launch is two-level (its extra steps are skipped).
-// When the directory is kept, it goes out with each entry's exclusive prefix (coarse:
-// first compact index; fine or flat: first slot) for the numeric phase.
-template <int G, bool LONG>
-__global__ __launch_bounds__(BLOCK) void k_symbolic_lds(const int *__restrict__ rows,
-                                                                       const int *__restrict__ count_p, int slice_bytes,
-                                                                       Operands op, int *__restrict__ rnnz, int tshift,
-                                                                       int two_level, unsigned *queue)
+// ---- rows that share a wave ----------------------------------------------------------------
+//
+// Rows of few products, G = 8, 16 or 32 lanes each (small_layout): the row's elements of B
+// are loaded once, SMALL_U pairs per lane, and stay in registers.  Their columns mark the
+// row's words (32 columns each) in a coarse bitmap; a scan gives the marked words compact
+// places, where the columns are marked in turn; a second scan gives nnz(C_i) -- all the
+// symbolic phase wants -- and each word's first slot.  The numeric phase then adds every
+// product at its column's rank (ds_add_f64), puts the column there too, and the row goes
+// out in order.
+// Against staging the A entries in LDS and walking B's tiles twice for the directory and
+// its rows a third time for the products, a lane or two per row of B (512 Laplacians of
+// 7.5 M rows; that kernel spent 52% of its time in vector instructions, 62% in the L1 and
+// 39% in LDS, two thirds of it bank conflicts): numeric 2,860 -> 1,850 us,
+// symbolic 1,044 -> 1,007 us, the call 5.74 -> 4.70 ms; a 47^3 stencil 178 -> 150 us, a random
+// product of ragged rows 261 -> 207 us. Now bound by vector instructions (symbolic 66% of the
+// time, numeric 46%).
+struct SmallNone { // symbolic: no values
+    typedef float V;
+};
+template <int G, typename P>
+__global__ __launch_bounds__(BLOCK) void k_small_rows(const int *__restrict__ rows, const int *__restrict__ count_p,
+                                                      int slice_bytes, Operands op, int *__restrict__ rnnz,
+                                                      const long long *__restrict__ crp, int *__restrict__ Ccol,
+                                                      typename P::V *__restrict__ Cval, int *err, unsigned *queue)
 {
-    static_assert(G < BLOCK, "rows that share a workgroup");
-    constexpr int RPB = BLOCK / G;
+    typedef typename P::V V;
+    constexpr bool NUM = !std::is_same<P, SmallNone>::value;
+    constexpr int RPB = BLOCK / G, U = SMALL_U;
     extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ unsigned redu[16];
     __shared__ int grp_s[2];
     const int g = threadIdx.x / G, l = threadIdx.x & (G - 1);
     unsigned char *slice = lds + (size_t)g * slice_bytes;
+    const V *__restrict__ Aval = (const V *)op.Aval;
+    const V *__restrict__ Bval = (const V *)op.Bval;
+    const unsigned nB = (unsigned)op.nnzB;
     const int nrows = *count_p;
+    // bits of a word below a column, or of a step's ends below a lane
+    auto under = [](unsigned m, int c) { return m & ((1u << (c & 31)) - 1u); };
     for (GroupWalk gw(queue, (nrows + RPB - 1) / RPB, grp_s, c_nxcd); gw.more(); gw.next()) {
         const int idx = gw.grp * RPB + g;
         const int row = idx < nrows ? rows[idx] : -1;
-        int S = 0, mn = 0, a0 = 0, nA = 0, tp = 0;
+        int S = 0, w0 = 0, n = 0, a0 = 0, nA = 0, p = 0;
+        long long cb = 0;
         if (row >= 0) {
-            mn = op.rmin[row];
-            S = op.rmax[row] - mn + 1;
+            w0 = 2 * op.rmin[row];
+            S = op.rmax[row] - (w0 >> 1) + 1;
             a0 = op.Arp[row];
             nA = op.Arp[row + 1] - a0;
-            tp = op.rtp[row];
+            p = (int)op.rprod[row];
+            if constexpr (NUM) {
+                cb = crp[row];
+                n = (int)(crp[row + 1] - cb);
+            }
         }
-        const bool sparse = use_sparse(S, tp);
-        const int W = sparse ? (S + 63) >> 6 : S; // entries of the first level
-        const RowLayout L = row_layout(0, S, 0, nA, tp, LONG);
-        u64 *dm = (u64 *)(slice + L.dm);
-        unsigned *doff = (unsigned *)(slice + L.doff);
-        int *tlen = (int *)(slice + L.tlen);
-        int *t0 = (int *)(slice + L.t0);
-        for (int t = l; t < W; t += G)
-            dm[t] = 0;
-        stage_row<G, false>(op, a0, nA, t0, tlen, nullptr, nullptr, nullptr);
+        const SmallLayout L = small_layout(NUM, S, n, nA, p);
+        uint2 *coarse = (uint2 *)(slice + L.coarse); // words of the row: marked words, those before
+        uint2 *fine = (uint2 *)(slice + L.fine);     // marked words: columns, slots before
+        double *vals = (double *)(slice + L.vals);
+        int *cols = (int *)(slice + L.cols);
+        uint4 *rec = (uint4 *)(slice + L.rec);
+        unsigned *ends = (unsigned *)(slice + L.ends); // per step of G pairs: it ends an entry
+        // this lane's entry of A
+        int start = 0, len = 0;
+        u64 a = 0;
+        if (l < nA) {
+            const typename Vec2<int>::type b = load2(op.Brp + op.Acol[a0 + l]);
+            start = b.x;
+            len = b.y - b.x;
+            if constexpr (NUM)
+                a = (u64)__double_as_longlong((double)Aval[a0 + l]);
+        }
+        const int CW = L.ncoarse, FW = L.nfine;
+        for (int q = l; q < CW; q += G)
+            coarse[q] = make_uint2(0, 0);
+        for (int q = l; q < FW; q += G)
+            fine[q] = make_uint2(0, 0);
+        if constexpr (NUM)
+            for (int q = l; q < n; q += G)
+                vals[q] = 0.0;
+        if (l < U)
+            ends[l] = 0;
+        // its pairs among the row's
+        const unsigned cnt = (unsigned)(len + 1) >> 1;
+        unsigned tot;
+        const unsigned ex = group_excl_scan<G, unsigned>(cnt | (cnt ? 1u << 16 : 0u), nullptr, tot);
+        const unsigned first = ex & 0xffff, total = tot & 0xffff;
         __syncthreads();
-        if (sparse)
-            or_tiles<G, OR_COARSE>(op, t0, tlen, nA, dm, nullptr, nullptr, mn, tshift);
-        else
-            or_tiles<G, OR_FLAT>(op, t0, tlen, nA, dm, nullptr, nullptr, mn, tshift);
+        if (cnt) {
+            const unsigned last = first + cnt - 1;
+            atomicOr(&ends[last / G], 1u << (last & (G - 1)));
+            rec[ex >> 16] = make_uint4((unsigned)start - STREAM_V * first, (unsigned)(start + len), (unsigned)a,
+                                       (unsigned)(a >> 32));
+        }
         __syncthreads();
-        const ChunkScan cs = scan_popcounts<G>(dm, W, redu);
-        const unsigned tot = cs.tot;
-        const long long rd = (row >= 0 && op.dir_mask) ? op.rdir[row] & ~RDIR_TWO : -1;
-        unsigned nnz = tot;
-        if (sparse)
-            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64 w) {
-                doff[t] = p;
-                if (rd >= 0) {
-                    op.dir_mask[rd + t] = w;
-                    op.dir_off[rd + t] = p;
+        // element 0 of a live pair is always the row's (at the array's end it is the load's
+        // second), element 1 if the entry has it
+        int c0[U], c1[U];
+        V v0[U], v1[U];
+        double av[U];
+        bool live[U], two[U];
+        unsigned e = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned bits = ends[u];
+            const unsigned q = u * G + l;
+            live[u] = q < total;
+            two[u] = false;
+            c0[u] = c1[u] = 0;
+            if (live[u]) {
+                const uint4 r = rec[e + __popc(under(bits, l))];
+                const unsigned k = r.x + STREAM_V * q, at = k < nB - 2 ? k : nB - 2;
+                const typename Vec2<int>::type c = load2(op.Bcol + at);
+                c0[u] = at == k ? c.x : c.y;
+                c1[u] = c.y;
+                two[u] = k + 1 < r.y;
+                if constexpr (NUM) {
+                    const typename Vec2<V>::type v = load2(Bval + at);
+                    v0[u] = at == k ? v.x : v.y;
+                    v1[u] = v.y;
+                    av[u] = __longlong_as_double((long long)(((u64)r.w << 32) | r.z));
                 }
-            });
-        else if (rd >= 0)
-            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64 w) {
-                op.dir_mask[rd + t] = w;
-                op.dir_off[rd + t] = p;
-            });
-        if (two_level) {
-            // two-level rows: tot = non-empty tiles; build and count the fine level
-            u64 *fm = dm + W;
-            __syncthreads();
-            if (sparse)
-                for (int k = l; k < (int)tot; k += G)
-                    fm[k] = 0;
-            __syncthreads();
-            if (sparse)
-                or_tiles<G, OR_FINE>(op, t0, tlen, nA, dm, doff, fm, mn, tshift);
-            __syncthreads();
-            const int F = sparse ? (int)tot : 0;
-            const ChunkScan fs = scan_popcounts<G>(fm, F, redu);
-            if (sparse)
-                nnz = fs.tot;
-            if (rd >= 0)
-                chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64 w) {
-                    op.dir_mask[rd + W + k] = w;
-                    op.dir_off[rd + W + k] = p;
-                });
+            }
+            e += __popc(bits);
         }
-        if (row >= 0 && l == 0)
-            rnnz[row] = (int)nnz;
+        // mark the words
+        auto word = [&](int c) { return (c >> 5) - w0; };
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (live[u]) {
+                const int w = word(c0[u]);
+                atomicOr(&coarse[w >> 5].x, 1u << (w & 31));
+            }
+            if (two[u]) {
+                const int w = word(c1[u]);
+                atomicOr(&coarse[w >> 5].x, 1u << (w & 31));
+            }
+        }
+        __syncthreads();
+        // exclusive prefix of n words' bits in their second halves; the sum
+        auto prefix = [&](uint2 *m, int nw) {
+            unsigned sum = 0;
+            for (int q0 = 0; __any(q0 < nw); q0 += G) {
+                const int q = q0 + l;
+                unsigned t;
+                const unsigned x = group_excl_scan<G, unsigned>(q < nw ? __popc(m[q].x) : 0u, nullptr, t);
+                if (q < nw)
+                    m[q].y = sum + x;
+                sum += t;
+            }
+            return sum;
+        };
+        const int nf = (int)prefix(coarse, CW);
+        __syncthreads();
+        // mark the columns
+        unsigned f0[U], f1[U];
+        auto fine_of = [&](int c) {
+            const int w = word(c);
+            const uint2 m = coarse[w >> 5];
+            return m.y + (unsigned)__popc(under(m.x, w));
+        };
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            f0[u] = f1[u] = 0;
+            if (live[u]) {
+                f0[u] = fine_of(c0[u]);
+                atomicOr(&fine[f0[u]].x, 1u << (c0[u] & 31));
+            }
+            if (two[u]) {
+                f1[u] = fine_of(c1[u]);
+                atomicOr(&fine[f1[u]].x, 1u << (c1[u] & 31));
+            }
+        }
+        __syncthreads();
+        const int nnz = (int)prefix(fine, nf);
+        if constexpr (!NUM) {
+            if (row >= 0 && l == 0)
+                rnnz[row] = nnz;
+        } else {
+            const bool ok = nnz == n;
+            if (row >= 0 && !ok && l == 0)
+                raise_internal(err);
+            __syncthreads();
+            if (ok) {
+                auto put = [&](unsigned f, int c, double x) {
+                    const uint2 m = fine[f];
+                    const unsigned slot = m.y + (unsigned)__popc(under(m.x, c));
+                    cols[slot] = c;
+                    P::put(vals, slot, x);
+                };
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (live[u])
+                        put(f0[u], c0[u], P::prep(av[u], v0[u]));
+                    if (two[u])
+                        put(f1[u], c1[u], P::prep(av[u], v1[u]));
+                }
+            }
+            __syncthreads();
+            if (ok)
+                for (int q = l; q < n; q += G) {
+                    Ccol[cb + q] = cols[q];
+                    Cval[cb + q] = P::result(vals, (unsigned)q);
+                }
+        }
         __syncthreads();
     }
 }
 
-// The same for a row with a workgroup to itself: the tiles of its B rows are walked as one
-// stream of pairs.  Bound by the loads of column and mask per tile (a load instruction costs
+// nnz(C_i) for a row with a workgroup to itself: the tiles of its B rows, walked as one
+// stream of pairs, are ORed into the row's tile directory (ds_or_b64), and its bits counted.
+// Flat rows: one pass into a directory over the whole span.  Two-level rows: pass 1 marks
+// the non-empty tiles in the coarse bitmap, a scan gives their compact indices, pass 2 ORs
+// the masks into the compact fine level.  Bound by the loads of column and mask per tile (a load instruction costs
 // the same for any number of active lanes: B rows of a few tiles left most of a sub-group
 // idle, and staging entries in LDS doubled a row's need) and then by the LDS ORs.  Symbolic
 // stage of R-MAT squares, before and after: scale 16 938 and 434 us, scale 18 8.5 and
@@ -870,175 +865,6 @@ __global__ __launch_bounds__(1024) void k_symbolic_wide(const int *__restrict__ 
 }
 
 // ---- numeric -------------------------------------------------------------------------------
-
-// The HSMU accumulator in LDS for rows that share a workgroup of one wave (G = 8, 16 or 32
-// lanes per row; slice layout: row_layout).  The row's tile directory is loaded (kept by
-// the symbolic phase) or rebuilt as there, every product is added with ds_add_f64 into its
-// slot, and the row of C is written in column order, a lane per tile walking its set bits.
-// Directory forms: flat (slot from the tile's entry), dense (one slot per column of the
-// span) and two-level (the tile's entry found through the coarse bitmap first); two_level =
-// 0 when no row of the launch uses it.
-template <int G, typename P, bool LONG>
-__global__ __launch_bounds__(BLOCK) void k_numeric_lds(const int *__restrict__ rows,
-                                                                      const int *__restrict__ count_p, int slice_bytes,
-                                                                      Operands op, const long long *__restrict__ crp,
-                                                                      int *__restrict__ Ccol, typename P::V *__restrict__ Cval,
-                                                                      int bshift, int tshift, int two_level, int *err,
-                                                                      unsigned *queue)
-{
-    static_assert(G < BLOCK, "rows that share a workgroup");
-    constexpr int RPB = BLOCK / G;
-    extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ unsigned redu[16];
-    __shared__ int grp_s[2];
-    const int g = threadIdx.x / G, l = threadIdx.x & (G - 1);
-    unsigned char *slice = lds + (size_t)g * slice_bytes;
-    const int nrows = *count_p;
-    for (GroupWalk gw(queue, (nrows + RPB - 1) / RPB, grp_s, c_nxcd); gw.more(); gw.next()) {
-        const int idx = gw.grp * RPB + g;
-        const int row = idx < nrows ? rows[idx] : -1;
-        int S = 0, mn = 0, n = 0, a0 = 0, nA = 0, tp = 0;
-        long long cb = 0;
-        if (row >= 0) {
-            mn = op.rmin[row];
-            S = op.rmax[row] - mn + 1;
-            cb = crp[row];
-            n = (int)(crp[row + 1] - cb);
-            a0 = op.Arp[row];
-            nA = op.Arp[row + 1] - a0;
-            tp = op.rtp[row];
-        }
-        const bool sparse = use_sparse(S, tp);
-        const int W = sparse ? (S + 63) >> 6 : S; // entries of the first level
-        const RowLayout L = row_layout(1, S, n, nA, tp, LONG);
-        u64 *dm = (u64 *)(slice + L.dm);
-        unsigned *doff = (unsigned *)(slice + L.doff);
-        unsigned *ft = (unsigned *)(slice + L.ft);
-        double *vals = (double *)(slice + L.vals);
-        double *av = (double *)(slice + L.av);
-        int *tlen = (int *)(slice + L.tlen);
-        int *t0 = (int *)(slice + L.t0);
-        int *blen = (int *)(slice + L.blen);
-        int *b0 = (int *)(slice + L.b0);
-        int *lidx = (int *)(slice + L.lidx);
-        int *lcnt = (int *)(slice + L.lcnt);
-        // fine level: the flat directory itself, or the compact entries after the coarse words
-        u64 *fm = sparse ? dm + W : dm;
-        unsigned *foff = sparse ? doff + W : doff;
-        const bool dense = !sparse && use_dense(S, n);
-        const int nv = dense ? 64 * S : n;
-        const long long rd = (row >= 0 && op.dir_mask) ? kept_dir(op, row, sparse) : -1;
-        for (int q = l; q < nv; q += G)
-            vals[q] = 0.0;
-        if (LONG && l == 0)
-            *lcnt = 0;
-        if (rd >= 0) {
-            // directory kept by the symbolic phase: load its first level, stage only B's ranges
-            for (int t = l; t < W; t += G) {
-                dm[t] = op.dir_mask[rd + t];
-                doff[t] = op.dir_off[rd + t];
-            }
-            stage_row<G, true>(op, a0, nA, nullptr, nullptr, b0, blen, av);
-        } else {
-            for (int t = l; t < W; t += G)
-                dm[t] = 0;
-            stage_row<G, true>(op, a0, nA, t0, tlen, b0, blen, av);
-        }
-        __syncthreads();
-        // entries with long rows of B, walked by whole waves
-        if constexpr (LONG) {
-            for (int k = l; k < nA; k += G)
-                if (blen[k] >= LONG_SEG)
-                    lidx[atomicAdd(lcnt, 1)] = k;
-        }
-        if (rd < 0) {
-            if (sparse)
-                or_tiles<G, OR_COARSE>(op, t0, tlen, nA, dm, nullptr, nullptr, mn, tshift);
-            else
-                or_tiles<G, OR_FLAT>(op, t0, tlen, nA, dm, nullptr, nullptr, mn, tshift);
-        }
-        // first level: flat slot offsets (rebuilt) or coarse compact indices (rebuilt), and
-        // the total (flat: nnz(C_i); two-level: non-empty tiles)
-        __syncthreads();
-        const ChunkScan cs = scan_popcounts<G>(dm, W, redu);
-        const unsigned tot = cs.tot;
-        if (rd < 0)
-            chunk_offsets<G>(dm, cs, [&](int t, unsigned p, u64) { doff[t] = p; });
-        unsigned nnz = tot;
-        const int F = sparse ? (int)tot : S; // fine entries
-        if (two_level) {
-            __syncthreads();
-            if (sparse) {
-                if (rd >= 0) {
-                    for (int k = l; k < F; k += G) {
-                        fm[k] = op.dir_mask[rd + W + k];
-                        foff[k] = op.dir_off[rd + W + k];
-                    }
-                } else {
-                    for (int k = l; k < F; k += G)
-                        fm[k] = 0;
-                }
-                // tile of every fine entry, from the coarse bitmap
-                for (int w = l; w < W; w += G) {
-                    u64 m = dm[w];
-                    unsigned k = doff[w];
-                    while (m) {
-                        ft[k++] = (unsigned)((w << 6) + __ffsll((unsigned long long)m) - 1);
-                        m &= m - 1;
-                    }
-                }
-            }
-            __syncthreads();
-            if (sparse && rd < 0)
-                or_tiles<G, OR_FINE>(op, t0, tlen, nA, dm, doff, fm, mn, tshift);
-            __syncthreads();
-            const ChunkScan fs = scan_popcounts<G>(fm, sparse ? F : 0, redu);
-            if (sparse) {
-                nnz = fs.tot;
-                if (rd < 0)
-                    chunk_offsets<G>(fm, fs, [&](int k, unsigned p, u64) { foff[k] = p; });
-            }
-        }
-        const bool ok = (int)nnz == n;
-        if (row >= 0 && !ok && l == 0)
-            raise_internal(err);
-        __syncthreads();
-        if (row >= 0 && ok) {
-            const int nlong = LONG ? *lcnt : 0;
-            if (dense)
-                add_products<G, SLOT_DENSE, P, LONG>(op, b0, blen, av, nA, lidx, nlong, nullptr, nullptr, fm, foff, vals,
-                                                     mn, bshift);
-            else if (sparse)
-                add_products<G, SLOT_TWO_LEVEL, P, LONG>(op, b0, blen, av, nA, lidx, nlong, dm, doff, fm, foff, vals,
-                                                         mn, bshift);
-            else
-                add_products<G, SLOT_FLAT, P, LONG>(op, b0, blen, av, nA, lidx, nlong, nullptr, nullptr, fm, foff, vals,
-                                                    mn, bshift);
-        }
-        __syncthreads();
-        if (row >= 0 && ok) {
-            // a lane per tile, then the values in slot order
-            for (int t0 = l; t0 < F; t0 += G) {
-                u64 m = fm[t0];
-                unsigned pos = foff[t0];
-                const int t = sparse ? (int)ft[t0] : t0;
-                const int c0 = (mn + t) << 6;
-                while (m) {
-                    const int b = __ffsll((unsigned long long)m) - 1;
-                    Ccol[cb + pos] = c0 + b;
-                    if (dense)
-                        Cval[cb + pos] = P::result(vals, (t << 6) + b);
-                    ++pos;
-                    m &= m - 1;
-                }
-            }
-            if (!dense)
-                for (int q = l; q < n; q += G)
-                    Cval[cb + q] = P::result(vals, q);
-        }
-        __syncthreads();
-    }
-}
 
 // The same for a row with a workgroup to itself (G = 64 to 1024 lanes): its B rows are
 // walked as one element stream.  What bounds it: the L1's rate for loads (12 bytes per
@@ -2001,18 +1827,42 @@ static int64_t row_grid(Kern kernel, int bs, size_t lds, int64_t groups, int num
     return blocks < 1 ? 1 : blocks;
 }
 
-template <int G, bool LONG>
-static void symbolic_g(const int *rows, const int *count_dev, int count, int max_need, const Operands &op, int *rnnz,
-                       int tshift, int two_level, int num_cus, unsigned *queue, hipStream_t s)
+// LDS of a row that shares a workgroup: the lanes of the workgroup's rows walk their slices
+// in step, 8 bytes a lane, so slices an odd multiple of 8 G bytes apart keep them on
+// different banks (padding that a small workgroup's LDS has room for).
+template <int G> static int row_slice(int need)
+{
+    const int step = 8 * G, odd = ((need + step - 1) / step | 1) * step;
+    return odd * (BLOCK / G) <= 32 * 1024 ? odd : (need + 15) & ~15;
+}
+
+template <int G, typename P>
+static void small_g(const int *rows, const int *count_dev, int count, int max_need, const Operands &op, int *rnnz,
+                    const long long *crp, int *Ccol, void *Cval, int *err, int num_cus, unsigned *queue,
+                    unsigned long long *lds_bytes, hipStream_t s)
 {
     constexpr int RPB = BLOCK / G;
-    const int slice = (max_need + 15) & ~15;
+    const int slice = row_slice<G>(max_need);
     const size_t lds = (size_t)slice * RPB;
-    const int64_t blocks =
-        row_grid(k_symbolic_lds<G, LONG>, BLOCK, lds, ((int64_t)count + RPB - 1) / RPB, num_cus, queue);
-    const int lg = __builtin_ctz(G);
-    hipLaunchKernelGGL((k_symbolic_lds<G, LONG>), dim3((unsigned)blocks), dim3(BLOCK), lds, s, rows, count_dev, slice,
-                       op, rnnz, tshift > lg ? lg : tshift, two_level, queue);
+    const int64_t blocks = row_grid(k_small_rows<G, P>, BLOCK, lds, ((int64_t)count + RPB - 1) / RPB, num_cus, queue);
+    *lds_bytes += (unsigned long long)blocks * lds;
+    hipLaunchKernelGGL((k_small_rows<G, P>), dim3((unsigned)blocks), dim3(BLOCK), lds, s, rows, count_dev, slice, op,
+                       rnnz, crp, Ccol, (typename P::V *)Cval, err, queue);
+}
+
+template <typename P>
+static void small_rows(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
+                       int *rnnz, const long long *crp, int *Ccol, void *Cval, int *err, int num_cus, unsigned *queue,
+                       unsigned long long *lds_bytes, hipStream_t s)
+{
+#define SMALL(B, G)                                                                                                    \
+    case B:                                                                                                            \
+        small_g<G, P>(rows, count_dev, count, max_need, op, rnnz, crp, Ccol, Cval, err, num_cus, queue, lds_bytes, s); \
+        break;
+    switch (bin) {
+        SMALL(0, 8) SMALL(1, 16) SMALL(2, 32)
+    }
+#undef SMALL
 }
 
 template <int G, bool TL>
@@ -2038,7 +1888,7 @@ static void symbolic_rows(int bin, const int *rows, const int *count_dev, int co
 }
 
 hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
-                           int *rnnz, int tshift, int two_level, int long_rows, u64 *gws, long long gws_stride,
+                           int *rnnz, int tshift, int two_level, u64 *gws, long long gws_stride,
                            int num_cus, int gws_blocks, int lds_dyn, unsigned *queue, hipStream_t s)
 {
     if (count <= 0)
@@ -2053,55 +1903,19 @@ hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int c
             hipLaunchKernelGGL(k_symbolic_global, dim3(blocks), dim3(1024), 0, s, rows, count_dev, op, rnnz,
                                tshift > 10 ? 10 : tshift, gws, gws_stride);
     } else if (bin >= 0 && bin < NLDS) {
-#define SYM(B, G, LONG)                                                                                                \
-    case B: symbolic_g<G, LONG>(rows, count_dev, count, max_need, op, rnnz, tshift, two_level, num_cus, queue, s); break;
         if (bin >= 3 && two_level)
             symbolic_rows<true>(bin, rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s);
         else if (bin >= 3)
             symbolic_rows<false>(bin, rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s);
-        else if (long_rows)
-            switch (bin) { SYM(0, 8, true) SYM(1, 16, true) SYM(2, 32, true) }
-        else
-            switch (bin) { SYM(0, 8, false) SYM(1, 16, false) SYM(2, 32, false) }
-#undef SYM
+        else {
+            unsigned long long ignored = 0;
+            small_rows<SmallNone>(bin, rows, count_dev, count, max_need, op, rnnz, nullptr, nullptr, nullptr, nullptr,
+                                  num_cus, queue, &ignored, s);
+        }
     } else {
         return hipErrorInvalidValue;
     }
     return hipGetLastError();
-}
-
-template <int G, typename P, bool LONG>
-static void numeric_g(const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
-                      const long long *crp, int *Ccol, void *Cval, int bshift, int tshift, int two_level, int *err,
-                      int num_cus, unsigned *queue, unsigned long long *lds_bytes, hipStream_t s)
-{
-    constexpr int BS = G < BLOCK ? BLOCK : G;
-    constexpr int RPB = BS / G;
-    const int slice = (max_need + 15) & ~15;
-    const size_t lds = (size_t)slice * RPB;
-    const int64_t blocks =
-        row_grid(k_numeric_lds<G, P, LONG>, BS, lds, ((int64_t)count + RPB - 1) / RPB, num_cus, queue);
-    *lds_bytes += (unsigned long long)blocks * lds;
-    const int lg = __builtin_ctz(G);
-    hipLaunchKernelGGL((k_numeric_lds<G, P, LONG>), dim3((unsigned)blocks), dim3(BS), lds, s, rows, count_dev, slice,
-                       op, crp, Ccol, (typename P::V *)Cval, bshift > lg ? lg : bshift, tshift > lg ? lg : tshift,
-                       two_level, err, queue);
-}
-
-template <typename P, bool LONG>
-static void numeric_l(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
-                      const long long *crp, int *Ccol, void *Cval, int bshift, int tshift, int two_level, int *err,
-                      int num_cus, unsigned *queue, unsigned long long *lds_bytes, hipStream_t s)
-{
-#define NUM(B, G)                                                                                                      \
-    case B:                                                                                                            \
-        numeric_g<G, P, LONG>(rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, tshift, two_level, err,   \
-                              num_cus, queue, lds_bytes, s);                                                           \
-        break;
-    switch (bin) {
-        NUM(0, 8) NUM(1, 16) NUM(2, 32)
-    }
-#undef NUM
 }
 
 template <int G, typename P, bool TL>
@@ -2134,8 +1948,8 @@ static void numeric_rows(int bin, const int *rows, const int *count_dev, int cou
 
 template <typename P>
 static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
-                            const long long *crp, int *Ccol, void *Cval, int bshift, int tshift, int two_level,
-                            int long_rows, const WideRows &wide, int *err, int num_cus, unsigned *queue,
+                            const long long *crp, int *Ccol, void *Cval, int bshift, int two_level,
+                            const WideRows &wide, int *err, int num_cus, unsigned *queue,
                             unsigned long long *lds_bytes, hipStream_t s)
 {
     if (bin == BIN_GLOBAL) {
@@ -2175,12 +1989,8 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
             numeric_rows<P, false>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, err, num_cus, queue,
                                    lds_bytes, s);
     } else if (bin >= 0 && bin < NLDS) {
-        if (long_rows)
-            numeric_l<P, true>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, tshift, two_level,
-                               err, num_cus, queue, lds_bytes, s);
-        else
-            numeric_l<P, false>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, tshift, two_level,
-                                err, num_cus, queue, lds_bytes, s);
+        small_rows<P>(bin, rows, count_dev, count, max_need, op, nullptr, crp, Ccol, Cval, err, num_cus, queue,
+                      lds_bytes, s);
     } else {
         return hipErrorInvalidValue;
     }
@@ -2188,8 +1998,7 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
 }
 
 hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_dev, int count, int max_need,
-                          const Operands &op, const long long *crp, int *Ccol, void *Cval, int bshift, int tshift,
-                          int two_level, int long_rows, const WideRows &wide, int *err, int num_cus, unsigned *queue,
+                          const Operands &op, const long long *crp, int *Ccol, void *Cval, int bshift, int two_level, const WideRows &wide, int *err, int num_cus, unsigned *queue,
                           unsigned long long *lds_bytes, hipStream_t s)
 {
     if (count <= 0)
@@ -2198,10 +2007,8 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
     if (!lds_bytes)
         lds_bytes = &ignored;
     if (fp32c)
-        return numeric_p<PrecF32C>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, tshift, two_level,
-                                   long_rows, wide, err, num_cus, queue, lds_bytes, s);
-    return numeric_p<PrecF64>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, tshift, two_level,
-                              long_rows, wide, err, num_cus, queue, lds_bytes, s);
+        return numeric_p<PrecF32C>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, two_level, wide, err, num_cus, queue, lds_bytes, s);
+    return numeric_p<PrecF64>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, two_level, wide, err, num_cus, queue, lds_bytes, s);
 }
 
 int wide_item_blocks(int count, int num_cus)
@@ -2225,21 +2032,16 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
         if (r != hipSuccess)                                                                                           \
             e = r;                                                                                                     \
     }
-#define CFGL(L)                                                                                                        \
-    CFG((k_symbolic_lds<8, L>)) CFG((k_symbolic_lds<16, L>)) CFG((k_symbolic_lds<32, L>))
+#define CFGL(P) CFG((k_small_rows<8, P>)) CFG((k_small_rows<16, P>)) CFG((k_small_rows<32, P>))
 #define CFGS(TL)                                                                                                       \
     CFG((k_symbolic_row<64, TL>)) CFG((k_symbolic_row<128, TL>)) CFG((k_symbolic_row<256, TL>))                        \
     CFG((k_symbolic_row<512, TL>)) CFG((k_symbolic_row<1024, TL>))
-#define CFGP(P, L)                                                                                                     \
-    CFG((k_numeric_lds<8, P, L>)) CFG((k_numeric_lds<16, P, L>)) CFG((k_numeric_lds<32, P, L>))
 #define CFGR(P, TL)                                                                                                    \
     CFG((k_numeric_row<64, P, TL>)) CFG((k_numeric_row<128, P, TL>)) CFG((k_numeric_row<256, P, TL>))                  \
     CFG((k_numeric_row<512, P, TL>)) CFG((k_numeric_row<1024, P, TL>))
-    CFGL(false) CFGL(true) CFGS(false) CFGS(true)
-    CFGP(PrecF64, false) CFGP(PrecF64, true) CFGP(PrecF32C, false) CFGP(PrecF32C, true)
+    CFGL(SmallNone) CFGL(PrecF64) CFGL(PrecF32C) CFGS(false) CFGS(true)
     CFGR(PrecF64, false) CFGR(PrecF32C, false) CFGR(PrecF64, true) CFGR(PrecF32C, true)
 #undef CFGR
-#undef CFGP
 #undef CFGL
 #undef CFGS
     CFG(k_symbolic_wide)

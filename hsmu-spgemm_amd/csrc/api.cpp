@@ -776,8 +776,6 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     if (tlanes > 64)
         tlanes = 64;
     const int bshift = ilog2(blanes), tshift = ilog2(tlanes);
-    // B has rows long enough for the whole-wave walks (the binning sized LDS for them)
-    const int long_rows = h1.max_brow >= LONG_TILES ? 1 : 0;
 
     Operands op;
     op.Arp = P.Arp;
@@ -822,7 +820,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         keep_dirs = mode.plan->dirs_kept;
     } else {
         unsigned long long tile_products = 0;
-        for (int b = 0; b < NBINS; ++b)
+        for (int b = BIN_SHARED; b < NBINS; ++b) // (rows that share a wave keep none)
             tile_products += h1.sym.work[b];
         const bool worth = 2 * dir_total <= tile_products || h1.sym.count[BIN_GLOBAL] > 0 ||
                            h1.num_wide_hint > 0;
@@ -863,7 +861,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         if (cnt <= 0)
             continue;
         HIP_TRY(launch_symbolic(b, binrows + (size_t)b * M, &dst->sym.count[b], cnt, h1.sym.max_need[b], op, rnnz,
-                                tshift, h1.sym.nsparse[b] > 0 ? 1 : 0, long_rows, gws, gws_stride, c->num_cus,
+                                tshift, h1.sym.nsparse[b] > 0 ? 1 : 0, gws, gws_stride, c->num_cus,
                                 gws_blocks, (int)bp.lds_row_max,
                                 opts.persistent ? dst->queue[0][b] : nullptr, s));
     }
@@ -984,7 +982,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         if (timing)
             HIP_TRY(hipEventRecord(c->evb[b][0], s));
         HIP_TRY(launch_numeric(b, fp32 ? 1 : 0, binrows + (size_t)b * M, &dst->num.count[b], cnt, h2.num.max_need[b], op,
-                               crp, Ccol, Cval, bshift, tshift, h2.num.nsparse[b] > 0 ? 1 : 0, long_rows, wide, errp,
+                               crp, Ccol, Cval, bshift, h2.num.nsparse[b] > 0 ? 1 : 0, wide, errp,
                                c->num_cus,
                                opts.persistent ? dst->queue[1][b] : nullptr, &lds_launched, s));
         if (timing)

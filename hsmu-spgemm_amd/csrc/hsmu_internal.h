@@ -64,7 +64,6 @@ struct DevStats {
     int err;
     int ntiles_b;
     int pad;
-    int max_brow; // longest row of B (counted from LONG_TILES on)
     unsigned long long num_wide_hint; // rows whose numeric need may exceed LDS (symbolic binning)
     unsigned long long wide_items; // windows the wide rows may need, at most (numeric binning)
     BinStats sym;
@@ -139,75 +138,52 @@ HSMU_HD inline int dir_entries(int S, int tp) { return use_sparse(S, tp) ? ((S +
 constexpr int LAYOUT_CAP = 1 << 18;
 constexpr int LAYOUT_NONE = 1 << 30;
 
-// LDS slice of one row in the LDS kernels (byte offsets), for a row whose C row spans
-// S tiles, has n = nnz(C_i) entries, nA entries in A and tp tile-products; E =
-// dir_entries(S, tp):
-//   dm   u64[E]     tile masks (flat), or coarse words then fine masks (two-level)
-//   doff u32[E]     slot of each tile's first column (numeric), coarse offsets (two-level)
-//   ft   u32[R]     numeric, two-level: tile of each fine entry, relative to rmin
-//   vals f64[n]     numeric: accumulators (64*S of them in the dense form)
-//   av   f64[nA]    numeric: a_ij of the row's entries
-//   tlen i32[nA]    tiles(B_j) for each entry j of the row
-//   t0   i32[nA]    first tile of B_j
-//   blen i32[nA]    numeric: nnz(B_j)
-//   b0   i32[nA]    numeric: first stored element of B_j
-//   lidx i32[nA]    with_long: entries whose B_j (numeric) or tile row (symbolic) is
-//                   long, walked by whole waves
-//   lcnt i32        with_long: their number (16 bytes reserved)
-// The size is rounded up to 16 bytes so per-row slices of a workgroup stay aligned.
-struct RowLayout {
-    int dm, doff, ft, vals, av, tlen, t0, blen, b0, lidx, lcnt, bytes;
-};
-
-// Rows of B at least this long (LONG_TILES for the tile OR) are walked by a whole wave:
-// with_long = the longest row of B reaches LONG_TILES, so the kernels list such entries.
+// A B row with at least this many elements left in a window is walked by a whole wave (rows
+// wider than LDS without an index of B).
 constexpr int LONG_SEG = 256;
-constexpr int LONG_TILES = 128;
 
-HSMU_HD inline RowLayout row_layout(int numeric, int S, int n, int nA, int tp, bool with_long)
+// ---- rows that share a wave ------------------------------------------------------------------
+//
+// G = 8, 16 or 32 lanes per row, each with SMALL_U pairs of elements of its B rows (a pair
+// of an entry's odd last element is half empty) and at most one entry of A:
+//   coarse 8[...]   per 32 words (of 32 columns) of the span: which are marked, those before
+//   fine   8[F]     per marked word, F <= min(p, words): its columns, slots before
+//   rec    16[nA]   entries with elements: first less STREAM_V times the first pair, end, a_ij
+//   vals   f64[n]   numeric: accumulators
+//   cols   i32[n]   numeric: columns
+//   ends   u32[U]   a bit per pair of each step of G: it ends an entry
+constexpr int SMALL_U = 4;
+struct SmallLayout {
+    int coarse, fine, rec, vals, cols, ends, ncoarse, nfine, bytes;
+};
+HSMU_HD inline SmallLayout small_layout(bool numeric, int S, int n, int nA, int p)
 {
-    RowLayout L = {};
-    const bool sparse = use_sparse(S, tp);
-    const int E = dir_entries(S, tp);
-    if (E > LAYOUT_CAP || n > LAYOUT_CAP || nA > LAYOUT_CAP) {
-        L.bytes = LAYOUT_NONE;
-        return L;
-    }
+    SmallLayout L = {};
+    L.ncoarse = (2 * S + 31) >> 5;
+    L.nfine = p < 2 * S ? p : 2 * S;
     int o = 0;
-    L.dm = o;
-    o += 8 * E;
-    L.doff = o;
-    if (numeric || sparse)
-        o += 4 * E;
-    L.ft = o;
-    if (numeric && sparse)
-        o += 4 * fine_cap(S, tp);
-    o = (o + 7) & ~7;
+    L.rec = o;
+    o += 16 * nA;
+    L.ends = o;
+    o += 4 * SMALL_U;
+    L.coarse = o;
+    o += 8 * L.ncoarse;
+    L.fine = o;
+    o += 8 * L.nfine;
     L.vals = o;
     if (numeric)
-        o += 8 * (!sparse && use_dense(S, n) ? 64 * S : n);
-    L.av = o;
+        o += 8 * n;
+    L.cols = o;
     if (numeric)
-        o += 8 * nA;
-    L.tlen = o;
-    o += 4 * nA;
-    L.t0 = o;
-    o += 4 * nA;
-    L.blen = o;
-    if (numeric)
-        o += 4 * nA;
-    L.b0 = o;
-    if (numeric)
-        o += 4 * nA;
-    L.lidx = o;
-    if (with_long)
-        o += 4 * nA;
-    o = (o + 15) & ~15;
-    L.lcnt = o;
-    if (with_long)
-        o += 16;
+        o += 4 * n;
     L.bytes = (o + 15) & ~15;
     return L;
+}
+// LDS of such a row on G lanes, if it is one: all its pairs fit
+HSMU_HD inline int small_need(bool numeric, int G, int S, int n, int nA, long long p)
+{
+    return nA <= G && p + nA <= 2 * SMALL_U * G && S <= LAYOUT_CAP ? small_layout(numeric, S, n, nA, (int)p).bytes
+                                                                  : LAYOUT_NONE;
 }
 
 // ---- one row per workgroup (64 lanes or more): the element stream ------------------------
@@ -298,18 +274,18 @@ HSMU_HD inline StreamLayout sym_stream_layout(int G, int S, int nA, int tp)
     return L;
 }
 
-// LDS a row needs in symbolic bin `bin`
-HSMU_HD inline int sym_need(int bin, int S, int nA, int tp, bool with_long)
+constexpr int BIN_SHARED = 3; // bins of rows that share a wave: 8, 16, 32 lanes
+
+// LDS a row with p products needs in symbolic bin `bin`
+HSMU_HD inline int sym_need(int bin, int S, int nA, int tp, long long p)
 {
-    return (8 << bin) >= BLOCK ? sym_stream_layout(8 << bin, S, nA, tp).bytes
-                               : row_layout(0, S, 0, nA, tp, with_long).bytes;
+    return bin >= BIN_SHARED ? sym_stream_layout(8 << bin, S, nA, tp).bytes : small_need(false, 8 << bin, S, 0, nA, p);
 }
 
-// LDS a row with p products needs in numeric bin `bin`
-HSMU_HD inline int num_need(int bin, int S, int n, int nA, int tp, long long p, bool with_long)
+// ... and in numeric bin `bin`
+HSMU_HD inline int num_need(int bin, int S, int n, int nA, int tp, long long p)
 {
-    return (8 << bin) >= BLOCK ? stream_layout(8 << bin, S, n, nA, tp, p).bytes
-                               : row_layout(1, S, n, nA, tp, with_long).bytes;
+    return bin >= BIN_SHARED ? stream_layout(8 << bin, S, n, nA, tp, p).bytes : small_need(true, 8 << bin, S, n, nA, p);
 }
 
 // LDS kept back from the dynamic allocation for the kernels' static __shared__ arrays
@@ -386,7 +362,7 @@ struct Operands {
 // lds_dyn: LDS a row may use (lds_row_max); BIN_GLOBAL rows keep their flat directory in
 // LDS when gws_stride masks fit it (gws is then unused).
 hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int count,
-                           int max_need, const Operands &op, int *rnnz, int tshift, int two_level, int long_rows,
+                           int max_need, const Operands &op, int *rnnz, int tshift, int two_level,
                            unsigned long long *gws, long long gws_stride, int num_cus,
                            int gws_blocks, int lds_dyn, unsigned *queue, hipStream_t s);
 
@@ -470,9 +446,7 @@ size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks);
 // window by window and are not counted.
 hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_dev, int count,
                           int max_need, const Operands &op, const long long *crp, int *Ccol,
-                          void *Cval, int bshift, int tshift, int two_level, int long_rows,
-                          const WideRows &wide,
-                          int *err, int num_cus, unsigned *queue, unsigned long long *lds_bytes,
+                          void *Cval, int bshift, int two_level, const WideRows &wide, int *err, int num_cus, unsigned *queue, unsigned long long *lds_bytes,
                           hipStream_t s);
 
 // A B of fewer than STREAM_V entries (n of them, at least one), copied to arrays of

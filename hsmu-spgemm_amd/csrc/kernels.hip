@@ -217,21 +217,14 @@ __global__ __launch_bounds__(BT_BS) void k_btiles(int64_t K, int64_t N, int64_t 
     const int64_t e0 = (int64_t)b * BT_N;
     const int64_t e1 = e0 + BT_N < nnz ? e0 + BT_N : nnz;
     int bad = 0;
-    // this block's share of the row pointers: in range and nondecreasing; the longest row,
-    // counted only from LONG_TILES on (all the kernels need to know)
+    // this block's share of the row pointers: in range and nondecreasing
     {
         const int64_t v0 = K * b / nb, v1 = K * (b + 1) / nb;
-        int longest = 0;
         for (int64_t r = v0 + t; r < v1; r += BT_BS) {
             const int s = rp[r], e = rp[r + 1];
             if (s < 0 || e < s || (int64_t)e > nnz)
                 bad |= ERR_ROWPTR;
-            else if (e - s >= LONG_TILES)
-                longest = e - s > longest ? e - s : longest;
         }
-        longest = wave_max(longest);
-        if (lane == 0 && longest)
-            atomicMax(&st->max_brow, longest);
     }
     // rows whose first entry is in [e0, e1): [r0, r1); the last block takes the rest
     if (w == 0) {
@@ -380,23 +373,21 @@ hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const
 // same per item at every width from 64 lanes, and a start and an end per row that narrow
 // groups spread over more rows, so both phases give a lane 32 items by default (symbolic
 // stage at 4 / 16 / 32 tiles per lane: R-MAT squares of scale 16 746 / 476 / 439 us and of
-// scale 18 6.67 / 4.28 / 3.52 ms, banded rows of 100 tiles 116 / 72 / 66 us).  Symbolic rows that share a wave walk their entries one after the other, in step
-// with the longest of them: beyond 16 tiles per lane their own wave is faster.  16 waves
-// per CU, where LDS limits the workgroups, take 17.8 ms on the square of scale 18 against
-// 19.2 ms with 8; 24 slow a banded square by 4%.
-constexpr int SHARED_PER_LANE = 16;
+// scale 18 6.67 / 4.28 / 3.52 ms, banded rows of 100 tiles 116 / 72 / 66 us).  Rows whose
+// elements fit the registers of 8, 16 or 32 lanes share a wave.  16 waves per CU, where LDS
+// limits the workgroups, take 17.8 ms on the square of scale 18 against 19.2 ms with 8; 24
+// slow a banded square by 4%.
 template <typename Need>
-DEVI int choose_bin(int numeric, long long work, Need need, const BinParams &bp)
+DEVI int choose_bin(long long work, Need need, const BinParams &bp)
 {
     if (bp.force_global)
         return BIN_GLOBAL;
-    const int shared = !numeric && bp.per_lane > SHARED_PER_LANE ? SHARED_PER_LANE : bp.per_lane;
     int b = 0;
-    while (b < NLDS - 1 && (8LL << b) * ((8 << b) < BLOCK ? shared : bp.per_lane) < work)
+    while (b < NLDS - 1 && (8LL << b) * bp.per_lane < work)
         ++b;
     // the budget limits only workgroups that pack several rows: a one-row workgroup needs
     // the row's LDS whatever its width
-    while ((8 << b) < BLOCK) {
+    while (b < BIN_SHARED) {
         const int nd = need(b);
         if (nd <= bp.lds_row_max && nd * (BLOCK >> (b + 3)) <= bp.lds_block_budget)
             break;
@@ -405,7 +396,7 @@ DEVI int choose_bin(int numeric, long long work, Need need, const BinParams &bp)
     // a one-row workgroup's LDS decides how many fit a CU: widen the row's group until
     // those workgroups hold min_waves waves, to hide the latency of the gathers from B
     int nd = need(b);
-    while (b < NLDS - 1 && (8 << b) >= BLOCK) {
+    while (b < NLDS - 1) {
         const int waves = (8 << b) / 64, wgs = (bp.min_waves + waves - 1) / waves;
         if ((long long)nd * wgs <= bp.lds_cu)
             break;
@@ -454,7 +445,7 @@ struct BinPlace {
 };
 
 // One row per lane of a wave (every lane of the wave calls it; r.prod == 0: no row).
-DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, bool with_long, const BinParams &bp, DevStats *st)
+DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams &bp, DevStats *st)
 {
     BinPlace at;
     int sp = 0;
@@ -464,20 +455,24 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, bool with_long,
     if (r.prod > 0) {
         if (numeric) {
             work = r.prod;
-            auto nd = [&](int bin) { return num_need(bin, r.S, r.nc, r.nA, r.tp, r.prod, with_long); };
-            at.b = choose_bin(numeric, work, nd, bp);
+            auto nd = [&](int bin) { return num_need(bin, r.S, r.nc, r.nA, r.tp, r.prod); };
+            at.b = choose_bin(work, nd, bp);
             need = nd(at.b);
         } else {
             work = r.tp;
-            auto nd = [&](int bin) { return sym_need(bin, r.S, r.nA, r.tp, with_long); };
-            at.b = choose_bin(numeric, work, nd, bp);
-            need = nd(at.b);
-            // the numeric need with nnz(C_i) <= min(products, 64 * span)
+            // the numeric need with nnz(C_i) <= min(products, 64 * span): a row that may be wide
+            // there keeps a directory, which rows that share a wave do not make
             const long long nub = r.prod < 64LL * r.S ? r.prod : 64LL * r.S;
-            wide = num_need(NLDS - 1, r.S, (int)(nub < INT_MAX ? nub : INT_MAX), r.nA, r.tp, r.prod, with_long) > bp.lds_row_max;
+            const int most = bp.lds_row_max < WINDOW_ROW_MIN ? bp.lds_row_max : WINDOW_ROW_MIN;
+            wide = num_need(NLDS - 1, r.S, (int)(nub < INT_MAX ? nub : INT_MAX), r.nA, r.tp, r.prod) > most;
+            auto nd = [&](int bin) {
+                return wide && bin < BIN_SHARED ? LAYOUT_NONE : sym_need(bin, r.S, r.nA, r.tp, r.prod);
+            };
+            at.b = choose_bin(work, nd, bp);
+            need = nd(at.b);
             // directory entries kept for the numeric phase: the row's form in an LDS bin, the
             // flat span for rows the symbolic phase handles in global memory
-            E = at.b < BIN_GLOBAL ? dir_entries(r.S, r.tp) : r.S;
+            E = at.b < BIN_SHARED ? 0 : at.b < BIN_GLOBAL ? dir_entries(r.S, r.tp) : r.S;
         }
         sp = use_sparse(r.S, r.tp) ? 1 : 0;
     }
@@ -785,7 +780,6 @@ __global__ __launch_bounds__(RI_BS) void k_row_info(int64_t M, int64_t K, int64_
     if (bad)
         atomicOr(&st->err, bad);
     // the rows' values, and their bins
-    const bool with_long = st->max_brow >= LONG_TILES;
     BinPlace at[ROWS_MAX / RI_BS];
 #pragma unroll
     for (int u = 0; u < ROWS_MAX / RI_BS; ++u) {
@@ -807,7 +801,7 @@ __global__ __launch_bounds__(RI_BS) void k_row_info(int64_t M, int64_t K, int64_
             if (r.prod == 0)
                 rnnz[i] = 0;
         }
-        at[u] = bin_row(B, 0, r, with_long, bp, st);
+        at[u] = bin_row(B, 0, r, bp, st);
     }
     __syncthreads();
     bin_reserve(B, 0, st, sums);
@@ -895,7 +889,6 @@ __global__ __launch_bounds__(RP_BS) void k_rowptr_bin(int64_t M, const int *__re
         if (t == 0)
             s_pre = before;
     }
-    const bool with_long = st->max_brow >= LONG_TILES;
     BinRow r = {0, 0, 0, 0, 0};
     if (i < M) {
         r.prod = rprod[i];
@@ -904,7 +897,7 @@ __global__ __launch_bounds__(RP_BS) void k_rowptr_bin(int64_t M, const int *__re
         r.nA = Arp[i + 1] - Arp[i];
         r.tp = rtp[i];
     }
-    const BinPlace at = bin_row(B, 1, r, with_long, bp, st);
+    const BinPlace at = bin_row(B, 1, r, bp, st);
     __syncthreads();
     if (i < M) {
         const u64 at0 = s_pre + pre, end = at0 + (u64)(unsigned)nc;
@@ -1210,8 +1203,7 @@ __global__ void k_plan_check(DevStats *st, const DevStats *expect, int stage)
         same = same && a.count[k] == b.count[k] && a.max_need[k] == b.max_need[k] && a.max_span[k] == b.max_span[k] &&
                a.nsparse[k] == b.nsparse[k] && a.max_na[k] == b.max_na[k];
     if (stage == 0)
-        same = same && st->dir_total == expect->dir_total && st->ntiles_b == expect->ntiles_b &&
-               st->max_brow == expect->max_brow;
+        same = same && st->dir_total == expect->dir_total && st->ntiles_b == expect->ntiles_b;
     else
         same = same && st->nnz_c == expect->nnz_c && st->wide_items == expect->wide_items;
     if (!same)

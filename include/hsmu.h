@@ -115,16 +115,16 @@ typedef struct hsmu_opts {
     int32_t lds_block_budget; /* LDS bytes per workgroup for bins that pack several rows
                                  into one workgroup (one wave); 0 = default (8 KiB) */
     int32_t products_per_lane;/* numeric work per lane that sets a row's lane count; 0 = 32 */
-    int32_t tiles_per_lane;   /* symbolic work per lane that sets a row's lane count (rows that
-                                 share a wave: at most 16); 0 = 32 */
+    int32_t tiles_per_lane;   /* symbolic work per lane that sets a row's lane count; 0 = 32 */
     int32_t timing;           /* hipEvents into hsmu_stats (each costs the device a few us):
                                  1 = per stage and per numeric bin (the default), 2 = per
                                  numeric bin only, 0 = none (stage and bin times read 0) */
-    int32_t b_lanes;          /* lanes that walk one row of B in the numeric phase, for rows that
-                                 share a workgroup (power of two, 1..64); 0 = a quarter of the
-                                 mean row length of B */
-    int32_t t_lanes;          /* lanes that walk one row of B's tiles in the tile OR (power
-                                 of two, 1..64); 0 = from the mean tiles per row of B */
+    int32_t b_lanes;          /* lanes that walk one row of B for rows wider than LDS that are
+                                 not cut into windows (power of two, 1..64); 0 = a quarter of
+                                 the mean row length of B */
+    int32_t t_lanes;          /* lanes that walk one row of B's tiles in the tile OR of rows
+                                 wider than LDS (power of two, 1..64); 0 = from the mean tiles
+                                 per row of B */
     int32_t rebuild_dirs;     /* 1: the numeric phase rebuilds each row's tile directory
                                  instead of reusing the one the symbolic phase kept */
     int32_t persistent;       /* 1: the LDS row kernels run as persistent workgroups (as
