@@ -481,15 +481,16 @@ DEVI void stream_or(const Stream<G> &st, long long w0, const Operands &op, u64 *
 // Against staging the A entries in LDS and walking B's tiles twice for the directory and
 // its rows a third time for the products, a lane or two per row of B (512 Laplacians of
 // 7.5 M rows; that kernel spent 52% of its time in vector instructions, 62% in the L1 and
-// 39% in LDS, two thirds of it bank conflicts): numeric 2,860 -> 1,850 us,
-// symbolic 1,044 -> 1,007 us, the call 5.74 -> 4.70 ms; a 47^3 stencil 178 -> 150 us, a random
-// product of ragged rows 261 -> 207 us. Now bound by vector instructions (symbolic 66% of the
-// time, numeric 46%).
+// 39% in LDS, two thirds of it bank conflicts): numeric 2,860 -> 1,670 us, symbolic 1,044
+// -> 880 us, the call 5.74 -> 4.41 ms; a 47^3 stencil 178 -> 147 us, a random product of
+// ragged rows 261 -> 197 us.  Now bound by vector instructions (about half of the time) and
+// the chain of loads, row to entries to B.  5 waves per SIMD (102 registers): at 4 the
+// batch's numeric phase takes 1,760 us, at 6 it spills (3,040 us).
 struct SmallNone { // symbolic: no values
     typedef float V;
 };
 template <int G, typename P>
-__global__ __launch_bounds__(BLOCK) void k_small_rows(const int *__restrict__ rows, const int *__restrict__ count_p,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_small_rows(const int *__restrict__ rows, const int *__restrict__ count_p,
                                                       int slice_bytes, Operands op, int *__restrict__ rnnz,
                                                       const long long *__restrict__ crp, int *__restrict__ Ccol,
                                                       typename P::V *__restrict__ Cval, int *err, unsigned *queue)
@@ -540,16 +541,10 @@ __global__ __launch_bounds__(BLOCK) void k_small_rows(const int *__restrict__ ro
             if constexpr (NUM)
                 a = (u64)__double_as_longlong((double)Aval[a0 + l]);
         }
-        const int CW = L.ncoarse, FW = L.nfine;
-        for (int q = l; q < CW; q += G)
-            coarse[q] = make_uint2(0, 0);
-        for (int q = l; q < FW; q += G)
-            fine[q] = make_uint2(0, 0);
-        if constexpr (NUM)
-            for (int q = l; q < n; q += G)
-                vals[q] = 0.0;
-        if (l < U)
-            ends[l] = 0;
+        // (the last 16 bytes may reach into cols, which is written later, or past the layout's
+        // end, which is a multiple of 16)
+        for (int q = L.ends + 16 * l; q < (NUM ? L.cols : L.vals); q += 16 * G)
+            *(uint4 *)(slice + q) = make_uint4(0, 0, 0, 0);
         // its pairs among the row's
         const unsigned cnt = (unsigned)(len + 1) >> 1;
         unsigned tot;
@@ -607,20 +602,28 @@ __global__ __launch_bounds__(BLOCK) void k_small_rows(const int *__restrict__ ro
             }
         }
         __syncthreads();
-        // exclusive prefix of n words' bits in their second halves; the sum
+        // exclusive prefix of the words' bits in their second halves, four words a lane; the sum
         auto prefix = [&](uint2 *m, int nw) {
             unsigned sum = 0;
-            for (int q0 = 0; __any(q0 < nw); q0 += G) {
-                const int q = q0 + l;
+            for (int q0 = 0; __any(q0 < nw); q0 += 4 * G) {
+                const int q = q0 + 4 * l;
+                uint4 a = make_uint4(0, 0, 0, 0), b = a;
+                if (q < nw) {
+                    a = *(uint4 *)(m + q);
+                    b = *(uint4 *)(m + q + 2);
+                }
+                const unsigned k0 = __popc(a.x), k1 = k0 + __popc(a.z), k2 = k1 + __popc(b.x);
                 unsigned t;
-                const unsigned x = group_excl_scan<G, unsigned>(q < nw ? __popc(m[q].x) : 0u, nullptr, t);
-                if (q < nw)
-                    m[q].y = sum + x;
+                const unsigned x = sum + group_excl_scan<G, unsigned>(k2 + __popc(b.z), nullptr, t);
+                if (q < nw) {
+                    *(uint4 *)(m + q) = make_uint4(a.x, x, a.z, x + k0);
+                    *(uint4 *)(m + q + 2) = make_uint4(b.x, x + k1, b.z, x + k2);
+                }
                 sum += t;
             }
             return sum;
         };
-        const int nf = (int)prefix(coarse, CW);
+        const int nf = (int)prefix(coarse, L.ncoarse);
         __syncthreads();
         // mark the columns
         unsigned f0[U], f1[U];
@@ -642,12 +645,15 @@ __global__ __launch_bounds__(BLOCK) void k_small_rows(const int *__restrict__ ro
             }
         }
         __syncthreads();
-        const int nnz = (int)prefix(fine, nf);
         if constexpr (!NUM) {
+            unsigned k = 0;
+            for (int q = l; q < nf; q += G)
+                k += __popc(fine[q].x);
+            k = group_sum<G>(k);
             if (row >= 0 && l == 0)
-                rnnz[row] = nnz;
+                rnnz[row] = (int)k;
         } else {
-            const bool ok = nnz == n;
+            const bool ok = (int)prefix(fine, nf) == n;
             if (row >= 0 && !ok && l == 0)
                 raise_internal(err);
             __syncthreads();
@@ -1836,6 +1842,9 @@ template <int G> static int row_slice(int need)
     return odd * (BLOCK / G) <= 32 * 1024 ? odd : (need + 15) & ~15;
 }
 
+// Waves per CU of a launch: a few times what is resident, so that a wave's start is paid for
+// several groups of rows and the last ones to end are short.
+constexpr int SMALL_WAVES = 128;
 template <int G, typename P>
 static void small_g(const int *rows, const int *count_dev, int count, int max_need, const Operands &op, int *rnnz,
                     const long long *crp, int *Ccol, void *Cval, int *err, int num_cus, unsigned *queue,
@@ -1844,7 +1853,9 @@ static void small_g(const int *rows, const int *count_dev, int count, int max_ne
     constexpr int RPB = BLOCK / G;
     const int slice = row_slice<G>(max_need);
     const size_t lds = (size_t)slice * RPB;
-    const int64_t blocks = row_grid(k_small_rows<G, P>, BLOCK, lds, ((int64_t)count + RPB - 1) / RPB, num_cus, queue);
+    int64_t blocks = row_grid(k_small_rows<G, P>, BLOCK, lds, ((int64_t)count + RPB - 1) / RPB, num_cus, queue);
+    if (blocks > (int64_t)SMALL_WAVES * num_cus)
+        blocks = (int64_t)SMALL_WAVES * num_cus;
     *lds_bytes += (unsigned long long)blocks * lds;
     hipLaunchKernelGGL((k_small_rows<G, P>), dim3((unsigned)blocks), dim3(BLOCK), lds, s, rows, count_dev, slice, op,
                        rnnz, crp, Ccol, (typename P::V *)Cval, err, queue);

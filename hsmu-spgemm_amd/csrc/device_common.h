@@ -100,9 +100,22 @@ DEVI int wave_max(int v)
 // Map the hardware block index so that each XCD (blocks are dealt round-robin over the
 // nx XCDs of the device: 8 on an MI355X) works on a contiguous range of logical blocks:
 // neighbouring rows, which share rows of B, then share one XCD's L2.
+// (a division costs 20 vector instructions: nx is a power of two on full devices)
 DEVI int xcd_block(int b, int n, int nx)
 {
-    const int x = b % nx, q = b / nx, per = n / nx, rem = n % nx;
+    int x, q, per, rem;
+    if ((nx & (nx - 1)) == 0) {
+        const int sh = __builtin_ctz(nx);
+        x = b & (nx - 1);
+        q = b >> sh;
+        per = n >> sh;
+        rem = n & (nx - 1);
+    } else {
+        x = b % nx;
+        q = b / nx;
+        per = n / nx;
+        rem = n % nx;
+    }
     return x * per + (x < rem ? x : rem) + q;
 }
 
@@ -147,12 +160,13 @@ struct GroupWalk {
     int *s; // two ints of LDS
 
     DEVI GroupWalk(unsigned *queue, int ngroups, int *lds2, int nxcd)
-        : q(queue), n(ngroups), nx(nxcd), xq(blockIdx.x % nxcd), s(lds2)
+        : q(queue), n(ngroups), chunk(1), nx(nxcd), xq(0), s(lds2)
     {
-        // chunks of about an eighth of a workgroup's share of its XCD's range
-        const long long per = (long long)ngroups / ((long long)gridDim.x * 8);
-        chunk = per > 1 ? (int)per : 1;
         if (q) {
+            // chunks of about an eighth of a workgroup's share of its XCD's range
+            const long long per = (long long)ngroups / ((long long)gridDim.x * 8);
+            chunk = per > 1 ? (int)per : 1;
+            xq = blockIdx.x % nxcd;
             pull_chunk(q, n, chunk, nx, xq, s);
             grp = s[0];
             end = s[1];

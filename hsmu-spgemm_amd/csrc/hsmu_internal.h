@@ -146,30 +146,31 @@ constexpr int LONG_SEG = 256;
 //
 // G = 8, 16 or 32 lanes per row, each with SMALL_U pairs of elements of its B rows (a pair
 // of an entry's odd last element is half empty) and at most one entry of A:
+//   rec    16[nA]   entries with elements: first less STREAM_V times the first pair, end, a_ij
+//   ends   u32[U]   a bit per pair of each step of G: it ends an entry
 //   coarse 8[...]   per 32 words (of 32 columns) of the span: which are marked, those before
 //   fine   8[F]     per marked word, F <= min(p, words): its columns, slots before
-//   rec    16[nA]   entries with elements: first less STREAM_V times the first pair, end, a_ij
 //   vals   f64[n]   numeric: accumulators
 //   cols   i32[n]   numeric: columns
-//   ends   u32[U]   a bit per pair of each step of G: it ends an entry
+// (from ends to vals zeroed together, 16 bytes at a time; coarse and fine in fours)
 constexpr int SMALL_U = 4;
 struct SmallLayout {
-    int coarse, fine, rec, vals, cols, ends, ncoarse, nfine, bytes;
+    int rec, ends, coarse, fine, vals, cols, ncoarse, bytes;
 };
 HSMU_HD inline SmallLayout small_layout(bool numeric, int S, int n, int nA, int p)
 {
     SmallLayout L = {};
     L.ncoarse = (2 * S + 31) >> 5;
-    L.nfine = p < 2 * S ? p : 2 * S;
+    const int f = p < 2 * S ? p : 2 * S;
     int o = 0;
     L.rec = o;
     o += 16 * nA;
     L.ends = o;
     o += 4 * SMALL_U;
     L.coarse = o;
-    o += 8 * L.ncoarse;
+    o += 8 * ((L.ncoarse + 3) & ~3);
     L.fine = o;
-    o += 8 * L.nfine;
+    o += 8 * ((f + 3) & ~3);
     L.vals = o;
     if (numeric)
         o += 8 * n;
