@@ -736,7 +736,23 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
 
     // ---- 1. B -> tiles ----
     unsigned long long *words = chain_words(dw);
-    HIP_TRY(launch_btiles(K, N, P.nnzB, P.Brp, P.Bcol, tptr, tcol, tmask, brow, words, &dw->ticket[0], dst, s));
+    // Rows that share a wave do without B's tiles: where B's rows are short enough for all of
+    // C's to be such rows, only the rows' records are made here, and the tiles when some row
+    // does want them.
+    bool tiled = P.nnzB > 8 * K;
+    auto make_tiles = [&](const BinStats &bins) -> hipError_t {
+        int wanted = 0; // rows outside the bins that share waves
+        for (int b = BIN_SHARED; b < NBINS; ++b)
+            wanted |= bins.count[b];
+        if (tiled || !wanted)
+            return hipSuccess;
+        tiled = true;
+        return launch_btiles(K, N, P.nnzB, P.Brp, P.Bcol, tptr, tcol, tmask, nullptr, words, &dw->ticket[0], dst, s);
+    };
+    if (tiled)
+        HIP_TRY(launch_btiles(K, N, P.nnzB, P.Brp, P.Bcol, tptr, tcol, tmask, brow, words, &dw->ticket[0], dst, s));
+    else
+        HIP_TRY(launch_brows(K, N, P.nnzB, P.Brp, P.Bcol, brow, dst, c->num_cus, s));
     HIP_TRY(mark(c->ev[EV_CONV]));
 
     // ---- 2. row analysis + symbolic binning ----
@@ -856,6 +872,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     }
 
     // ---- 3. symbolic ----
+    HIP_TRY(make_tiles(h1.sym));
     for (int b = 0; b < NBINS; ++b) {
         const int cnt = h1.sym.count[b];
         if (cnt <= 0)
@@ -947,6 +964,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     HIP_TRY(mark(c->ev[EV_ALLOC]));
 
     // ---- 5. numeric ----
+    HIP_TRY(make_tiles(h2.num));
     if (!cap)
         c->host->err = 0;
     int *errp = cap ? &dst->err : &c->host->err;

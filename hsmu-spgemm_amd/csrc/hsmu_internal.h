@@ -301,6 +301,9 @@ hipError_t launch_fill_zero(void *p, size_t bytes, hipStream_t s);
 struct alignas(16) BRow {
     int len, ntiles, first, last;
 };
+// The records alone (and the number of tiles), for a B whose tiles may not be wanted.
+hipError_t launch_brows(int64_t K, int64_t N, int64_t nnz, const int *rp, const int *col, BRow *brow, DevStats *st,
+                        int num_cus, hipStream_t s);
 // B -> tiles: tptr (K + 1), tcol and tmask (room for nnz), brow (K, may be null).  words:
 // btiles_blocks(nnz) zeroed words, *ticket = 0.
 int64_t btiles_blocks(int64_t nnz);

@@ -362,6 +362,148 @@ hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const
     return hipGetLastError();
 }
 
+// ---- B's rows without their tiles -----------------------------------------------------------
+//
+// The records of B's rows (length, tiles, first and last tile) and the checks of k_btiles,
+// for a B of short rows: rows of C that share a wave read B itself, so the tiles are made
+// only once a row turns out to want them.  8 lanes per row, BR_U rows at a time; rows of
+// more than BR_LONG entries a wave each, of more than BR_BLOCK the block.  Bound by the
+// chain row pointer -> columns; 45 M entries in 7.5 M rows take 180 us, their tiles 477.
+constexpr int BR_BS = 256;
+constexpr int BR_G = 8;
+constexpr int BR_U = 4;
+constexpr int BR_ROWS = 256; // rows of a block at a time
+constexpr int BR_LONG = 64;
+constexpr int BR_BLOCK = 16384;
+
+__global__ __launch_bounds__(BR_BS) void k_brows(int64_t K, int64_t N, int64_t nnz, const int *__restrict__ rp,
+                                                 const int *__restrict__ col, BRow *__restrict__ brow, DevStats *st)
+{
+    __shared__ int s_long, s_tiles, s_part;
+    __shared__ unsigned short s_list[BR_ROWS];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, g = t / BR_G, l = t & (BR_G - 1);
+    int bad = 0, total = 0; // tiles counted by this thread
+    // entry k of a row from s: is it its tile's first?
+    auto head = [&](int64_t k, int64_t s, int c, int before) {
+        if ((unsigned)c >= (unsigned long long)N)
+            bad |= ERR_BCOL;
+        if (k > s && before > c)
+            bad |= ERR_UNSORTED;
+        return k == s || (before >> 6) != (c >> 6) ? 1 : 0;
+    };
+    auto store = [&](int64_t r, int s, int e, int tiles, int c0, int c1) {
+        brow[r] = e > s ? BRow{e - s, tiles, c0 >> 6, c1 >> 6} : BRow{0, 0, INT_MAX, -1};
+    };
+    if (blockIdx.x == 0) { // entries of no row (row pointers that do not start at 0 or end at nnz)
+        const int64_t a = rp[0] < nnz ? rp[0] : nnz, b = rp[K] > 0 ? rp[K] : 0;
+        for (int64_t k = t; k < a; k += BR_BS)
+            (void)head(k, 0, col[k], k > 0 ? col[k - 1] : 0);
+        for (int64_t k = b + t; k < nnz; k += BR_BS)
+            (void)head(k, 0, col[k], k > 0 ? col[k - 1] : 0);
+    }
+    if (t == 0)
+        s_tiles = 0;
+    for (int64_t i0 = (int64_t)blockIdx.x * BR_ROWS; i0 < K; i0 += (int64_t)gridDim.x * BR_ROWS) {
+        const int n = (int)(K - i0 < BR_ROWS ? K - i0 : BR_ROWS);
+        if (t == 0)
+            s_long = 0;
+        __syncthreads();
+        for (int q0 = g; q0 < n; q0 += BR_U * (BR_BS / BR_G)) {
+            int s[BR_U], e[BR_U], c[BR_U];
+#pragma unroll
+            for (int u = 0; u < BR_U; ++u) {
+                const int q = q0 + u * (BR_BS / BR_G);
+                s[u] = e[u] = 0;
+                if (q < n) {
+                    s[u] = rp[i0 + q];
+                    e[u] = rp[i0 + q + 1];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < BR_U; ++u) {
+                if (s[u] < 0 || e[u] < s[u] || (int64_t)e[u] > nnz) {
+                    bad |= ERR_ROWPTR;
+                    e[u] = s[u] = 0;
+                }
+                c[u] = s[u] + l < e[u] && e[u] - s[u] <= BR_LONG ? col[s[u] + l] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < BR_U; ++u) {
+                const int q = q0 + u * (BR_BS / BR_G);
+                const bool lng = e[u] - s[u] > BR_LONG;
+                const int before = __builtin_amdgcn_update_dpp(0, c[u], 0x138, 0xf, 0xf, false); // wave_shr:1
+                int sum = 0, last = c[u]; // (sorted: the largest)
+                if (!lng) {
+                    if (s[u] + l < e[u])
+                        sum = head(s[u] + l, s[u], c[u], before);
+                    for (int k = s[u] + l + BR_G; k < e[u]; k += BR_G) {
+                        const int cc = col[k];
+                        sum += head(k, s[u], cc, col[k - 1]);
+                        last = cc;
+                    }
+                    total += sum;
+                }
+                sum = group_sum<BR_G>(sum);
+                last = group_max<BR_G>(last);
+                if (l == 0 && q < n) {
+                    if (lng)
+                        s_list[atomicAdd(&s_long, 1)] = (unsigned short)q;
+                    else
+                        store(i0 + q, s[u], e[u], sum, c[u], last);
+                }
+            }
+        }
+        __syncthreads();
+        const int nlong = s_long;
+        for (int i = 0; i < nlong; ++i) {
+            const int q = s_list[i];
+            const int s = rp[i0 + q], e = rp[i0 + q + 1];
+            const bool block = e - s > BR_BLOCK; // (the same in every thread)
+            if (!block && (i & (BR_BS / 64 - 1)) != w)
+                continue;
+            int sum = 0;
+#pragma unroll 4
+            for (int64_t k = (int64_t)s + (block ? t : lane); k < e; k += block ? BR_BS : 64)
+                sum += head(k, s, col[k], k > s ? col[k - 1] : 0);
+            total += sum;
+            sum = wave_sum(sum);
+            if (!block) {
+                if (lane == 0)
+                    store(i0 + q, s, e, sum, col[s], col[e - 1]);
+                continue;
+            }
+            if (t == 0)
+                s_part = 0;
+            __syncthreads();
+            if (lane == 0)
+                atomicAdd(&s_part, sum);
+            __syncthreads();
+            if (t == 0)
+                store(i0 + q, s, e, s_part, col[s], col[e - 1]);
+            __syncthreads();
+        }
+        __syncthreads();
+    }
+    if (bad)
+        atomicOr(&st->err, bad);
+    total = wave_sum(total);
+    __syncthreads();
+    if (lane == 0)
+        atomicAdd(&s_tiles, total);
+    __syncthreads();
+    if (t == 0 && s_tiles)
+        atomicAdd(&st->ntiles_b, s_tiles);
+}
+
+hipError_t launch_brows(int64_t K, int64_t N, int64_t nnz, const int *rp, const int *col, BRow *brow, DevStats *st,
+                        int num_cus, hipStream_t s)
+{
+    const int64_t chunks = (K + BR_ROWS - 1) / BR_ROWS, most = 32 * (int64_t)num_cus;
+    hipLaunchKernelGGL(k_brows, dim3((unsigned)(chunks < 1 ? 1 : chunks < most ? chunks : most)), dim3(BR_BS), 0, s, K, N,
+                       nnz, rp, col, brow, st);
+    return hipGetLastError();
+}
+
 // ---- binning -----------------------------------------------------------------------------
 
 // Bin of one row: lanes from work (per_lane items per lane, 8..1024 lanes), then fewer

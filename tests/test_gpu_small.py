@@ -49,3 +49,27 @@ def test_small_rows(ctx, N, opts, fp32):
     bound = 2.0 ** -23 * np.abs(ref.val) + 1e-10 * ref.absval if fp32 else 1e-12 * ref.absval
     assert np.all(np.abs(C.val.astype(np.float64) - ref.val) <= bound)
     assert min(st["num_bin_rows"][:3]) > 0 or N == 1 << 20
+
+
+@pytest.mark.parametrize("opts", [dict(), dict(rebuild_dirs=1), dict(force_global=1), dict(lds_block_budget=64)])
+def test_rows_of_short_b(ctx, opts):
+    """A B of short rows on average, whose tiles are made when a row of C wants them: rows of
+    one lane group, a wave (over 64 entries) and a block (over 16,384) in B; rows of C that
+    share waves, alone and beside rows that do not."""
+    rng = np.random.default_rng(17)
+    print(f"[gpu-case] short B {opts}", flush=True)
+    N, K = 30000, 6000
+    lens = rng.integers(0, 9, K)
+    lens[[5, 255, 256, 4000]] = [65, 64, 16385, 300]
+    lens[-1] = 7
+    B = csr([rng.choice(N, n, replace=False) for n in lens], N, rng)
+    assert len(B.col) <= 8 * K
+    small = [rng.choice(np.arange(300, 3000), n, replace=False) for n in rng.integers(0, 8, 700)] + [[K - 1]]
+    for rows in (small, small + [[5], [256, 5], np.arange(0, K, 7), [255, 4000]]):
+        A = csr(rows, K, rng)
+        C, st = ctx.spgemm(A, B, **opts)
+        ref = oracle.spgemm(A, B)
+        assert np.array_equal(np.asarray(C.rowptr, np.int64), ref.rowptr) and np.array_equal(C.col, ref.col)
+        assert np.all(np.abs(C.val - ref.val) <= 1e-12 * ref.absval)
+        tiles = sum(len(np.unique(np.asarray(B.col[B.rowptr[j]:B.rowptr[j + 1]]) >> 6)) for j in range(K))
+        assert st["tiles_b"] == tiles
