@@ -728,9 +728,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     int *binrows = ar.get<int>((size_t)NBINS * (size_t)M);
     long long *rdir = ar.get<long long>((size_t)M);
     BRow *brow = ar.get<BRow>((size_t)(K > 0 ? K : 1));
-    const int64_t nsums = std::max(row_info_blocks(M, P.nnzA, c->num_cus), rowptr_blocks(M));
-    BinSum *sums = ar.get<BinSum>((size_t)nsums * NBINS);
-    if (!sums || !tptr || !tcol || !tmask || !rprod || !rtp || !rmin || !rmax || !rnnz || !binrows || !rdir ||
+    if (!tptr || !tcol || !tmask || !rprod || !rtp || !rmin || !rmax || !rnnz || !binrows || !rdir ||
         !brow)
         return fail(HSMU_ERR_NOMEM, "workspace allocation");
 
@@ -772,7 +770,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     bp.lds_cu = lds_dyn;
     bp.min_waves = opts.min_waves > 0 ? opts.min_waves : 16;
     HIP_TRY(launch_row_info(M, K, P.nnzA, P.Arp, P.Acol, brow, tptr, rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, dst,
-                            sums, &dw->done[0], host, c->num_cus, s));
+                            dw->sums[0], &dw->done[0], host, c->num_cus, s));
     HIP_TRY(mark(c->ev[EV_ANALYSIS]));
     DevStats h1;
     rc = checkpoint(c, mode, dst, 0, h1);
@@ -934,7 +932,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
                     wide_list_bytes(c->num_cus)))
         bp.lds_row_max = WINDOW_ROW_MIN;
     HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp, rp64 || batch ? nullptr : (int *)Crp, bp,
-                              binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, sums, &dw->done[1], host, s));
+                              binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1], host, s));
     HIP_TRY(mark(c->ev[EV_SYMBOLIC]));
     DevStats h2;
     rc = checkpoint(c, mode, dst, 1, h2);

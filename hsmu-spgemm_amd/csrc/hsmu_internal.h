@@ -72,17 +72,19 @@ struct DevStats {
     unsigned queue[2][NBINS][MAX_XCDS];
 };
 
-// One block's part of a binning's sums and maxima, for one bin.
+// A part of a binning's sums and maxima, for one bin: block b of the binning adds to part
+// b % BIN_PARTS.
 struct BinSum {
     unsigned long long work, nnz_c, nnz_a;
-    unsigned long long need_span; // max_need | max_span << 32
-    unsigned long long na_sparse; // max_na | nsparse << 32
+    unsigned need, span, na_max, nsparse;
 };
+constexpr int BIN_PARTS = 16;
 
 // Everything on the device that a call needs zeroed: the counters, the blocks done and the
 // places taken of each binning or scan, and (behind it) the words of the two chained scans.
 struct DevWork {
     DevStats st;
+    BinSum sums[2][BIN_PARTS * NBINS]; // symbolic, numeric
     unsigned done[2], ticket[2];
     // followed by btiles_blocks(nnz(B)) + rowptr_blocks(M) 64-bit words
 };
@@ -314,13 +316,11 @@ hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const
 // Per row of A: products, tile-products, tile span (from the BRow of each B_j it names), and
 // the rows' symbolic bins: binrows, and each LDS-bin row's directory range: rdir[i] = offset
 // (span entries), -1 for rows not in an LDS bin; st->dir_total = entries reserved.  host (may
-// be null): the counters are copied there at the end (device-accessible host memory).  sums:
-// NBINS per block (row_info_blocks).
+// be null): the counters are copied there at the end (device-accessible host memory).
 hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, const int *Acol,
                            const BRow *brow, const int *tptr, long long *rprod, int *rtp, int *rmin,
                            int *rmax, int *rnnz, BinParams bp, int *binrows, long long *rdir, DevStats *st,
                            BinSum *sums, unsigned *done, DevStats *host, int num_cus, hipStream_t s);
-int64_t row_info_blocks(int64_t M, int64_t nnzA, int num_cus);
 
 // C's row pointers (crp, and out32 when given: M + 1 each) from rnnz, and the numeric bins.
 // words: rowptr_blocks(M) zeroed words, *ticket = 0.  sums, host as above (rowptr_blocks).

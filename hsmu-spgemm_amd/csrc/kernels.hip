@@ -560,8 +560,9 @@ struct BinRow {
 // The blocks of one binning: their counts in LDS, then one global atomic per bin and block
 // for the rows' places (atomics on one address retire one every few nanoseconds
 // device-wide: with one more for each sum and maximum they were the binning's whole time).
-// The sums and maxima go to the block's own BinSum, and the last block to finish adds those
-// up and, given `host`, writes the totals there.
+// The sums and maxima go to one of BIN_PARTS parts, and the last block to finish adds those
+// up and, given `host`, writes the totals there.  (With a part of its own for every block,
+// that last addition kept a batch of 7.5 M rows waiting for 130 us, in each of the phases.)
 struct BinBlock {
     int cnt[NBINS], need[NBINS], span[NBINS], base[NBINS], sparse[NBINS], na_max[NBINS];
     u64 work[NBINS], nc[NBINS], na[NBINS];
@@ -679,12 +680,18 @@ DEVI void bin_reserve(BinBlock &B, int numeric, DevStats *st, BinSum *sums)
     if (t < NBINS) {
         const int c = B.cnt[t];
         B.base[t] = c ? atomicAdd(&bs->count[t], c) : 0;
-        BinSum *s = sums + (size_t)blockIdx.x * NBINS + t;
-        device_store(&s->work, B.work[t]);
-        device_store(&s->nnz_c, B.nc[t]);
-        device_store(&s->nnz_a, B.na[t]);
-        device_store(&s->need_span, (u64)(unsigned)B.need[t] | ((u64)(unsigned)B.span[t] << 32));
-        device_store(&s->na_sparse, (u64)(unsigned)B.na_max[t] | ((u64)(unsigned)B.sparse[t] << 32));
+        if (c && gridDim.x > 1) {
+            BinSum *s = sums + (blockIdx.x % BIN_PARTS) * NBINS + t;
+            atomicAdd(&s->work, B.work[t]);
+            atomicAdd(&s->nnz_a, B.na[t]);
+            if (numeric)
+                atomicAdd(&s->nnz_c, B.nc[t]);
+            atomicMax(&s->need, (unsigned)B.need[t]);
+            atomicMax(&s->span, (unsigned)B.span[t]);
+            atomicMax(&s->na_max, (unsigned)B.na_max[t]);
+            if (B.sparse[t])
+                atomicAdd(&s->nsparse, (unsigned)B.sparse[t]);
+        }
     }
     if (!numeric && t == NBINS)
         B.dir_base = B.dir ? atomicAdd(&st->dir_total, B.dir) : 0;
@@ -709,29 +716,17 @@ DEVI void bin_finish(BinBlock &B, int numeric, DevStats *st, const BinSum *sums,
             return;
         bin_clear(B);
         __syncthreads();
-        const int parts = (int)blockDim.x / NBINS, bin = t % NBINS;
-        if (t / NBINS < parts) {
-            u64 w = 0, nc = 0, na = 0;
-            unsigned need = 0, span = 0, nam = 0, sp = 0;
-#pragma unroll 4
-            for (int q = t / NBINS; q < nblk; q += parts) {
-                const BinSum *s = sums + (size_t)q * NBINS + bin;
-                w += device_load(&s->work);
-                nc += device_load(&s->nnz_c);
-                na += device_load(&s->nnz_a);
-                const u64 x = device_load(&s->need_span), y = device_load(&s->na_sparse);
-                need = (unsigned)x > need ? (unsigned)x : need;
-                span = (unsigned)(x >> 32) > span ? (unsigned)(x >> 32) : span;
-                nam = (unsigned)y > nam ? (unsigned)y : nam;
-                sp += (unsigned)(y >> 32);
-            }
-            atomicAdd(&B.work[bin], w);
-            atomicAdd(&B.nc[bin], nc);
-            atomicAdd(&B.na[bin], na);
-            atomicMax(&B.need[bin], (int)need);
-            atomicMax(&B.span[bin], (int)span);
-            atomicMax(&B.na_max[bin], (int)nam);
-            atomicAdd(&B.sparse[bin], (int)sp);
+        static_assert(BIN_PARTS * NBINS <= 256, "a thread per part and bin");
+        if (t < BIN_PARTS * NBINS) {
+            const int bin = t % NBINS;
+            const BinSum *s = sums + t;
+            atomicAdd(&B.work[bin], device_load(&s->work));
+            atomicAdd(&B.nc[bin], device_load(&s->nnz_c));
+            atomicAdd(&B.na[bin], device_load(&s->nnz_a));
+            atomicMax(&B.need[bin], (int)device_load(&s->need));
+            atomicMax(&B.span[bin], (int)device_load(&s->span));
+            atomicMax(&B.na_max[bin], (int)device_load(&s->na_max));
+            atomicAdd(&B.sparse[bin], (int)device_load(&s->nsparse));
         }
         __syncthreads();
     }
@@ -761,18 +756,23 @@ DEVI void bin_finish(BinBlock &B, int numeric, DevStats *st, const BinSum *sums,
 // [rmin, rmax] of tile columns of row i of C (rows of B are sorted, so each B row's first
 // and last tile bound it); then the symbolic binning of the block's rows.  Reference:
 // k_compute_flop, src/small/mask.cuh:14-51.
-// A group of G lanes per row; a block takes `rows` rows, 256 / G at a time, and bins them
+// A group of G lanes per row; a block takes `rows` rows, a lane group each at a time, and bins them
 // together, so that the binning's atomics are few and hide behind other blocks' gathers.
 // Rows of more than LONG_A entries per lane are listed and left to whole waves, those of
 // more than LONG_WAVE entries to the whole block (at 2,048 entries for every group width,
 // a hub row's 16 lanes kept an R-MAT graph's analysis waiting).
 constexpr int LONG_A = 16;
 constexpr int LONG_WAVE = 4096;
-constexpr int RI_BS = 1024;
-constexpr int ROWS_MAX = 2048; // rows of a block
+// Short rows (G = 8) take blocks of 512 lanes, of which twice as many overlap on a CU, and at
+// least 128 rows each, as more blocks queue at the bins' counters: 7.5 M rows of 6 entries
+// take 464 us with 1,024 lanes and 330 with 512, 16,384 rows 10.8 and, with 64 rows per
+// block, 11.6.  Longer rows gather more per row: an R-MAT graph of scale 18 takes 383 us with
+// 1,024 lanes and 595 with 512.
+constexpr int ri_lanes(int G) { return G == 8 ? 512 : 1024; }
+constexpr int ri_rows_max(int G) { return 2 * ri_lanes(G); } // rows of a block
 
 template <int G>
-__global__ __launch_bounds__(RI_BS) void k_row_info(int64_t M, int64_t K, int64_t nnzA, int rows,
+__global__ __launch_bounds__(ri_lanes(G)) void k_row_info(int64_t M, int64_t K, int64_t nnzA, int rows,
                                                   const int *__restrict__ Arp, const int *__restrict__ Acol,
                                                   const BRow *__restrict__ brow, const int *__restrict__ tptr,
                                                   long long *__restrict__ rprod, int *__restrict__ rtp, int *__restrict__ rmin,
@@ -780,7 +780,7 @@ __global__ __launch_bounds__(RI_BS) void k_row_info(int64_t M, int64_t K, int64_
                                                   int *__restrict__ binrows, long long *__restrict__ rdir,
                                                   DevStats *st, BinSum *sums, unsigned *done, DevStats *host)
 {
-    constexpr int RPB = RI_BS / G, NW = RI_BS / 64;
+    constexpr int RI_BS = ri_lanes(G), ROWS_MAX = ri_rows_max(G), RPB = RI_BS / G, NW = RI_BS / 64;
     __shared__ long long s_prod[ROWS_MAX];
     __shared__ int s_tp[ROWS_MAX], s_mn[ROWS_MAX], s_mx[ROWS_MAX];
     __shared__ BinBlock B;
@@ -969,14 +969,14 @@ static int row_info_lanes(int64_t M, int64_t nnzA)
 // block's LDS holds, for fewer atomics per row.
 static int row_info_rows(int64_t M, int64_t nnzA, int num_cus)
 {
-    const int rpb = RI_BS / row_info_lanes(M, nnzA);
+    const int G = row_info_lanes(M, nnzA), rpb = ri_lanes(G) / G;
     const int64_t full = (int64_t)rpb * 2 * num_cus;
-    int64_t passes = (M + full - 1) / full;
-    passes = passes < 1 ? 1 : (passes > ROWS_MAX / rpb ? ROWS_MAX / rpb : passes);
-    return (int)passes * rpb;
+    const int64_t least = G == 8 ? 2 : 1, most = ri_rows_max(G) / rpb;
+    const int64_t passes = (M + full - 1) / full;
+    return (int)(passes < least ? least : passes > most ? most : passes) * rpb;
 }
 
-int64_t row_info_blocks(int64_t M, int64_t nnzA, int num_cus)
+static int64_t row_info_blocks(int64_t M, int64_t nnzA, int num_cus)
 {
     const int rows = row_info_rows(M, nnzA, num_cus);
     return (M + rows - 1) / rows;
@@ -991,7 +991,7 @@ hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, c
     const unsigned blocks = (unsigned)row_info_blocks(M, nnzA, num_cus);
 #define ROW_INFO(G)                                                                                                    \
     case G:                                                                                                            \
-        hipLaunchKernelGGL((k_row_info<G>), dim3(blocks), dim3(RI_BS), 0, s, M, K, nnzA, rows, Arp, Acol, brow, tptr,  \
+        hipLaunchKernelGGL((k_row_info<G>), dim3(blocks), dim3(ri_lanes(G)), 0, s, M, K, nnzA, rows, Arp, Acol, brow, tptr,  \
                            rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, st, sums, done, host);                     \
         break;
     switch (row_info_lanes(M, nnzA)) {
@@ -1001,9 +1001,15 @@ hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, c
     return hipGetLastError();
 }
 
-// C's row pointers from nnz(C_i) (chained scan) and the numeric binning, a lane per row.  out32 (may be null): the row pointers as int32 too, for the caller.
+// C's row pointers from nnz(C_i) (chained scan) and the numeric binning, T rows per lane.
+// out32 (may be null): the row pointers as int32 too, for the caller.  Each block takes a
+// place, then places in the bins, and waits for the blocks before it, so many rows go two to
+// a lane (7.5 M rows: 196 us with one, 172 with two); up to RP_FEW go one to a lane, on
+// more CUs.
 constexpr int RP_BS = 1024;
+constexpr int RP_FEW = 1 << 19;
 
+template <int T>
 __global__ __launch_bounds__(RP_BS) void k_rowptr_bin(int64_t M, const int *__restrict__ Arp,
                                                     const long long *__restrict__ rprod, const int *__restrict__ rtp,
                                                     const int *__restrict__ rmin, const int *__restrict__ rmax,
@@ -1022,44 +1028,67 @@ __global__ __launch_bounds__(RP_BS) void k_rowptr_bin(int64_t M, const int *__re
         s_b = gridDim.x > 1 ? (int)atomicAdd(ticket, 1u) : 0;
     __syncthreads();
     const int b = uniform(s_b);
-    const int64_t i = (int64_t)b * RP_BS + t;
-    const int nc = i < M ? rnnz[i] : 0;
-    u64 total;
-    const u64 pre = group_excl_scan<RP_BS, u64>((u64)(unsigned)nc, red, total);
+    const int64_t i0 = (int64_t)b * (T * RP_BS) + t;
+    int nc[T];
+    u64 pre[T], total = 0; // entries of the block's rows before this one's
+#pragma unroll
+    for (int u = 0; u < T; ++u)
+        nc[u] = i0 + u * RP_BS < M ? rnnz[i0 + u * RP_BS] : 0;
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+        u64 tot;
+        pre[u] = total + group_excl_scan<RP_BS, u64>((u64)(unsigned)nc[u], red, tot);
+        total += tot;
+    }
     if (t < 64) {
         const u64 before = chain_prefix(words, b, total);
         if (t == 0)
             s_pre = before;
     }
-    BinRow r = {0, 0, 0, 0, 0};
-    if (i < M) {
-        r.prod = rprod[i];
-        r.nc = nc;
-        r.S = rmax[i] - rmin[i] + 1;
-        r.nA = Arp[i + 1] - Arp[i];
-        r.tp = rtp[i];
+    BinPlace at[T];
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+        const int64_t i = i0 + u * RP_BS;
+        BinRow r = {0, 0, 0, 0, 0};
+        if (i < M) {
+            r.prod = rprod[i];
+            r.nc = nc[u];
+            r.S = rmax[i] - rmin[i] + 1;
+            r.nA = Arp[i + 1] - Arp[i];
+            r.tp = rtp[i];
+        }
+        at[u] = bin_row(B, 1, r, bp, st);
     }
-    const BinPlace at = bin_row(B, 1, r, bp, st);
     __syncthreads();
-    if (i < M) {
-        const u64 at0 = s_pre + pre, end = at0 + (u64)(unsigned)nc;
-        crp[i] = (long long)at0;
-        if (out32)
-            out32[i] = (int)at0;
-        if (i == M - 1) {
-            crp[M] = (long long)end;
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+        const int64_t i = i0 + u * RP_BS;
+        if (i < M) {
+            const u64 at0 = s_pre + pre[u], end = at0 + (u64)(unsigned)nc[u];
+            crp[i] = (long long)at0;
             if (out32)
-                out32[M] = (int)end;
-            device_store(&st->nnz_c, (long long)end);
+                out32[i] = (int)at0;
+            if (i == M - 1) {
+                crp[M] = (long long)end;
+                if (out32)
+                    out32[M] = (int)end;
+                device_store(&st->nnz_c, (long long)end);
+            }
         }
     }
     bin_reserve(B, 1, st, sums);
-    if (at.b >= 0)
-        binrows[(int64_t)at.b * M + B.base[at.b] + at.pos] = (int)i;
+#pragma unroll
+    for (int u = 0; u < T; ++u)
+        if (at[u].b >= 0)
+            binrows[(int64_t)at[u].b * M + B.base[at[u].b] + at[u].pos] = (int)(i0 + u * RP_BS);
     bin_finish(B, 1, st, sums, done, host);
 }
 
-int64_t rowptr_blocks(int64_t M) { return (M + RP_BS - 1) / RP_BS; }
+int64_t rowptr_blocks(int64_t M)
+{
+    const int64_t rows = M > RP_FEW ? 2 * RP_BS : RP_BS;
+    return (M + rows - 1) / rows;
+}
 
 hipError_t launch_rowptr_bin(int64_t M, const int *Arp, const long long *rprod, const int *rtp, const int *rmin,
                              const int *rmax, const int *rnnz, long long *crp, int *out32, BinParams bp, int *binrows,
@@ -1068,8 +1097,9 @@ hipError_t launch_rowptr_bin(int64_t M, const int *Arp, const long long *rprod, 
 {
     if (M <= 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_rowptr_bin, dim3((unsigned)rowptr_blocks(M)), dim3(RP_BS), 0, s, M, Arp, rprod, rtp, rmin, rmax,
-                       rnnz, crp, out32, bp, binrows, words, ticket, st, sums, done, host);
+    hipLaunchKernelGGL(M > RP_FEW ? k_rowptr_bin<2> : k_rowptr_bin<1>, dim3((unsigned)rowptr_blocks(M)), dim3(RP_BS), 0,
+                       s, M, Arp, rprod, rtp, rmin, rmax, rnnz, crp, out32, bp, binrows, words, ticket, st, sums, done,
+                       host);
     return hipGetLastError();
 }
 
