@@ -11,6 +11,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
@@ -174,7 +175,7 @@ enum { EV_START, EV_CONV, EV_ANALYSIS, EV_SYMBOLIC, EV_ALLOC, EV_NUMERIC, EV_COU
 // Pinned host memory the device writes: the counters of the last checkpoint, and the
 // numeric kernels' error word.
 struct HostBlock {
-    DevStats st;
+    HostStats stats;
     int err;
 };
 
@@ -183,6 +184,7 @@ struct hsmu_ctx {
     hipStream_t stream = nullptr;
     Pool pool;
     HostBlock *host = nullptr; // pinned; the device writes its counters there
+    unsigned seq = 0;          // number of the last checkpoint
     hipEvent_t ev[EV_COUNT] = {};
     hipEvent_t evb[NBINS][2] = {};
     int num_cus = 0;
@@ -245,7 +247,9 @@ int hsmu_ctx_create(int device, hsmu_ctx **out)
     }
     // every failure from here on releases what was already created
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess &&
-              hipHostMalloc((void **)&c->host, sizeof(HostBlock), hipHostMallocDefault) == hipSuccess;
+              hipHostMalloc((void **)&c->host, sizeof(HostBlock), hipHostMallocCoherent) == hipSuccess;
+    if (ok)
+        *c->host = HostBlock{};
     for (int i = 0; ok && i < EV_COUNT; ++i)
         ok = hipEventCreate(&c->ev[i]) == hipSuccess;
     for (int b = 0; ok && b < NBINS; ++b)
@@ -494,9 +498,9 @@ extern "C" int hsmu_btiles(hsmu_ctx *c, const hsmu_csr *B, hsmu_tiles *T)
     HIP_TRY(launch_fill_zero(dw, work_bytes, c->stream));
     HIP_TRY(launch_btiles(K, B->N, B->nnz, (const int *)B->rowptr, B->col, tptr, tcol, tmask, nullptr, chain_words(dw),
                           &dw->ticket[0], &dw->st, c->stream));
-    HIP_TRY(hipMemcpyAsync(&c->host->st, &dw->st, sizeof(DevStats), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipMemcpyAsync(&c->host->stats.st, &dw->st, sizeof(DevStats), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    rc = device_error_status(c->host->st.err);
+    rc = device_error_status(c->host->stats.st.err);
     if (rc) {
         c->pool.release(tptr);
         c->pool.release(tcol);
@@ -504,7 +508,7 @@ extern "C" int hsmu_btiles(hsmu_ctx *c, const hsmu_csr *B, hsmu_tiles *T)
         return rc;
     }
     T->M = K;
-    T->ntiles = c->host->st.ntiles_b;
+    T->ntiles = c->host->stats.st.ntiles_b;
     T->tptr = tptr;
     T->tcol = tcol;
     T->tmask = (uint64_t *)tmask;
@@ -663,8 +667,19 @@ int checkpoint(hsmu_ctx *c, const RunMode &m, DevStats *dst, int k, DevStats &ou
         out = m.plan->rec[k];
         return HSMU_OK;
     }
-    HIP_TRY(hipStreamSynchronize(s)); // the last kernel has written the counters to the host
-    out = c->host->st;
+    // the binning kernel writes the counters to the host and then the checkpoint's number:
+    // short waits end there, some 5 us before the stream knows that the kernel has; long ones
+    // are the runtime's (as are failures)
+    const volatile unsigned *seq = &c->host->stats.seq;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(100);
+    bool there = *seq == c->seq;
+    while (!there && std::chrono::steady_clock::now() < until)
+        for (int k = 0; k < 32 && !there; ++k)
+            there = *seq == c->seq;
+    if (!there)
+        HIP_TRY(hipStreamSynchronize(s));
+    std::atomic_thread_fence(std::memory_order_acquire);
+    out = c->host->stats.st;
     if (m.plan)
         m.plan->rec[k] = out;
     return device_error_status(out.err);
@@ -714,7 +729,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     auto mark = [&](hipEvent_t e) -> hipError_t { return stage_timing ? hipEventRecord(e, s) : hipSuccess; };
     int rc;
     DevStats *dst = &dw->st;
-    DevStats *host = cap ? nullptr : &c->host->st;
+    HostStats *host = cap ? nullptr : &c->host->stats;
 
     int *tptr = ar.get<int>((size_t)K + 1);
     const size_t ntcap = P.nnzB > STREAM_V ? (size_t)P.nnzB : STREAM_V; // loaded STREAM_V at a time
@@ -770,7 +785,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     bp.lds_cu = lds_dyn;
     bp.min_waves = opts.min_waves > 0 ? opts.min_waves : 16;
     HIP_TRY(launch_row_info(M, K, P.nnzA, P.Arp, P.Acol, brow, tptr, rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, dst,
-                            dw->sums[0], &dw->done[0], host, c->num_cus, s));
+                            dw->sums[0], &dw->done[0], host, ++c->seq, c->num_cus, s));
     HIP_TRY(mark(c->ev[EV_ANALYSIS]));
     DevStats h1;
     rc = checkpoint(c, mode, dst, 0, h1);
@@ -932,7 +947,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
                     wide_list_bytes(c->num_cus)))
         bp.lds_row_max = WINDOW_ROW_MIN;
     HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp, rp64 || batch ? nullptr : (int *)Crp, bp,
-                              binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1], host, s));
+                              binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1], host, ++c->seq, s));
     HIP_TRY(mark(c->ev[EV_SYMBOLIC]));
     DevStats h2;
     rc = checkpoint(c, mode, dst, 1, h2);

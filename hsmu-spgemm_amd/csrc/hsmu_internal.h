@@ -72,6 +72,13 @@ struct DevStats {
     unsigned queue[2][NBINS][MAX_XCDS];
 };
 
+// The counters as a binning hands them to the host (pinned memory): seq, a number of the
+// caller's, follows them.
+struct HostStats {
+    DevStats st;
+    unsigned seq;
+};
+
 // A part of a binning's sums and maxima, for one bin: block b of the binning adds to part
 // b % BIN_PARTS.
 struct BinSum {
@@ -320,7 +327,7 @@ hipError_t launch_btiles(int64_t K, int64_t N, int64_t nnz, const int *rp, const
 hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, const int *Acol,
                            const BRow *brow, const int *tptr, long long *rprod, int *rtp, int *rmin,
                            int *rmax, int *rnnz, BinParams bp, int *binrows, long long *rdir, DevStats *st,
-                           BinSum *sums, unsigned *done, DevStats *host, int num_cus, hipStream_t s);
+                           BinSum *sums, unsigned *done, HostStats *host, unsigned seq, int num_cus, hipStream_t s);
 
 // C's row pointers (crp, and out32 when given: M + 1 each) from rnnz, and the numeric bins.
 // words: rowptr_blocks(M) zeroed words, *ticket = 0.  sums, host as above (rowptr_blocks).
@@ -329,7 +336,7 @@ hipError_t launch_rowptr_bin(int64_t M, const int *Arp, const long long *rprod, 
                              const int *rmin, const int *rmax, const int *rnnz, long long *crp,
                              int *out32, BinParams bp, int *binrows, unsigned long long *words,
                              unsigned *ticket, DevStats *st, BinSum *sums, unsigned *done,
-                             DevStats *host, hipStream_t s);
+                             HostStats *host, unsigned seq, hipStream_t s);
 
 // A kept directory that is two-level has this bit in rdir (the form follows from use_sparse
 // for rows the symbolic phase held in LDS; it keeps flat ones for the others).

@@ -700,7 +700,7 @@ DEVI void bin_reserve(BinBlock &B, int numeric, DevStats *st, BinSum *sums)
 
 // The end of a binning: the last block adds the blocks' sums up and hands the counters to
 // the host.  Every thread of the block (of blockDim.x >= NBINS).
-DEVI void bin_finish(BinBlock &B, int numeric, DevStats *st, const BinSum *sums, unsigned *done, DevStats *host)
+DEVI void bin_finish(BinBlock &B, int numeric, DevStats *st, const BinSum *sums, unsigned *done, HostStats *host, unsigned seq)
 {
     const int t = threadIdx.x;
     const int nblk = (int)gridDim.x;
@@ -744,10 +744,16 @@ DEVI void bin_finish(BinBlock &B, int numeric, DevStats *st, const BinSum *sums,
         return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    // the counters arrive before the number that follows them: the host, which waits for it,
+    // goes on without the end of the kernel
     const unsigned *from = (const unsigned *)st;
-    unsigned *to = (unsigned *)host;
+    unsigned *to = (unsigned *)&host->st;
     for (unsigned q = t; q < sizeof(DevStats) / sizeof(unsigned); q += blockDim.x)
-        to[q] = device_load(&from[q]);
+        __hip_atomic_store(&to[q], device_load(&from[q]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (t == 0)
+        __hip_atomic_store(&host->seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---- row analysis of A ---------------------------------------------------------------
@@ -778,7 +784,7 @@ __global__ __launch_bounds__(ri_lanes(G)) void k_row_info(int64_t M, int64_t K, 
                                                   long long *__restrict__ rprod, int *__restrict__ rtp, int *__restrict__ rmin,
                                                   int *__restrict__ rmax, int *__restrict__ rnnz, BinParams bp,
                                                   int *__restrict__ binrows, long long *__restrict__ rdir,
-                                                  DevStats *st, BinSum *sums, unsigned *done, DevStats *host)
+                                                  DevStats *st, BinSum *sums, unsigned *done, HostStats *host, unsigned seq)
 {
     constexpr int RI_BS = ri_lanes(G), ROWS_MAX = ri_rows_max(G), RPB = RI_BS / G, NW = RI_BS / 64;
     __shared__ long long s_prod[ROWS_MAX];
@@ -956,7 +962,7 @@ __global__ __launch_bounds__(ri_lanes(G)) void k_row_info(int64_t M, int64_t K, 
             binrows[(int64_t)at[u].b * M + B.base[at[u].b] + at[u].pos] = (int)(i0 + q);
         rdir[i0 + q] = at[u].dloc >= 0 ? (long long)B.dir_base + at[u].dloc : -1;
     }
-    bin_finish(B, 0, st, sums, done, host);
+    bin_finish(B, 0, st, sums, done, host, seq);
 }
 
 static int row_info_lanes(int64_t M, int64_t nnzA)
@@ -984,7 +990,7 @@ static int64_t row_info_blocks(int64_t M, int64_t nnzA, int num_cus)
 
 hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, const int *Acol, const BRow *brow,
                            const int *tptr, long long *rprod, int *rtp, int *rmin, int *rmax, int *rnnz, BinParams bp,
-                           int *binrows, long long *rdir, DevStats *st, BinSum *sums, unsigned *done, DevStats *host,
+                           int *binrows, long long *rdir, DevStats *st, BinSum *sums, unsigned *done, HostStats *host, unsigned seq,
                            int num_cus, hipStream_t s)
 {
     const int rows = row_info_rows(M, nnzA, num_cus);
@@ -992,7 +998,7 @@ hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, c
 #define ROW_INFO(G)                                                                                                    \
     case G:                                                                                                            \
         hipLaunchKernelGGL((k_row_info<G>), dim3(blocks), dim3(ri_lanes(G)), 0, s, M, K, nnzA, rows, Arp, Acol, brow, tptr,  \
-                           rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, st, sums, done, host);                     \
+                           rprod, rtp, rmin, rmax, rnnz, bp, binrows, rdir, st, sums, done, host, seq);                     \
         break;
     switch (row_info_lanes(M, nnzA)) {
         ROW_INFO(8) ROW_INFO(16) ROW_INFO(32) ROW_INFO(64)
@@ -1016,7 +1022,7 @@ __global__ __launch_bounds__(RP_BS) void k_rowptr_bin(int64_t M, const int *__re
                                                     const int *__restrict__ rnnz, long long *__restrict__ crp,
                                                     int *__restrict__ out32, BinParams bp, int *__restrict__ binrows,
                                                     u64 *words, unsigned *ticket, DevStats *st, BinSum *sums,
-                                                    unsigned *done, DevStats *host)
+                                                    unsigned *done, HostStats *host, unsigned seq)
 {
     __shared__ BinBlock B;
     __shared__ u64 red[RP_BS / 64];
@@ -1081,7 +1087,7 @@ __global__ __launch_bounds__(RP_BS) void k_rowptr_bin(int64_t M, const int *__re
     for (int u = 0; u < T; ++u)
         if (at[u].b >= 0)
             binrows[(int64_t)at[u].b * M + B.base[at[u].b] + at[u].pos] = (int)(i0 + u * RP_BS);
-    bin_finish(B, 1, st, sums, done, host);
+    bin_finish(B, 1, st, sums, done, host, seq);
 }
 
 int64_t rowptr_blocks(int64_t M)
@@ -1092,14 +1098,14 @@ int64_t rowptr_blocks(int64_t M)
 
 hipError_t launch_rowptr_bin(int64_t M, const int *Arp, const long long *rprod, const int *rtp, const int *rmin,
                              const int *rmax, const int *rnnz, long long *crp, int *out32, BinParams bp, int *binrows,
-                             u64 *words, unsigned *ticket, DevStats *st, BinSum *sums, unsigned *done, DevStats *host,
+                             u64 *words, unsigned *ticket, DevStats *st, BinSum *sums, unsigned *done, HostStats *host, unsigned seq,
                              hipStream_t s)
 {
     if (M <= 0)
         return hipSuccess;
     hipLaunchKernelGGL(M > RP_FEW ? k_rowptr_bin<2> : k_rowptr_bin<1>, dim3((unsigned)rowptr_blocks(M)), dim3(RP_BS), 0,
                        s, M, Arp, rprod, rtp, rmin, rmax, rnnz, crp, out32, bp, binrows, words, ticket, st, sums, done,
-                       host);
+                       host, seq);
     return hipGetLastError();
 }
 
