@@ -886,7 +886,9 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
 
     // ---- 3. symbolic ----
     HIP_TRY(make_tiles(h1.sym));
-    for (int b = 0; b < NBINS; ++b) {
+    HIP_TRY(launch_small(SMALL_SYMBOLIC, binrows, M, &dst->sym, h1.sym.count, h1.sym.max_need, op, rnnz, nullptr, nullptr,
+                         nullptr, nullptr, c->num_cus, opts.persistent ? dst->queue[0] : nullptr, nullptr, s));
+    for (int b = BIN_SHARED; b < NBINS; ++b) {
         const int cnt = h1.sym.count[b];
         if (cnt <= 0)
             continue;
@@ -982,7 +984,20 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         c->host->err = 0;
     int *errp = cap ? &dst->err : &c->host->err;
     unsigned long long lds_launched = 0;
-    for (int b = 0; b < NBINS; ++b) {
+    // rows that share a wave: one launch, or one for each bin where the bins are timed
+    for (int b = 0; b < (timing ? BIN_SHARED : 1); ++b) {
+        int count[BIN_SHARED] = {};
+        for (int k = 0; k < BIN_SHARED; ++k)
+            count[k] = !timing || k == b ? h2.num.count[k] : 0;
+        if (timing && count[b] > 0)
+            HIP_TRY(hipEventRecord(c->evb[b][0], s));
+        HIP_TRY(launch_small(fp32 ? SMALL_F32C : SMALL_F64, binrows, M, &dst->num, count, h2.num.max_need, op, nullptr,
+                             crp, Ccol, Cval, errp, c->num_cus, opts.persistent ? dst->queue[1] : nullptr,
+                             &lds_launched, s));
+        if (timing && count[b] > 0)
+            HIP_TRY(hipEventRecord(c->evb[b][1], s));
+    }
+    for (int b = BIN_SHARED; b < NBINS; ++b) {
         const int cnt = h2.num.count[b];
         if (cnt <= 0)
             continue;

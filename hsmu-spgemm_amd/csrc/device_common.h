@@ -152,26 +152,27 @@ DEVI void pull_chunk(unsigned *q, int n, int chunk, int nx, int &xq, int *s)
 }
 
 // The row groups a workgroup of a row kernel works on: with a queue, chunks pulled from
-// it; without, groups xcd_block(blockIdx) + k * gridDim (one group at a time).
+// it; without, groups xcd_block(block) + k * blocks (one group at a time).
 // nx: XCDs of the device (1..MAX_XCDS).
 struct GroupWalk {
     unsigned *q;
-    int n, chunk, nx, xq, grp, end;
+    int n, chunk, nx, xq, step, grp, end;
     int *s; // two ints of LDS
 
-    DEVI GroupWalk(unsigned *queue, int ngroups, int *lds2, int nxcd)
-        : q(queue), n(ngroups), chunk(1), nx(nxcd), xq(0), s(lds2)
+    // this workgroup is the block-th of `blocks` (all of the grid's, or a part of it)
+    DEVI GroupWalk(unsigned *queue, int ngroups, int *lds2, int nxcd, int block = blockIdx.x, int blocks = gridDim.x)
+        : q(queue), n(ngroups), chunk(1), nx(nxcd), xq(0), step(blocks), s(lds2)
     {
         if (q) {
             // chunks of about an eighth of a workgroup's share of its XCD's range
-            const long long per = (long long)ngroups / ((long long)gridDim.x * 8);
+            const long long per = (long long)ngroups / ((long long)blocks * 8);
             chunk = per > 1 ? (int)per : 1;
-            xq = blockIdx.x % nxcd;
+            xq = block % nxcd;
             pull_chunk(q, n, chunk, nx, xq, s);
             grp = s[0];
             end = s[1];
         } else {
-            grp = xcd_block(blockIdx.x, gridDim.x, nx);
+            grp = xcd_block(block, blocks, nx);
             end = grp + 1;
         }
     }
@@ -185,7 +186,7 @@ struct GroupWalk {
             grp = s[0];
             end = s[1];
         } else {
-            grp += (int)gridDim.x - 1;
+            grp += step - 1;
             end = grp + 1;
         }
     }

@@ -364,6 +364,13 @@ struct Operands {
     unsigned *dir_off;
 };
 
+// Rows that share a wave, those of the bins with count[b] > 0 in one launch (bin b's list at
+// rows + b * stride).  Symbolic: rnnz; numeric: the rows of C, lds_bytes as launch_numeric.
+enum { SMALL_SYMBOLIC, SMALL_F64, SMALL_F32C };
+hipError_t launch_small(int form, const int *rows, long long stride, const BinStats *bins_dev, const int *count,
+                        const int *max_need, const Operands &op, int *rnnz, const long long *crp, int *Ccol, void *Cval,
+                        int *err, int num_cus, unsigned (*queue)[MAX_XCDS], unsigned long long *lds_bytes, hipStream_t s);
+
 // Global-memory workspace (bin BIN_GLOBAL): gws_blocks regions of gws_stride u64 each;
 // a region holds gws_tiles 64-bit masks followed by gws_tiles 32-bit offsets, with
 // gws_tiles >= the widest tile span in the bin.
