@@ -395,7 +395,9 @@ constexpr int WIDE_UNIT = 4096;
 // per CU they are slower in one piece.  R-MAT squares of scale 16 (FP32) / 18 with rows of up
 // to 160 KB in LDS 2.35 / 17.1 ms, 80 KB 2.34 / 16.9, 64 KB 2.11 / 16.5, 48 KB 2.11 / 16.7.
 constexpr int WINDOW_ROW_MIN = 64 * 1024;
-constexpr int WIDE_UMAX = 16;
+// (the masks and slots of 24 units leave room for three workgroups per CU; R-MAT scale 18 with 4 /
+// 8 / 16 / 24 units 17.8 / 17.8 / 16.4 / 16.2 ms, 4 and 8 in an earlier state that took 17.4 with 16)
+constexpr int WIDE_UMAX = 24;
 constexpr int WIDE_TILES = WIDE_UNIT / 64;     // tiles of a unit
 constexpr int WIDE_BUCKETS = 32;               // windows are listed by their place in C's columns
 constexpr int WIDE_LISTS = 1 + 2 * WIDE_BUCKETS;
