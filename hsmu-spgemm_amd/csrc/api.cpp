@@ -928,7 +928,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
             return fail(HSMU_ERR_NOMEM, "C row pointers");
         outs.p.push_back(Crp);
     }
-    bp.per_lane = opts.products_per_lane > 0 ? opts.products_per_lane : 32;
+    bp.per_lane = opts.products_per_lane > 0 ? opts.products_per_lane : 48;
     // The column index of B that cuts wide rows into windows, and whether it and `list` bytes
     // of the windows' lists can be had.
     const long long units = wide_units(N);

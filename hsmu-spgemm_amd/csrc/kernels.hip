@@ -513,9 +513,11 @@ hipError_t launch_brows(int64_t K, int64_t N, int64_t nnz, const int *rp, const 
 // (numeric).
 // Lanes per row: the stream that rows with a workgroup of their own walk costs about the
 // same per item at every width from 64 lanes, and a start and an end per row that narrow
-// groups spread over more rows, so both phases give a lane 32 items by default (symbolic
+// groups spread over more rows, so a lane gets 32 tiles or 48 products by default (symbolic
 // stage at 4 / 16 / 32 tiles per lane: R-MAT squares of scale 16 746 / 476 / 439 us and of
-// scale 18 6.67 / 4.28 / 3.52 ms, banded rows of 100 tiles 116 / 72 / 66 us).  Rows whose
+// scale 18 6.67 / 4.28 / 3.52 ms, banded rows of 100 tiles 116 / 72 / 66 us; numeric bins at
+// 32 / 48 / 64 / 96 products: banded rows of 4,096 products 553 / 483 / 484 us, R-MAT scale 15
+// 681 / 658 / 662 / 690).  Rows whose
 // elements fit the registers of 8, 16 or 32 lanes share a wave.  16 waves per CU, where LDS
 // limits the workgroups, take 17.8 ms on the square of scale 18 against 19.2 ms with 8; 24
 // slow a banded square by 4%.
