@@ -542,7 +542,7 @@ def main():
                    "fp64_errors": fp64_err},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(achieved / PEAK_HBM_GBS, 4), "traffic": traffic,
-                     "kernel": f"k_numeric_lds bin {dom}" if dom < 8 else "wide-row bin",
+                     "kernel": ("k_small_bin" if dom < 3 else "k_numeric_row") + f" bin {dom}" if dom < 8 else "wide-row bin",
                      "kernel_ms": round(dom_ms, 4), "alg_bytes_per_launch": dom_bytes,
                      "frac_end_to_end": round(e2e_gbs / PEAK_HBM_GBS, 4),
                      "alg_bytes_end_to_end": st0["alg_bytes"],
