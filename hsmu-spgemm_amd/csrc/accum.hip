@@ -1925,7 +1925,9 @@ hipError_t launch_small(int form, const int *rows, long long stride, const BinSt
     unsigned long long ignored = 0;
     if (!lds_bytes)
         lds_bytes = &ignored;
-    auto *f = form == SMALL_SYMBOLIC ? small_launch<SmallNone> : form == SMALL_F64 ? small_launch<PrecF64> : small_launch<PrecF32C>;
+    auto *f = form == SMALL_SYMBOLIC ? small_launch<SmallNone>
+              : form == SMALL_F64    ? small_launch<PrecF64>
+                                     : small_launch<PrecF32C>;
     return f(rows, stride, bins_dev, count, max_need, op, rnnz, crp, Ccol, Cval, err, num_cus, queue, lds_bytes, s);
 }
 
@@ -2054,7 +2056,8 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
 }
 
 hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_dev, int count, int max_need,
-                          const Operands &op, const long long *crp, int *Ccol, void *Cval, int bshift, int two_level, const WideRows &wide, int *err, int num_cus, unsigned *queue,
+                          const Operands &op, const long long *crp, int *Ccol, void *Cval, int bshift, int two_level,
+                          const WideRows &wide, int *err, int num_cus, unsigned *queue,
                           unsigned long long *lds_bytes, hipStream_t s)
 {
     if (count <= 0)
@@ -2063,8 +2066,10 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
     if (!lds_bytes)
         lds_bytes = &ignored;
     if (fp32c)
-        return numeric_p<PrecF32C>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, two_level, wide, err, num_cus, queue, lds_bytes, s);
-    return numeric_p<PrecF64>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, two_level, wide, err, num_cus, queue, lds_bytes, s);
+        return numeric_p<PrecF32C>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, two_level, wide,
+                                   err, num_cus, queue, lds_bytes, s);
+    return numeric_p<PrecF64>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, two_level, wide, err,
+                              num_cus, queue, lds_bytes, s);
 }
 
 int wide_item_blocks(int count, int num_cus)

@@ -792,12 +792,10 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     if (rc)
         return rc;
 
-    // lanes per A entry: walk one B row (numeric) / one B tile row (tile OR)
+    // lanes that walk one row of B (its tiles in the symbolic phase) for rows wider than LDS that
+    // take no windows
     const long long avg_b = P.nnzB / (K > 0 ? K : 1);
     const long long avg_t = (long long)h1.ntiles_b / (K > 0 ? K : 1);
-    // about four products per lane per B row: shorter sub-groups keep more A entries in
-    // flight per wave and idle fewer lanes on ragged B rows (measured on the banded
-    // workload: 16 lanes for 64-entry rows beats 64 lanes by 1.2x in the numeric phase)
     int blanes = opts.b_lanes > 0 ? opts.b_lanes : pow2_floor(avg_b / 4 > 0 ? avg_b / 4 : 1);
     int tlanes = opts.t_lanes > 0 ? opts.t_lanes : pow2_floor(avg_t > 0 ? avg_t : 1);
     if (blanes > 64)
@@ -949,7 +947,8 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
                     wide_list_bytes(c->num_cus)))
         bp.lds_row_max = WINDOW_ROW_MIN;
     HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp, rp64 || batch ? nullptr : (int *)Crp, bp,
-                              binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1], host, ++c->seq, s));
+                              binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1],
+                              host, ++c->seq, s));
     HIP_TRY(mark(c->ev[EV_SYMBOLIC]));
     DevStats h2;
     rc = checkpoint(c, mode, dst, 1, h2);

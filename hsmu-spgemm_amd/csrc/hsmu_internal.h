@@ -466,7 +466,8 @@ size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks);
 // window by window and are not counted.
 hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_dev, int count,
                           int max_need, const Operands &op, const long long *crp, int *Ccol,
-                          void *Cval, int bshift, int two_level, const WideRows &wide, int *err, int num_cus, unsigned *queue, unsigned long long *lds_bytes,
+                          void *Cval, int bshift, int two_level, const WideRows &wide, int *err, int num_cus,
+                          unsigned *queue, unsigned long long *lds_bytes,
                           hipStream_t s);
 
 // A B of fewer than STREAM_V entries (n of them, at least one), copied to arrays of

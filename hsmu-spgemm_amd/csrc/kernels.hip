@@ -2,7 +2,8 @@
 //
 // Pipeline for C = A * B (all on one stream; host synchronises twice, to validate the
 // input / size the symbolic launches and to size C):
-//   1. B -> 64-column tiles (k_btiles: one pass, chained scan).
+//   1. B -> 64-column tiles (k_btiles: one pass, chained scan; for a B of short rows only
+//      the rows' records, k_brows, unless a row of C wants the tiles).
 //      Reference: src/compressed/compressed_mask64.cuh:61-424.  Tiles of a row come out
 //      sorted by tile column (the reference's order is whatever LDS atomics give).
 //   2. Row analysis of A (k_row_info): products, tile-products and the tile span
@@ -10,12 +11,13 @@
 //   3. Binning (in k_row_info, and in k_rowptr_bin for the numeric phase) by work and LDS
 //      need, wave/workgroup-aggregated appends.  Reference: src/bining.cuh:1-395 (fixed
 //      ranges there; derived from LDS need here).
-//   4. Symbolic (k_symbolic_lds / k_symbolic_global): OR of B's tile masks over the A row
-//      into a dense mask directory over the row's tile span, nnz(C_i) = sum popcount.
+//   4. Symbolic (k_symbolic_row / _wide / _global): OR of B's tile masks over the A row
+//      into a mask directory over the row's tile span, nnz(C_i) = sum popcount; rows of few
+//      products (k_small_bin, k_small_rows) mark their columns directly.
 //      Reference: compressed_tilePtr_symbolic.cuh + compressed_tileOR.cuh, which do the
 //      same in two hash passes; the dense directory needs one pass and no hashing.
 //   5. Scan of nnz(C_i) to row pointers (k_rowptr_bin).
-//   6. Numeric (k_numeric_lds / k_numeric_window): the HSMU accumulator.  The row's
+//   6. Numeric (k_numeric_row, k_small_bin, k_numeric_windows): the HSMU accumulator.  The row's
 //      value array is exactly nnz(C_i) long; the slot of column c is
 //        off[t] + popcount(mask[t] & ((1 << (c & 63)) - 1)),  t = (c >> 6) - rmin,
 //      i.e. the rank of c among C's sorted columns, found in O(1) from the tile
@@ -25,8 +27,7 @@
 //      replaces the reference's separate O(n^2) rank-sort pass
 //      (src/compressed/compressed_Ccol_symbolic.cuh:4-63).
 //   Rows whose directory + values do not fit LDS: the symbolic tile OR runs on a global
-//   workspace, the numeric phase slides a dense LDS window over the row's columns (the
-//   reference's bin-13 dense spECK path, src/external/spECK/dense_acc.cu:246-267, whose
+//   workspace, the numeric phase takes the row in windows of its columns (the reference's bin-13 dense spECK path, src/external/spECK/dense_acc.cu:246-267, whose
 //   early return leaves rows unwritten; every row is written here).
 
 #include <hip/hip_runtime.h>
@@ -702,7 +703,8 @@ DEVI void bin_reserve(BinBlock &B, int numeric, DevStats *st, BinSum *sums)
 
 // The end of a binning: the last block adds the blocks' sums up and hands the counters to
 // the host.  Every thread of the block (of blockDim.x >= NBINS).
-DEVI void bin_finish(BinBlock &B, int numeric, DevStats *st, const BinSum *sums, unsigned *done, HostStats *host, unsigned seq)
+DEVI void bin_finish(BinBlock &B, int numeric, DevStats *st, const BinSum *sums, unsigned *done, HostStats *host,
+                     unsigned seq)
 {
     const int t = threadIdx.x;
     const int nblk = (int)gridDim.x;
@@ -992,7 +994,8 @@ static int64_t row_info_blocks(int64_t M, int64_t nnzA, int num_cus)
 
 hipError_t launch_row_info(int64_t M, int64_t K, int64_t nnzA, const int *Arp, const int *Acol, const BRow *brow,
                            const int *tptr, long long *rprod, int *rtp, int *rmin, int *rmax, int *rnnz, BinParams bp,
-                           int *binrows, long long *rdir, DevStats *st, BinSum *sums, unsigned *done, HostStats *host, unsigned seq,
+                           int *binrows, long long *rdir, DevStats *st, BinSum *sums, unsigned *done, HostStats *host,
+                           unsigned seq,
                            int num_cus, hipStream_t s)
 {
     const int rows = row_info_rows(M, nnzA, num_cus);
@@ -1100,7 +1103,8 @@ int64_t rowptr_blocks(int64_t M)
 
 hipError_t launch_rowptr_bin(int64_t M, const int *Arp, const long long *rprod, const int *rtp, const int *rmin,
                              const int *rmax, const int *rnnz, long long *crp, int *out32, BinParams bp, int *binrows,
-                             u64 *words, unsigned *ticket, DevStats *st, BinSum *sums, unsigned *done, HostStats *host, unsigned seq,
+                             u64 *words, unsigned *ticket, DevStats *st, BinSum *sums, unsigned *done, HostStats *host,
+                             unsigned seq,
                              hipStream_t s)
 {
     if (M <= 0)

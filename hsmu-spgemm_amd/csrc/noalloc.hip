@@ -1,7 +1,7 @@
 // noalloc.hip -- the workspace of hsmu_spgemm_noalloc: one file-scope device array.
 //
 // hsmu_spgemm takes its workspace (B's tiles, per-row analysis, bins, row directories,
-// wide-row work items) from the context's caching pool, which calls hipMalloc the first
+// the wide rows' index and windows) from the context's caching pool, which calls hipMalloc the first
 // time a size is needed.  Callers that may not allocate device memory at all (code under
 // stream capture, serving loops, harnesses that forbid it) use hsmu_spgemm_noalloc, whose
 // workspace is this array instead: NOALLOC_SCRATCH_BYTES of device memory that every GPU
