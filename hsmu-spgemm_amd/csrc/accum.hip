@@ -1479,14 +1479,21 @@ __global__ __launch_bounds__(1024) void k_numeric_wcompact(const int *__restrict
 
 // The first element of every B row at each unit's start (and the row's end): index[j * (U + 1)
 // + u] = first element of row j with a column of unit u or later.  A lane per (row, unit),
-// binary search in the row (neighbouring lanes search one row).
-__global__ __launch_bounds__(256) void k_wide_index(long long K, long long U, const int *__restrict__ rp,
-                                                    const int *__restrict__ col, int *__restrict__ index)
+// binary search in the row (neighbouring lanes search one row).  In a replayed plan the row
+// pointers are the inputs' current ones: without wide rows (as after a failed check of the
+// plan) nothing is read, and what is read lies within B's nnz entries.
+__global__ __launch_bounds__(256) void k_wide_index(const int *__restrict__ count_p, long long K, long long U, int nnz,
+                                                    const int *__restrict__ rp, const int *__restrict__ col,
+                                                    int *__restrict__ index)
 {
+    if (*count_p == 0)
+        return;
     const long long n = K * (U + 1), stride = (long long)gridDim.x * 256;
     for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < n; q += stride) {
         const long long j = q / (U + 1), u = q - j * (U + 1);
         int lo = rp[j], hi = rp[j + 1];
+        lo = lo < 0 ? 0 : lo < nnz ? lo : nnz;
+        hi = hi < 0 ? 0 : hi < nnz ? hi : nnz;
         if (u == 0)
             hi = lo;
         else if (u == U)
@@ -2018,8 +2025,8 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
         if (op.dir_mask && wide.items) { // windows
             const long long nix = wide.K * (wide.nunits + 1);
             const long long gx = (nix + 255) / 256;
-            hipLaunchKernelGGL(k_wide_index, dim3((unsigned)(gx < 65536 ? gx : 65536)), dim3(256), 0, s, wide.K,
-                               wide.nunits, op.Brp, op.Bcol, wide.index);
+            hipLaunchKernelGGL(k_wide_index, dim3((unsigned)(gx < 65536 ? gx : 65536)), dim3(256), 0, s,
+                               count_dev, wide.K, wide.nunits, op.nnzB, op.Brp, op.Bcol, wide.index);
             const unsigned gi = (unsigned)wide_item_blocks(count, num_cus);
             hipLaunchKernelGGL(k_wide_items<false>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
                                wide.items, wide.items_cap, wide.places, err);
