@@ -916,7 +916,9 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     }
     if (!crp)
         return fail(HSMU_ERR_NOMEM, "C row pointers");
-    // C's int32 row pointers, when they are the caller's (a batch splits them afterwards)
+    // C's int32 row pointers, when they are the caller's (a batch splits them afterwards).  An
+    // allocation-free call's arrays are written once C is known to fit them.
+    const bool narrow_later = ar.fixed() && !rp64;
     void *Crp = nullptr;
     if (rp64 && !batch) {
         Crp = crp;
@@ -946,9 +948,10 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         windows_fit((unsigned long long)M * wide_row_items(n_most, n_most / 64 + 1) * sizeof(WideItem) +
                     wide_list_bytes(c->num_cus)))
         bp.lds_row_max = WINDOW_ROW_MIN;
-    HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp, rp64 || batch ? nullptr : (int *)Crp, bp,
-                              binrows, words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1],
-                              host, ++c->seq, s));
+    HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp,
+                              rp64 || batch || narrow_later ? nullptr : (int *)Crp, bp, binrows,
+                              words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1], host,
+                              ++c->seq, s));
     HIP_TRY(mark(c->ev[EV_SYMBOLIC]));
     DevStats h2;
     rc = checkpoint(c, mode, dst, 1, h2);
@@ -1033,6 +1036,8 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         if (timing)
             HIP_TRY(hipEventRecord(c->evb[b][1], s));
     }
+    if (narrow_later)
+        HIP_TRY(launch_rowptr_narrow(crp, M + 1, (int *)Crp, s));
     if (batch)
         HIP_TRY(launch_batch_split(batch->count, batch->off, crp, Crp, rp64 ? 1 : 0, bases, M + batch->count, s));
     HIP_TRY(mark(c->ev[EV_NUMERIC]));

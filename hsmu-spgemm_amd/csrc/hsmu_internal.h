@@ -474,6 +474,8 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
 // STREAM_V entries whose last one repeats: the element stream loads STREAM_V at a time.
 hipError_t launch_pad_b(const int *col, const void *val, int val32, int n, int *pcol, void *pval, hipStream_t s);
 
+// int64 row pointers that fit int32, as int32
+hipError_t launch_rowptr_narrow(const long long *in, int64_t n, int *out, hipStream_t s);
 // out[i] = in[i] - in[0] for i < n (row pointers of a row panel, rebased to 0)
 hipError_t launch_rowptr_rebase(const int *in, int64_t n, int *out, hipStream_t s);
 // sum[i] and asum[i] = sum of the values / of their magnitudes in row i of a CSR matrix

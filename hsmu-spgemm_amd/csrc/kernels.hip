@@ -1136,7 +1136,22 @@ hipError_t launch_pad_b(const int *col, const void *val, int val32, int n, int *
     return hipGetLastError();
 }
 
-// ---- row panels and row sums ------------------------------------------------------------
+// ---- row pointers, row panels and row sums -------------------------------------------------
+
+__global__ __launch_bounds__(256) void k_rowptr_narrow(const long long *__restrict__ in, int64_t n, int *__restrict__ out)
+{
+    const int64_t stride = (int64_t)gridDim.x * 256;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride)
+        out[i] = (int)in[i];
+}
+
+hipError_t launch_rowptr_narrow(const long long *in, int64_t n, int *out, hipStream_t s)
+{
+    const int64_t blocks = (n + 255) / 256;
+    hipLaunchKernelGGL(k_rowptr_narrow, dim3((unsigned)(blocks < 1 ? 1 : blocks < 8192 ? blocks : 8192)), dim3(256), 0, s,
+                       in, n, out);
+    return hipGetLastError();
+}
 
 __global__ __launch_bounds__(256) void k_rowptr_rebase(const int *__restrict__ in, int64_t n, int *__restrict__ out)
 {
