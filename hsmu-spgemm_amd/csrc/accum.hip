@@ -1909,7 +1909,8 @@ static hipError_t small_launch(const int *rows, long long stride, const BinStats
         // whole rounds over the XCDs, so that each bin's blocks start at the first
         b.blocks[k] = (int)((blocks + MAX_XCDS - 1) / MAX_XCDS * MAX_XCDS);
         grid += b.blocks[k];
-        *lds_bytes += (unsigned long long)blocks * bytes;
+        // a workgroup per group, as without the limit; a queue's workgroups are what runs
+        *lds_bytes += (unsigned long long)(queue ? blocks : groups) * bytes;
     }
     if (grid == 0)
         return hipSuccess;
