@@ -1477,6 +1477,19 @@ __global__ __launch_bounds__(1024) void k_numeric_wcompact(const int *__restrict
 
 // ---- wide rows as windows -----------------------------------------------------------------
 
+// The first element of [lo, hi) of a sorted row whose column is c or later.
+DEVI int first_element(const int *__restrict__ col, int lo, int hi, int c)
+{
+    while (lo < hi) {
+        const int mid = lo + ((hi - lo) >> 1);
+        if (col[mid] < c)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
 // The first element of every B row at each unit's start (and the row's end): index[j * (U + 1)
 // + u] = first element of row j with a column of unit u or later.  A lane per (row, unit),
 // binary search in the row (neighbouring lanes search one row).  In a replayed plan the row
@@ -1494,19 +1507,7 @@ __global__ __launch_bounds__(256) void k_wide_index(const int *__restrict__ coun
         int lo = rp[j], hi = rp[j + 1];
         lo = lo < 0 ? 0 : lo < nnz ? lo : nnz;
         hi = hi < 0 ? 0 : hi < nnz ? hi : nnz;
-        if (u == 0)
-            hi = lo;
-        else if (u == U)
-            lo = hi;
-        const int c = (int)(u * WIDE_UNIT < INT_MAX ? u * WIDE_UNIT : INT_MAX);
-        while (lo < hi) {
-            const int mid = lo + ((hi - lo) >> 1);
-            if (col[mid] < c)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        index[q] = lo;
+        index[q] = u == 0 ? lo : u == U ? hi : first_element(col, lo, hi, (int)(u * WIDE_UNIT));
     }
 }
 
@@ -1715,7 +1716,7 @@ template <int BS, bool DENSE> constexpr int ww_lds()
     return WIDE_UNIT * 8 + BS * 16 + words * 10 + (DENSE ? 0 : WW_TILES * 10);
 }
 
-template <typename P, int BS, bool DENSE>
+template <typename P, int BS, bool DENSE, bool INDEX>
 __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restrict__ items,
                                                         const WideCount *__restrict__ listed, unsigned *taken,
                                                         Operands op, const int *__restrict__ index, long long U,
@@ -1760,9 +1761,17 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
         auto segment = [&](int e, int col) {
             if (e >= nA)
                 return Segment{0, 0, 0};
-            const int *ix = index + (long long)col * (U + 1);
-            const int s0 = ix[u0];
-            return Segment{s0, ix[u1] - s0, (u64)__double_as_longlong((double)Aval[a0 + e])};
+            int s0, s1;
+            if constexpr (INDEX) {
+                const int *ix = index + (long long)col * (U + 1);
+                s0 = ix[u0];
+                s1 = ix[u1];
+            } else {
+                const typename Vec2<int>::type r = load2(op.Brp + col);
+                s0 = first_element(op.Bcol, r.x, r.y, u0 * WIDE_UNIT);
+                s1 = u1 < U ? first_element(op.Bcol, s0, r.y, u1 * WIDE_UNIT) : r.y;
+            }
+            return Segment{s0, s1 - s0, (u64)__double_as_longlong((double)Aval[a0 + e])};
         };
         const Segment first = segment(l, j);
         // dense: lane i of wave w holds tile w * TW + i
@@ -2024,24 +2033,30 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
     if (bin == BIN_GLOBAL) {
         const int blocks = count < wide.blocks ? count : wide.blocks;
         if (op.dir_mask && wide.items) { // windows
-            const long long nix = wide.K * (wide.nunits + 1);
-            const long long gx = (nix + 255) / 256;
-            hipLaunchKernelGGL(k_wide_index, dim3((unsigned)(gx < 65536 ? gx : 65536)), dim3(256), 0, s,
-                               count_dev, wide.K, wide.nunits, op.nnzB, op.Brp, op.Bcol, wide.index);
+            if (wide.index) {
+                const long long gx = (wide.K * (wide.nunits + 1) + 255) / 256;
+                hipLaunchKernelGGL(k_wide_index, dim3((unsigned)(gx < 65536 ? gx : 65536)), dim3(256), 0, s, count_dev,
+                                   wide.K, wide.nunits, op.nnzB, op.Brp, op.Bcol, wide.index);
+            }
             const unsigned gi = (unsigned)wide_item_blocks(count, num_cus);
             hipLaunchKernelGGL(k_wide_items<false>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
                                wide.items, wide.items_cap, wide.places, err);
             hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(1024), 0, s, wide.places, (int)gi, wide.ctr);
             hipLaunchKernelGGL(k_wide_items<true>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
                                wide.items, wide.items_cap, wide.places, err);
-            hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, true>),
-                               dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, true>()))), dim3(WW_BS),
-                               (ww_lds<WW_BS, true>()), s, wide.items, wide.ctr, wide.ctr->taken, op, wide.index,
-                               wide.nunits, crp, Ccol, (typename P::V *)Cval);
-            hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, false>),
-                               dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, false>()))), dim3(WW_BS),
-                               (ww_lds<WW_BS, false>()), s, wide.items, wide.ctr, wide.ctr->taken + 1, op, wide.index,
-                               wide.nunits, crp, Ccol, (typename P::V *)Cval);
+#define WINDOWS(DENSE, INDEX, TAKEN)                                                                                   \
+    hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, DENSE, INDEX>),                                                    \
+                       dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, DENSE>()))), dim3(WW_BS),                     \
+                       (ww_lds<WW_BS, DENSE>()), s, wide.items, wide.ctr, wide.ctr->taken + TAKEN, op, wide.index,     \
+                       wide.nunits, crp, Ccol, (typename P::V *)Cval)
+            if (wide.index) {
+                WINDOWS(true, true, 0);
+                WINDOWS(false, true, 1);
+            } else {
+                WINDOWS(true, false, 0);
+                WINDOWS(false, false, 1);
+            }
+#undef WINDOWS
         } else if (op.dir_mask)
             hipLaunchKernelGGL(k_numeric_wcompact<P>, dim3(blocks), dim3(1024), CW_LDS, s, rows, count_dev, op, crp,
                                Ccol, (typename P::V *)Cval, bshift > 6 ? 6 : bshift, wide.ws, wide.cur_stride,
@@ -2117,8 +2132,8 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
     CFG(k_numeric_window<PrecF64>) CFG(k_numeric_window<PrecF32C>)
     CFG(k_numeric_wcompact<PrecF64>) CFG(k_numeric_wcompact<PrecF32C>) 
 #define CFGW(P)                                                                                                        \
-    CFG((k_numeric_windows<P, WW_BS, false>))                                                                          \
-    CFG((k_numeric_windows<P, WW_BS, true>))
+    CFG((k_numeric_windows<P, WW_BS, false, false>)) CFG((k_numeric_windows<P, WW_BS, false, true>))                   \
+    CFG((k_numeric_windows<P, WW_BS, true, false>)) CFG((k_numeric_windows<P, WW_BS, true, true>))
     CFGW(PrecF64) CFGW(PrecF32C)
 #undef CFGW
 #undef CFG

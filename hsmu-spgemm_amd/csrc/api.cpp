@@ -850,7 +850,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         for (int b = BIN_SHARED; b < NBINS; ++b) // (rows that share a wave keep none)
             tile_products += h1.sym.work[b];
         const bool worth = 2 * dir_total <= tile_products || h1.sym.count[BIN_GLOBAL] > 0 ||
-                           h1.num_wide_hint > 0;
+                           h1.num_wide_work > 0;
         unsigned long long budget = c->total_mem / 4 > (1ull << 31) ? c->total_mem / 4 : (1ull << 31);
         // allocation-free: at most half of the workspace left, the rest serves C's row
         // pointers and the numeric phase
@@ -929,24 +929,27 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         outs.p.push_back(Crp);
     }
     bp.per_lane = opts.products_per_lane > 0 ? opts.products_per_lane : 48;
-    // The column index of B that cuts wide rows into windows, and whether it and `list` bytes
-    // of the windows' lists can be had.
+    // Wide rows are cut into windows when there is room for `list` bytes of the windows' lists,
+    // with the column index of B where its places cost little beside the rows' products.
     const long long units = wide_units(N);
-    const unsigned long long index_bytes = (unsigned long long)K * (units + 1) * sizeof(int);
+    const unsigned long long places = (unsigned long long)K * (units + 1), index_bytes = places * sizeof(int);
     auto windows_fit = [&](unsigned long long list) {
-        const unsigned long long left = ar.remaining(); // allocation-free: of the workspace
+        return keep_dirs && list <= ar.remaining() && units < (1 << 24); // allocation-free: the workspace left
+    };
+    auto index_pays = [&](unsigned long long products, unsigned long long list) {
+        const unsigned long long left = ar.remaining();
         unsigned long long most =
             opts.wide_scratch_mb > 0 ? (unsigned long long)opts.wide_scratch_mb << 20 : c->total_mem / 4;
         if (most > left / 2)
             most = left / 2;
-        return keep_dirs && index_bytes <= most && list <= left - index_bytes && units < (1 << 24);
+        return places <= products / WIDE_INDEX_WORK && index_bytes <= most && list <= left - index_bytes;
     };
-    // rows of more than WINDOW_ROW_MIN are wide where windows are certain: with room for the
-    // lists of M full rows
+    // rows of more than WINDOW_ROW_MIN are wide where windows with the index are certain: with
+    // room for the lists of M full rows
     const int n_most = (int)(N < INT_MAX ? N : INT_MAX);
-    if (bp.lds_row_max > WINDOW_ROW_MIN &&
-        windows_fit((unsigned long long)M * wide_row_items(n_most, n_most / 64 + 1) * sizeof(WideItem) +
-                    wide_list_bytes(c->num_cus)))
+    const unsigned long long list_most =
+        (unsigned long long)M * wide_row_items(n_most, n_most / 64 + 1) * sizeof(WideItem) + wide_list_bytes(c->num_cus);
+    if (bp.lds_row_max > WINDOW_ROW_MIN && windows_fit(list_most) && index_pays(h1.num_wide_work, list_most))
         bp.lds_row_max = WINDOW_ROW_MIN;
     HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp,
                               rp64 || batch || narrow_later ? nullptr : (int *)Crp, bp, binrows,
@@ -1003,18 +1006,19 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         const int cnt = h2.num.count[b];
         if (cnt <= 0)
             continue;
-        // wide rows: with kept directories and room for the index of B, windows of their
-        // columns on a persistent grid; else a workgroup per row, with a workspace for the
-        // tiles of a two-level directory and the cursors of its row's A entries
+        // wide rows: with kept directories, windows of their columns on a persistent grid; else
+        // a workgroup per row, with a workspace for the tiles of a two-level directory and the
+        // cursors of its row's A entries
         WideRows wide = {};
         if (b == BIN_GLOBAL) {
-            const bool windows = h2.wide_items < (1ull << 31) &&
-                                 windows_fit(h2.wide_items * sizeof(WideItem) + wide_list_bytes(c->num_cus));
+            const unsigned long long list = h2.wide_items * sizeof(WideItem) + wide_list_bytes(c->num_cus);
+            const bool windows = h2.wide_items < (1ull << 31) && windows_fit(list);
+            const bool indexed = windows && index_pays(h2.num.work[b], list);
             wide.blocks = cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt;
             if (windows) {
                 wide.nunits = units;
                 wide.K = K;
-                wide.index = (int *)ar.raw((size_t)index_bytes);
+                wide.index = indexed ? (int *)ar.raw((size_t)index_bytes) : nullptr;
                 wide.items_cap = (long long)h2.wide_items;
                 wide.items = ar.get<WideItem>((size_t)wide.items_cap);
                 wide.places = ar.get<unsigned>((size_t)wide_item_blocks(cnt, c->num_cus) * WIDE_LISTS);
@@ -1024,7 +1028,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
                 wide.ft_stride = keep_dirs ? (((long long)h2.num.max_span[b] + 63) & ~63LL) : 0;
                 wide.ws = ar.get<int>(wide_ws_ints(wide.cur_stride, wide.ft_stride, wide.blocks) + 1);
             }
-            if (windows ? (!wide.index || !wide.items || !wide.places || !wide.ctr) : !wide.ws)
+            if (windows ? ((indexed && !wide.index) || !wide.items || !wide.places || !wide.ctr) : !wide.ws)
                 return fail(HSMU_ERR_NOMEM, "wide-row workspace");
         }
         if (timing)

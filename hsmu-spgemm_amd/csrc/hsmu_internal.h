@@ -64,7 +64,7 @@ struct DevStats {
     int err;
     int ntiles_b;
     int pad;
-    unsigned long long num_wide_hint; // rows whose numeric need may exceed LDS (symbolic binning)
+    unsigned long long num_wide_work; // products of rows that may be wide in the numeric phase (symbolic binning)
     unsigned long long wide_items; // windows the wide rows may need, at most (numeric binning)
     BinStats sym;
     BinStats num;
@@ -389,15 +389,23 @@ hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int c
 // (aligned, so that all rows' windows share their boundaries) that holds at most WIDE_UNIT
 // entries of C_i and spans at most WIDE_UMAX units, one workgroup each.  The index gives
 // every B row's first element at each unit's start, so a window's elements are known without
-// a search.
+// a search; where it does not pay, a window searches the B rows it names.
 constexpr int WIDE_UNIT = 4096;
-// Rows of more LDS than this are wide where windows can be had: with one or two workgroups
+// Rows of more LDS than this are wide where the index pays: with one or two workgroups
 // per CU they are slower in one piece.  R-MAT squares of scale 16 (FP32) / 18 with rows of up
 // to 160 KB in LDS 2.35 / 17.1 ms, 80 KB 2.34 / 16.9, 64 KB 2.11 / 16.5, 48 KB 2.11 / 16.7.
 constexpr int WINDOW_ROW_MIN = 64 * 1024;
 // (the masks and slots of 24 units leave room for three workgroups per CU; R-MAT scale 18 with 4 /
 // 8 / 16 / 24 units 17.8 / 17.8 / 16.4 / 16.2 ms, 4 and 8 in an earlier state that took 17.4 with 16)
 constexpr int WIDE_UMAX = 24;
+// The index costs a place per row of B and unit (2 to 3.4 ps each), whatever the wide rows are;
+// a search costs 0.8 (Zipf panel) to 4 ps (R-MAT scale 16) per product of theirs.  So it is made
+// where they have this many products for each place.  With the index and without: R-MAT squares
+// of scale 16 / 18 2.06 / 16.2 and 2.60 / 20.7 ms, a Zipf panel 4.14 and 5.38 (115 products per
+// place or more); a grid of 1 M rows, one of them with 20,000 entries, 1.47 and 0.81 ms, of 4 M
+// rows 13.7 and 4.6 ms and 15 GB (less than 0.01); one row with 1 M entries the same with both
+// (0.04).
+constexpr unsigned long long WIDE_INDEX_WORK = 4;
 constexpr int WIDE_TILES = WIDE_UNIT / 64;     // tiles of a unit
 constexpr int WIDE_BUCKETS = 32;               // windows are listed by their place in C's columns
 constexpr int WIDE_LISTS = 1 + 2 * WIDE_BUCKETS;
@@ -446,7 +454,7 @@ struct WideRows {
     WideItem *items;
     unsigned *places;
     WideCount *ctr;
-    int *index; // K rows of nunits + 1
+    int *index; // K rows of nunits + 1, or null: search
     long long nunits;
     long long K;
 };

@@ -623,9 +623,11 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
         sp = use_sparse(r.S, r.tp) ? 1 : 0;
     }
     const int lane = threadIdx.x & 63;
-    const u64 wides = __ballot(wide);
-    if (lane == 0 && wides)
-        atomicAdd(&st->num_wide_hint, (u64)__popcll(wides));
+    if (__ballot(wide)) {
+        const u64 products = wave_sum(wide ? (u64)r.prod : 0ull);
+        if (lane == 0)
+            atomicAdd(&st->num_wide_work, products);
+    }
     if (numeric && __ballot(at.b == BIN_GLOBAL)) { // room for the wide rows' windows
         const u64 items = wave_sum(at.b == BIN_GLOBAL ? (u64)wide_row_items(r.nc, r.S) : 0ull);
         if (lane == 0)

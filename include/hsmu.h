@@ -134,9 +134,10 @@ typedef struct hsmu_opts {
                                  this many waves per CU at the occupancy its LDS allows (at
                                  most 1024 lanes); 0 = 16 */
     int32_t wide_scratch_mb;  /* rows wider than LDS: MiB the column index of B may take that cuts
-                                 them into windows (4 bytes per row of B and 4,096 columns);
-                                 0 = a quarter of device memory.  Beyond it those rows take one
-                                 workgroup each, which is slower */
+                                 them into windows (4 bytes per row of B and 4,096 columns; made
+                                 where those rows have products enough to pay for it); 0 = a
+                                 quarter of device memory.  Beyond it their windows search each
+                                 row of B, which is slower */
     int32_t wide_window;      /* accepted, without effect: 0, 4096 or 8192 (windows of rows wider
                                  than LDS hold 4,096 entries of C) */
 } hsmu_opts;
