@@ -540,6 +540,10 @@ extern "C" int hsmu_csr_free(hsmu_ctx *c, hsmu_csr *C)
     return HSMU_OK;
 }
 
+// Forms of the wide rows, by the memory they want: windows with the column index of B, windows
+// that search B's rows, a workgroup per row.
+enum { WIDE_INDEXED, WIDE_SEARCHED, WIDE_PER_ROW, WIDE_NONE };
+
 // A plan: the recorded run of one batch (or one SpGEMM) and its captured HIP graph.
 struct hsmu_plan {
     hsmu_ctx *c = nullptr;
@@ -551,6 +555,7 @@ struct hsmu_plan {
     hsmu_stats stats0;            // statistics of the recording run
     bool empty = false;           // product with no entries: nothing to replay
     bool dirs_kept = false;       // the recording run kept the row directories
+    int wide_form = 0;            // the form its wide rows took
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
@@ -608,6 +613,20 @@ class Arena {
         return p;
     }
     template <typename T> T *get(size_t n) { return (T *)raw(n * sizeof(T)); }
+    // Give back what was taken since mark() (not in a capture pass, which repeats the requests
+    // that were kept).
+    struct Mark {
+        size_t blocks, off, shortage;
+    };
+    Mark mark() const { return {keep_ ? keep_->size() : taken_.size(), off_, short_}; }
+    void rewind(const Mark &m)
+    {
+        std::vector<void *> &v = keep_ ? *keep_ : taken_;
+        for (; v.size() > m.blocks; v.pop_back())
+            c_->pool.release(v.back());
+        off_ = m.off;
+        short_ = m.shortage;
+    }
     // bytes a further workspace request may take (unbounded unless allocation-free)
     size_t remaining() const { return base_ ? (off_ < size_ ? size_ - off_ : 0) : SIZE_MAX; }
     bool fixed() const { return fixed_ != nullptr; }
@@ -1012,24 +1031,42 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         WideRows wide = {};
         if (b == BIN_GLOBAL) {
             const unsigned long long list = h2.wide_items * sizeof(WideItem) + wide_list_bytes(c->num_cus);
-            const bool windows = h2.wide_items < (1ull << 31) && windows_fit(list);
-            const bool indexed = windows && index_pays(h2.num.work[b], list);
-            wide.blocks = cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt;
-            if (windows) {
-                wide.nunits = units;
-                wide.K = K;
-                wide.index = indexed ? (int *)ar.raw((size_t)index_bytes) : nullptr;
-                wide.items_cap = (long long)h2.wide_items;
-                wide.items = ar.get<WideItem>((size_t)wide.items_cap);
-                wide.places = ar.get<unsigned>((size_t)wide_item_blocks(cnt, c->num_cus) * WIDE_LISTS);
-                wide.ctr = ar.get<WideCount>(1);
-            } else {
-                wide.cur_stride = ((long long)h2.num.max_na[b] + 63) & ~63LL;
-                wide.ft_stride = keep_dirs ? (((long long)h2.num.max_span[b] + 63) & ~63LL) : 0;
-                wide.ws = ar.get<int>(wide_ws_ints(wide.cur_stride, wide.ft_stride, wide.blocks) + 1);
+            // the widest form whose memory can be had: a plan's capture pass repeats the one
+            // the recording run found
+            int form = h2.wide_items >= (1ull << 31) || !windows_fit(list) ? WIDE_PER_ROW
+                       : index_pays(h2.num.work[b], list)                  ? WIDE_INDEXED
+                                                                           : WIDE_SEARCHED;
+            if (cap)
+                form = mode.plan->wide_form;
+            const Arena::Mark before = ar.mark();
+            for (; form != WIDE_NONE; ++form) {
+                wide = {};
+                wide.blocks = cnt > 2 * c->num_cus ? 2 * c->num_cus : cnt;
+                if (form == WIDE_PER_ROW) {
+                    wide.cur_stride = ((long long)h2.num.max_na[b] + 63) & ~63LL;
+                    wide.ft_stride = keep_dirs ? (((long long)h2.num.max_span[b] + 63) & ~63LL) : 0;
+                    wide.ws = ar.get<int>(wide_ws_ints(wide.cur_stride, wide.ft_stride, wide.blocks) + 1);
+                    if (wide.ws)
+                        break;
+                } else {
+                    wide.nunits = units;
+                    wide.K = K;
+                    wide.index = form == WIDE_INDEXED ? (int *)ar.raw((size_t)index_bytes) : nullptr;
+                    wide.items_cap = (long long)h2.wide_items;
+                    wide.items = ar.get<WideItem>((size_t)wide.items_cap);
+                    wide.places = ar.get<unsigned>((size_t)wide_item_blocks(cnt, c->num_cus) * WIDE_LISTS);
+                    wide.ctr = ar.get<WideCount>(1);
+                    if ((wide.index || form == WIDE_SEARCHED) && wide.items && wide.places && wide.ctr)
+                        break;
+                }
+                if (cap)
+                    return fail(HSMU_ERR_NOMEM, "wide-row workspace");
+                ar.rewind(before);
             }
-            if (windows ? ((indexed && !wide.index) || !wide.items || !wide.places || !wide.ctr) : !wide.ws)
+            if (form == WIDE_NONE)
                 return fail(HSMU_ERR_NOMEM, "wide-row workspace");
+            if (mode.plan)
+                mode.plan->wide_form = form;
         }
         if (timing)
             HIP_TRY(hipEventRecord(c->evb[b][0], s));
