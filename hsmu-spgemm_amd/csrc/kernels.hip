@@ -1229,24 +1229,60 @@ DEVI int find_instance(const long long *__restrict__ off, int count, long long x
     return lo;
 }
 
-// The stacking kernels take chunks of STACK_CHUNK places per workgroup, and in a chunk one
-// instance after the other: the search for the first and the instance's fields are scalar,
-// and a lane's loads need no lookup.  (A lookup per entry, stepping through the offsets in
-// memory, kept 512 Laplacians' 45 M entries at 684 us for A and B, and a binary search per
-// row their pointers at 75 us; now 252, one pass for both, and 20.)  each(i, lo, hi): places [lo, hi) are
-// instance i's.
+// The stacking kernels take chunks of STACK_CHUNK places per workgroup.  A chunk of few
+// instances goes one instance after the other: the search for the first and the instance's
+// fields are scalar, and a lane's loads need no lookup.  (A lookup per entry, stepping through
+// the offsets in memory, kept 512 Laplacians' 45 M entries at 684 us for A and B, and a binary
+// search per row their pointers at 75 us; now 252, one pass for both, and 20.)  In a chunk of
+// more than STACK_FEW instances, where that is a chain of short waits, every lane finds its
+// places' instances in a copy of the offsets in LDS: calls of 100,000 instances of 1 row 7.0 ms
+// one after the other and 1.3 so, 20,000 of 9 rows 0.88 and 0.5, 4,000 of 64 rows 345 and 330 us,
+// with 4, 16 or 64 as the limit.
+// each(i, q, hi): this lane's places of instance i are q, q + 256, ... below hi.
 constexpr int STACK_CHUNK = 4096;
+constexpr int STACK_FEW = 16;
 constexpr int STACK_U = 4; // loads in flight per lane
 template <typename Each>
 DEVI void stack_chunks(const long long *__restrict__ off, int step, int count, int64_t n, Each each)
 {
+    __shared__ unsigned short first[STACK_CHUNK]; // of the instances in the chunk, in it
+    const int t = threadIdx.x;
     for (int64_t base = (int64_t)blockIdx.x * STACK_CHUNK; base < n; base += (int64_t)gridDim.x * STACK_CHUNK) {
         const int64_t end = base + STACK_CHUNK < n ? base + STACK_CHUNK : n;
-        for (int i = find_instance(off, count, base, step); i < count; ++i) {
-            const int64_t i0 = off[i] + (int64_t)i * step, i1 = off[i + 1] + (int64_t)(i + 1) * step;
-            if (i0 >= end)
-                break;
-            each(i, i0 > base ? i0 : base, i1 < end ? i1 : end);
+        const int a = find_instance(off, count, base, step), more = a + STACK_FEW;
+        if (more >= count || off[more] + (int64_t)more * step >= end) {
+            for (int i = a; i < count; ++i) {
+                const int64_t i0 = off[i] + (int64_t)i * step, i1 = off[i + 1] + (int64_t)(i + 1) * step;
+                if (i0 >= end)
+                    break;
+                each(i, (i0 > base ? i0 : base) + t, i1 < end ? i1 : end);
+            }
+            continue;
+        }
+        const int b = find_instance(off, count, end - 1, step);
+        const bool fit = b - a < STACK_CHUNK; // (more only with empty instances among them)
+        if (fit) {
+            __syncthreads();
+            for (int i = t; i <= b - a; i += 256) // (the first starts at the chunk's start or before)
+                first[i] = (unsigned short)(i ? off[a + i] + (int64_t)(a + i) * step - base : 0);
+            __syncthreads();
+        }
+        for (int64_t q = base + t; q < end; q += 256) {
+            int i = a;
+            if (fit) {
+                int lo = 0, hi = b - a; // the last instance that starts at q or before
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (first[mid] <= (unsigned)(q - base))
+                        lo = mid;
+                    else
+                        hi = mid - 1;
+                }
+                i += lo;
+            } else {
+                i = find_instance(off, count, q, step);
+            }
+            each(i, q, q + 1);
         }
     }
 }
@@ -1256,14 +1292,14 @@ __global__ __launch_bounds__(256) void k_batch_rowptr(int which, int count, cons
                                                       const long long *__restrict__ eoff, int64_t nrows, int64_t nnz,
                                                       int *__restrict__ out, DevStats *st)
 {
-    stack_chunks(roff, 0, count, nrows, [&](int i, int64_t lo, int64_t hi) {
+    stack_chunks(roff, 0, count, nrows, [&](int i, int64_t q, int64_t hi) {
         const BatchInst &I = inst[i];
         const int64_t r0 = roff[i];
         const int *__restrict__ rp = (which ? I.Brp : I.Arp) - r0;
         const int e0 = (int)eoff[i];
-        for (int64_t g = lo + threadIdx.x; g < hi; g += 256)
+        for (int64_t g = q; g < hi; g += 256)
             out[g] = e0 + rp[g];
-        if (lo == r0 && threadIdx.x == 0 && lo < hi &&
+        if (q == r0 && q < hi && // the instance's first row
             (rp[r0] != 0 || (long long)rp[r0 + (which ? I.K : I.M)] != eoff[i + 1] - eoff[i]))
             atomicOr(&st->err, ERR_ROWPTR);
     });
@@ -1272,9 +1308,9 @@ __global__ __launch_bounds__(256) void k_batch_rowptr(int which, int count, cons
 }
 
 template <typename T>
-DEVI void copy_entries(const T *__restrict__ src, T *__restrict__ dst, int64_t lo, int64_t hi)
+DEVI void copy_entries(const T *__restrict__ src, T *__restrict__ dst, int64_t q, int64_t hi)
 {
-    for (int64_t e = lo + threadIdx.x; e < hi; e += STACK_U * 256) {
+    for (int64_t e = q; e < hi; e += STACK_U * 256) {
         T v[STACK_U];
 #pragma unroll
         for (int u = 0; u < STACK_U; ++u)
@@ -1294,12 +1330,12 @@ __global__ __launch_bounds__(256) void k_batch_entries(int which, int count, con
                                                        void *__restrict__ val, DevStats *st)
 {
     int bad = 0;
-    stack_chunks(eoff, 0, count, nnz, [&](int i, int64_t lo, int64_t hi) {
+    stack_chunks(eoff, 0, count, nnz, [&](int i, int64_t q, int64_t hi) {
         const BatchInst &I = inst[i];
         const int64_t e0 = eoff[i];
         const int *__restrict__ src = (which ? I.Bcol : I.Acol) - e0;
         const int K = I.K, N = I.N, k0 = (int)koff[i];
-        for (int64_t e = lo + threadIdx.x; e < hi; e += STACK_U * 256) {
+        for (int64_t e = q; e < hi; e += STACK_U * 256) {
             int c[STACK_U];
 #pragma unroll
             for (int u = 0; u < STACK_U; ++u)
@@ -1322,9 +1358,9 @@ __global__ __launch_bounds__(256) void k_batch_entries(int which, int count, con
         }
         const void *from = which ? I.Bval : I.Aval;
         if (val32)
-            copy_entries((const float *)from - e0, (float *)val, lo, hi);
+            copy_entries((const float *)from - e0, (float *)val, q, hi);
         else
-            copy_entries((const double *)from - e0, (double *)val, lo, hi);
+            copy_entries((const double *)from - e0, (double *)val, q, hi);
     });
     if (bad)
         atomicOr(&st->err, bad);
@@ -1335,10 +1371,10 @@ __global__ __launch_bounds__(256) void k_batch_split(int count, const long long 
                                                      int rp64, long long *__restrict__ bases)
 {
     // C_i's M_i + 1 pointers lie from mo[i] + i
-    stack_chunks(mo, 1, count, mo[count] + count, [&](int i, int64_t lo, int64_t hi) {
+    stack_chunks(mo, 1, count, mo[count] + count, [&](int i, int64_t first, int64_t hi) {
         const long long *__restrict__ rp = crp - i;
         const long long v0 = crp[mo[i]];
-        for (int64_t q = lo + threadIdx.x; q < hi; q += 256) {
+        for (int64_t q = first; q < hi; q += 256) {
             const long long v = rp[q] - v0;
             if (rp64)
                 ((long long *)out)[q] = v;
@@ -1346,9 +1382,8 @@ __global__ __launch_bounds__(256) void k_batch_split(int count, const long long 
                 ((int *)out)[q] = (int)v;
         }
     });
-    if (blockIdx.x == 0)
-        for (int i = threadIdx.x; i <= count; i += 256)
-            bases[i] = crp[mo[i]];
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i <= count; i += (int64_t)gridDim.x * 256)
+        bases[i] = crp[mo[i]];
 }
 
 static unsigned stack_grid(int64_t n)
