@@ -489,7 +489,8 @@ DEVI void stream_or(const Stream<G> &st, long long w0, const Operands &op, u64 *
 struct SmallNone { // symbolic: no values
     typedef float V;
 };
-template <int G, typename P>
+// TOPS: some row of the launch may have a third level (which costs registers).
+template <int G, typename P, bool TOPS>
 DEVI void small_rows(const int *__restrict__ rows, const int *__restrict__ count_p, int slice_bytes, const Operands &op,
                      int *__restrict__ rnnz, const long long *__restrict__ crp, int *__restrict__ Ccol,
                      typename P::V *__restrict__ Cval, int *err, unsigned *queue, int block, int blocks)
@@ -523,38 +524,47 @@ DEVI void small_rows(const int *__restrict__ rows, const int *__restrict__ count
                 n = (int)(crp[row + 1] - cb);
             }
         }
-        const SmallLayout L = small_layout(NUM, S, n, nA, p);
+        const SmallLayout L = small_layout(NUM, TOPS, S, n, nA, p);
+        uint2 *tops = (uint2 *)(slice + L.top);
         uint2 *coarse = (uint2 *)(slice + L.coarse); // words of the row: marked words, those before
         uint2 *fine = (uint2 *)(slice + L.fine);     // marked words: columns, slots before
         double *vals = (double *)(slice + L.vals);
         int *cols = (int *)(slice + L.cols);
         uint4 *rec = (uint4 *)(slice + L.rec);
         unsigned *ends = (unsigned *)(slice + L.ends); // per step of G pairs: it ends an entry
-        // this lane's entry of A
-        int start = 0, len = 0;
-        u64 a = 0;
-        if (l < nA) {
-            const typename Vec2<int>::type b = load2(op.Brp + op.Acol[a0 + l]);
-            start = b.x;
-            len = b.y - b.x;
-            if constexpr (NUM)
-                a = (u64)__double_as_longlong((double)Aval[a0 + l]);
-        }
         // (the last 16 bytes may reach into cols, which is written later, or past the layout's
         // end, which is a multiple of 16)
-        for (int q = L.ends + 16 * l; q < (NUM ? L.cols : L.vals); q += 16 * G)
-            *(uint4 *)(slice + q) = make_uint4(0, 0, 0, 0);
-        // its pairs among the row's
-        const unsigned cnt = (unsigned)(len + 1) >> 1;
-        unsigned tot;
-        const unsigned ex = group_excl_scan<G, unsigned>(cnt | (cnt ? 1u << 16 : 0u), nullptr, tot);
-        const unsigned first = ex & 0xffff, total = tot & 0xffff;
-        __syncthreads();
-        if (cnt) {
-            const unsigned last = first + cnt - 1;
-            atomicOr(&ends[last / G], 1u << (last & (G - 1)));
-            rec[ex >> 16] = make_uint4((unsigned)start - STREAM_V * first, (unsigned)(start + len), (unsigned)a,
-                                       (unsigned)(a >> 32));
+        auto clear = [&]() {
+            for (int q = L.ends + 16 * l; q < (NUM ? L.cols : L.vals); q += 16 * G)
+                *(uint4 *)(slice + q) = make_uint4(0, 0, 0, 0);
+        };
+        // the entries of A, one per lane at a time: their pairs among the row's
+        unsigned total = 0, nrec = 0;
+        for (int c = 0; c == 0 || (G == 32 && __any(c < nA)); c += G) {
+            int start = 0, len = 0;
+            u64 a = 0;
+            if (c + l < nA) {
+                const typename Vec2<int>::type b = load2(op.Brp + op.Acol[a0 + c + l]);
+                start = b.x;
+                len = b.y - b.x;
+                if constexpr (NUM)
+                    a = (u64)__double_as_longlong((double)Aval[a0 + c + l]);
+            }
+            if (c == 0)
+                clear();
+            const unsigned cnt = (unsigned)(len + 1) >> 1;
+            unsigned tot;
+            const unsigned ex = group_excl_scan<G, unsigned>(cnt | (cnt ? 1u << 16 : 0u), nullptr, tot);
+            const unsigned first = total + (ex & 0xffff);
+            __syncthreads();
+            if (cnt) {
+                const unsigned last = first + cnt - 1;
+                atomicOr(&ends[last / G], 1u << (last & (G - 1)));
+                rec[nrec + (ex >> 16)] = make_uint4((unsigned)start - STREAM_V * first, (unsigned)(start + len),
+                                                    (unsigned)a, (unsigned)(a >> 32));
+            }
+            total += tot & 0xffff;
+            nrec += tot >> 16;
         }
         __syncthreads();
         // element 0 of a live pair is always the row's (at the array's end it is the load's
@@ -587,20 +597,6 @@ DEVI void small_rows(const int *__restrict__ rows, const int *__restrict__ count
             }
             e += __popc(bits);
         }
-        // mark the words
-        auto word = [&](int c) { return (c >> 5) - w0; };
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (live[u]) {
-                const int w = word(c0[u]);
-                atomicOr(&coarse[w >> 5].x, 1u << (w & 31));
-            }
-            if (two[u]) {
-                const int w = word(c1[u]);
-                atomicOr(&coarse[w >> 5].x, 1u << (w & 31));
-            }
-        }
-        __syncthreads();
         // exclusive prefix of the words' bits in their second halves, four words a lane; the sum
         auto prefix = [&](uint2 *m, int nw) {
             unsigned sum = 0;
@@ -622,25 +618,64 @@ DEVI void small_rows(const int *__restrict__ rows, const int *__restrict__ count
             }
             return sum;
         };
-        const int nf = (int)prefix(coarse, L.ncoarse);
-        __syncthreads();
+        // a column's word, and its place in the coarse and fine level once those above are done
+        auto word = [&](int c) { return (c >> 5) - w0; };
+        auto place = [&](const uint2 *m, int w) {
+            const uint2 x = m[w >> 5];
+            return x.y + (unsigned)__popc(under(x.x, w));
+        };
+        auto coarse_of = [&](int w) { return TOPS && L.ntop ? place(tops, w >> 5) : (unsigned)w >> 5; };
+        auto mark = [&](uint2 *m, unsigned at, int bit) { atomicOr(&m[at].x, 1u << (bit & 31)); };
+        int nc = L.ncoarse;
+        if constexpr (TOPS) {
+            if (__any(L.ntop > 0)) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (live[u] && L.ntop)
+                        mark(tops, (unsigned)word(c0[u]) >> 10, word(c0[u]) >> 5);
+                    if (two[u] && L.ntop)
+                        mark(tops, (unsigned)word(c1[u]) >> 10, word(c1[u]) >> 5);
+                }
+                __syncthreads();
+                const int marked = (int)prefix(tops, L.ntop);
+                nc = L.ntop ? marked : nc;
+                __syncthreads();
+            }
+        }
+        // mark the words
+        int nf = 2 * S;
+        if (__any(!L.flat)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (live[u] && !L.flat)
+                    mark(coarse, coarse_of(word(c0[u])), word(c0[u]));
+                if (two[u] && !L.flat)
+                    mark(coarse, coarse_of(word(c1[u])), word(c1[u]));
+            }
+            __syncthreads();
+            const int marked = (int)prefix(coarse, nc);
+            nf = L.flat ? nf : marked;
+            __syncthreads();
+        }
         // mark the columns
         unsigned f0[U], f1[U];
         auto fine_of = [&](int c) {
             const int w = word(c);
-            const uint2 m = coarse[w >> 5];
-            return m.y + (unsigned)__popc(under(m.x, w));
+            if (L.flat)
+                return (unsigned)w;
+            const uint2 x = coarse[coarse_of(w)];
+            return x.y + (unsigned)__popc(under(x.x, w));
         };
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             f0[u] = f1[u] = 0;
             if (live[u]) {
                 f0[u] = fine_of(c0[u]);
-                atomicOr(&fine[f0[u]].x, 1u << (c0[u] & 31));
+                mark(fine, f0[u], c0[u]);
             }
             if (two[u]) {
                 f1[u] = fine_of(c1[u]);
-                atomicOr(&fine[f1[u]].x, 1u << (c1[u] & 31));
+                mark(fine, f1[u], c1[u]);
             }
         }
         __syncthreads();
@@ -686,13 +721,13 @@ DEVI void small_rows(const int *__restrict__ rows, const int *__restrict__ count
 // widest groups first (a launch of a few thousand rows is all start and end: a random product
 // of 30,011 ragged rows takes 164 us in place of 199; but with the registers of the widest
 // form a batch whose rows are all of one bin takes 3.79 ms in place of 3.70).
-template <int G, typename P>
+template <int G, typename P, bool TOPS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_small_bin(
     const int *__restrict__ rows, const int *__restrict__ count, int slice, Operands op, int *__restrict__ rnnz,
     const long long *__restrict__ crp, int *__restrict__ Ccol, typename P::V *__restrict__ Cval, int *err,
     unsigned *queue)
 {
-    small_rows<G, P>(rows, count, slice, op, rnnz, crp, Ccol, Cval, err, queue, blockIdx.x, gridDim.x);
+    small_rows<G, P, TOPS>(rows, count, slice, op, rnnz, crp, Ccol, Cval, err, queue, blockIdx.x, gridDim.x);
 }
 
 struct SmallBins {
@@ -700,7 +735,7 @@ struct SmallBins {
     unsigned *queue[BIN_SHARED];
     int slice[BIN_SHARED], blocks[BIN_SHARED];
 };
-template <typename P>
+template <typename P, bool TOPS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_small_rows(
     SmallBins bins, Operands op, int *__restrict__ rnnz, const long long *__restrict__ crp, int *__restrict__ Ccol,
     typename P::V *__restrict__ Cval, int *err)
@@ -708,8 +743,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void
     int block = blockIdx.x;
 #define SMALL(B, G)                                                                                                    \
     if (block < bins.blocks[B])                                                                                        \
-        return small_rows<G, P>(bins.rows[B], bins.count[B], bins.slice[B], op, rnnz, crp, Ccol, Cval, err,            \
-                                bins.queue[B], block, bins.blocks[B]);                                                 \
+        return small_rows<G, P, TOPS>(bins.rows[B], bins.count[B], bins.slice[B], op, rnnz, crp, Ccol, Cval, err,      \
+                                      bins.queue[B], block, bins.blocks[B]);                                           \
     block -= bins.blocks[B];
     SMALL(2, 32) SMALL(1, 16) SMALL(0, 8)
 #undef SMALL
@@ -1893,9 +1928,9 @@ template <int G> static int row_slice(int need)
 // Waves per CU of a bin: a few times what is resident, so that a wave's start is paid for
 // several groups of rows and the last ones to end are short.
 constexpr int SMALL_WAVES = 128;
-template <typename P>
+template <typename P, bool TOPS>
 static hipError_t small_launch(const int *rows, long long stride, const BinStats *bins_dev, const int *count,
-                               const int *max_need, const Operands &op, int *rnnz, const long long *crp, int *Ccol,
+                               const BinStats &bins, const Operands &op, int *rnnz, const long long *crp, int *Ccol,
                                void *Cval, int *err, int num_cus, unsigned (*queue)[MAX_XCDS],
                                unsigned long long *lds_bytes, hipStream_t s)
 {
@@ -1905,15 +1940,15 @@ static hipError_t small_launch(const int *rows, long long stride, const BinStats
     for (int k = 0; k < BIN_SHARED; ++k) {
         if (count[k] <= 0)
             continue;
-        const int rpb = BLOCK >> (k + 3);
+        const int rpb = BLOCK >> (k + 3), need = bins.max_need[k];
         b.rows[k] = rows + k * stride;
         b.count[k] = &bins_dev->count[k];
         b.queue[k] = queue ? queue[k] : nullptr;
-        b.slice[k] = k == 0 ? row_slice<8>(max_need[k]) : k == 1 ? row_slice<16>(max_need[k]) : row_slice<32>(max_need[k]);
+        b.slice[k] = k == 0 ? row_slice<8>(need) : k == 1 ? row_slice<16>(need) : row_slice<32>(need);
         const size_t bytes = (size_t)b.slice[k] * rpb;
         lds = lds > bytes ? lds : bytes;
         const int64_t groups = ((int64_t)count[k] + rpb - 1) / rpb, most = (int64_t)SMALL_WAVES * num_cus;
-        int64_t blocks = row_grid(k_small_rows<P>, BLOCK, bytes, groups, num_cus, b.queue[k]);
+        int64_t blocks = row_grid(k_small_rows<P, TOPS>, BLOCK, bytes, groups, num_cus, b.queue[k]);
         blocks = blocks < most ? blocks : most;
         // whole rounds over the XCDs, so that each bin's blocks start at the first
         b.blocks[k] = (int)((blocks + MAX_XCDS - 1) / MAX_XCDS * MAX_XCDS);
@@ -1925,27 +1960,30 @@ static hipError_t small_launch(const int *rows, long long stride, const BinStats
         return hipSuccess;
 #define SMALL(B, G)                                                                                                    \
     if (b.blocks[B] == grid)                                                                                           \
-        hipLaunchKernelGGL((k_small_bin<G, P>), dim3((unsigned)grid), dim3(BLOCK), lds, s, b.rows[B], b.count[B],      \
+        hipLaunchKernelGGL((k_small_bin<G, P, TOPS>), dim3((unsigned)grid), dim3(BLOCK), lds, s, b.rows[B], b.count[B],      \
                            b.slice[B], op, rnnz, crp, Ccol, (typename P::V *)Cval, err, b.queue[B]);                   \
     else
     SMALL(0, 8) SMALL(1, 16) SMALL(2, 32)
 #undef SMALL
-    hipLaunchKernelGGL((k_small_rows<P>), dim3((unsigned)grid), dim3(BLOCK), lds, s, b, op, rnnz, crp, Ccol,
+    hipLaunchKernelGGL((k_small_rows<P, TOPS>), dim3((unsigned)grid), dim3(BLOCK), lds, s, b, op, rnnz, crp, Ccol,
                        (typename P::V *)Cval, err);
     return hipGetLastError();
 }
 
 hipError_t launch_small(int form, const int *rows, long long stride, const BinStats *bins_dev, const int *count,
-                        const int *max_need, const Operands &op, int *rnnz, const long long *crp, int *Ccol, void *Cval,
+                        const BinStats &bins, const Operands &op, int *rnnz, const long long *crp, int *Ccol, void *Cval,
                         int *err, int num_cus, unsigned (*queue)[MAX_XCDS], unsigned long long *lds_bytes, hipStream_t s)
 {
     unsigned long long ignored = 0;
     if (!lds_bytes)
         lds_bytes = &ignored;
-    auto *f = form == SMALL_SYMBOLIC ? small_launch<SmallNone>
-              : form == SMALL_F64    ? small_launch<PrecF64>
-                                     : small_launch<PrecF32C>;
-    return f(rows, stride, bins_dev, count, max_need, op, rnnz, crp, Ccol, Cval, err, num_cus, queue, lds_bytes, s);
+    bool tops = false; // a row may have a third level
+    for (int k = 0; k < BIN_SHARED; ++k)
+        tops |= count[k] > 0 && small_coarse(bins.max_span[k]) > SMALL_DIRECT;
+    auto *f = form == SMALL_SYMBOLIC ? (tops ? small_launch<SmallNone, true> : small_launch<SmallNone, false>)
+              : form == SMALL_F64    ? (tops ? small_launch<PrecF64, true> : small_launch<PrecF64, false>)
+                                     : (tops ? small_launch<PrecF32C, true> : small_launch<PrecF32C, false>);
+    return f(rows, stride, bins_dev, count, bins, op, rnnz, crp, Ccol, Cval, err, num_cus, queue, lds_bytes, s);
 }
 
 template <int G, bool TL>
@@ -2116,7 +2154,9 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
         if (r != hipSuccess)                                                                                           \
             e = r;                                                                                                     \
     }
-#define CFGL(P) CFG(k_small_rows<P>) CFG((k_small_bin<8, P>)) CFG((k_small_bin<16, P>)) CFG((k_small_bin<32, P>))
+#define CFGT(P, T)                                                                                                     \
+    CFG((k_small_rows<P, T>)) CFG((k_small_bin<8, P, T>)) CFG((k_small_bin<16, P, T>)) CFG((k_small_bin<32, P, T>))
+#define CFGL(P) CFGT(P, false) CFGT(P, true)
 #define CFGS(TL)                                                                                                       \
     CFG((k_symbolic_row<64, TL>)) CFG((k_symbolic_row<128, TL>)) CFG((k_symbolic_row<256, TL>))                        \
     CFG((k_symbolic_row<512, TL>)) CFG((k_symbolic_row<1024, TL>))
@@ -2127,6 +2167,7 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
     CFGR(PrecF64, false) CFGR(PrecF32C, false) CFGR(PrecF64, true) CFGR(PrecF32C, true)
 #undef CFGR
 #undef CFGL
+#undef CFGT
 #undef CFGS
     CFG(k_symbolic_wide)
     CFG(k_numeric_window<PrecF64>) CFG(k_numeric_window<PrecF32C>)

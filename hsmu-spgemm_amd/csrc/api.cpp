@@ -903,7 +903,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
 
     // ---- 3. symbolic ----
     HIP_TRY(make_tiles(h1.sym));
-    HIP_TRY(launch_small(SMALL_SYMBOLIC, binrows, M, &dst->sym, h1.sym.count, h1.sym.max_need, op, rnnz, nullptr, nullptr,
+    HIP_TRY(launch_small(SMALL_SYMBOLIC, binrows, M, &dst->sym, h1.sym.count, h1.sym, op, rnnz, nullptr, nullptr,
                          nullptr, nullptr, c->num_cus, opts.persistent ? dst->queue[0] : nullptr, nullptr, s));
     for (int b = BIN_SHARED; b < NBINS; ++b) {
         const int cnt = h1.sym.count[b];
@@ -1015,7 +1015,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
             count[k] = !timing || k == b ? h2.num.count[k] : 0;
         if (timing && count[b] > 0)
             HIP_TRY(hipEventRecord(c->evb[b][0], s));
-        HIP_TRY(launch_small(fp32 ? SMALL_F32C : SMALL_F64, binrows, M, &dst->num, count, h2.num.max_need, op, nullptr,
+        HIP_TRY(launch_small(fp32 ? SMALL_F32C : SMALL_F64, binrows, M, &dst->num, count, h2.num, op, nullptr,
                              crp, Ccol, Cval, errp, c->num_cus, opts.persistent ? dst->queue[1] : nullptr,
                              &lds_launched, s));
         if (timing && count[b] > 0)

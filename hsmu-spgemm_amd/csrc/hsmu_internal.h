@@ -147,6 +147,9 @@ HSMU_HD inline int dir_entries(int S, int tp) { return use_sparse(S, tp) ? ((S +
 constexpr int LAYOUT_CAP = 1 << 18;
 constexpr int LAYOUT_NONE = 1 << 30;
 
+// Tiles a row that shares a wave may span (its top words alone would fill a workgroup's LDS).
+constexpr int SMALL_SPAN = 1 << 22;
+
 // A B row with at least this many elements left in a window is walked by a whole wave (rows
 // wider than LDS without an index of B).
 constexpr int LONG_SEG = 256;
@@ -154,30 +157,47 @@ constexpr int LONG_SEG = 256;
 // ---- rows that share a wave ------------------------------------------------------------------
 //
 // G = 8, 16 or 32 lanes per row, each with SMALL_U pairs of elements of its B rows (a pair
-// of an entry's odd last element is half empty) and at most one entry of A:
+// of an entry's odd last element is half empty) and one entry of A (32 lanes: or more):
 //   rec    16[nA]   entries with elements: first less STREAM_V times the first pair, end, a_ij
 //   ends   u32[U]   a bit per pair of each step of G: it ends an entry
-//   coarse 8[...]   per 32 words (of 32 columns) of the span: which are marked, those before
-//   fine   8[F]     per marked word, F <= min(p, words): its columns, slots before
+//   top    8[...]   per 32 coarse words: which are marked, those before
+//   coarse 8[...]   per 32 words (of 32 columns): which are marked, those before
+//   fine   8[F]     per word: its columns, slots before
 //   vals   f64[n]   numeric: accumulators
 //   cols   i32[n]   numeric: columns
-// (from ends to vals zeroed together, 16 bytes at a time; coarse and fine in fours)
+// (from ends to vals zeroed together, 16 bytes at a time; levels in fours)
+// The fine level holds the marked words, at most one per product; with a word or less per
+// product in the span it holds them all, and no level above it is needed (where all lanes
+// would mark the same few bits).  The coarse level holds the span's coarse words, or, for a
+// span of more than SMALL_DIRECT of them that the row leaves mostly empty, the marked ones.
 constexpr int SMALL_U = 4;
+constexpr int SMALL_DIRECT = 128;
 struct SmallLayout {
-    int rec, ends, coarse, fine, vals, cols, ncoarse, bytes;
+    int rec, ends, top, coarse, fine, vals, cols, ntop, ncoarse, bytes;
+    bool flat;
 };
-HSMU_HD inline SmallLayout small_layout(bool numeric, int S, int n, int nA, int p)
+HSMU_HD inline int small_coarse(int S) { return (2 * S + 31) >> 5; }
+HSMU_HD inline SmallLayout small_layout(bool numeric, bool tops, int S, int n, int nA, int p)
 {
     SmallLayout L = {};
-    L.ncoarse = (2 * S + 31) >> 5;
-    const int f = p < 2 * S ? p : 2 * S;
+    const int words = 2 * S;
+    L.flat = words <= p;
+    const int f = L.flat ? words : p;
+    int nc = L.flat ? 0 : small_coarse(S);
+    if (tops && nc > SMALL_DIRECT && nc > 2 * (((nc + 31) >> 5) + p)) {
+        L.ntop = (nc + 31) >> 5;
+        nc = p;
+    }
+    L.ncoarse = nc;
     int o = 0;
     L.rec = o;
     o += 16 * nA;
     L.ends = o;
     o += 4 * SMALL_U;
+    L.top = o;
+    o += 8 * ((L.ntop + 3) & ~3);
     L.coarse = o;
-    o += 8 * ((L.ncoarse + 3) & ~3);
+    o += 8 * ((nc + 3) & ~3);
     L.fine = o;
     o += 8 * ((f + 3) & ~3);
     L.vals = o;
@@ -192,8 +212,9 @@ HSMU_HD inline SmallLayout small_layout(bool numeric, int S, int n, int nA, int 
 // LDS of such a row on G lanes, if it is one: all its pairs fit
 HSMU_HD inline int small_need(bool numeric, int G, int S, int n, int nA, long long p)
 {
-    return nA <= G && p + nA <= 2 * SMALL_U * G && S <= LAYOUT_CAP ? small_layout(numeric, S, n, nA, (int)p).bytes
-                                                                  : LAYOUT_NONE;
+    return (nA <= G || G == 32) && p + nA <= 2 * SMALL_U * G && S <= SMALL_SPAN
+               ? small_layout(numeric, true, S, n, nA, (int)p).bytes
+               : LAYOUT_NONE;
 }
 
 // ---- one row per workgroup (64 lanes or more): the element stream ------------------------
@@ -365,10 +386,11 @@ struct Operands {
 };
 
 // Rows that share a wave, those of the bins with count[b] > 0 in one launch (bin b's list at
-// rows + b * stride).  Symbolic: rnnz; numeric: the rows of C, lds_bytes as launch_numeric.
+// rows + b * stride, its needs and spans in bins).  Symbolic: rnnz; numeric: the rows of C,
+// lds_bytes as launch_numeric.
 enum { SMALL_SYMBOLIC, SMALL_F64, SMALL_F32C };
 hipError_t launch_small(int form, const int *rows, long long stride, const BinStats *bins_dev, const int *count,
-                        const int *max_need, const Operands &op, int *rnnz, const long long *crp, int *Ccol, void *Cval,
+                        const BinStats &bins, const Operands &op, int *rnnz, const long long *crp, int *Ccol, void *Cval,
                         int *err, int num_cus, unsigned (*queue)[MAX_XCDS], unsigned long long *lds_bytes, hipStream_t s);
 
 // Global-memory workspace (bin BIN_GLOBAL): gws_blocks regions of gws_stride u64 each;
