@@ -1931,7 +1931,7 @@ constexpr int SMALL_WAVES = 128;
 template <typename P, bool TOPS>
 static hipError_t small_launch(const int *rows, long long stride, const BinStats *bins_dev, const int *count,
                                const BinStats &bins, const Operands &op, int *rnnz, const long long *crp, int *Ccol,
-                               void *Cval, int *err, int num_cus, unsigned (*queue)[MAX_XCDS],
+                               void *Cval, int *err, int num_cus, unsigned (*queue)[QUEUE_INTS],
                                unsigned long long *lds_bytes, hipStream_t s)
 {
     SmallBins b = {};
@@ -1972,7 +1972,7 @@ static hipError_t small_launch(const int *rows, long long stride, const BinStats
 
 hipError_t launch_small(int form, const int *rows, long long stride, const BinStats *bins_dev, const int *count,
                         const BinStats &bins, const Operands &op, int *rnnz, const long long *crp, int *Ccol, void *Cval,
-                        int *err, int num_cus, unsigned (*queue)[MAX_XCDS], unsigned long long *lds_bytes, hipStream_t s)
+                        int *err, int num_cus, unsigned (*queue)[QUEUE_INTS], unsigned long long *lds_bytes, hipStream_t s)
 {
     unsigned long long ignored = 0;
     if (!lds_bytes)

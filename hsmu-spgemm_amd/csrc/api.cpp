@@ -904,7 +904,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     // ---- 3. symbolic ----
     HIP_TRY(make_tiles(h1.sym));
     HIP_TRY(launch_small(SMALL_SYMBOLIC, binrows, M, &dst->sym, h1.sym.count, h1.sym, op, rnnz, nullptr, nullptr,
-                         nullptr, nullptr, c->num_cus, opts.persistent ? dst->queue[0] : nullptr, nullptr, s));
+                         nullptr, nullptr, c->num_cus, opts.persistent ? dw->queue[0] : nullptr, nullptr, s));
     for (int b = BIN_SHARED; b < NBINS; ++b) {
         const int cnt = h1.sym.count[b];
         if (cnt <= 0)
@@ -912,7 +912,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         HIP_TRY(launch_symbolic(b, binrows + (size_t)b * M, &dst->sym.count[b], cnt, h1.sym.max_need[b], op, rnnz,
                                 tshift, h1.sym.nsparse[b] > 0 ? 1 : 0, gws, gws_stride, c->num_cus,
                                 gws_blocks, (int)bp.lds_row_max,
-                                opts.persistent ? dst->queue[0][b] : nullptr, s));
+                                opts.persistent ? dw->queue[0][b] : nullptr, s));
     }
     // Arrays of C handed to the caller; dropped again (one-shot calls) on any failure.
     struct Outs {
@@ -1016,7 +1016,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         if (timing && count[b] > 0)
             HIP_TRY(hipEventRecord(c->evb[b][0], s));
         HIP_TRY(launch_small(fp32 ? SMALL_F32C : SMALL_F64, binrows, M, &dst->num, count, h2.num, op, nullptr,
-                             crp, Ccol, Cval, errp, c->num_cus, opts.persistent ? dst->queue[1] : nullptr,
+                             crp, Ccol, Cval, errp, c->num_cus, opts.persistent ? dw->queue[1] : nullptr,
                              &lds_launched, s));
         if (timing && count[b] > 0)
             HIP_TRY(hipEventRecord(c->evb[b][1], s));
@@ -1073,7 +1073,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         HIP_TRY(launch_numeric(b, fp32 ? 1 : 0, binrows + (size_t)b * M, &dst->num.count[b], cnt, h2.num.max_need[b], op,
                                crp, Ccol, Cval, bshift, h2.num.nsparse[b] > 0 ? 1 : 0, wide, errp,
                                c->num_cus,
-                               opts.persistent ? dst->queue[1][b] : nullptr, &lds_launched, s));
+                               opts.persistent ? dw->queue[1][b] : nullptr, &lds_launched, s));
         if (timing)
             HIP_TRY(hipEventRecord(c->evb[b][1], s));
     }

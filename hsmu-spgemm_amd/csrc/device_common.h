@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "hsmu_internal.h"
+
 namespace hsmu {
 
 typedef unsigned long long u64;
@@ -120,7 +122,7 @@ DEVI int xcd_block(int b, int n, int nx)
 }
 
 // Device work queue of the persistent row kernels: the n row groups of a launch are cut
-// into nx contiguous ranges, one per XCD, each with a counter q[x] (zero at launch) that
+// into nx contiguous ranges, one per XCD, each with a counter q[x * QUEUE_STRIDE] (zero at launch) that
 // hands out chunks of `chunk` consecutive groups.  A workgroup takes the next chunk of its
 // own XCD's range (xq starts at blockIdx.x % nx) and, once that range is used up, of the
 // following ranges in turn, so the groups one XCD works on stay neighbours (shared rows
@@ -135,9 +137,9 @@ DEVI void pull_chunk(unsigned *q, int n, int chunk, int nx, int &xq, int *s)
             const int x = (xq + k) % nx;
             const int lo = (int)((long long)n * x / nx), hi = (int)((long long)n * (x + 1) / nx);
             const unsigned nch = (unsigned)((hi - lo + chunk - 1) / chunk);
-            if (__hip_atomic_load(&q[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= nch)
+            if (__hip_atomic_load(&q[x * QUEUE_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= nch)
                 continue;
-            const unsigned v = atomicAdd(&q[x], 1u);
+            const unsigned v = atomicAdd(&q[x * QUEUE_STRIDE], 1u);
             if (v < nch) {
                 got = lo + (int)v * chunk;
                 end = got + chunk < hi ? got + chunk : hi;

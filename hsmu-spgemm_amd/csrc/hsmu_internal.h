@@ -68,8 +68,6 @@ struct DevStats {
     unsigned long long wide_items; // windows the wide rows may need, at most (numeric binning)
     BinStats sym;
     BinStats num;
-    // work-queue counters of the persistent LDS kernels: [phase][bin][XCD]
-    unsigned queue[2][NBINS][MAX_XCDS];
 };
 
 // The counters as a binning hands them to the host (pinned memory): seq, a number of the
@@ -87,10 +85,19 @@ struct BinSum {
 };
 constexpr int BIN_PARTS = 16;
 
-// Everything on the device that a call needs zeroed: the counters, the blocks done and the
-// places taken of each binning or scan, and (behind it) the words of the two chained scans.
+// Work-queue counters of a persistent LDS kernel, one per XCD, each on a cache line of its own
+// (on one line the pulls of all XCDs wait for each other: 200,000 rows of 8 entries times 24
+// into 64 columns, 100,000 groups in each phase, 6.3 ms, so 1.6; 24 times 24 into 100,000
+// columns 5.2 and 2.7).
+constexpr int QUEUE_STRIDE = 32;
+constexpr int QUEUE_INTS = MAX_XCDS * QUEUE_STRIDE;
+
+// Everything on the device that a call needs zeroed: the counters, those of the work queues
+// [phase][bin], the blocks done and the places taken of each binning or scan, and (behind it)
+// the words of the two chained scans.
 struct DevWork {
     DevStats st;
+    alignas(128) unsigned queue[2][NBINS][QUEUE_INTS];
     BinSum sums[2][BIN_PARTS * NBINS]; // symbolic, numeric
     unsigned done[2], ticket[2];
     // followed by btiles_blocks(nnz(B)) + rowptr_blocks(M) 64-bit words
@@ -391,7 +398,7 @@ struct Operands {
 enum { SMALL_SYMBOLIC, SMALL_F64, SMALL_F32C };
 hipError_t launch_small(int form, const int *rows, long long stride, const BinStats *bins_dev, const int *count,
                         const BinStats &bins, const Operands &op, int *rnnz, const long long *crp, int *Ccol, void *Cval,
-                        int *err, int num_cus, unsigned (*queue)[MAX_XCDS], unsigned long long *lds_bytes, hipStream_t s);
+                        int *err, int num_cus, unsigned (*queue)[QUEUE_INTS], unsigned long long *lds_bytes, hipStream_t s);
 
 // Global-memory workspace (bin BIN_GLOBAL): gws_blocks regions of gws_stride u64 each;
 // a region holds gws_tiles 64-bit masks followed by gws_tiles 32-bit offsets, with

@@ -113,7 +113,7 @@ LAUNCH(launch_copy, const void *, void *, size_t, int, hipStream_t)
 LAUNCH(launch_brows, int64_t, int64_t, int64_t, ci, ci, BRow *, DevStats *, int, hipStream_t)
 LAUNCH(launch_pad_b, ci, const void *, int, int, int *, void *, hipStream_t)
 LAUNCH(launch_small, int, ci, long long, const BinStats *, ci, const BinStats &, const Operands &, int *, const long long *, int *,
-       void *, int *, int, unsigned (*)[MAX_XCDS], u64 *, hipStream_t)
+       void *, int *, int, unsigned (*)[QUEUE_INTS], u64 *, hipStream_t)
 LAUNCH(launch_btiles, int64_t, int64_t, int64_t, ci, ci, int *, int *, u64 *, BRow *, u64 *, unsigned *, DevStats *,
        hipStream_t)
 LAUNCH(launch_symbolic, int, ci, ci, int, int, const Operands &, int *, int, int, u64 *, long long, int, int, int,
