@@ -799,6 +799,10 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     bp.lds_block_budget = opts.lds_block_budget > 0 ? opts.lds_block_budget : 8 * 1024;
     if (bp.lds_block_budget > lds_dyn)
         bp.lds_block_budget = lds_dyn;
+    // two rows of a workgroup may take 16 KiB: rows of 192 products over 2 M columns, 12 KB for
+    // two, take 672 us per 200,000 so and 1,490 with a wave or two each (10 KB), over 100,000
+    // columns 498 and 781
+    bp.lds_pair_budget = opts.lds_block_budget > 0 ? bp.lds_block_budget : 16 * 1024;
     bp.per_lane = opts.tiles_per_lane > 0 ? opts.tiles_per_lane : 32;
     bp.force_global = opts.force_global;
     bp.lds_cu = lds_dyn;

@@ -33,6 +33,7 @@ constexpr int ERR_PLAN = 32;    // a replayed plan's inputs changed structure
 
 struct BinParams {
     int lds_block_budget; // LDS bytes per workgroup for bins with several rows per workgroup
+    int lds_pair_budget;  // the same for two rows per workgroup
     int lds_row_max;      // LDS bytes one row may use
     int per_lane;         // work items per lane
     int lds_cu;           // LDS bytes of a CU

@@ -534,7 +534,7 @@ DEVI int choose_bin(long long work, Need need, const BinParams &bp)
     // the row's LDS whatever its width
     while (b < BIN_SHARED) {
         const int nd = need(b);
-        if (nd <= bp.lds_row_max && nd * (BLOCK >> (b + 3)) <= bp.lds_block_budget)
+        if (nd <= bp.lds_row_max && nd * (BLOCK >> (b + 3)) <= (b < BIN_SHARED - 1 ? bp.lds_block_budget : bp.lds_pair_budget))
             break;
         ++b;
     }

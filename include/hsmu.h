@@ -113,7 +113,8 @@ typedef struct hsmu_opts {
                                  global-memory path; 0 = device maximum (in the numeric phase
                                  64 KiB where wide rows can be cut into windows) */
     int32_t lds_block_budget; /* LDS bytes per workgroup for bins that pack several rows
-                                 into one workgroup (one wave); 0 = default (8 KiB) */
+                                 into one workgroup (one wave); 0 = default (8 KiB, 16 for two
+                                 rows) */
     int32_t products_per_lane;/* numeric work per lane that sets a row's lane count; 0 = 48 */
     int32_t tiles_per_lane;   /* symbolic work per lane that sets a row's lane count; 0 = 32 */
     int32_t timing;           /* hipEvents into hsmu_stats (each costs the device a few us):
