@@ -796,6 +796,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     // 8 KiB per one-wave workgroup that packs several rows: 20 such workgroups fit a CU's
     // 160 KiB; rows needing more move up to a bin with fewer rows per workgroup (measured
     // best on the batched Laplacians)
+    bp.lds_window_max = bp.lds_row_max;
     bp.lds_block_budget = opts.lds_block_budget > 0 ? opts.lds_block_budget : 8 * 1024;
     if (bp.lds_block_budget > lds_dyn)
         bp.lds_block_budget = lds_dyn;
@@ -967,13 +968,13 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
             most = left / 2;
         return places <= products / WIDE_INDEX_WORK && index_bytes <= most && list <= left - index_bytes;
     };
-    // rows of more than WINDOW_ROW_MIN are wide where windows with the index are certain: with
-    // room for the lists of M full rows
+    // rows of more than WINDOW_ROW_MIN that fill their windows are wide where windows with the
+    // index are certain: with room for the lists of M full rows
     const int n_most = (int)(N < INT_MAX ? N : INT_MAX);
     const unsigned long long list_most =
         (unsigned long long)M * wide_row_items(n_most, n_most / 64 + 1) * sizeof(WideItem) + wide_list_bytes(c->num_cus);
     if (bp.lds_row_max > WINDOW_ROW_MIN && windows_fit(list_most) && index_pays(h1.num_wide_work, list_most))
-        bp.lds_row_max = WINDOW_ROW_MIN;
+        bp.lds_window_max = WINDOW_ROW_MIN;
     HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp,
                               rp64 || batch || narrow_later ? nullptr : (int *)Crp, bp, binrows,
                               words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1], host,

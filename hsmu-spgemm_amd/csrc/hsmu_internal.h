@@ -35,6 +35,7 @@ struct BinParams {
     int lds_block_budget; // LDS bytes per workgroup for bins with several rows per workgroup
     int lds_pair_budget;  // the same for two rows per workgroup
     int lds_row_max;      // LDS bytes one row may use
+    int lds_window_max;   // the same for a row whose windows would be filled (window_filled)
     int per_lane;         // work items per lane
     int lds_cu;           // LDS bytes of a CU
     int force_global;
@@ -452,6 +453,14 @@ constexpr int WIDE_DENSE = WIDE_UNIT / 4;
 constexpr int WIDE_DENSE_WORK = 3 * WIDE_UNIT;
 constexpr unsigned WIDE_DENSE_MIN = 8192;
 constexpr int WIDE_HEAVY = 16 * WIDE_UNIT;
+// Entries enough to fill a quarter of the row's windows; spread out further, it runs faster in one
+// piece as long as LDS holds it (2,000 rows of 6,400 entries over 2 M columns: 738 us as 20 windows
+// of 320 entries each, 320 us in LDS; an eighth or half in place of a quarter: the R-MAT square of
+// scale 18 takes 16.15 and 16.64 ms, with a quarter 16.16).
+HSMU_HD inline bool window_filled(int n, int S)
+{
+    return 4LL * n * WIDE_TILES * WIDE_UMAX >= (long long)S * WIDE_UNIT;
+}
 struct __attribute__((aligned(16))) WideItem {
     int row;
     unsigned units;     // first unit | number of units << 24

@@ -509,7 +509,7 @@ hipError_t launch_brows(int64_t K, int64_t N, int64_t nnz, const int *rp, const 
 
 // Bin of one row: lanes from work (per_lane items per lane, 8..1024 lanes), then fewer
 // rows per workgroup until the workgroup's LDS fits the budget; rows whose own need
-// exceeds lds_row_max go to the global-memory bin.  need(b): the row's LDS in bin b.
+// exceeds row_max go to the global-memory bin.  need(b): the row's LDS in bin b.
 // Reference ranges being replaced: src/bining.cuh:12 (symbolic), :121 (tile OR), :228
 // (numeric).
 // Lanes per row: the stream that rows with a workgroup of their own walk costs about the
@@ -523,7 +523,7 @@ hipError_t launch_brows(int64_t K, int64_t N, int64_t nnz, const int *rp, const 
 // limits the workgroups, take 17.8 ms on the square of scale 18 against 19.2 ms with 8; 24
 // slow a banded square by 4%.
 template <typename Need>
-DEVI int choose_bin(long long work, Need need, const BinParams &bp)
+DEVI int choose_bin(long long work, Need need, int row_max, const BinParams &bp)
 {
     if (bp.force_global)
         return BIN_GLOBAL;
@@ -534,7 +534,7 @@ DEVI int choose_bin(long long work, Need need, const BinParams &bp)
     // the row's LDS whatever its width
     while (b < BIN_SHARED) {
         const int nd = need(b);
-        if (nd <= bp.lds_row_max && nd * (BLOCK >> (b + 3)) <= (b < BIN_SHARED - 1 ? bp.lds_block_budget : bp.lds_pair_budget))
+        if (nd <= row_max && nd * (BLOCK >> (b + 3)) <= (b < BIN_SHARED - 1 ? bp.lds_block_budget : bp.lds_pair_budget))
             break;
         ++b;
     }
@@ -546,12 +546,12 @@ DEVI int choose_bin(long long work, Need need, const BinParams &bp)
         if ((long long)nd * wgs <= bp.lds_cu)
             break;
         const int wider = need(b + 1);
-        if (wider > bp.lds_row_max)
+        if (wider > row_max)
             break; // (the stream's tables grow a little with the width)
         nd = wider;
         ++b;
     }
-    return nd > bp.lds_row_max ? BIN_GLOBAL : b;
+    return nd > row_max ? BIN_GLOBAL : b;
 }
 
 // One row as the binning sees it.
@@ -602,7 +602,7 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
         if (numeric) {
             work = r.prod;
             auto nd = [&](int bin) { return num_need(bin, r.S, r.nc, r.nA, r.tp, r.prod); };
-            at.b = choose_bin(work, nd, bp);
+            at.b = choose_bin(work, nd, window_filled(r.nc, r.S) ? bp.lds_window_max : bp.lds_row_max, bp);
             need = nd(at.b);
         } else {
             work = r.tp;
@@ -614,7 +614,7 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
             auto nd = [&](int bin) {
                 return wide && bin < BIN_SHARED ? LAYOUT_NONE : sym_need(bin, r.S, r.nA, r.tp, r.prod);
             };
-            at.b = choose_bin(work, nd, bp);
+            at.b = choose_bin(work, nd, bp.lds_row_max, bp);
             need = nd(at.b);
             // directory entries kept for the numeric phase: the row's form in an LDS bin, the
             // flat span for rows the symbolic phase handles in global memory

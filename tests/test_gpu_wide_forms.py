@@ -71,3 +71,22 @@ def test_hub_row_takes_no_index():
         finally:
             ctx.close()
     assert held[1] - held[0] < 45e6
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_rows_that_fill_their_windows(ctx, fp32):
+    """Rows of 130 KB of LDS at the span up to which they are cut into windows (a quarter full),
+    and a tile wider, which stay in LDS."""
+    rng = np.random.default_rng(13)
+    N, n = 64 * 7600, 5000
+    print(f"[gpu-case] rows at a quarter of their windows, fp32 {fp32}", flush=True)
+
+    def row(tiles, first):  # n columns over exactly that many tiles
+        inner = rng.choice(np.arange(first * 64 + 64, (first + tiles - 1) * 64), n - 2, replace=False)
+        return np.concatenate([[first * 64 + 63], inner, [(first + tiles - 1) * 64]])
+
+    B = csr([row(7500, 0), row(7501, 0), row(7500, 77), row(7501, 99)], N, rng)
+    A = csr([[0], [1], [2], [3], [0], [3]], 4, rng)
+    C, st = ctx.spgemm(A, B, precision=hsmu.HSMU_FP32_COMP if fp32 else hsmu.HSMU_FP64)
+    check(C, A, B, fp32)
+    assert st["num_bin_rows"][8] == 3 and st["rows_nonempty"] == 6
