@@ -788,16 +788,23 @@ __global__ __launch_bounds__(G) void k_symbolic_row(const int *__restrict__ rows
         st.red = red;
         const int words = (L.doff - L.bits) >> 3;
         const long long rd = op.dir_mask ? uniform64(op.rdir[row]) & ~RDIR_TWO : -1;
+        auto tiles = [&](int e) {
+            const int j = op.Acol[a0 + e];
+            const typename Vec2<int>::type t = load2(op.tptr + j);
+            return Segment{t.x, t.y - t.x, 0};
+        };
+        // two-level rows walk their tiles twice: the lane's first entry is kept (with more lanes
+        // that costs an R-MAT square of scale 18 0.5%)
+        constexpr bool KEEP = TL && G <= 128;
+        Segment mine = {0, 0, 0};
+        if (KEEP && l < nA)
+            mine = tiles(l);
         for (int t = l; t < W; t += G)
             dm[t] = 0;
         for (int q = l; q < words; q += G)
             st.bits[q] = 0;
         __syncthreads();
-        auto tiles_of = [&](int e) {
-            const int j = op.Acol[a0 + e];
-            const typename Vec2<int>::type t = load2(op.tptr + j);
-            return Segment{t.x, t.y - t.x, 0};
-        };
+        auto tiles_of = [&](int e) { return KEEP && e < G ? mine : tiles(e); };
         if (!sparse)
             st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
                 stream_or<G, OR_FLAT>(t, w0, op, dm, nullptr, nullptr, mn);
@@ -990,6 +997,26 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
         const int nv = dense ? 64 * S : n;
         const long long rd = op.dir_mask ? uniform64(kept_dir(op, row, sparse)) : -1;
         const int words = (L.doff - L.bits) >> 3;
+        auto tiles = [&](int e) {
+            const int j = op.Acol[a0 + e];
+            const typename Vec2<int>::type t = load2(op.tptr + j);
+            return Segment{t.x, t.y - t.x, 0};
+        };
+        auto entries = [&](int e) {
+            const int j = op.Acol[a0 + e];
+            const typename Vec2<int>::type b = load2(op.Brp + j);
+            const double a = (double)Aval[a0 + e];
+            return Segment{b.x, b.y - b.x, (u64)__double_as_longlong(a)};
+        };
+        // two-level rows may walk their tiles twice and then their elements: the lane's first
+        // entry is kept
+        constexpr bool KEEP = TL && G <= 128;
+        Segment my_tiles = {0, 0, 0}, mine = {0, 0, 0};
+        if (KEEP && l < nA) {
+            if (rd < 0)
+                my_tiles = tiles(l);
+            mine = entries(l);
+        }
         for (int q = 2 * l; q < nv; q += 2 * G) // (the array is padded to 16 bytes)
             *(double2 *)(vals + q) = make_double2(0.0, 0.0);
         for (int q = l; q < words; q += G)
@@ -1004,11 +1031,7 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
                 dm[t] = 0;
         }
         __syncthreads();
-        auto tiles_of = [&](int e) {
-            const int j = op.Acol[a0 + e];
-            const typename Vec2<int>::type t = load2(op.tptr + j);
-            return Segment{t.x, t.y - t.x, 0};
-        };
+        auto tiles_of = [&](int e) { return KEEP && e < G ? my_tiles : tiles(e); };
         auto rezero = [&]() { // the stream's bits, for its next run
             __syncthreads();
             for (int q = l; q < words; q += G)
@@ -1073,12 +1096,7 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
             raise_internal(err);
         __syncthreads();
         if (ok) { // uniform
-            auto rows_of = [&](int e) {
-                const int j = op.Acol[a0 + e];
-                const typename Vec2<int>::type b = load2(op.Brp + j);
-                const double a = (double)Aval[a0 + e];
-                return Segment{b.x, b.y - b.x, (u64)__double_as_longlong(a)};
-            };
+            auto rows_of = [&](int e) { return KEEP && e < G ? mine : entries(e); };
             if (dense)
                 st.run(nA, rows_of, [&](const Stream<G> &t, long long w0) {
                     stream_add<G, SLOT_DENSE, P>(t, w0, op, nullptr, nullptr, fm, foff, vals, mn);
