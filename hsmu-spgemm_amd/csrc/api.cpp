@@ -966,20 +966,22 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     auto windows_fit = [&](unsigned long long list) {
         return keep_dirs && list <= ar.remaining() && units < (1 << 24); // allocation-free: the workspace left
     };
-    auto index_pays = [&](unsigned long long products, unsigned long long list) {
+    auto index_fits = [&](unsigned long long list) {
         const unsigned long long left = ar.remaining();
         unsigned long long most =
             opts.wide_scratch_mb > 0 ? (unsigned long long)opts.wide_scratch_mb << 20 : c->total_mem / 4;
         if (most > left / 2)
             most = left / 2;
-        return places <= products / WIDE_INDEX_WORK && index_bytes <= most && list <= left - index_bytes;
+        return index_bytes <= most && list <= left - index_bytes;
     };
     // rows of more than WINDOW_ROW_MIN that fill their windows are wide where windows with the
-    // index are certain: with room for the lists of M full rows
+    // index are worth it (a product of theirs per place) and certain: with room for the lists of M
+    // full rows
     const int n_most = (int)(N < INT_MAX ? N : INT_MAX);
     const unsigned long long list_most =
         (unsigned long long)M * wide_row_items(n_most, n_most / 64 + 1) * sizeof(WideItem) + wide_list_bytes(c->num_cus);
-    if (bp.lds_row_max > WINDOW_ROW_MIN && windows_fit(list_most) && index_pays(h1.num_wide_work, list_most))
+    if (bp.lds_row_max > WINDOW_ROW_MIN && places <= h1.num_wide_work && windows_fit(list_most) &&
+        index_fits(list_most))
         bp.lds_window_max = WINDOW_ROW_MIN;
     HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp,
                               rp64 || batch || narrow_later ? nullptr : (int *)Crp, bp, binrows,
@@ -1044,9 +1046,15 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
             const unsigned long long list = h2.wide_items * sizeof(WideItem) + wide_list_bytes(c->num_cus);
             // the widest form whose memory can be had: a plan's capture pass repeats the one
             // the recording run found
-            int form = h2.wide_items >= (1ull << 31) || !windows_fit(list) ? WIDE_PER_ROW
-                       : index_pays(h2.num.work[b], list)                  ? WIDE_INDEXED
-                                                                           : WIDE_SEARCHED;
+            const unsigned long long rows = (unsigned long long)cnt, entries = h2.num.nnz_a[b];
+            // what a search takes: per window (half of their bound) and WIDE_STEP entries of A, the
+            // halvings of a row of B of the mean length beyond two
+            const unsigned long long windows = h2.wide_items / (2 * rows) + 1;
+            const int halvings = 64 - __builtin_clzll(h2.num.work[b] / entries + 1);
+            const unsigned long long loads = (entries / WIDE_STEP + rows) * windows * (halvings > 2 ? halvings - 2 : 0);
+            int form = h2.wide_items >= (1ull << 31) || !windows_fit(list)       ? WIDE_PER_ROW
+                       : places <= WIDE_INDEX_PLACES * loads && index_fits(list) ? WIDE_INDEXED
+                                                                                 : WIDE_SEARCHED;
             if (cap)
                 form = mode.plan->wide_form;
             const Arena::Mark before = ar.mark();

@@ -429,14 +429,18 @@ constexpr int WINDOW_ROW_MIN = 64 * 1024;
 // (the masks and slots of 24 units leave room for three workgroups per CU; R-MAT scale 18 with 4 /
 // 8 / 16 / 24 units 17.8 / 17.8 / 16.4 / 16.2 ms, 4 and 8 in an earlier state that took 17.4 with 16)
 constexpr int WIDE_UMAX = 24;
-// The index costs a place per row of B and unit (2 to 3.4 ps each), whatever the wide rows are;
-// a search costs 0.8 (Zipf panel) to 4 ps (R-MAT scale 16) per product of theirs.  So it is made
-// where they have this many products for each place.  With the index and without: R-MAT squares
-// of scale 16 / 18 2.06 / 16.2 and 2.60 / 20.7 ms, a Zipf panel 4.14 and 5.38 (115 products per
-// place or more); a grid of 1 M rows, one of them with 20,000 entries, 1.47 and 0.81 ms, of 4 M
-// rows 13.7 and 4.6 ms and 15 GB (less than 0.01); one row with 1 M entries the same with both
-// (0.04).
-constexpr unsigned long long WIDE_INDEX_WORK = 4;
+// The index costs a place per row of B and unit (2 to 3.4 ps each), whatever the wide rows are.
+// A search costs a chain of loads per WIDE_STEP entries of A in a window, as long as a row of B
+// takes halvings; with few entries in B's rows (up to two halvings) it costs what the index's two
+// reads do.  The line lies between the products on both sides of it: rows of R-MAT scale 20 take
+// with the index and without 3.8 and 4.1 ms (4 rows, 1,070 places per halving), 4.2 and 5.0 (16
+// rows, 590), 8.9 and 14.3 (1,024 rows); rows of a Zipf panel 257 and 221 us (2 rows), 307 and 299
+// (16 rows, 400), 420 and 426 (64 rows, 100), 4.14 and 5.38 ms (2,000 rows); R-MAT squares of
+// scale 16 / 18 2.06 / 16.2 and 2.60 / 20.7 ms; a grid of 1 M rows, one of them with 20,000
+// entries, 1.47 and 0.81 ms, of 4 M rows 13.7 (and 15 GB) and 4.6 ms; 200 rows of 50,000 entries
+// times single ones 4.9 and 3.0 ms.
+constexpr unsigned long long WIDE_INDEX_PLACES = 700;
+constexpr int WIDE_STEP = 256;
 constexpr int WIDE_TILES = WIDE_UNIT / 64;     // tiles of a unit
 constexpr int WIDE_BUCKETS = 32;               // windows are listed by their place in C's columns
 constexpr int WIDE_LISTS = 1 + 2 * WIDE_BUCKETS;

@@ -192,6 +192,7 @@ int main()
         g_stats[0].dir_total = 4096;
         g_stats[0].num_wide_work = g_stats[1].num.work[BIN_GLOBAL] = 1ull << 30;
         g_stats[0].sym.count[NLDS - 1] = g_stats[1].num.count[BIN_GLOBAL] = 4;
+        g_stats[1].num.nnz_a[BIN_GLOBAL] = 1 << 24;
         g_stats[1].num.max_na[BIN_GLOBAL] = t.na;
         g_stats[1].num.max_span[BIN_GLOBAL] = 960;
         g_stats[1].wide_items = t.items;
