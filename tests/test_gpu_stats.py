@@ -10,7 +10,7 @@ def test_lds_of_rows_that_share_a_wave(ctx):
     """lds_launched is the LDS all row groups ask for: the same per row on a small grid and on
     one of more groups than there are workgroups (their 8-lane rows differ only at the rim)."""
     per_row = []
-    for n in (150, 900):
+    for n in (300, 900):
         A = hsmu.gen_laplace2d(n)
         print(f"[gpu-case] lds_launched of a {n} x {n} grid", flush=True)
         _, st = ctx.spgemm(A, A)
