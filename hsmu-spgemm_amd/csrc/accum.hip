@@ -1634,7 +1634,8 @@ template <bool FILL>
 __global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ rows, const int *__restrict__ count_p,
                                                       Operands op, const long long *__restrict__ crp, long long U,
                                                       WideItem *__restrict__ items, long long cap,
-                                                      unsigned *__restrict__ places, int *err)
+                                                      unsigned *__restrict__ places, unsigned *__restrict__ hot,
+                                                      long long hot_cap, long long hot_min, WideCount *ctr, int *err)
 {
     __shared__ unsigned cnt[WIDE_LISTS]; // heavy windows, others, dense ones
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1648,7 +1649,9 @@ __global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ ro
         const unsigned n = (unsigned)(uniform64(crp[row + 1]) - uniform64(crp[row]));
         const WideDir d(op, uniform(op.rmin[row]), uniform(op.rmax[row]), uniform64(op.rdir[row]));
         const int F = d.entries();
-        const float work = (float)uniform64(op.rprod[row]) / (float)n; // products per entry of C_i
+        const long long prod = uniform64(op.rprod[row]);
+        const float work = (float)prod / (float)n; // products per entry of C_i
+        const int nA = uniform(op.Arp[row + 1]) - uniform(op.Arp[row]);
         const int U0 = d.mn / WIDE_TILES, U1 = (d.mn + d.S - 1) / WIDE_TILES + 1; // units of the row
         int wu = 0, wv = 0; // lane i holds the i-th window found: its units [wu, wv) and
         unsigned wa = 0, we = 0; // the entries before its start and end
@@ -1665,6 +1668,11 @@ __global__ __launch_bounds__(WI_BS) void k_wide_items(const int *__restrict__ ro
                         items[q] = WideItem{row, (unsigned)wu | ((unsigned)(wv - wu) << 24), wa, we - wa};
                     else // cannot happen: wide_row_items bounds them
                         raise_internal(err);
+                    if (hot && q < cap && prod - (n - (we - wa)) > hot_min && (long long)nA * (we - wa) >= hot_min) {
+                        const unsigned h = atomicAdd(&ctr->hot, 1u);
+                        if (h < hot_cap) // (as above)
+                            hot[h] = q;
+                    }
                 }
             }
             nw = 0;
@@ -1736,6 +1744,22 @@ __global__ __launch_bounds__(1024) void k_wide_order(unsigned *__restrict__ plac
         ctr->dense = done - dense_s >= WIDE_DENSE_MIN ? dense_s : done;
         ctr->listed = done;
         ctr->taken[0] = ctr->taken[1] = 0;
+        ctr->hot = ctr->sums = 0;
+        ctr->parts = 0;
+    }
+}
+
+// The elements of B's row j in units [u0, u1).
+template <bool INDEX>
+DEVI int2 window_elements(const Operands &op, const int *__restrict__ index, long long U, int u0, int u1, int j)
+{
+    if constexpr (INDEX) {
+        const int *ix = index + (long long)j * (U + 1);
+        return make_int2(ix[u0], ix[u1]);
+    } else {
+        const typename Vec2<int>::type r = load2(op.Brp + j);
+        const int s0 = first_element(op.Bcol, r.x, r.y, u0 * WIDE_UNIT);
+        return make_int2(s0, u1 < U ? first_element(op.Bcol, s0, r.y, u1 * WIDE_UNIT) : r.y);
     }
 }
 
@@ -1807,24 +1831,15 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
         const unsigned units = uniform(item.y), base = uniform(item.z);
         const int cnt = (int)uniform(item.w);
         const int u0 = (int)(units & 0xffffffu), u1 = DENSE ? u0 + 1 : u0 + (int)(units >> 24);
-        const int a0 = uniform(ra), nA = uniform(rb) - a0;
+        const int a0 = uniform(ra), nA = cnt ? uniform(rb) - a0 : 0; // (0: cut into parts)
         const WideDir d(op, uniform(rmn), uniform(rmx), uniform64(rrd));
         const long long cb = uniform64(rcb) + base;
         const int T0 = u0 * WIDE_TILES, nt = (u1 - u0) * WIDE_TILES;
         auto segment = [&](int e, int col) {
             if (e >= nA)
                 return Segment{0, 0, 0};
-            int s0, s1;
-            if constexpr (INDEX) {
-                const int *ix = index + (long long)col * (U + 1);
-                s0 = ix[u0];
-                s1 = ix[u1];
-            } else {
-                const typename Vec2<int>::type r = load2(op.Brp + col);
-                s0 = first_element(op.Bcol, r.x, r.y, u0 * WIDE_UNIT);
-                s1 = u1 < U ? first_element(op.Bcol, s0, r.y, u1 * WIDE_UNIT) : r.y;
-            }
-            return Segment{s0, s1 - s0, (u64)__double_as_longlong((double)Aval[a0 + e])};
+            const int2 r = window_elements<INDEX>(op, index, U, u0, u1, col);
+            return Segment{r.x, r.y - r.x, (u64)__double_as_longlong((double)Aval[a0 + e])};
         };
         const Segment first = segment(l, j);
         // dense: lane i of wave w holds tile w * TW + i
@@ -1833,6 +1848,7 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
         unsigned to = 0;
         if constexpr (DENSE) {
             tm = d.tile(T0 + w * TW + (lane < TW ? lane : TW - 1) - d.mn, to);
+            tm = cnt ? tm : 0;
         } else {
             for (int t = l; t < nt; t += BS) {
                 unsigned off;
@@ -1907,6 +1923,144 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
         }
         __syncthreads();
     }
+}
+
+// Windows that may be hot, a wave each: the parts of those that are, which leave the list (no
+// entries, no units).  An estimate that is off only makes the parts uneven; a window for whose
+// parts or sums there is no room stays whole.
+template <bool INDEX>
+__global__ __launch_bounds__(256) void k_wide_cut(const unsigned *__restrict__ hot, unsigned hot_cap, long long hot_min,
+                                                  WideItem *__restrict__ items, WideCount *ctr, Operands op,
+                                                  const int *__restrict__ index, long long U,
+                                                  const long long *__restrict__ crp, WidePart *__restrict__ parts,
+                                                  u64 part_cap, WideSum *__restrict__ sums, double *__restrict__ sum_val,
+                                                  unsigned sum_cap)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned n = ctr->hot < hot_cap ? ctr->hot : hot_cap;
+    for (unsigned i = blockIdx.x * 4 + w; i < n; i += gridDim.x * 4) {
+        const unsigned place = uniform(hot[i]);
+        const WideItem it = items[place];
+        const int row = uniform(it.row);
+        const unsigned units = uniform(it.units), base = uniform(it.base), cnt = uniform(it.cnt);
+        const int u0 = (int)(units & 0xffffffu), u1 = u0 + (int)(units >> 24);
+        const int a0 = uniform(op.Arp[row]), nA = uniform(op.Arp[row + 1]) - a0;
+        const int ns = nA < WIDE_SAMPLE ? nA : WIDE_SAMPLE;
+        long long found = 0;
+        for (int q = lane; q < ns; q += 64) {
+            const int2 r = window_elements<INDEX>(op, index, U, u0, u1, op.Acol[a0 + (int)((long long)q * nA / ns)]);
+            found += r.y - r.x;
+        }
+        const long long est = wave_sum(found) * nA / ns;
+        if (est < hot_min)
+            continue;
+        const long long want = est / (hot_min / WIDE_PARTS), most = want < nA ? want : nA;
+        const int k = (int)(most < 4096 ? most : 4096);
+        unsigned sum = 0;
+        u64 at = 0;
+        if (lane == 0) {
+            sum = atomicAdd(&ctr->sums, 1u);
+            if (sum < sum_cap)
+                at = atomicAdd(&ctr->parts, (u64)k);
+        }
+        sum = uniform(sum);
+        at = uniform64(at);
+        if (sum >= sum_cap)
+            continue;
+        const bool fits = at + (u64)k <= part_cap;
+        if (lane == 0)
+            sums[sum] = WideSum{crp[row] + base, fits ? (long long)cnt : 0};
+        if (!fits) { // (every place below ctr->parts is read)
+            for (u64 q = at + lane; q < part_cap; q += 64)
+                parts[q] = WidePart{row, (unsigned)u0, base, 0, 1, 1, (int)sum, 0};
+            continue;
+        }
+        if (lane == 0)
+            items[place] = WideItem{row, (unsigned)u0, base, 0};
+        for (int q = lane; q < k; q += 64)
+            parts[at + q] = WidePart{row, units, base, cnt, (int)((long long)nA * q / k), (int)((long long)nA * (q + 1) / k),
+                                     (int)sum, 0};
+        for (unsigned q = lane; q < cnt; q += 64)
+            sum_val[(size_t)sum * WIDE_UNIT + q] = 0.0;
+    }
+}
+
+// The parts of hot windows: as k_numeric_windows' compact form, over a range of the row's entries.
+// Their sums meet by atomics in sum_val (k_wide_sums takes them to C); a window's first part writes
+// its columns.
+template <typename P, int BS, bool INDEX>
+__global__ __launch_bounds__(BS) void k_numeric_parts(const WidePart *__restrict__ parts,
+                                                      const WideCount *__restrict__ ctr, u64 part_cap, Operands op,
+                                                      const int *__restrict__ index, long long U,
+                                                      const long long *__restrict__ crp, int *__restrict__ Ccol,
+                                                      double *sum_val)
+{
+    typedef typename P::V V;
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ u64 red[16];
+    constexpr int NW = BS / 64, words = stream_window(BS) / 64;
+    double *vals = (double *)lds;
+    Stream<BS> st;
+    st.rec = (uint4 *)(vals + WIDE_UNIT);
+    st.bits = (u64 *)(st.rec + BS);
+    u64 *wm = st.bits + words;
+    unsigned short *wo = (unsigned short *)(wm + WW_TILES);
+    st.wb = wo + WW_TILES;
+    st.red = red;
+    const int l = threadIdx.x, lane = l & 63, w = uniform((int)(threadIdx.x >> 6));
+    const V *__restrict__ Aval = (const V *)op.Aval;
+    const u64 n = ctr->parts < part_cap ? ctr->parts : part_cap;
+    for (u64 i = blockIdx.x; i < n; i += gridDim.x) {
+        const WidePart p = parts[i];
+        const int row = uniform(p.row), sum = uniform(p.sum), e0 = uniform(p.e0), cnt = (int)uniform(p.cnt);
+        const unsigned units = uniform(p.units), base = uniform(p.base);
+        const int u0 = (int)(units & 0xffffffu), u1 = u0 + (int)(units >> 24);
+        const int a0 = uniform(op.Arp[row]) + e0, nA = uniform(p.e1) - e0;
+        const WideDir d(op, uniform(op.rmin[row]), uniform(op.rmax[row]), uniform64(op.rdir[row]));
+        const long long cb = uniform64(crp[row]) + base;
+        const int T0 = u0 * WIDE_TILES, nt = (u1 - u0) * WIDE_TILES;
+        for (int t = l; t < nt; t += BS) {
+            unsigned off;
+            wm[t] = d.tile(T0 + t - d.mn, off);
+            wo[t] = (unsigned short)(off - base);
+        }
+        for (int q = 2 * l; q < cnt; q += 2 * BS) // (WIDE_UNIT is even)
+            *(double2 *)(vals + q) = make_double2(0.0, 0.0);
+        for (int q = l; q < words; q += BS)
+            st.bits[q] = 0;
+        __syncthreads();
+        st.run(
+            nA,
+            [&](int e) {
+                const int2 r = window_elements<INDEX>(op, index, U, u0, u1, op.Acol[a0 + e]);
+                return Segment{r.x, r.y - r.x, (u64)__double_as_longlong((double)Aval[a0 + e])};
+            },
+            [&](const Stream<BS> &t, long long w0) {
+                stream_add<BS, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, wm, wo, vals, T0);
+            });
+        __syncthreads();
+        double *sv = sum_val + (size_t)sum * WIDE_UNIT;
+        for (int q = l; q < cnt; q += BS)
+            unsafeAtomicAdd(&sv[q], vals[q]);
+        if (e0 == 0)
+            for (int t = w; t < nt; t += NW) {
+                const u64 m = uniform64(wm[t]);
+                if ((m >> lane) & 1ull)
+                    Ccol[cb + wo[t] + (unsigned)mbcnt(m)] = ((T0 + t) << 6) + lane;
+            }
+        __syncthreads();
+    }
+}
+
+template <typename P>
+__global__ __launch_bounds__(256) void k_wide_sums(const WideSum *__restrict__ sums, const WideCount *__restrict__ ctr,
+                                                   unsigned sum_cap, const double *__restrict__ sum_val,
+                                                   typename P::V *__restrict__ Cval)
+{
+    const unsigned n = ctr->sums < sum_cap ? ctr->sums : sum_cap;
+    for (unsigned i = blockIdx.x; i < n; i += gridDim.x)
+        for (long long q = threadIdx.x; q < sums[i].cnt; q += 256)
+            Cval[sums[i].at + q] = P::result(sum_val + (size_t)i * WIDE_UNIT, (unsigned)q);
 }
 
 // workgroups of a windows' kernel that a CU holds
@@ -2096,10 +2250,29 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
             }
             const unsigned gi = (unsigned)wide_item_blocks(count, num_cus);
             hipLaunchKernelGGL(k_wide_items<false>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
-                               wide.items, wide.items_cap, wide.places, err);
+                               wide.items, wide.items_cap, wide.places, wide.hot, wide.hot_cap, wide.hot_min, wide.ctr, err);
             hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(1024), 0, s, wide.places, (int)gi, wide.ctr);
             hipLaunchKernelGGL(k_wide_items<true>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
-                               wide.items, wide.items_cap, wide.places, err);
+                               wide.items, wide.items_cap, wide.places, wide.hot, wide.hot_cap, wide.hot_min, wide.ctr, err);
+            if (wide.hot) {
+                const unsigned gh = (unsigned)(8 * num_cus);
+#define HOT(INDEX)                                                                                                     \
+    hipLaunchKernelGGL((k_wide_cut<INDEX>), dim3(gh), dim3(256), 0, s, wide.hot, (unsigned)wide.hot_cap,               \
+                       wide.hot_min, wide.items, wide.ctr, op, wide.index, wide.nunits, crp, wide.parts, (u64)wide.part_cap, wide.sums,          \
+                       wide.sum_val, (unsigned)wide.sum_cap);                                                          \
+    hipLaunchKernelGGL((k_numeric_parts<P, WW_BS, INDEX>),                                                             \
+                       dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, false>()))), dim3(WW_BS),                     \
+                       (ww_lds<WW_BS, false>()), s, wide.parts, wide.ctr, (u64)wide.part_cap, op, wide.index,          \
+                       wide.nunits, crp, Ccol, wide.sum_val)
+                if (wide.index) {
+                    HOT(true);
+                } else {
+                    HOT(false);
+                }
+#undef HOT
+                hipLaunchKernelGGL(k_wide_sums<P>, dim3(gh), dim3(256), 0, s, wide.sums, wide.ctr, (unsigned)wide.sum_cap,
+                                   wide.sum_val, (typename P::V *)Cval);
+            }
 #define WINDOWS(DENSE, INDEX, TAKEN)                                                                                   \
     hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, DENSE, INDEX>),                                                    \
                        dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, DENSE>()))), dim3(WW_BS),                     \
@@ -2192,7 +2365,8 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
     CFG(k_numeric_wcompact<PrecF64>) CFG(k_numeric_wcompact<PrecF32C>) 
 #define CFGW(P)                                                                                                        \
     CFG((k_numeric_windows<P, WW_BS, false, false>)) CFG((k_numeric_windows<P, WW_BS, false, true>))                   \
-    CFG((k_numeric_windows<P, WW_BS, true, false>)) CFG((k_numeric_windows<P, WW_BS, true, true>))
+    CFG((k_numeric_windows<P, WW_BS, true, false>)) CFG((k_numeric_windows<P, WW_BS, true, true>))                     \
+    CFG((k_numeric_parts<P, WW_BS, false>)) CFG((k_numeric_parts<P, WW_BS, true>))
     CFGW(PrecF64) CFGW(PrecF32C)
 #undef CFGW
 #undef CFG

@@ -556,6 +556,7 @@ struct hsmu_plan {
     bool empty = false;           // product with no entries: nothing to replay
     bool dirs_kept = false;       // the recording run kept the row directories
     int wide_form = 0;            // the form its wide rows took
+    bool wide_cut = false;        // the windows of hot rows are cut into parts
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
@@ -1086,6 +1087,36 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
                 return fail(HSMU_ERR_NOMEM, "wide-row workspace");
             if (mode.plan)
                 mode.plan->wide_form = form;
+            // hot rows: without the memory their windows stay whole
+            const unsigned long long share = 2 * h2.num.work[b] / (3 * (unsigned long long)c->num_cus);
+            const unsigned long long hot_min = share > WIDE_HOT ? share : WIDE_HOT;
+            const unsigned long long sums = h2.num.work[b] / hot_min + 1; // (at most 385 on 256 CUs)
+            const unsigned long long parts = (2 * sums + 16) * WIDE_PARTS;
+            const unsigned long long hot_bytes = h2.hot_items * sizeof(unsigned) + parts * sizeof(WidePart) +
+                                                 sums * (WIDE_UNIT * sizeof(double) + sizeof(WideSum)) + 2048;
+            if (form < WIDE_PER_ROW && h2.hot_most + WIDE_UNIT >= hot_min && hot_bytes <= ar.remaining() &&
+                (!cap || mode.plan->wide_cut)) {
+                const Arena::Mark whole = ar.mark();
+                wide.hot_min = (long long)hot_min;
+                wide.hot_cap = (long long)h2.hot_items;
+                wide.part_cap = (long long)parts;
+                wide.sum_cap = (long long)sums;
+                wide.hot = ar.get<unsigned>((size_t)h2.hot_items);
+                wide.parts = ar.get<WidePart>((size_t)parts);
+                wide.sums = ar.get<WideSum>((size_t)sums);
+                wide.sum_val = ar.get<double>((size_t)sums * WIDE_UNIT);
+                if (!wide.hot || !wide.parts || !wide.sums || !wide.sum_val) {
+                    if (cap)
+                        return fail(HSMU_ERR_NOMEM, "wide-row workspace");
+                    ar.rewind(whole);
+                    wide.hot = nullptr;
+                    wide.parts = nullptr;
+                    wide.sums = nullptr;
+                    wide.sum_val = nullptr;
+                }
+                if (mode.plan)
+                    mode.plan->wide_cut = wide.hot != nullptr;
+            }
         }
         if (timing)
             HIP_TRY(hipEventRecord(c->evb[b][0], s));

@@ -68,6 +68,8 @@ struct DevStats {
     int pad;
     unsigned long long num_wide_work; // products of rows that may be wide in the numeric phase (symbolic binning)
     unsigned long long wide_items; // windows the wide rows may need, at most (numeric binning)
+    unsigned long long hot_items;  // those of them that belong to hot rows
+    unsigned long long hot_most;   // products beyond its entries of C of the hottest
     BinStats sym;
     BinStats num;
 };
@@ -471,9 +473,37 @@ struct __attribute__((aligned(16))) WideItem {
     unsigned base, cnt; // the row's entries before the window, and in it
 };
 // The list: windows with compact slots, from `dense` on those with a slot per column, its
-// end; how many of each form are taken.
+// end; how many of each form are taken.  Windows that may be hot, the windows that are cut, their
+// parts.
 struct WideCount {
     unsigned dense, listed, taken[2];
+    unsigned hot, sums;
+    unsigned long long parts;
+};
+// A hot row has WIDE_HOT products more than entries of C_i, and entries of A for as many on a
+// window's entries of C_i (each takes one product of an entry of A at most, unless B's rows repeat
+// columns): one of its windows may hold as many, which kept a workgroup busy long after the others
+// had ended.  Such windows are estimated from WIDE_SAMPLE of the row's entries of A and, with
+// WIDE_HOT products or more and twice a workgroup's share of all wide rows' (less is no tail: cutting
+// it slows an R-MAT square of scale 18 by 1.6%), cut into WIDE_PARTS or more ranges of entries of A,
+// whose FP64 sums meet in memory.  3,000 rows of B with 900 of their 1,000 entries in one unit: a row
+// of C with all of them 2.12 ms whole and 0.37 cut, 64 such rows 3.97 and 0.59.
+constexpr unsigned long long WIDE_HOT = 512 * 1024;
+constexpr int WIDE_PARTS = 4;
+constexpr int WIDE_SAMPLE = 256;
+HSMU_HD inline bool wide_hot(long long p, long long n, int nA)
+{
+    return p - n > (long long)WIDE_HOT && (long long)nA * WIDE_UNIT >= (long long)WIDE_HOT;
+}
+struct __attribute__((aligned(16))) WidePart {
+    int row;
+    unsigned units, base, cnt; // as the window's
+    int e0, e1;                // entries of A
+    int sum, pad;              // its place among the cut windows
+};
+struct WideSum { // where a cut window's values go in C, how many
+    long long at;
+    long long cnt;
 };
 HSMU_HD inline long long wide_units(long long N) { return (N + WIDE_UNIT - 1) / WIDE_UNIT; }
 // windows of a row of n entries over S tiles, at most: two neighbouring ones hold more than
@@ -500,6 +530,14 @@ struct WideRows {
     int *index; // K rows of nunits + 1, or null: search
     long long nunits;
     long long K;
+    // hot rows (null hot: none): their windows' places in the list, parts, cut windows with
+    // WIDE_UNIT sums each; capacities
+    unsigned *hot;
+    WidePart *parts;
+    WideSum *sums;
+    double *sum_val;
+    long long hot_cap, part_cap, sum_cap;
+    long long hot_min; // products of a window that is cut
 };
 // workgroups that list the windows of count rows
 int wide_item_blocks(int count, int num_cus);

@@ -629,9 +629,20 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
             atomicAdd(&st->num_wide_work, products);
     }
     if (numeric && __ballot(at.b == BIN_GLOBAL)) { // room for the wide rows' windows
-        const u64 items = wave_sum(at.b == BIN_GLOBAL ? (u64)wide_row_items(r.nc, r.S) : 0ull);
+        const u64 mine = at.b == BIN_GLOBAL ? (u64)wide_row_items(r.nc, r.S) : 0ull;
+        const u64 items = wave_sum(mine);
         if (lane == 0)
             atomicAdd(&st->wide_items, items);
+        const bool hot = at.b == BIN_GLOBAL && wide_hot(r.prod, r.nc, r.nA);
+        if (__ballot(hot)) {
+            const u64 hots = wave_sum(hot ? mine : 0ull);
+            const u64 most = wave_last(wave_incl_scan(hot ? (u64)(r.prod - r.nc) : 0ull, (u64)0,
+                                                      [](u64 a, u64 b) { return a > b ? a : b; }));
+            if (lane == 0) {
+                atomicAdd(&st->hot_items, hots);
+                atomicMax(&st->hot_most, most);
+            }
+        }
     }
     // the lanes that chose one bin (neighbouring rows usually share it) add up first
     u64 pending = __ballot(at.b >= 0);
@@ -1441,7 +1452,8 @@ __global__ void k_plan_check(DevStats *st, const DevStats *expect, int stage)
     if (stage == 0)
         same = same && st->dir_total == expect->dir_total && st->ntiles_b == expect->ntiles_b;
     else
-        same = same && st->nnz_c == expect->nnz_c && st->wide_items == expect->wide_items;
+        same = same && st->nnz_c == expect->nnz_c && st->wide_items == expect->wide_items &&
+               st->hot_items == expect->hot_items;
     if (!same)
         st->err |= ERR_PLAN;
     if (st->err) {

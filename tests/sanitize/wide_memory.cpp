@@ -196,6 +196,8 @@ int main()
         g_stats[1].num.max_na[BIN_GLOBAL] = t.na;
         g_stats[1].num.max_span[BIN_GLOBAL] = 960;
         g_stats[1].wide_items = t.items;
+        g_stats[1].hot_items = 16 << 20; // a list of 64 MiB
+        g_stats[1].hot_most = 1ull << 30;
         g_stats[1].nnz_c = 1000;
         hsmu_ctx_trim(ctx);
         g_limit = t.limit;
@@ -209,6 +211,7 @@ int main()
         ok = ok && g_wide.size() == (t.form < 3 ? 2u : 0u);
         for (const WideRows &w : g_wide) // recording, capture: the same form in the same blocks
             ok = ok && (w.items != nullptr) == (t.form < 2) && (w.index != nullptr) == (t.form == 0) &&
+                 (w.hot != nullptr) == (t.form == 0) && w.hot == g_wide[0].hot && w.sum_val == g_wide[0].sum_val &&
                  (t.form != 2 || w.ws) && w.items == g_wide[0].items && w.index == g_wide[0].index &&
                  w.ws == g_wide[0].ws && w.ctr == g_wide[0].ctr;
         hsmu_plan_destroy(plan);
