@@ -316,6 +316,17 @@ template <typename T> struct Vec2 {
 };
 template <typename T> DEVI typename Vec2<T>::type load2(const T *p) { return *(const typename Vec2<T>::type *)p; }
 
+// Entry e of a row of nA entries from a0: its column, and the tiles of that row of B (none past
+// the row's end).
+DEVI int col_of(const Operands &op, int a0, int e, int nA) { return e < nA ? op.Acol[a0 + e] : 0; }
+DEVI Segment tile_range(const Operands &op, int e, int nA, int j)
+{
+    if (e >= nA)
+        return Segment{0, 0, 0};
+    const typename Vec2<int>::type t = load2(op.tptr + j);
+    return Segment{t.x, t.y - t.x, 0};
+}
+
 // A lane's elements k, k + 1 of an array of n: loaded from k or, at the array's end, from
 // n - 2; in0 / in1: element 0 / 1 of the load belongs to [k, end).
 struct Pair {
@@ -761,7 +772,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void
 // 3.5 ms; banded rows of 100 tiles 147 and 131 us.  TL: some row of the launch has a two-level directory.  A kept directory
 // goes out coalesced: the masks first, then each entry's slot offset, written over its mask
 // in LDS (coarse level: into doff, which the fine pass reads).
-template <int G, bool TL>
+template <int G, bool TL, bool LONG = false>
 __global__ __launch_bounds__(G) void k_symbolic_row(const int *__restrict__ rows, const int *__restrict__ count_p,
                                                     Operands op, int *__restrict__ rnnz, unsigned *queue)
 {
@@ -788,11 +799,7 @@ __global__ __launch_bounds__(G) void k_symbolic_row(const int *__restrict__ rows
         st.red = red;
         const int words = (L.doff - L.bits) >> 3;
         const long long rd = op.dir_mask ? uniform64(op.rdir[row]) & ~RDIR_TWO : -1;
-        auto tiles = [&](int e) {
-            const int j = op.Acol[a0 + e];
-            const typename Vec2<int>::type t = load2(op.tptr + j);
-            return Segment{t.x, t.y - t.x, 0};
-        };
+        auto tiles = [&](int e) { return tile_range(op, e, nA, op.Acol[a0 + e]); };
         // two-level rows walk their tiles twice: the lane's first entry is kept (with more lanes
         // that costs an R-MAT square of scale 18 0.5%)
         constexpr bool KEEP = TL && G <= 128;
@@ -804,14 +811,21 @@ __global__ __launch_bounds__(G) void k_symbolic_row(const int *__restrict__ rows
         for (int q = l; q < words; q += G)
             st.bits[q] = 0;
         __syncthreads();
-        auto tiles_of = [&](int e) { return KEEP && e < G ? mine : tiles(e); };
+        auto walk_tiles = [&](auto body) {
+            if constexpr (LONG)
+                st.run(
+                    nA, tile_range(op, l, nA, col_of(op, a0, l, nA)), [&](int e) { return col_of(op, a0, e, nA); },
+                    [&](int e, int j) { return tile_range(op, e, nA, j); }, body);
+            else
+                st.run(nA, [&](int e) { return KEEP && e < G ? mine : tiles(e); }, body);
+        };
         if (!sparse)
-            st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+            walk_tiles([&](const Stream<G> &t, long long w0) {
                 stream_or<G, OR_FLAT>(t, w0, op, dm, nullptr, nullptr, mn);
             });
         if constexpr (TL) {
             if (sparse)
-                st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                walk_tiles([&](const Stream<G> &t, long long w0) {
                     stream_or<G, OR_COARSE>(t, w0, op, dm, nullptr, nullptr, mn);
                 });
         }
@@ -838,7 +852,7 @@ __global__ __launch_bounds__(G) void k_symbolic_row(const int *__restrict__ rows
                 for (int q = l; q < words; q += G)
                     st.bits[q] = 0;
                 __syncthreads();
-                st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                walk_tiles([&](const Stream<G> &t, long long w0) {
                     stream_or<G, OR_FINE>(t, w0, op, dm, doff, fm, mn);
                 });
                 const ChunkScan fs = scan_popcounts<G>(fm, F, (unsigned *)red);
@@ -958,7 +972,7 @@ __global__ __launch_bounds__(1024) void k_symbolic_wide(const int *__restrict__ 
 // TL: some row of the launch has a two-level directory (the form costs registers, so
 // launches without one run a kernel without it).  At 5 waves per SIMD (96 registers) ten
 // banded rows of 128 lanes fit a CU as their LDS does.
-template <int G, typename P, bool TL>
+template <int G, typename P, bool TL, bool LONG = false>
 __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5))) void k_numeric_row(
     const int *__restrict__ rows, const int *__restrict__ count_p, Operands op, const long long *__restrict__ crp,
     int *__restrict__ Ccol, typename P::V *__restrict__ Cval, int *err, unsigned *queue)
@@ -997,17 +1011,15 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
         const int nv = dense ? 64 * S : n;
         const long long rd = op.dir_mask ? uniform64(kept_dir(op, row, sparse)) : -1;
         const int words = (L.doff - L.bits) >> 3;
-        auto tiles = [&](int e) {
-            const int j = op.Acol[a0 + e];
-            const typename Vec2<int>::type t = load2(op.tptr + j);
-            return Segment{t.x, t.y - t.x, 0};
-        };
-        auto entries = [&](int e) {
-            const int j = op.Acol[a0 + e];
+        auto tiles = [&](int e) { return tile_range(op, e, nA, op.Acol[a0 + e]); };
+        auto entry = [&](int e, int j) {
+            if (e >= nA)
+                return Segment{0, 0, 0};
             const typename Vec2<int>::type b = load2(op.Brp + j);
             const double a = (double)Aval[a0 + e];
             return Segment{b.x, b.y - b.x, (u64)__double_as_longlong(a)};
         };
+        auto entries = [&](int e) { return entry(e, op.Acol[a0 + e]); };
         // two-level rows may walk their tiles twice and then their elements: the lane's first
         // entry is kept
         constexpr bool KEEP = TL && G <= 128;
@@ -1031,7 +1043,14 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
                 dm[t] = 0;
         }
         __syncthreads();
-        auto tiles_of = [&](int e) { return KEEP && e < G ? my_tiles : tiles(e); };
+        auto walk_tiles = [&](auto body) {
+            if constexpr (LONG)
+                st.run(
+                    nA, tile_range(op, l, nA, col_of(op, a0, l, nA)), [&](int e) { return col_of(op, a0, e, nA); },
+                    [&](int e, int j) { return tile_range(op, e, nA, j); }, body);
+            else
+                st.run(nA, [&](int e) { return KEEP && e < G ? my_tiles : tiles(e); }, body);
+        };
         auto rezero = [&]() { // the stream's bits, for its next run
             __syncthreads();
             for (int q = l; q < words; q += G)
@@ -1042,12 +1061,12 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
         if (rd < 0) {
             if constexpr (TL) {
                 if (sparse)
-                    st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                    walk_tiles([&](const Stream<G> &t, long long w0) {
                         stream_or<G, OR_COARSE>(t, w0, op, dm, nullptr, nullptr, mn);
                     });
             }
             if (!sparse)
-                st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                walk_tiles([&](const Stream<G> &t, long long w0) {
                     stream_or<G, OR_FLAT>(t, w0, op, dm, nullptr, nullptr, mn);
                 });
             rezero();
@@ -1082,7 +1101,7 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
             }
             __syncthreads();
             if (rd < 0) {
-                st.run(nA, tiles_of, [&](const Stream<G> &t, long long w0) {
+                walk_tiles([&](const Stream<G> &t, long long w0) {
                     stream_or<G, OR_FINE>(t, w0, op, dm, doff, fm, mn);
                 });
                 rezero();
@@ -1096,18 +1115,24 @@ __global__ __launch_bounds__(G) __attribute__((amdgpu_waves_per_eu(TL ? 4 : 5)))
             raise_internal(err);
         __syncthreads();
         if (ok) { // uniform
-            auto rows_of = [&](int e) { return KEEP && e < G ? mine : entries(e); };
+            auto walk_rows = [&](auto body) {
+                if constexpr (LONG)
+                    st.run(
+                        nA, entry(l, col_of(op, a0, l, nA)), [&](int e) { return col_of(op, a0, e, nA); }, entry, body);
+                else
+                    st.run(nA, [&](int e) { return KEEP && e < G ? mine : entries(e); }, body);
+            };
             if (dense)
-                st.run(nA, rows_of, [&](const Stream<G> &t, long long w0) {
+                walk_rows([&](const Stream<G> &t, long long w0) {
                     stream_add<G, SLOT_DENSE, P>(t, w0, op, nullptr, nullptr, fm, foff, vals, mn);
                 });
             else if (!sparse)
-                st.run(nA, rows_of, [&](const Stream<G> &t, long long w0) {
+                walk_rows([&](const Stream<G> &t, long long w0) {
                     stream_add<G, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, fm, foff, vals, mn);
                 });
             if constexpr (TL) {
                 if (sparse)
-                    st.run(nA, rows_of, [&](const Stream<G> &t, long long w0) {
+                    walk_rows([&](const Stream<G> &t, long long w0) {
                         stream_add<G, SLOT_TWO_LEVEL, P>(t, w0, op, dm, doff, fm, foff, vals, mn);
                     });
             }
@@ -2158,20 +2183,27 @@ hipError_t launch_small(int form, const int *rows, long long stride, const BinSt
     return f(rows, stride, bins_dev, count, bins, op, rnnz, crp, Ccol, Cval, err, num_cus, queue, lds_bytes, s);
 }
 
-template <int G, bool TL>
+// Rows of 1,024 lanes that stage their entries in so many turns load the next turn's meanwhile.
+constexpr int LONG_NA = 8 * 1024;
+
+template <int G, bool TL, bool LONG = false>
 static void symbolic_row(const int *rows, const int *count_dev, int count, int max_need, const Operands &op, int *rnnz,
                          int num_cus, unsigned *queue, hipStream_t s)
 {
     const size_t lds = (size_t)((max_need + 15) & ~15);
-    const int64_t blocks = row_grid(k_symbolic_row<G, TL>, G, lds, count, num_cus, queue);
-    hipLaunchKernelGGL((k_symbolic_row<G, TL>), dim3((unsigned)blocks), dim3(G), lds, s, rows, count_dev, op, rnnz,
+    const int64_t blocks = row_grid(k_symbolic_row<G, TL, LONG>, G, lds, count, num_cus, queue);
+    hipLaunchKernelGGL((k_symbolic_row<G, TL, LONG>), dim3((unsigned)blocks), dim3(G), lds, s, rows, count_dev, op, rnnz,
                        queue);
 }
 
 template <bool TL>
-static void symbolic_rows(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
-                          int *rnnz, int num_cus, unsigned *queue, hipStream_t s)
+static void symbolic_rows(int bin, const int *rows, const int *count_dev, int count, int max_need, int max_na,
+                          const Operands &op, int *rnnz, int num_cus, unsigned *queue, hipStream_t s)
 {
+    if (bin == NLDS - 1 && max_na >= LONG_NA) {
+        symbolic_row<1024, TL, true>(rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s);
+        return;
+    }
 #define SYM(B, G)                                                                                                      \
     case B: symbolic_row<G, TL>(rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s); break;
     switch (bin) {
@@ -2180,8 +2212,8 @@ static void symbolic_rows(int bin, const int *rows, const int *count_dev, int co
 #undef SYM
 }
 
-hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
-                           int *rnnz, int tshift, int two_level, u64 *gws, long long gws_stride,
+hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int count, int max_need, int max_na,
+                           const Operands &op, int *rnnz, int tshift, int two_level, u64 *gws, long long gws_stride,
                            int num_cus, int gws_blocks, int lds_dyn, unsigned *queue, hipStream_t s)
 {
     if (count <= 0)
@@ -2197,32 +2229,38 @@ hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int c
                                tshift > 10 ? 10 : tshift, gws, gws_stride);
     } else if (bin >= BIN_SHARED && bin < NLDS) {
         if (two_level)
-            symbolic_rows<true>(bin, rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s);
+            symbolic_rows<true>(bin, rows, count_dev, count, max_need, max_na, op, rnnz, num_cus, queue, s);
         else
-            symbolic_rows<false>(bin, rows, count_dev, count, max_need, op, rnnz, num_cus, queue, s);
+            symbolic_rows<false>(bin, rows, count_dev, count, max_need, max_na, op, rnnz, num_cus, queue, s);
     } else {
         return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
-template <int G, typename P, bool TL>
+template <int G, typename P, bool TL, bool LONG = false>
 static void numeric_row(const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
                         const long long *crp, int *Ccol, void *Cval, int *err, int num_cus, unsigned *queue,
                         unsigned long long *lds_bytes, hipStream_t s)
 {
     const size_t lds = (size_t)((max_need + 15) & ~15);
-    const int64_t blocks = row_grid(k_numeric_row<G, P, TL>, G, lds, count, num_cus, queue);
+    const int64_t blocks = row_grid(k_numeric_row<G, P, TL, LONG>, G, lds, count, num_cus, queue);
     *lds_bytes += (unsigned long long)blocks * lds;
-    hipLaunchKernelGGL((k_numeric_row<G, P, TL>), dim3((unsigned)blocks), dim3(G), lds, s, rows, count_dev, op, crp,
+    hipLaunchKernelGGL((k_numeric_row<G, P, TL, LONG>), dim3((unsigned)blocks), dim3(G), lds, s, rows, count_dev, op, crp,
                        Ccol, (typename P::V *)Cval, err, queue);
 }
 
 template <typename P, bool TL>
-static void numeric_rows(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
+static void numeric_rows(int bin, const int *rows, const int *count_dev, int count, int max_need, int max_na,
+                         const Operands &op,
                          const long long *crp, int *Ccol, void *Cval, int *err, int num_cus, unsigned *queue,
                          unsigned long long *lds_bytes, hipStream_t s)
 {
+    if (bin == NLDS - 1 && max_na >= LONG_NA) {
+        numeric_row<1024, P, TL, true>(rows, count_dev, count, max_need, op, crp, Ccol, Cval, err, num_cus, queue,
+                                       lds_bytes, s);
+        return;
+    }
 #define NUM(B, G)                                                                                                      \
     case B:                                                                                                            \
         numeric_row<G, P, TL>(rows, count_dev, count, max_need, op, crp, Ccol, Cval, err, num_cus, queue, lds_bytes,   \
@@ -2235,7 +2273,8 @@ static void numeric_rows(int bin, const int *rows, const int *count_dev, int cou
 }
 
 template <typename P>
-static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int count, int max_need, const Operands &op,
+static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int count, int max_need, int max_na,
+                            const Operands &op,
                             const long long *crp, int *Ccol, void *Cval, int bshift, int two_level,
                             const WideRows &wide, int *err, int num_cus, unsigned *queue,
                             unsigned long long *lds_bytes, hipStream_t s)
@@ -2296,10 +2335,10 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
                                err);
     } else if (bin >= 3 && bin < NLDS) {
         if (two_level)
-            numeric_rows<P, true>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, err, num_cus, queue,
+            numeric_rows<P, true>(bin, rows, count_dev, count, max_need, max_na, op, crp, Ccol, Cval, err, num_cus, queue,
                                   lds_bytes, s);
         else
-            numeric_rows<P, false>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, err, num_cus, queue,
+            numeric_rows<P, false>(bin, rows, count_dev, count, max_need, max_na, op, crp, Ccol, Cval, err, num_cus, queue,
                                    lds_bytes, s);
     } else {
         return hipErrorInvalidValue;
@@ -2307,7 +2346,7 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
     return hipGetLastError();
 }
 
-hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_dev, int count, int max_need,
+hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_dev, int count, int max_need, int max_na,
                           const Operands &op, const long long *crp, int *Ccol, void *Cval, int bshift, int two_level,
                           const WideRows &wide, int *err, int num_cus, unsigned *queue,
                           unsigned long long *lds_bytes, hipStream_t s)
@@ -2318,9 +2357,9 @@ hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_
     if (!lds_bytes)
         lds_bytes = &ignored;
     if (fp32c)
-        return numeric_p<PrecF32C>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, two_level, wide,
+        return numeric_p<PrecF32C>(bin, rows, count_dev, count, max_need, max_na, op, crp, Ccol, Cval, bshift, two_level, wide,
                                    err, num_cus, queue, lds_bytes, s);
-    return numeric_p<PrecF64>(bin, rows, count_dev, count, max_need, op, crp, Ccol, Cval, bshift, two_level, wide, err,
+    return numeric_p<PrecF64>(bin, rows, count_dev, count, max_need, max_na, op, crp, Ccol, Cval, bshift, two_level, wide, err,
                               num_cus, queue, lds_bytes, s);
 }
 
@@ -2350,10 +2389,10 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
 #define CFGL(P) CFGT(P, false) CFGT(P, true)
 #define CFGS(TL)                                                                                                       \
     CFG((k_symbolic_row<64, TL>)) CFG((k_symbolic_row<128, TL>)) CFG((k_symbolic_row<256, TL>))                        \
-    CFG((k_symbolic_row<512, TL>)) CFG((k_symbolic_row<1024, TL>))
+    CFG((k_symbolic_row<512, TL>)) CFG((k_symbolic_row<1024, TL>)) CFG((k_symbolic_row<1024, TL, true>))
 #define CFGR(P, TL)                                                                                                    \
     CFG((k_numeric_row<64, P, TL>)) CFG((k_numeric_row<128, P, TL>)) CFG((k_numeric_row<256, P, TL>))                  \
-    CFG((k_numeric_row<512, P, TL>)) CFG((k_numeric_row<1024, P, TL>))
+    CFG((k_numeric_row<512, P, TL>)) CFG((k_numeric_row<1024, P, TL>)) CFG((k_numeric_row<1024, P, TL, true>))
     CFGL(SmallNone) CFGL(PrecF64) CFGL(PrecF32C) CFGS(false) CFGS(true)
     CFGR(PrecF64, false) CFGR(PrecF32C, false) CFGR(PrecF64, true) CFGR(PrecF32C, true)
 #undef CFGR

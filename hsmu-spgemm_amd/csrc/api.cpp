@@ -921,7 +921,8 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         const int cnt = h1.sym.count[b];
         if (cnt <= 0)
             continue;
-        HIP_TRY(launch_symbolic(b, binrows + (size_t)b * M, &dst->sym.count[b], cnt, h1.sym.max_need[b], op, rnnz,
+        HIP_TRY(launch_symbolic(b, binrows + (size_t)b * M, &dst->sym.count[b], cnt, h1.sym.max_need[b],
+                                h1.sym.max_na[b], op, rnnz,
                                 tshift, h1.sym.nsparse[b] > 0 ? 1 : 0, gws, gws_stride, c->num_cus,
                                 gws_blocks, (int)bp.lds_row_max,
                                 opts.persistent ? dw->queue[0][b] : nullptr, s));
@@ -1120,7 +1121,8 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         }
         if (timing)
             HIP_TRY(hipEventRecord(c->evb[b][0], s));
-        HIP_TRY(launch_numeric(b, fp32 ? 1 : 0, binrows + (size_t)b * M, &dst->num.count[b], cnt, h2.num.max_need[b], op,
+        HIP_TRY(launch_numeric(b, fp32 ? 1 : 0, binrows + (size_t)b * M, &dst->num.count[b], cnt, h2.num.max_need[b],
+                               h2.num.max_na[b], op,
                                crp, Ccol, Cval, bshift, h2.num.nsparse[b] > 0 ? 1 : 0, wide, errp,
                                c->num_cus,
                                opts.persistent ? dw->queue[1][b] : nullptr, &lds_launched, s));

@@ -413,7 +413,7 @@ hipError_t launch_small(int form, const int *rows, long long stride, const BinSt
 // lds_dyn: LDS a row may use (lds_row_max); BIN_GLOBAL rows keep their flat directory in
 // LDS when gws_stride masks fit it (gws is then unused).
 hipError_t launch_symbolic(int bin, const int *rows, const int *count_dev, int count,
-                           int max_need, const Operands &op, int *rnnz, int tshift, int two_level,
+                           int max_need, int max_na, const Operands &op, int *rnnz, int tshift, int two_level,
                            unsigned long long *gws, long long gws_stride, int num_cus,
                            int gws_blocks, int lds_dyn, unsigned *queue, hipStream_t s);
 
@@ -554,7 +554,7 @@ size_t wide_ws_ints(long long cur_stride, long long ft_stride, int blocks);
 // compressed_Cval.cuh:202-533); the wide-row kernels' persistent workgroups reuse their LDS
 // window by window and are not counted.
 hipError_t launch_numeric(int bin, int fp32c, const int *rows, const int *count_dev, int count,
-                          int max_need, const Operands &op, const long long *crp, int *Ccol,
+                          int max_need, int max_na, const Operands &op, const long long *crp, int *Ccol,
                           void *Cval, int bshift, int two_level, const WideRows &wide, int *err, int num_cus,
                           unsigned *queue, unsigned long long *lds_bytes,
                           hipStream_t s);

@@ -116,7 +116,7 @@ LAUNCH(launch_small, int, ci, long long, const BinStats *, ci, const BinStats &,
        void *, int *, int, unsigned (*)[QUEUE_INTS], u64 *, hipStream_t)
 LAUNCH(launch_btiles, int64_t, int64_t, int64_t, ci, ci, int *, int *, u64 *, BRow *, u64 *, unsigned *, DevStats *,
        hipStream_t)
-LAUNCH(launch_symbolic, int, ci, ci, int, int, const Operands &, int *, int, int, u64 *, long long, int, int, int,
+LAUNCH(launch_symbolic, int, ci, ci, int, int, int, const Operands &, int *, int, int, u64 *, long long, int, int, int,
        unsigned *, hipStream_t)
 LAUNCH(launch_row_sums, int64_t, const void *, int, const void *, int, double *, double *, hipStream_t)
 LAUNCH(launch_plan_bases, const long long *, const long long *, int64_t, DevStats *, hipStream_t)
@@ -158,7 +158,7 @@ hipError_t launch_rowptr_bin(int64_t, ci, const long long *, ci, ci, ci, ci, lon
 {
     return counters(host, seq, 1);
 }
-hipError_t launch_numeric(int bin, int, ci, ci, int, int, const Operands &, const long long *, int *, void *, int, int,
+hipError_t launch_numeric(int bin, int, ci, ci, int, int, int, const Operands &, const long long *, int *, void *, int, int,
                           const WideRows &w, int *, int, unsigned *, u64 *, hipStream_t)
 {
     if (bin == BIN_GLOBAL)
