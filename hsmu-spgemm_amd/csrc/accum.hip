@@ -1788,12 +1788,74 @@ DEVI int2 window_elements(const Operands &op, const int *__restrict__ index, lon
     }
 }
 
+// The parts of hot windows that are this workgroup's: as k_numeric_windows' compact form, over a range
+// of the row's entries.  Their sums meet by atomics in sum_val (k_wide_sums takes them to C); a
+// window's first part writes its columns.
+struct WideCut {
+    const WidePart *parts;
+    const WideCount *ctr;
+    u64 part_cap;
+    double *sum_val;
+};
+template <typename P, int BS, bool INDEX>
+DEVI void window_parts(const WideCut &cut, const Operands &op, const int *__restrict__ index, long long U,
+                       const long long *__restrict__ crp, int *__restrict__ Ccol, double *vals, Stream<BS> &st, u64 *wm,
+                       unsigned short *wo)
+{
+    typedef typename P::V V;
+    constexpr int NW = BS / 64, words = stream_window(BS) / 64;
+    const int l = threadIdx.x, lane = l & 63, w = uniform((int)(threadIdx.x >> 6));
+    const V *__restrict__ Aval = (const V *)op.Aval;
+    const u64 n = cut.ctr->parts < cut.part_cap ? cut.ctr->parts : cut.part_cap;
+    for (u64 i = blockIdx.x; i < n; i += gridDim.x) {
+        const WidePart p = cut.parts[i];
+        const int row = uniform(p.row), sum = uniform(p.sum), e0 = uniform(p.e0), cnt = (int)uniform(p.cnt);
+        const unsigned units = uniform(p.units), base = uniform(p.base);
+        const int u0 = (int)(units & 0xffffffu), u1 = u0 + (int)(units >> 24);
+        const int a0 = uniform(op.Arp[row]) + e0, nA = uniform(p.e1) - e0;
+        const WideDir d(op, uniform(op.rmin[row]), uniform(op.rmax[row]), uniform64(op.rdir[row]));
+        const long long cb = uniform64(crp[row]) + base;
+        const int T0 = u0 * WIDE_TILES, nt = (u1 - u0) * WIDE_TILES;
+        for (int t = l; t < nt; t += BS) {
+            unsigned off;
+            wm[t] = d.tile(T0 + t - d.mn, off);
+            wo[t] = (unsigned short)(off - base);
+        }
+        for (int q = 2 * l; q < cnt; q += 2 * BS) // (WIDE_UNIT is even)
+            *(double2 *)(vals + q) = make_double2(0.0, 0.0);
+        for (int q = l; q < words; q += BS)
+            st.bits[q] = 0;
+        __syncthreads();
+        st.run(
+            nA,
+            [&](int e) {
+                const int2 r = window_elements<INDEX>(op, index, U, u0, u1, op.Acol[a0 + e]);
+                return Segment{r.x, r.y - r.x, (u64)__double_as_longlong((double)Aval[a0 + e])};
+            },
+            [&](const Stream<BS> &t, long long w0) {
+                stream_add<BS, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, wm, wo, vals, T0);
+            });
+        __syncthreads();
+        double *sv = cut.sum_val + (size_t)sum * WIDE_UNIT;
+        for (int q = l; q < cnt; q += BS)
+            unsafeAtomicAdd(&sv[q], vals[q]);
+        if (e0 == 0)
+            for (int t = w; t < nt; t += NW) {
+                const u64 m = uniform64(wm[t]);
+                if ((m >> lane) & 1ull)
+                    Ccol[cb + wo[t] + (unsigned)mbcnt(m)] = ((T0 + t) << 6) + lane;
+            }
+        __syncthreads();
+    }
+}
+
 // Wide rows as windows: the compact accumulator over one window's entries of C_i, its part
 // of the row's directory (expanded to one mask and slot per tile of the window) and its
 // elements of the B rows as one stream, their ranges read from the index.  Workgroups take
 // windows from the list until it is used up.  Neither a search nor atomics in C nor a
 // second round: every window's elements are known when it starts, and a window belongs to
 // one workgroup.
+// CUT: the parts of hot windows first, which then run beside the others.
 // DENSE: a slot per column of the unit, with no masks in LDS: the element's column is its
 // slot, and a tile goes out as one store of columns and one of values by a wave.
 // No single unit bounds the compact form (Zipf panel: vector ALU 41%, LDS 32%, L1 47% of the
@@ -1818,12 +1880,12 @@ template <int BS, bool DENSE> constexpr int ww_lds()
     return WIDE_UNIT * 8 + BS * 16 + words * 10 + (DENSE ? 0 : WW_TILES * 10);
 }
 
-template <typename P, int BS, bool DENSE, bool INDEX>
+template <typename P, int BS, bool DENSE, bool INDEX, bool CUT = false>
 __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restrict__ items,
                                                         const WideCount *__restrict__ listed, unsigned *taken,
                                                         Operands op, const int *__restrict__ index, long long U,
                                                         const long long *__restrict__ crp, int *__restrict__ Ccol,
-                                                        typename P::V *__restrict__ Cval)
+                                                        typename P::V *__restrict__ Cval, WideCut cut)
 {
     typedef typename P::V V;
     extern __shared__ __align__(16) unsigned char lds[];
@@ -1841,6 +1903,8 @@ __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restri
     int *stage = (int *)vals; // columns, once the values are out
     const int l = threadIdx.x, lane = l & 63, w = uniform((int)(threadIdx.x >> 6));
     const V *__restrict__ Aval = (const V *)op.Aval;
+    if constexpr (CUT)
+        window_parts<P, BS, INDEX>(cut, op, index, U, crp, Ccol, vals, st, wm, wo);
     const unsigned i0 = DENSE ? listed->dense : 0u, i1 = DENSE ? listed->listed : listed->dense;
     unsigned it = i0 + blockIdx.x;
     if (it >= i1)
@@ -1979,7 +2043,10 @@ __global__ __launch_bounds__(256) void k_wide_cut(const unsigned *__restrict__ h
         const long long est = wave_sum(found) * nA / ns;
         if (est < hot_min)
             continue;
-        const long long want = est / (hot_min / WIDE_PARTS), most = want < nA ? want : nA;
+        const int by_na = nA / WIDE_PART_NA < WIDE_NA_PARTS ? nA / WIDE_PART_NA : WIDE_NA_PARTS;
+        long long most = est / (hot_min / WIDE_PARTS);
+        most = most > by_na ? most : by_na;
+        most = most < nA ? most : nA;
         const int k = (int)(most < 4096 ? most : 4096);
         unsigned sum = 0;
         u64 at = 0;
@@ -2007,73 +2074,6 @@ __global__ __launch_bounds__(256) void k_wide_cut(const unsigned *__restrict__ h
                                      (int)sum, 0};
         for (unsigned q = lane; q < cnt; q += 64)
             sum_val[(size_t)sum * WIDE_UNIT + q] = 0.0;
-    }
-}
-
-// The parts of hot windows: as k_numeric_windows' compact form, over a range of the row's entries.
-// Their sums meet by atomics in sum_val (k_wide_sums takes them to C); a window's first part writes
-// its columns.
-template <typename P, int BS, bool INDEX>
-__global__ __launch_bounds__(BS) void k_numeric_parts(const WidePart *__restrict__ parts,
-                                                      const WideCount *__restrict__ ctr, u64 part_cap, Operands op,
-                                                      const int *__restrict__ index, long long U,
-                                                      const long long *__restrict__ crp, int *__restrict__ Ccol,
-                                                      double *sum_val)
-{
-    typedef typename P::V V;
-    extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ u64 red[16];
-    constexpr int NW = BS / 64, words = stream_window(BS) / 64;
-    double *vals = (double *)lds;
-    Stream<BS> st;
-    st.rec = (uint4 *)(vals + WIDE_UNIT);
-    st.bits = (u64 *)(st.rec + BS);
-    u64 *wm = st.bits + words;
-    unsigned short *wo = (unsigned short *)(wm + WW_TILES);
-    st.wb = wo + WW_TILES;
-    st.red = red;
-    const int l = threadIdx.x, lane = l & 63, w = uniform((int)(threadIdx.x >> 6));
-    const V *__restrict__ Aval = (const V *)op.Aval;
-    const u64 n = ctr->parts < part_cap ? ctr->parts : part_cap;
-    for (u64 i = blockIdx.x; i < n; i += gridDim.x) {
-        const WidePart p = parts[i];
-        const int row = uniform(p.row), sum = uniform(p.sum), e0 = uniform(p.e0), cnt = (int)uniform(p.cnt);
-        const unsigned units = uniform(p.units), base = uniform(p.base);
-        const int u0 = (int)(units & 0xffffffu), u1 = u0 + (int)(units >> 24);
-        const int a0 = uniform(op.Arp[row]) + e0, nA = uniform(p.e1) - e0;
-        const WideDir d(op, uniform(op.rmin[row]), uniform(op.rmax[row]), uniform64(op.rdir[row]));
-        const long long cb = uniform64(crp[row]) + base;
-        const int T0 = u0 * WIDE_TILES, nt = (u1 - u0) * WIDE_TILES;
-        for (int t = l; t < nt; t += BS) {
-            unsigned off;
-            wm[t] = d.tile(T0 + t - d.mn, off);
-            wo[t] = (unsigned short)(off - base);
-        }
-        for (int q = 2 * l; q < cnt; q += 2 * BS) // (WIDE_UNIT is even)
-            *(double2 *)(vals + q) = make_double2(0.0, 0.0);
-        for (int q = l; q < words; q += BS)
-            st.bits[q] = 0;
-        __syncthreads();
-        st.run(
-            nA,
-            [&](int e) {
-                const int2 r = window_elements<INDEX>(op, index, U, u0, u1, op.Acol[a0 + e]);
-                return Segment{r.x, r.y - r.x, (u64)__double_as_longlong((double)Aval[a0 + e])};
-            },
-            [&](const Stream<BS> &t, long long w0) {
-                stream_add<BS, SLOT_FLAT, P>(t, w0, op, nullptr, nullptr, wm, wo, vals, T0);
-            });
-        __syncthreads();
-        double *sv = sum_val + (size_t)sum * WIDE_UNIT;
-        for (int q = l; q < cnt; q += BS)
-            unsafeAtomicAdd(&sv[q], vals[q]);
-        if (e0 == 0)
-            for (int t = w; t < nt; t += NW) {
-                const u64 m = uniform64(wm[t]);
-                if ((m >> lane) & 1ull)
-                    Ccol[cb + wo[t] + (unsigned)mbcnt(m)] = ((T0 + t) << 6) + lane;
-            }
-        __syncthreads();
     }
 }
 
@@ -2293,37 +2293,32 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
             hipLaunchKernelGGL(k_wide_order, dim3(1), dim3(1024), 0, s, wide.places, (int)gi, wide.ctr);
             hipLaunchKernelGGL(k_wide_items<true>, dim3(gi), dim3(WI_BS), 0, s, rows, count_dev, op, crp, wide.nunits,
                                wide.items, wide.items_cap, wide.places, wide.hot, wide.hot_cap, wide.hot_min, wide.ctr, err);
-            if (wide.hot) {
-                const unsigned gh = (unsigned)(8 * num_cus);
-#define HOT(INDEX)                                                                                                     \
-    hipLaunchKernelGGL((k_wide_cut<INDEX>), dim3(gh), dim3(256), 0, s, wide.hot, (unsigned)wide.hot_cap,               \
-                       wide.hot_min, wide.items, wide.ctr, op, wide.index, wide.nunits, crp, wide.parts, (u64)wide.part_cap, wide.sums,          \
-                       wide.sum_val, (unsigned)wide.sum_cap);                                                          \
-    hipLaunchKernelGGL((k_numeric_parts<P, WW_BS, INDEX>),                                                             \
-                       dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, false>()))), dim3(WW_BS),                     \
-                       (ww_lds<WW_BS, false>()), s, wide.parts, wide.ctr, (u64)wide.part_cap, op, wide.index,          \
-                       wide.nunits, crp, Ccol, wide.sum_val)
-                if (wide.index) {
-                    HOT(true);
-                } else {
-                    HOT(false);
-                }
-#undef HOT
-                hipLaunchKernelGGL(k_wide_sums<P>, dim3(gh), dim3(256), 0, s, wide.sums, wide.ctr, (unsigned)wide.sum_cap,
-                                   wide.sum_val, (typename P::V *)Cval);
-            }
-#define WINDOWS(DENSE, INDEX, TAKEN)                                                                                   \
-    hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, DENSE, INDEX>),                                                    \
+            const unsigned gh = (unsigned)(8 * num_cus);
+            const WideCut cut = {wide.parts, wide.ctr, (u64)wide.part_cap, wide.sum_val};
+#define WINDOWS(DENSE, INDEX, CUT, TAKEN)                                                                              \
+    hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, DENSE, INDEX, CUT>),                                               \
                        dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, DENSE>()))), dim3(WW_BS),                     \
                        (ww_lds<WW_BS, DENSE>()), s, wide.items, wide.ctr, wide.ctr->taken + TAKEN, op, wide.index,     \
-                       wide.nunits, crp, Ccol, (typename P::V *)Cval)
+                       wide.nunits, crp, Ccol, (typename P::V *)Cval, cut)
+#define FORM(INDEX)                                                                                                    \
+    if (wide.hot)                                                                                                      \
+        hipLaunchKernelGGL((k_wide_cut<INDEX>), dim3(gh), dim3(256), 0, s, wide.hot, (unsigned)wide.hot_cap,           \
+                           wide.hot_min, wide.items, wide.ctr, op, wide.index, wide.nunits, crp, wide.parts,           \
+                           (u64)wide.part_cap, wide.sums, wide.sum_val, (unsigned)wide.sum_cap);                       \
+    WINDOWS(true, INDEX, false, 0);                                                                                    \
+    if (wide.hot) {                                                                                                    \
+        WINDOWS(false, INDEX, true, 1);                                                                                \
+        hipLaunchKernelGGL(k_wide_sums<P>, dim3(gh), dim3(256), 0, s, wide.sums, wide.ctr, (unsigned)wide.sum_cap,     \
+                           wide.sum_val, (typename P::V *)Cval);                                                       \
+    } else {                                                                                                           \
+        WINDOWS(false, INDEX, false, 1);                                                                               \
+    }
             if (wide.index) {
-                WINDOWS(true, true, 0);
-                WINDOWS(false, true, 1);
+                FORM(true)
             } else {
-                WINDOWS(true, false, 0);
-                WINDOWS(false, false, 1);
+                FORM(false)
             }
+#undef FORM
 #undef WINDOWS
         } else if (op.dir_mask)
             hipLaunchKernelGGL(k_numeric_wcompact<P>, dim3(blocks), dim3(1024), CW_LDS, s, rows, count_dev, op, crp,
@@ -2405,7 +2400,7 @@ hipError_t configure_kernels(int lds_max, int num_xcds)
 #define CFGW(P)                                                                                                        \
     CFG((k_numeric_windows<P, WW_BS, false, false>)) CFG((k_numeric_windows<P, WW_BS, false, true>))                   \
     CFG((k_numeric_windows<P, WW_BS, true, false>)) CFG((k_numeric_windows<P, WW_BS, true, true>))                     \
-    CFG((k_numeric_parts<P, WW_BS, false>)) CFG((k_numeric_parts<P, WW_BS, true>))
+    CFG((k_numeric_windows<P, WW_BS, false, false, true>)) CFG((k_numeric_windows<P, WW_BS, false, true, true>))
     CFGW(PrecF64) CFGW(PrecF32C)
 #undef CFGW
 #undef CFG

@@ -798,6 +798,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     // 160 KiB; rows needing more move up to a bin with fewer rows per workgroup (measured
     // best on the batched Laplacians)
     bp.lds_window_max = bp.lds_row_max;
+    bp.giant_min = INT64_MAX;
     bp.lds_block_budget = opts.lds_block_budget > 0 ? opts.lds_block_budget : 8 * 1024;
     if (bp.lds_block_budget > lds_dyn)
         bp.lds_block_budget = lds_dyn;
@@ -870,6 +871,14 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     op.dir_mask = nullptr;
     op.dir_off = nullptr;
     const unsigned long long dir_total = h1.dir_total;
+    // a row far beyond a CU's share of the products is wide, if there is room for that
+    unsigned long long products = 0;
+    for (int b = 0; b < NBINS; ++b)
+        products += h1.sym.nnz_c[b];
+    const unsigned long long share2 = 2 * products / (unsigned long long)c->num_cus;
+    const unsigned long long giant_min = share2 > WIDE_GIANT ? share2 : WIDE_GIANT;
+    const bool giant = h1.prod_most >= giant_min &&
+                       ar.remaining() >= 12 * dir_total + 8 * (unsigned long long)M + (96ull << 20);
     bool keep_dirs;
     if (cap) {
         keep_dirs = mode.plan->dirs_kept;
@@ -881,7 +890,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
         }
         const bool worth = 2 * dir_total <= tile_products ||
                            (2 * dir_total <= 3 * tile_products && tile_products <= 10 * entries) ||
-                           h1.sym.count[BIN_GLOBAL] > 0 || h1.num_wide_work > 0;
+                           h1.sym.count[BIN_GLOBAL] > 0 || h1.num_wide_work > 0 || giant;
         unsigned long long budget = c->total_mem / 4 > (1ull << 31) ? c->total_mem / 4 : (1ull << 31);
         // allocation-free: at most half of the workspace left, the rest serves C's row
         // pointers and the numeric phase
@@ -985,6 +994,8 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     if (bp.lds_row_max > WINDOW_ROW_MIN && places <= h1.num_wide_work && windows_fit(list_most) &&
         index_fits(list_most))
         bp.lds_window_max = WINDOW_ROW_MIN;
+    if (giant && keep_dirs)
+        bp.giant_min = (long long)giant_min;
     HIP_TRY(launch_rowptr_bin(M, P.Arp, rprod, rtp, rmin, rmax, rnnz, crp,
                               rp64 || batch || narrow_later ? nullptr : (int *)Crp, bp, binrows,
                               words + btiles_blocks(P.nnzB), &dw->ticket[1], dst, dw->sums[1], &dw->done[1], host,
@@ -1092,7 +1103,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
             const unsigned long long share = 2 * h2.num.work[b] / (3 * (unsigned long long)c->num_cus);
             const unsigned long long hot_min = share > WIDE_HOT ? share : WIDE_HOT;
             const unsigned long long sums = h2.num.work[b] / hot_min + 1; // (at most 385 on 256 CUs)
-            const unsigned long long parts = (2 * sums + 16) * WIDE_PARTS;
+            const unsigned long long parts = (2 * sums + 16) * WIDE_NA_PARTS;
             const unsigned long long hot_bytes = h2.hot_items * sizeof(unsigned) + parts * sizeof(WidePart) +
                                                  sums * (WIDE_UNIT * sizeof(double) + sizeof(WideSum)) + 2048;
             if (form < WIDE_PER_ROW && h2.hot_most + WIDE_UNIT >= hot_min && hot_bytes <= ar.remaining() &&

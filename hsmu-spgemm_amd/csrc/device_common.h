@@ -99,6 +99,11 @@ DEVI int wave_max(int v)
     return wave_last(wave_incl_scan(v, 0, [](int a, int b) { return a > b ? a : b; }));
 }
 
+DEVI u64 wave_most(u64 v)
+{
+    return wave_last(wave_incl_scan(v, (u64)0, [](u64 a, u64 b) { return a > b ? a : b; }));
+}
+
 // Map the hardware block index so that each XCD (blocks are dealt round-robin over the
 // nx XCDs of the device: 8 on an MI355X) works on a contiguous range of logical blocks:
 // neighbouring rows, which share rows of B, then share one XCD's L2.

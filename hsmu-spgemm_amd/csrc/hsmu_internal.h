@@ -36,6 +36,7 @@ struct BinParams {
     int lds_pair_budget;  // the same for two rows per workgroup
     int lds_row_max;      // LDS bytes one row may use
     int lds_window_max;   // the same for a row whose windows would be filled (window_filled)
+    long long giant_min;  // products of a row that is wide whatever LDS it needs (wide_hot)
     int per_lane;         // work items per lane
     int lds_cu;           // LDS bytes of a CU
     int force_global;
@@ -47,7 +48,7 @@ struct BinStats {
     int max_need[NBINS]; // LDS bytes of the largest row in the bin
     int max_span[NBINS]; // tiles spanned by the widest row in the bin
     unsigned long long work[NBINS]; // products (numeric) or tile-products (symbolic)
-    unsigned long long nnz_c[NBINS];// nnz of C in the bin's rows (numeric)
+    unsigned long long nnz_c[NBINS];// nnz of C in the bin's rows (symbolic: their products)
     unsigned long long nnz_a[NBINS];// nnz of A in the bin's rows
     int nsparse[NBINS];             // rows with a two-level tile directory
     int max_na[NBINS];              // longest row of A in the bin
@@ -66,6 +67,7 @@ struct DevStats {
     int err;
     int ntiles_b;
     int pad;
+    unsigned long long prod_most;     // products of the largest row, if more than WIDE_GIANT
     unsigned long long num_wide_work; // products of rows that may be wide in the numeric phase (symbolic binning)
     unsigned long long wide_items; // windows the wide rows may need, at most (numeric binning)
     unsigned long long hot_items;  // those of them that belong to hot rows
@@ -318,9 +320,15 @@ HSMU_HD inline StreamLayout sym_stream_layout(int G, int S, int nA, int tp)
 
 constexpr int BIN_SHARED = 3; // bins of rows that share a wave: 8, 16, 32 lanes
 
+// Entries of A from which a row of few tiles per entry takes k_symbolic_wide: the stream's turns of
+// 1,024 entries are a chain, its sub-groups of lanes are not (a row of
+// 100,000 entries of 2 tiles 455 us as a stream, 235 so; 100 such rows, whole calls, 2.58 and 2.37 ms).
+constexpr int SYM_LONG = 32 * 1024;
 // LDS a row with p products needs in symbolic bin `bin`
 HSMU_HD inline int sym_need(int bin, int S, int nA, int tp, long long p)
 {
+    if (nA >= SYM_LONG && tp / 4 <= nA)
+        return LAYOUT_NONE;
     return bin >= BIN_SHARED ? sym_stream_layout(8 << bin, S, nA, tp).bytes : small_need(false, 8 << bin, S, 0, nA, p);
 }
 
@@ -485,16 +493,22 @@ struct WideCount {
 // columns): one of its windows may hold as many, which kept a workgroup busy long after the others
 // had ended.  Such windows are estimated from WIDE_SAMPLE of the row's entries of A and, with
 // WIDE_HOT products or more and twice a workgroup's share of all wide rows' (less is no tail: cutting
-// it slows an R-MAT square of scale 18 by 1.6%), cut into WIDE_PARTS or more ranges of entries of A,
-// whose FP64 sums meet in memory.  3,000 rows of B with 900 of their 1,000 entries in one unit: a row
+// it slows an R-MAT square of scale 18 by 1.6%), cut into WIDE_PARTS or more ranges of entries of A
+// (or of WIDE_PART_NA entries, up to WIDE_NA_PARTS of them: a workgroup takes 3.8 us for 256 entries
+// of few elements), whose FP64 sums meet in memory.  3,000 rows of B with 900 of their 1,000 entries in one unit: a row
 // of C with all of them 2.12 ms whole and 0.37 cut, 64 such rows 3.97 and 0.59.
 constexpr unsigned long long WIDE_HOT = 512 * 1024;
 constexpr int WIDE_PARTS = 4;
+constexpr int WIDE_PART_NA = 4096;
+constexpr int WIDE_NA_PARTS = 256;
 constexpr int WIDE_SAMPLE = 256;
 HSMU_HD inline bool wide_hot(long long p, long long n, int nA)
 {
     return p - n > (long long)WIDE_HOT && (long long)nA * WIDE_UNIT >= (long long)WIDE_HOT;
 }
+// A row of this many products, and of twice a CU's share of all products, that fits LDS is wide for
+// its windows to be cut: alone on a CU it ends long after the others.
+constexpr unsigned long long WIDE_GIANT = WIDE_HOT;
 struct __attribute__((aligned(16))) WidePart {
     int row;
     unsigned units, base, cnt; // as the window's

@@ -602,7 +602,8 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
         if (numeric) {
             work = r.prod;
             auto nd = [&](int bin) { return num_need(bin, r.S, r.nc, r.nA, r.tp, r.prod); };
-            at.b = choose_bin(work, nd, window_filled(r.nc, r.S) ? bp.lds_window_max : bp.lds_row_max, bp);
+            const bool giant = r.prod >= bp.giant_min && wide_hot(r.prod, r.nc, r.nA);
+            at.b = choose_bin(work, nd, giant ? 0 : window_filled(r.nc, r.S) ? bp.lds_window_max : bp.lds_row_max, bp);
             need = nd(at.b);
         } else {
             work = r.tp;
@@ -628,6 +629,11 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
         if (lane == 0)
             atomicAdd(&st->num_wide_work, products);
     }
+    if (!numeric && __ballot(r.prod > (long long)WIDE_GIANT)) {
+        const u64 most = wave_most((u64)r.prod);
+        if (lane == 0)
+            atomicMax(&st->prod_most, most);
+    }
     if (numeric && __ballot(at.b == BIN_GLOBAL)) { // room for the wide rows' windows
         const u64 mine = at.b == BIN_GLOBAL ? (u64)wide_row_items(r.nc, r.S) : 0ull;
         const u64 items = wave_sum(mine);
@@ -636,8 +642,7 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
         const bool hot = at.b == BIN_GLOBAL && wide_hot(r.prod, r.nc, r.nA);
         if (__ballot(hot)) {
             const u64 hots = wave_sum(hot ? mine : 0ull);
-            const u64 most = wave_last(wave_incl_scan(hot ? (u64)(r.prod - r.nc) : 0ull, (u64)0,
-                                                      [](u64 a, u64 b) { return a > b ? a : b; }));
+            const u64 most = wave_most(hot ? (u64)(r.prod - r.nc) : 0ull);
             if (lane == 0) {
                 atomicAdd(&st->hot_items, hots);
                 atomicMax(&st->hot_most, most);
@@ -654,7 +659,7 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
         pending &= ~same;
         const u64 wsum = wave_sum(mine ? (u64)work : 0ull);
         const u64 nas = wave_sum(mine ? (u64)r.nA : 0ull);
-        const u64 ncs = numeric ? wave_sum(mine ? (u64)r.nc : 0ull) : 0ull;
+        const u64 ncs = wave_sum(mine ? (numeric ? (u64)r.nc : (u64)r.prod) : 0ull);
         const int needm = wave_max(mine ? need : 0);
         const int spanm = wave_max(mine ? r.S : 0);
         const int nam = wave_max(mine ? r.nA : 0);
@@ -670,8 +675,7 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
             atomicMax(&B.na_max[bb], nam);
             atomicAdd(&B.work[bb], wsum);
             atomicAdd(&B.na[bb], nas);
-            if (ncs)
-                atomicAdd(&B.nc[bb], ncs);
+            atomicAdd(&B.nc[bb], ncs);
             if (sps)
                 atomicAdd(&B.sparse[bb], sps);
             if (dtot)
@@ -700,8 +704,7 @@ DEVI void bin_reserve(BinBlock &B, int numeric, DevStats *st, BinSum *sums)
             BinSum *s = sums + (blockIdx.x % BIN_PARTS) * NBINS + t;
             atomicAdd(&s->work, B.work[t]);
             atomicAdd(&s->nnz_a, B.na[t]);
-            if (numeric)
-                atomicAdd(&s->nnz_c, B.nc[t]);
+            atomicAdd(&s->nnz_c, B.nc[t]);
             atomicMax(&s->need, (unsigned)B.need[t]);
             atomicMax(&s->span, (unsigned)B.span[t]);
             atomicMax(&s->na_max, (unsigned)B.na_max[t]);

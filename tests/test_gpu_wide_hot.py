@@ -67,3 +67,48 @@ def test_hot_windows(ctx, case, indexed, fp32):
         plan.destroy()
         dA.free()
         dB.free()
+
+
+def giant(case):
+    rng = np.random.default_rng(71)
+    if case == "narrow":  # a row that LDS holds, of most of the products; 14 tiles
+        K, per, N, na = 200000, 4, 900, 200000
+        col = rng.integers(0, N, (K, per))
+    elif case == "spread":  # the same with a two-level directory
+        K, per, N, na = 200000, 4, 1000000, 200000
+        col = np.sort(rng.choice(N, 3000, replace=False))[rng.integers(0, 3000, (K, per))]
+    else:  # "long": entries enough for the symbolic form without turns, products too few to be cut
+        K, per, N, na = 60000, 3, 300000, 40000
+        col = np.sort(rng.choice(N, 2000, replace=False))[rng.integers(0, 2000, (K, per))]
+    col = np.sort(col, axis=1).astype(np.int32)
+    val = lambda n: rng.uniform(-1, 1, n).astype(np.float32).astype(np.float64)
+    B = hsmu.HostMatrix(K, N, (np.arange(K + 1) * per).astype(np.int32), col.ravel(), val(K * per))
+    rows = [rng.choice(K, 5) for _ in range(700)]
+    rows[300] = rng.choice(K, na, replace=False)
+    rows = [np.sort(r) for r in rows]
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    return hsmu.HostMatrix(len(rows), K, rp, np.concatenate(rows).astype(np.int32), val(rp[-1])), B
+
+
+@pytest.mark.parametrize("case", ["narrow", "spread", "long"])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_giant_rows(ctx, case, fp32):
+    A, B = giant(case)
+    ref = oracle.spgemm(A, B)
+    o = hsmu.default_opts(precision=hsmu.HSMU_FP32_COMP if fp32 else hsmu.HSMU_FP64)
+    dA, dB = ctx.matrix(A, fp32), ctx.matrix(B, fp32)
+    print(f"[gpu-case] giant row {case} fp32 {fp32}", flush=True)
+    plan = ctx.plan([dA], [dB], o)
+    try:
+        check(ctx.fetch(plan.results[0]), ref, fp32)
+        for _ in range(3):
+            plan.execute()
+            check(ctx.fetch(plan.results[0]), ref, fp32)
+        C, st = ctx.spgemm_device(dA, dB, o)
+        check(ctx.fetch(C), ref, fp32)
+        ctx.free_result(C)
+        assert st["sym_bin_rows"][8] == 1 and st["num_bin_rows"][8] == (case != "long")
+    finally:
+        plan.destroy()
+        dA.free()
+        dB.free()
