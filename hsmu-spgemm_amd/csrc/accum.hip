@@ -486,7 +486,8 @@ DEVI void stream_or(const Stream<G> &st, long long w0, const Operands &op, u64 *
 // are loaded once, SMALL_U pairs per lane, and stay in registers.  Their columns mark the
 // row's words (32 columns each) in a coarse bitmap; a scan gives the marked words compact
 // places, where the columns are marked in turn; a second scan gives nnz(C_i) -- all the
-// symbolic phase wants -- and each word's first slot.  The numeric phase then adds every
+// symbolic phase wants -- and each word's first slot.  (Narrow spans need no coarse level, wide
+// ones have another above it: small_layout.)  The numeric phase then adds every
 // product at its column's rank (ds_add_f64), puts the column there too, and the row goes
 // out in order.
 // Against staging the A entries in LDS and walking B's tiles twice for the directory and
@@ -672,10 +673,8 @@ DEVI void small_rows(const int *__restrict__ rows, const int *__restrict__ count
         unsigned f0[U], f1[U];
         auto fine_of = [&](int c) {
             const int w = word(c);
-            if (L.flat)
-                return (unsigned)w;
-            const uint2 x = coarse[coarse_of(w)];
-            return x.y + (unsigned)__popc(under(x.x, w));
+            const uint2 x = coarse[coarse_of(w)]; // (a flat row's lies in its fine level)
+            return L.flat ? (unsigned)w : x.y + (unsigned)__popc(under(x.x, w));
         };
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -731,7 +730,8 @@ DEVI void small_rows(const int *__restrict__ rows, const int *__restrict__ count
 // One bin of such rows; or, where several have rows, the three in one launch, those of the
 // widest groups first (a launch of a few thousand rows is all start and end: a random product
 // of 30,011 ragged rows takes 164 us in place of 199; but with the registers of the widest
-// form a batch whose rows are all of one bin takes 3.79 ms in place of 3.70).
+// form a batch whose rows are all of one bin takes 3.79 ms in place of 3.70).  That launch gets 4
+// waves per SIMD: at 5 it spills 34 registers (200,000 rows of 3 times 3 160 us, 154 at 4).
 template <int G, typename P, bool TOPS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_small_bin(
     const int *__restrict__ rows, const int *__restrict__ count, int slice, Operands op, int *__restrict__ rnnz,
@@ -747,7 +747,7 @@ struct SmallBins {
     int slice[BIN_SHARED], blocks[BIN_SHARED];
 };
 template <typename P, bool TOPS>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_small_rows(
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_small_rows(
     SmallBins bins, Operands op, int *__restrict__ rnnz, const long long *__restrict__ crp, int *__restrict__ Ccol,
     typename P::V *__restrict__ Cval, int *err)
 {

@@ -861,7 +861,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
     // them -- the directories hold at most half as many entries as the tile-products that
     // rebuild them (banded: 1.3M entries for 10M tile-products; the batched Laplacians:
     // about as many, and rebuilding is 0.6 ms faster there), or up to half as many again
-    // where rows of A name rows of B of ten tiles or fewer, whose walk is mostly its starts
+    // where rows of A name rows of B of five tiles or fewer, whose walk is mostly its starts
     // (200,000 rows of 80 entries times 3 over 100,000 columns: 1,750 us kept, 2,350 rebuilt;
     // of 24 times 24: 2,450 and 2,300) -- or when wide rows need them
     // for their windows, and they fit a quarter of the device memory (72 GB on an
@@ -889,7 +889,7 @@ int pipeline(hsmu_ctx *c, const Problem &P, const hsmu_opts &opts, Arena &ar, co
             entries += h1.sym.nnz_a[b];
         }
         const bool worth = 2 * dir_total <= tile_products ||
-                           (2 * dir_total <= 3 * tile_products && tile_products <= 10 * entries) ||
+                           (2 * dir_total <= 3 * tile_products && tile_products <= 5 * entries) ||
                            h1.sym.count[BIN_GLOBAL] > 0 || h1.num_wide_work > 0 || giant;
         unsigned long long budget = c->total_mem / 4 > (1ull << 31) ? c->total_mem / 4 : (1ull << 31);
         // allocation-free: at most half of the workspace left, the rest serves C's row
