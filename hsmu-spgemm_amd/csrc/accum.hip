@@ -66,10 +66,9 @@ DEVI void or_put(u64 *dm, const unsigned *coff, u64 *fm, int tt, u64 m)
         atomicOr(&fm[fine_index(dm, coff, tt)], m);
 }
 
-// Tiles [tb, te) of one B row by a group of gw lanes (this lane the gl-th), U tiles per
-// lane per step.
-template <int MODE, int U = UNROLL>
-DEVI void or_walk(const Operands &op, int tb, int te, int gw, int gl, u64 *dm, const unsigned *coff, u64 *fm, int mn)
+// Tiles [tb, te) of one B row into a flat directory by a group of gw lanes (this lane the gl-th),
+// U tiles per lane per step.
+template <int U> DEVI void or_walk(const Operands &op, int tb, int te, int gw, int gl, u64 *dm, int mn)
 {
     for (int t = tb + gl; t < te; t += U * gw) {
         int c[U];
@@ -81,14 +80,13 @@ DEVI void or_walk(const Operands &op, int tb, int te, int gw, int gl, u64 *dm, c
             m[u] = 0;
             if (tu < te) {
                 c[u] = op.tcol[tu];
-                if constexpr (MODE != OR_COARSE)
-                    m[u] = op.tmask[tu];
+                m[u] = op.tmask[tu];
             }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
             if (c[u] >= 0)
-                or_put<MODE>(dm, coff, fm, c[u] - mn, m[u]);
+                or_put<OR_FLAT>(dm, nullptr, nullptr, c[u] - mn, m[u]);
     }
 }
 
@@ -938,7 +936,7 @@ __global__ __launch_bounds__(1024) void k_symbolic_wide(const int *__restrict__ 
         const int a1 = op.Arp[row + 1];
         for (int e = op.Arp[row] + sg; e < a1; e += NSG) {
             const int j = op.Acol[e];
-            or_walk<OR_FLAT, 2 * UNROLL>(op, op.tptr[j], op.tptr[j + 1], SG, sl, dm, nullptr, nullptr, mn);
+            or_walk<2 * UNROLL>(op, op.tptr[j], op.tptr[j + 1], SG, sl, dm, mn);
         }
         __syncthreads();
         const ChunkScan cs = scan_popcounts<1024>(dm, S, red);
@@ -960,7 +958,7 @@ __global__ __launch_bounds__(1024) void k_symbolic_wide(const int *__restrict__ 
 
 // ---- numeric -------------------------------------------------------------------------------
 
-// The same for a row with a workgroup to itself (G = 64 to 1024 lanes): its B rows are
+// C's entries of a row with a workgroup to itself (G = 64 to 1024 lanes): its B rows are
 // walked as one element stream.  What bounds it: the L1's rate for loads (12 bytes per
 // product; see the stream's loads), the LDS's for ds_add_f64 (24 cycles per 64 products),
 // C's stores, and the chain of short phases of a row, which several workgroups per CU
@@ -1851,15 +1849,14 @@ DEVI void window_parts(const WideCut &cut, const Operands &op, const int *__rest
 
 // Wide rows as windows: the compact accumulator over one window's entries of C_i, its part
 // of the row's directory (expanded to one mask and slot per tile of the window) and its
-// elements of the B rows as one stream, their ranges read from the index.  Workgroups take
-// windows from the list until it is used up.  Neither a search nor atomics in C nor a
-// second round: every window's elements are known when it starts, and a window belongs to
-// one workgroup.
+// elements of the B rows as one stream, their ranges read from the index or searched.  Workgroups
+// take windows from the list until it is used up.  There are no atomics in C and no second round:
+// a window's elements are known when it starts, and a window belongs to one workgroup.
 // CUT: the parts of hot windows first, which then run beside the others.
 // DENSE: a slot per column of the unit, with no masks in LDS: the element's column is its
 // slot, and a tile goes out as one store of columns and one of values by a wave.
 // No single unit bounds the compact form (Zipf panel: vector ALU 41%, LDS 32%, L1 47% of the
-// time): a window's phases follow one another and 48 KB of LDS leave three workgroups per
+// time): a window's phases follow one another and 52 KB of LDS leave three workgroups per
 // CU, so the next window's item, row and columns of A, and the next 256 entries' ranges, are
 // loaded during the stream.  The dense form takes about a third fewer instructions and leaves
 // room for four: Zipf panels of 2,000 rows 4.80 -> 4.25 ms, of 777 rows FP32 1.85 -> 1.55 ms
@@ -1868,9 +1865,9 @@ DEVI void window_parts(const WideCut &cut, const Operands &op, const int *__rest
 // a kernel of its own they took 1.55 ms on the R-MAT square of scale 18.  Against items of up
 // to 512 A entries that kept cursors into the B rows and posted chunks of them window by
 // window (in rounds, with split rows meeting by atomics): scale 18 22.4 -> 8.6 ms, the Zipf
-// panel 7.6 -> 3.9 ms.  Compact form with 128 / 256 / 512 lanes: Zipf 6.3 / 4.8 / 5.0 ms,
-// scale 18 20.8 / 17.4 / 17.5 ms; windows of 2,048 entries and twice the workgroups 6.1 and
-// 18.4 ms.  Dense form with 512 lanes: Zipf 4.6 ms.
+// panel 7.6 -> 3.9 ms.  With windows of up to 16 units (48 KB): compact form with 128 / 256 / 512
+// lanes Zipf 6.3 / 4.8 / 5.0 ms, scale 18 20.8 / 17.4 / 17.5 ms; windows of 2,048 entries and twice
+// the workgroups 6.1 and 18.4 ms.  Dense form with 512 lanes: Zipf 4.6 ms.
 constexpr int WW_TILES = WIDE_TILES * WIDE_UMAX;
 constexpr int WW_BS = 256; // lanes of a workgroup
 constexpr int WW_PER_TILE = 16; // entries per tile from which a wave writes a tile's columns
@@ -1879,6 +1876,8 @@ template <int BS, bool DENSE> constexpr int ww_lds()
     constexpr int words = stream_window(BS) / 64;
     return WIDE_UNIT * 8 + BS * 16 + words * 10 + (DENSE ? 0 : WW_TILES * 10);
 }
+static_assert(3 * (ww_lds<WW_BS, false>() + LDS_STATIC_RESERVE) <= 160 * 1024, "three compact windows per CU");
+static_assert(4 * (ww_lds<WW_BS, true>() + LDS_STATIC_RESERVE) <= 160 * 1024, "four dense windows per CU");
 
 template <typename P, int BS, bool DENSE, bool INDEX, bool CUT = false>
 __global__ __launch_bounds__(BS) void k_numeric_windows(const WideItem *__restrict__ items,
@@ -2088,8 +2087,12 @@ __global__ __launch_bounds__(256) void k_wide_sums(const WideSum *__restrict__ s
             Cval[sums[i].at + q] = P::result(sum_val + (size_t)i * WIDE_UNIT, (unsigned)q);
 }
 
-// workgroups of a windows' kernel that a CU holds
-static int ww_per_cu(int lds) { return 160 * 1024 / (lds + LDS_STATIC_RESERVE); }
+// workgroups of a windows' kernel that a CU of lds_cu bytes holds
+static int ww_per_cu(int lds, int lds_cu)
+{
+    const int n = lds_cu / (lds + LDS_STATIC_RESERVE);
+    return n > 0 ? n : 1;
+}
 
 // ---- launchers -------------------------------------------------------------------------------
 
@@ -2297,7 +2300,7 @@ static hipError_t numeric_p(int bin, const int *rows, const int *count_dev, int 
             const WideCut cut = {wide.parts, wide.ctr, (u64)wide.part_cap, wide.sum_val};
 #define WINDOWS(DENSE, INDEX, CUT, TAKEN)                                                                              \
     hipLaunchKernelGGL((k_numeric_windows<P, WW_BS, DENSE, INDEX, CUT>),                                               \
-                       dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, DENSE>()))), dim3(WW_BS),                     \
+                       dim3((unsigned)(num_cus * ww_per_cu(ww_lds<WW_BS, DENSE>(), wide.lds_cu))), dim3(WW_BS),        \
                        (ww_lds<WW_BS, DENSE>()), s, wide.items, wide.ctr, wide.ctr->taken + TAKEN, op, wide.index,     \
                        wide.nunits, crp, Ccol, (typename P::V *)Cval, cut)
 #define FORM(INDEX)                                                                                                    \

@@ -12,11 +12,11 @@
 namespace hsmu {
 
 // Row bins.  Bins 0..7 keep a row in LDS with G = 8 << b lanes per row (rows per
-// workgroup = max(1, BLOCK / G)).  BIN_GLOBAL keeps the row's tile directory in global
-// memory and accumulates straight into C (rows whose LDS need exceeds the limit).
+// workgroup = max(1, BLOCK / G)).  BIN_GLOBAL holds the rows that LDS does not, or not well: their
+// directory is in global memory, and the numeric phase takes them in windows of C's columns.
 constexpr int NLDS = 8;
 constexpr int BIN_GLOBAL = 8;
-constexpr int NBINS = 10;  // slot 9 reserved
+constexpr int NBINS = 10; // as the public statistics (slot 9 stays empty)
 // Workgroup size of the bins that pack several rows per workgroup (G < 64 lanes per
 // row): one wave, so the phases of a row group are separated by single-wave barriers and
 // every wave runs at its own pace (measured: 4-wave workgroups of 8-lane rows spend most
@@ -460,9 +460,12 @@ constexpr int WIDE_LISTS = 1 + 2 * WIDE_BUCKETS;
 // masks nor slots per tile: a Zipf panel, whose windows hold 1.1 products per entry, takes
 // 4.25 ms against 4.80.  Windows with more products are the hot columns of skewed graphs,
 // where a slot per column puts more adds on one LDS bank: R-MAT squares of scale 16 and 18
-// take 2.62 and 17.7 ms with them against 2.53 and 17.45.
+// take 2.62 and 17.7 ms with them against 2.53 and 17.45.  Without the least number, scale 16 takes
+// 2.03 ms against 2.00; without the form, Zipf panels of 2,000 / 777 rows 4.72 / 1.83 against 4.17 /
+// 1.53.
 // Windows of more than WIDE_HEAVY products are listed first, so that none of them is the last
-// one running.
+// one running (one window of 1.1 M products, late in C's columns, among 541 M: 3.5 ms against 4.45;
+// R-MAT squares and Zipf panels take the same time without).
 constexpr int WIDE_DENSE = WIDE_UNIT / 4;
 constexpr int WIDE_DENSE_WORK = 3 * WIDE_UNIT;
 constexpr unsigned WIDE_DENSE_MIN = 8192;
@@ -535,6 +538,7 @@ struct WideRows {
     int *ws;
     long long cur_stride, ft_stride;
     int blocks;
+    int lds_cu; // LDS bytes of a CU
     // windows: their capacity and list, the place of each listing workgroup's windows per
     // bucket, and how many are listed and taken (null items: one workgroup per row)
     long long items_cap;

@@ -27,8 +27,9 @@
 //      replaces the reference's separate O(n^2) rank-sort pass
 //      (src/compressed/compressed_Ccol_symbolic.cuh:4-63).
 //   Rows whose directory + values do not fit LDS: the symbolic tile OR runs on a global
-//   workspace, the numeric phase takes the row in windows of its columns (the reference's bin-13 dense spECK path, src/external/spECK/dense_acc.cu:246-267, whose
-//   early return leaves rows unwritten; every row is written here).
+//   workspace, the numeric phase takes the row in windows of its columns (the reference's
+//   bin-13 dense spECK path, src/external/spECK/dense_acc.cu:246-267, whose early return
+//   leaves rows unwritten; every row is written here).
 
 #include <hip/hip_runtime.h>
 

@@ -57,8 +57,9 @@ enum hsmu_status {
 enum hsmu_precision {
     HSMU_FP64 = 0,      /* plain: FP64 products, FP64 LDS accumulation (the reference's value_t) */
     HSMU_FP32_COMP = 1  /* compensated FP32: FP32 values; products exact and their sums carried with
-                           more bits than a compensated FP32 pair (accumulated in FP64), rounded to
-                           FP32 once: within one FP32 rounding of the exact sum */
+                           more bits than a compensated FP32 pair (accumulated in FP64, in any
+                           order), rounded to FP32 once: an entry c that is the sum of n products
+                           is off by at most 2^-24 |c| + about n 2^-53 sum |a b| */
 };
 
 /* ---- matrices ---------------------------------------------------------------- */
@@ -111,7 +112,8 @@ typedef struct hsmu_opts {
                                  (exercises the fallback on small inputs) */
     int32_t lds_row_max;      /* bytes of LDS one row may use before it falls back to the
                                  global-memory path; 0 = device maximum (in the numeric phase
-                                 64 KiB where wide rows can be cut into windows) */
+                                 64 KiB for rows that are faster cut into windows, none for a
+                                 row of a large share of all products) */
     int32_t lds_block_budget; /* LDS bytes per workgroup for bins that pack several rows
                                  into one workgroup (one wave); 0 = default (8 KiB, 16 for two
                                  rows) */
