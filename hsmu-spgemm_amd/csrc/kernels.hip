@@ -523,25 +523,23 @@ hipError_t launch_brows(int64_t K, int64_t N, int64_t nnz, const int *rp, const 
 // elements fit the registers of 8, 16 or 32 lanes share a wave.  16 waves per CU, where LDS
 // limits the workgroups, take 17.8 ms on the square of scale 18 against 19.2 ms with 8; 24
 // slow a banded square by 4%.
+// (nd: the row's need in the bin chosen)
 template <typename Need>
-DEVI int choose_bin(long long work, Need need, int row_max, const BinParams &bp)
+DEVI int choose_bin(long long work, Need need, int row_max, const BinParams &bp, int &nd)
 {
-    if (bp.force_global)
-        return BIN_GLOBAL;
-    int b = 0;
+    int b = bp.force_global ? BIN_GLOBAL : 0;
     while (b < NLDS - 1 && (8LL << b) * bp.per_lane < work)
         ++b;
+    nd = need(b);
     // the budget limits only workgroups that pack several rows: a one-row workgroup needs
     // the row's LDS whatever its width
     while (b < BIN_SHARED) {
-        const int nd = need(b);
         if (nd <= row_max && nd * (BLOCK >> (b + 3)) <= (b < BIN_SHARED - 1 ? bp.lds_block_budget : bp.lds_pair_budget))
-            break;
-        ++b;
+            return b;
+        nd = need(++b);
     }
     // a one-row workgroup's LDS decides how many fit a CU: widen the row's group until
     // those workgroups hold min_waves waves, to hide the latency of the gathers from B
-    int nd = need(b);
     while (b < NLDS - 1) {
         const int waves = (8 << b) / 64, wgs = (bp.min_waves + waves - 1) / waves;
         if ((long long)nd * wgs <= bp.lds_cu)
@@ -552,7 +550,11 @@ DEVI int choose_bin(long long work, Need need, int row_max, const BinParams &bp)
         nd = wider;
         ++b;
     }
-    return nd > row_max ? BIN_GLOBAL : b;
+    if (b < BIN_GLOBAL && nd > row_max) {
+        b = BIN_GLOBAL;
+        nd = need(b);
+    }
+    return b;
 }
 
 // One row as the binning sees it.
@@ -604,8 +606,8 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
             work = r.prod;
             auto nd = [&](int bin) { return num_need(bin, r.S, r.nc, r.nA, r.tp, r.prod); };
             const bool giant = r.prod >= bp.giant_min && wide_hot(r.prod, r.nc, r.nA);
-            at.b = choose_bin(work, nd, giant ? 0 : window_filled(r.nc, r.S) ? bp.lds_window_max : bp.lds_row_max, bp);
-            need = nd(at.b);
+            at.b = choose_bin(work, nd, giant ? 0 : window_filled(r.nc, r.S) ? bp.lds_window_max : bp.lds_row_max, bp,
+                              need);
         } else {
             work = r.tp;
             // the numeric need with nnz(C_i) <= min(products, 64 * span): a row that may be wide
@@ -616,8 +618,7 @@ DEVI BinPlace bin_row(BinBlock &B, int numeric, const BinRow &r, const BinParams
             auto nd = [&](int bin) {
                 return wide && bin < BIN_SHARED ? LAYOUT_NONE : sym_need(bin, r.S, r.nA, r.tp, r.prod);
             };
-            at.b = choose_bin(work, nd, bp.lds_row_max, bp);
-            need = nd(at.b);
+            at.b = choose_bin(work, nd, bp.lds_row_max, bp, need);
             // directory entries kept for the numeric phase: the row's form in an LDS bin, the
             // flat span for rows the symbolic phase handles in global memory
             E = at.b < BIN_SHARED ? 0 : at.b < BIN_GLOBAL ? dir_entries(r.S, r.tp) : r.S;
