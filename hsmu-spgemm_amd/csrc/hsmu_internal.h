@@ -510,7 +510,8 @@ HSMU_HD inline bool wide_hot(long long p, long long n, int nA)
     return p - n > (long long)WIDE_HOT && (long long)nA * WIDE_UNIT >= (long long)WIDE_HOT;
 }
 // A row of this many products, and of twice a CU's share of all products, that fits LDS is wide for
-// its windows to be cut: alone on a CU it ends long after the others.
+// its windows to be cut: alone on a CU it ends long after the others (a row of 300,000 entries times
+// 3 over 1,000 columns 3.0 ms in LDS, 1.37 cut; 50 dense rows of 4.5 M products 1.32 and 0.53 ms).
 constexpr unsigned long long WIDE_GIANT = WIDE_HOT;
 struct __attribute__((aligned(16))) WidePart {
     int row;
